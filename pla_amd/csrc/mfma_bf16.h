@@ -89,5 +89,12 @@ __device__ __forceinline__ void pack2_pair(float x, float y, uint32_t& hi, uint3
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x - (float)h[0], y - (float)h[1]));
 }
+// The same for magnitudes far below the fp16 range: no clamp.
+__device__ __forceinline__ void pack2_pair_small(float x, float y, uint32_t& hi, uint32_t& lo) {
+  const f32x2_t c = {x, y};
+  const f16x2_t h = __builtin_convertvector(c, f16x2_t);
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x - (float)h[0], y - (float)h[1]));
+}
 
 }  // namespace pla

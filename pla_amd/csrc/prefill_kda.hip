@@ -73,84 +73,105 @@ struct KdaPrefillParams {
   unsigned char seq_order[INLINE_TABLE_SEQUENCES];
 };
 
+// Operand tiles go out past the caches: the sweeps read them after the whole call's tiles were written.
+__device__ __forceinline__ void nt_store16(uint16_t* p, const uint4 v) {
+  __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t*>(p));
+}
+
+constexpr float LOG2E = 1.4426950408889634f;
+
 // 52 KB, so that three workgroups share a CU.  The normalised q never goes through LDS: the thread that
 // normalised a piece of it also forms that piece of the decayed tile, and the wavefront that needs a row block
 // as an MFMA operand reads those rows again (they were fetched a moment ago) and scales them by the row's
 // inverse norm.  L takes over Kn's storage once every wavefront is done with its k operands (the M blocks wait
 // in registers for the barrier).
 struct __align__(16) KdaPrepShared {
-  float G[CHUNK][132];
+  float G[CHUNK][132];     // base 2: cumulative log-decay times log2 e
   union {
     uint16_t Kn[CHUNK][PITCH128];
     float L[CHUNK][68];
   };
   float B[CHUNK];
   float QI[CHUNK];         // 1 / |q_row|
+  float half_sum[128];     // per channel: sum of the gate over the first half of the rows
 };
 static_assert(sizeof(float[CHUNK][68]) <= sizeof(uint16_t[CHUNK][PITCH128]), "L must fit into Kn's storage");
 
-// Eight decayed elements of a bf16 row: x[c] * exp(sign * (G[c] - R[c])) for the lane's two
-// channel quads of contraction step s.
-__device__ __forceinline__ void decayed8(const uint16_t* xrow, const float* grow, const float* rrow, float sign,
-                                         int s, int kb, f32x4_t& a, f32x4_t& b) {
-  const int c0 = 32 * s + 4 * kb, c1 = c0 + 16;
-  const uint2 x0 = *reinterpret_cast<const uint2*>(xrow + c0);
-  const uint2 x1 = *reinterpret_cast<const uint2*>(xrow + c1);
-  const float4 g0 = *reinterpret_cast<const float4*>(grow + c0);
-  const float4 g1 = *reinterpret_cast<const float4*>(grow + c1);
-  const float4 r0 = *reinterpret_cast<const float4*>(rrow + c0);
-  const float4 r1 = *reinterpret_cast<const float4*>(rrow + c1);
-  a = f32x4_t{lo16<bf16_t>(x0.x) * __expf(sign * (g0.x - r0.x)), hi16<bf16_t>(x0.x) * __expf(sign * (g0.y - r0.y)),
-              lo16<bf16_t>(x0.y) * __expf(sign * (g0.z - r0.z)), hi16<bf16_t>(x0.y) * __expf(sign * (g0.w - r0.w))};
-  b = f32x4_t{lo16<bf16_t>(x1.x) * __expf(sign * (g1.x - r1.x)), hi16<bf16_t>(x1.x) * __expf(sign * (g1.y - r1.y)),
-              lo16<bf16_t>(x1.y) * __expf(sign * (g1.z - r1.z)), hi16<bf16_t>(x1.y) * __expf(sign * (g1.w - r1.w))};
+// Four channels x e^{a - b} of a bf16 row, a and b rows of G (base 2: one subtraction and one v_exp_f32 per element).
+__device__ __forceinline__ f32x4_t decay4(const float4 a, const float4 b) {
+  return f32x4_t{__builtin_amdgcn_exp2f(a.x - b.x), __builtin_amdgcn_exp2f(a.y - b.y), __builtin_amdgcn_exp2f(a.z - b.z),
+                 __builtin_amdgcn_exp2f(a.w - b.w)};
+}
+__device__ __forceinline__ f32x4_t widen4(const uint2 x) {
+  return f32x4_t{lo16<bf16_t>(x.x), hi16<bf16_t>(x.x), lo16<bf16_t>(x.y), hi16<bf16_t>(x.y)};
+}
+__device__ __forceinline__ f32x4_t times4(const f32x4_t a, const f32x4_t b) {
+  return f32x4_t{a[0] * b[0], a[1] * b[1], a[2] * b[2], a[3] * b[3]};
 }
 
+// Preparation of one (chunk, head).  What bounds it are its vector instructions (about 60 % of the SIMD cycles over the
+// launch, a further share in v_exp_f32; 12 wavefronts per CU by LDS), so the kernel counts them:
+//   G is kept in base 2 (scaled by log2 e where the gate is summed), so that a decay factor is one subtraction and
+//   one v_exp_f32; the gate's bound is applied in the scan's final addition; the masks of a chunk's missing rows are
+//   a branch that whole chunks skip; a thread owns the channels 32 s + 4 kb .. + 3 and the same + 16, both halves of one
+//   granule of the operand tiles, which it stores without an exchange; the scan runs over both halves of a chunk's rows
+//   in registers; the row blocks of phase 3 (1 to 4 blocks of work) rotate over the wavefronts.
+// Where the call's tiles exceed the caches it is bound by memory (131 KiB read and written per tile), and the order of
+// the workgroups matters: heads vary fastest, so that the workgroups in flight read whole token rows (with the chunks
+// fastest they read 256 bytes out of every row of the call).  Measured: 18 sequences of 121 to 999 tokens, 12 heads
+// 92 -> 85.6 us; 65 536 tokens, 32 heads 0.97-1.07 -> 0.88-0.91 ms (4.9 TB/s).
 __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillParams p) {
-  const int cb = staged_chunk(p.stg, p.stage, blockIdx.x, p.seq_chunk_off[p.N]);
-  const int h = blockIdx.y;
+  const int chunk = blockIdx.x / p.H, h = blockIdx.x - chunk * p.H;
+  const int cb = staged_chunk(p.stg, p.stage, chunk, p.seq_chunk_off[p.N]);
   if (cb < 0) return;
   const int t0 = p.chunk_tok[cb];
   const int len = p.chunk_len[cb];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kb = lane >> 4;
+  const unsigned turn = blockIdx.x >> 3;             // the workgroup's place among those of its XCD
+  const int bi = (int)((wave + turn + (turn >> 5)) & 3);
   __shared__ KdaPrepShared sh;
   const int64_t tile = (int64_t)cb * p.H + h;
 
-  uint32_t qn[4][4], kn[4][4];   // normalised bf16 pairs of rows tid / 16 + 16 u, channels 8 (tid % 16) .. + 7
+  // the thread's channels of rows tid / 16 + 16 u: ca .. ca + 3 and ca + 16 .. ca + 19, granule tid % 16 of an operand tile
+  const int nrow = tid >> 4, ca = 32 * ((tid & 15) >> 2) + 4 * (tid & 3);
+  uint2 qn[4][2], kn[4][2];      // normalised bf16
   uint2 qraw[4][2];
   // ---- phase 1: normalised q / k, per-channel log-decay, beta ---------------------------------
   {
-    // q, k: thread handles eight channels of rows tid / 16 + 16 u (a row is one 16-lane DPP row, so its
-    // sum of squares is a row reduction); all eight 16-byte loads are in flight at once
-    const int nrow = tid >> 4, nc0 = 8 * (tid & 15);
-    uint4 qv[4], kv[4];
+    // q, k: a row is one 16-lane DPP row, so its sum of squares is a row reduction; all loads are in flight at once
+    uint2 qv[4][2], kv[4][2], graw[4][2];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = nrow + 16 * u;
       const int64_t t = t0 + (j < len ? j : 0);
-      qv[u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.q) + t * p.stride_q + h * 128 + nc0);
-      kv[u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.k) + t * p.stride_k + h * 128 + nc0);
+      const uint16_t* const qsrc = reinterpret_cast<const uint16_t*>(p.q) + t * p.stride_q + h * 128 + ca;
+      const uint16_t* const ksrc = reinterpret_cast<const uint16_t*>(p.k) + t * p.stride_k + h * 128 + ca;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        qv[u][x] = *reinterpret_cast<const uint2*>(qsrc + 16 * x);
+        kv[u][x] = *reinterpret_cast<const uint2*>(ksrc + 16 * x);
+      }
     }
-    // gate: thread handles eight channels of rows tid / 16 + 16 u; requested together with q and k, so the
-    // phase costs one trip to memory
-    const int gc0 = 8 * (tid & 15);
-    uint4 graw[4];
+    // gate: requested together with q and k, so the phase costs one trip to memory
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int j = (tid >> 4) + 16 * u;
-      graw[u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.g) +
-                                                (int64_t)(t0 + (j < len ? j : 0)) * p.stride_g + h * 128 + gc0);
-    }
-    float dtb[8];
+      const int j = nrow + 16 * u;
+      const uint16_t* const gsrc = reinterpret_cast<const uint16_t*>(p.g) + (int64_t)(t0 + (j < len ? j : 0)) * p.stride_g + h * 128 + ca;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dtb[e] = p.dt_bias[h * 128 + gc0 + e];
+      for (int x = 0; x < 2; ++x) graw[u][x] = *reinterpret_cast<const uint2*>(gsrc + 16 * x);
+    }
+    f32x4_t dtb[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dtb[x][e] = p.dt_bias[h * 128 + ca + 16 * x + e];
     const float a_log = p.A_log[h];
     float braw = 0.f;
     if (tid < len) braw = to_float(reinterpret_cast<const bf16_t*>(p.beta)[(int64_t)(t0 + tid) * p.stride_beta + h]);
     // the q rows of this wavefront's row block in MFMA operand layout (phase 3), raw
     {
-      const int i_row = 16 * wave + r16;
+      const int i_row = 16 * bi + r16;
       const uint16_t* qrow = reinterpret_cast<const uint16_t*>(p.q) + (int64_t)(t0 + (i_row < len ? i_row : 0)) * p.stride_q + h * 128;
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
@@ -161,35 +182,46 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int j = nrow + 16 * u;
-      const uint32_t qw[4] = {qv[u].x, qv[u].y, qv[u].z, qv[u].w}, kw[4] = {kv[u].x, kv[u].y, kv[u].z, kv[u].w};
+      f32x4_t qw[2], kw[2];
       float qs = 0.f, ks = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float q0 = lo16<bf16_t>(qw[e]), q1 = hi16<bf16_t>(qw[e]), k0 = lo16<bf16_t>(kw[e]), k1 = hi16<bf16_t>(kw[e]);
-        qs += q0 * q0 + q1 * q1;
-        ks += k0 * k0 + k1 * k1;
-      }
-      const float qi = rsqrtf(row16_allreduce(qs) + 1e-6f), ki = rsqrtf(row16_allreduce(ks) + 1e-6f);
-      const bool ok = j < len;
+      for (int x = 0; x < 2; ++x) {
+        qw[x] = widen4(qv[u][x]);
+        kw[x] = widen4(kv[u][x]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        qn[u][e] = ok ? pack2<bf16_t>(lo16<bf16_t>(qw[e]) * qi, hi16<bf16_t>(qw[e]) * qi) : 0u;
-        kn[u][e] = ok ? pack2<bf16_t>(lo16<bf16_t>(kw[e]) * ki, hi16<bf16_t>(kw[e]) * ki) : 0u;
+        for (int e = 0; e < 4; ++e) {
+          qs += qw[x][e] * qw[x][e];
+          ks += kw[x][e] * kw[x][e];
+        }
       }
-      *reinterpret_cast<uint4*>(&sh.Kn[j][nc0]) = make_uint4(kn[u][0], kn[u][1], kn[u][2], kn[u][3]);
-      if ((tid & 15) == 0) sh.QI[j] = ok ? qi : 0.f;
+      float qi = rsqrtf(row16_allreduce(qs) + 1e-6f);
+      const float ki = rsqrtf(row16_allreduce(ks) + 1e-6f);
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        qn[u][x] = make_uint2(pack2<bf16_t>(qw[x][0] * qi, qw[x][1] * qi), pack2<bf16_t>(qw[x][2] * qi, qw[x][3] * qi));
+        kn[u][x] = make_uint2(pack2<bf16_t>(kw[x][0] * ki, kw[x][1] * ki), pack2<bf16_t>(kw[x][2] * ki, kw[x][3] * ki));
+      }
+      if (len < CHUNK && j >= len) {               // a row the chunk does not have
+        qn[u][0] = qn[u][1] = kn[u][0] = kn[u][1] = make_uint2(0u, 0u);
+        qi = 0.f;
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) *reinterpret_cast<uint2*>(&sh.Kn[j][ca + 16 * x]) = kn[u][x];
+      if ((tid & 15) == 0) sh.QI[j] = qi;
     }
-    const float eA = expf(a_log);
+    // the gate over its bound (the scan applies it): 1 / (1 + e^{-eA (g + dt_bias)})
+    const float eA2 = -expf(a_log) * LOG2E;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int j = (tid >> 4) + 16 * u;
-      const uint32_t w[4] = {graw[u].x, graw[u].y, graw[u].z, graw[u].w};
+      const int j = nrow + 16 * u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float g0 = p.lower_bound * fast_rcp(1.0f + __expf(-eA * (lo16<bf16_t>(w[e]) + dtb[2 * e])));
-        const float g1 = p.lower_bound * fast_rcp(1.0f + __expf(-eA * (hi16<bf16_t>(w[e]) + dtb[2 * e + 1])));
-        sh.G[j][gc0 + 2 * e] = j < len ? g0 : 0.f;
-        sh.G[j][gc0 + 2 * e + 1] = j < len ? g1 : 0.f;
+      for (int x = 0; x < 2; ++x) {
+        const f32x4_t w = widen4(graw[u][x]);
+        f32x4_t r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = fast_rcp(1.0f + __builtin_amdgcn_exp2f(eA2 * (w[e] + dtb[x][e])));
+        if (len < CHUNK && j >= len) r = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<f32x4_t*>(&sh.G[j][ca + 16 * x]) = r;
       }
     }
     if (tid < CHUNK) {
@@ -197,60 +229,61 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
     }
   }
   __syncthreads();
-  if (tid < 128) {
-    float cum = 0.f;
-    for (int j = 0; j < CHUNK; ++j) {
-      cum += sh.G[j][tid];
-      sh.G[j][tid] = cum;                 // rows beyond the chunk repeat G_last (their g is zero)
-    }
-    p.eGlast[tile * 128 + tid] = __expf(cum);
+  {
+    // inclusive sums per channel over the two halves of the rows, in registers; the second half starts from the first's sum
+    const float bound = p.lower_bound * LOG2E;
+    const int c = tid & 127, j0 = (CHUNK / 2) * (tid >> 7);
+    float x[CHUNK / 2];
+#pragma unroll
+    for (int j = 0; j < CHUNK / 2; ++j) x[j] = sh.G[j0 + j][c];
+#pragma unroll
+    for (int j = 1; j < CHUNK / 2; ++j) x[j] += x[j - 1];
+    if (j0 == 0) sh.half_sum[c] = x[CHUNK / 2 - 1];
+    __syncthreads();
+    const float base = j0 == 0 ? 0.f : bound * sh.half_sum[c];
+#pragma unroll
+    for (int j = 0; j < CHUNK / 2; ++j) sh.G[j0 + j][c] = fmaf(bound, x[j], base);   // missing rows repeat G_last (their gate is zero)
+    if (j0 != 0) p.eGlast[tile * 128 + c] = __builtin_amdgcn_exp2f(fmaf(bound, x[CHUNK / 2 - 1], base));
   }
   __syncthreads();
 
   // ---- phase 2: decayed operand tiles for the sequential kernel (fp16, row major) ---------------
   {
-    const float* const glast = &sh.G[CHUNK - 1][0];
+    float4 glast[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) glast[x] = *reinterpret_cast<const float4*>(&sh.G[CHUNK - 1][ca + 16 * x]);
+    const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int j = (tid >> 4) + 16 * u, c0 = 8 * (tid & 15);   // the rows and channels this thread normalised
-      const uint32_t* const kwv = kn[u];
-      const uint32_t* const qwv = qn[u];
+      const int j = nrow + 16 * u;                              // the rows and channels this thread normalised
       uint32_t kg[4], qg[4], kt[4], ktl[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float g0 = sh.G[j][c0 + 2 * e], g1 = sh.G[j][c0 + 2 * e + 1];
-        const float e0 = __expf(g0), e1 = __expf(g1);
-        const float k0 = lo16<bf16_t>(kwv[e]), k1 = hi16<bf16_t>(kwv[e]);
-        kg[e] = pack2<f16_t>(k0 * e0, k1 * e1);
-        qg[e] = pack2<f16_t>(p.scale * lo16<bf16_t>(qwv[e]) * e0, p.scale * hi16<bf16_t>(qwv[e]) * e1);
-        pack2_pair(k0 * __expf(glast[c0 + 2 * e] - g0), k1 * __expf(glast[c0 + 2 * e + 1] - g1), kt[e], ktl[e]);
+      for (int x = 0; x < 2; ++x) {
+        const float4 g = *reinterpret_cast<const float4*>(&sh.G[j][ca + 16 * x]);
+        const f32x4_t e = decay4(g, zero4), es = f32x4_t{p.scale * e[0], p.scale * e[1], p.scale * e[2], p.scale * e[3]};
+        const f32x4_t k4 = widen4(kn[u][x]);
+        const f32x4_t a = times4(k4, e), b = times4(widen4(qn[u][x]), es), c = times4(k4, decay4(glast[x], g));
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          kg[2 * x + y] = pack2<f16_t>(a[2 * y], a[2 * y + 1]);
+          qg[2 * x + y] = pack2<f16_t>(b[2 * y], b[2 * y + 1]);
+          pack2_pair_small(c[2 * y], c[2 * y + 1], kt[2 * x + y], ktl[2 * x + y]);
+        }
       }
       // The tiles leave in the layout the sweeps read from LDS (they copy them as linear memory): unpadded rows of
       // 256 bytes with the swizzle of prefill_common.h, columns permuted inside groups of 32 so that an operand granule
-      // holds channels 32 s + 4 kb .. + 3 and 32 s + 16 + 4 kb .. + 3.  The thread's channels c0 .. c0 + 3 and
-      // c0 + 4 .. c0 + 7 are the same half of two neighbouring granules, and the thread two lanes away holds the other
-      // halves: the two exchange one piece each (a quad permutation) and then each stores one whole granule, so a
-      // wavefront still writes whole rows with one 16-byte store per lane.
-      const int lc = tid & 15;
-      const bool upper = lc & 2;                       // this thread holds the second halves of its granules
-      const int granule = 4 * (lc >> 2) + 2 * (lc & 1) + (upper ? 1 : 0);
-      auto whole_granule = [&](const uint32_t (&x)[4]) {
-        const uint32_t s0 = upper ? x[0] : x[2], s1 = upper ? x[1] : x[3];
-        const uint32_t r0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s0, 0x4E, 0xF, 0xF, true);      // lane ^ 2
-        const uint32_t r1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s1, 0x4E, 0xF, 0xF, true);
-        return upper ? make_uint4(r0, r1, x[2], x[3]) : make_uint4(x[0], x[1], r0, r1);
-      };
-      const int64_t at = tile * 8192 + tile_offset(j, granule), at2 = tile * 16384 + tile_offset(j, granule);
-      *reinterpret_cast<uint4*>(p.Kg + at) = whole_granule(kg);
-      *reinterpret_cast<uint4*>(p.Qg + at) = whole_granule(qg);
-      *reinterpret_cast<uint4*>(p.Kt + at2) = whole_granule(kt);
-      *reinterpret_cast<uint4*>(p.Kt + at2 + 8192) = whole_granule(ktl);
+      // holds channels 32 s + 4 kb .. + 3 and 32 s + 16 + 4 kb .. + 3, which are the thread's: one 16-byte store per
+      // lane, whole rows per wavefront.
+      const int64_t at = tile * 8192 + tile_offset(j, tid & 15), at2 = tile * 16384 + tile_offset(j, tid & 15);
+      nt_store16(p.Kg + at, make_uint4(kg[0], kg[1], kg[2], kg[3]));
+      nt_store16(p.Qg + at, make_uint4(qg[0], qg[1], qg[2], qg[3]));
+      nt_store16(p.Kt + at2, make_uint4(kt[0], kt[1], kt[2], kt[3]));
+      nt_store16(p.Kt + at2 + 8192, make_uint4(ktl[0], ktl[1], ktl[2], ktl[3]));
     }
   }
 
   // ---- phase 3: M and P, wavefront w owns row block w (reference row = first row of the block) --
   {
-    const int bi = wave;
     const float* const R = &sh.G[16 * bi][0];
     const int i_row = 16 * bi + r16;
     HiLo Al[4];
@@ -261,22 +294,16 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
       const int c0 = 32 * s + 4 * kb, c1 = c0 + 16;
       const float4 g0 = *reinterpret_cast<const float4*>(&sh.G[i_row][c0]), g1 = *reinterpret_cast<const float4*>(&sh.G[i_row][c1]);
       const float4 r0 = *reinterpret_cast<const float4*>(R + c0), r1 = *reinterpret_cast<const float4*>(R + c1);
-      const f32x4_t e0 = {__expf(g0.x - r0.x), __expf(g0.y - r0.y), __expf(g0.z - r0.z), __expf(g0.w - r0.w)};
-      const f32x4_t e1 = {__expf(g1.x - r1.x), __expf(g1.y - r1.y), __expf(g1.z - r1.z), __expf(g1.w - r1.w)};
-      const uint2 k0 = *reinterpret_cast<const uint2*>(&sh.Kn[i_row][c0]), k1 = *reinterpret_cast<const uint2*>(&sh.Kn[i_row][c1]);
-      f32x4_t a = {lo16<bf16_t>(k0.x) * e0[0], hi16<bf16_t>(k0.x) * e0[1], lo16<bf16_t>(k0.y) * e0[2], hi16<bf16_t>(k0.y) * e0[3]};
-      f32x4_t b = {lo16<bf16_t>(k1.x) * e1[0], hi16<bf16_t>(k1.x) * e1[1], lo16<bf16_t>(k1.y) * e1[2], hi16<bf16_t>(k1.y) * e1[3]};
+      const f32x4_t e0 = decay4(g0, r0), e1 = decay4(g1, r1);
+      const f32x4_t a = times4(widen4(*reinterpret_cast<const uint2*>(&sh.Kn[i_row][c0])), e0);
+      const f32x4_t b = times4(widen4(*reinterpret_cast<const uint2*>(&sh.Kn[i_row][c1])), e1);
       Al[s] = split8(a, b);
       // the same normalised bf16 values as phase 1 formed: raw q times the row's inverse norm, rounded to bf16
       const float qi = sh.QI[i_row];
-      const uint2 x0 = qraw[s][0], x1 = qraw[s][1];
-      const uint32_t n0 = pack2<bf16_t>(lo16<bf16_t>(x0.x) * qi, hi16<bf16_t>(x0.x) * qi);
-      const uint32_t n1 = pack2<bf16_t>(lo16<bf16_t>(x0.y) * qi, hi16<bf16_t>(x0.y) * qi);
-      const uint32_t n2 = pack2<bf16_t>(lo16<bf16_t>(x1.x) * qi, hi16<bf16_t>(x1.x) * qi);
-      const uint32_t n3 = pack2<bf16_t>(lo16<bf16_t>(x1.y) * qi, hi16<bf16_t>(x1.y) * qi);
-      a = f32x4_t{lo16<bf16_t>(n0) * e0[0], hi16<bf16_t>(n0) * e0[1], lo16<bf16_t>(n1) * e0[2], hi16<bf16_t>(n1) * e0[3]};
-      b = f32x4_t{lo16<bf16_t>(n2) * e1[0], hi16<bf16_t>(n2) * e1[1], lo16<bf16_t>(n3) * e1[2], hi16<bf16_t>(n3) * e1[3]};
-      Ql[s] = round8(a, b);
+      const f32x4_t x0 = widen4(qraw[s][0]), x1 = widen4(qraw[s][1]);
+      const uint2 n0 = make_uint2(pack2<bf16_t>(x0[0] * qi, x0[1] * qi), pack2<bf16_t>(x0[2] * qi, x0[3] * qi));
+      const uint2 n1 = make_uint2(pack2<bf16_t>(x1[0] * qi, x1[1] * qi), pack2<bf16_t>(x1[2] * qi, x1[3] * qi));
+      Ql[s] = round8(times4(widen4(n0), e0), times4(widen4(n1), e1));
     }
     // P leaves in the six-block operand layout (prefill_common.h): its product is formed transposed (A = k rows j,
     // B = q rows i), so a lane holds four consecutive j of token i = 16 bi + r16, which is half of the 16 bytes it owns
@@ -291,9 +318,11 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
       f32x4_t m = {0.f, 0.f, 0.f, 0.f}, pq = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        f32x4_t a, b;
-        decayed8(&sh.Kn[j][0], &sh.G[j][0], R, -1.0f, s, kb, a, b);     // k_j e^{R - G_j}
-        const HiLo Br = split8(a, b);
+        const int c0 = 32 * s + 4 * kb, c1 = c0 + 16;                   // k_j e^{R - G_j}
+        const f32x4_t e0 = decay4(*reinterpret_cast<const float4*>(R + c0), *reinterpret_cast<const float4*>(&sh.G[j][c0]));
+        const f32x4_t e1 = decay4(*reinterpret_cast<const float4*>(R + c1), *reinterpret_cast<const float4*>(&sh.G[j][c1]));
+        const HiLo Br = split8(times4(widen4(*reinterpret_cast<const uint2*>(&sh.Kn[j][c0])), e0),
+                               times4(widen4(*reinterpret_cast<const uint2*>(&sh.Kn[j][c1])), e1));
         m = mfma16(Al[s].hi, Br.hi, m);
         m = mfma16(Al[s].lo, Br.hi, m);
         m = mfma16(Al[s].hi, Br.lo, m);
@@ -324,7 +353,7 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
 
   // ---- phase 4: W = L^-1 diag(beta) by blocks on one wavefront (which one rotates with the workgroup, so
   // that co-resident workgroups keep different SIMDs busy) -----------------------------------------
-  if (wave == (int)(blockIdx.x & 3)) {
+  if (bi == 0) {
     block_inverse_inplace(sh.L, lane);
     store_w_operand_blocks(sh.L, sh.B, lane, p.W + tile * (2 * TRI_BLOCKS * 512));
   }
@@ -1155,7 +1184,7 @@ static int kda_prefill_run(
                 segmented ? L.max_segments : N, o, H);
   const bool ok = launch_pipeline(
       s, stages, lease.get(), segmented, (unsigned)N * H, (unsigned)L.max_segments * H, &p.pass, &p.stage,
-      [&](hipStream_t ps) { hipLaunchKernelGGL(kda_prep_solve_kernel, dim3(L.NC_max, H), dim3(256), 0, ps, p); },
+      [&](hipStream_t ps) { hipLaunchKernelGGL(kda_prep_solve_kernel, dim3((unsigned)L.NC_max * H), dim3(256), 0, ps, p); },
       [&](unsigned grid) {
         // the first sweep over segments publishes no output: the lean variant, two workgroups per CU
         // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)
