@@ -17,6 +17,7 @@
 #include <optional>
 #include <string>
 #include <variant>
+#include <vector>
 
 #include "../../include/pla_gfx950.h"
 
@@ -400,6 +401,246 @@ void fused_kda_decode_mega_forward(const Tensor& x, const Tensor& weight, const 
       x.stride(0), raw_beta.stride(1), onorm_row, conv_state.stride(0), state.stride(0), stream_of(x)));
 }
 
+// ---- KDA replay: verify and commit of both runners ---------------------------------------------------------------
+// The facades (pla_amd/decode/kda_replayssm_*/__init__.py) offer every call to these functions first.  Each repeats the
+// facade's checks and returns false, with nothing launched, for a call that it does not take as it stands (a failed
+// check, an index vector that needs a copy): the facade then words the error or makes the copy.
+#define OFFER(cond) do { if (!(cond)) return false; } while (0)
+
+bool index_vector(const Tensor& t, const Tensor& ref) {
+  return t.device() == ref.device() && t.dim() == 1 && t.is_contiguous() && (t.scalar_type() == at::kInt || t.scalar_type() == at::kLong);
+}
+int wide(const Tensor& t) { return t.scalar_type() == at::kLong ? 1 : 0; }
+bool shaped(const Tensor& t, at::IntArrayRef shape, at::ScalarType dtype) { return t.sizes() == shape && t.scalar_type() == dtype; }
+bool at16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// The bytes between a tensor's first and last element.
+struct ByteSpan {
+  uintptr_t begin, end;
+  explicit ByteSpan(const Tensor& t) : begin(reinterpret_cast<uintptr_t>(t.data_ptr())), end(begin) {
+    if (t.numel() == 0) return;
+    int64_t extent = 1;
+    for (int64_t d = 0; d < t.dim(); ++d) extent += (t.size(d) - 1) * t.stride(d);
+    end += extent * t.element_size();
+  }
+  bool meets(const ByteSpan& o) const { return begin < o.end && o.begin < end; }
+};
+
+// Request-row verify over paged checkpoints (facade: kda_replay_verify).
+bool kda_replay_verify(const Tensor& x, const Tensor& raw_g, const Tensor& raw_beta, const Tensor& conv_weight, const Tensor& conv,
+                       const Tensor& state, const Tensor& A_log, const Tensor& dt_bias, const Tensor& out, const Tensor& rawv,
+                       const Tensor& rawk, const Tensor& rec_g, const Tensor& rec_beta, const Tensor& windows, const Tensor& cu,
+                       const Tensor& src, const std::string& layout, double lower_bound, double scale, int64_t null_block_id) {
+  constexpr int64_t D = 128;
+  OFFER(state.dim() == 4 && rawv.dim() == 4 && conv.dim() == 3 && (null_block_id == -1 || null_block_id == 0));
+  const int64_t slots = state.size(0), H = state.size(1), R = rawv.size(0), Q = rawv.size(2);
+  OFFER(state.is_cuda() && H > 0 && slots > 0 && shaped(state, {slots, H, D, D}, at::kFloat) && state.stride(3) == 1 &&
+        state.stride(2) == D && state.stride(1) == D * D && state.stride(0) >= H * D * D && state.stride(0) % 4 == 0 && at16(state));
+  OFFER(layout == "DS" || layout == "SD");
+  OFFER(conv.size(0) == slots && conv.scalar_type() == at::kBFloat16);
+  const int ch = layout == "DS" ? 1 : 2, tap = 3 - ch;                  // channel and history dimension
+  const int64_t c_slot = conv.stride(0), c_ch = conv.stride(ch), c_tap = conv.stride(tap), history = conv.size(tap);
+  OFFER(conv.size(ch) == 3 * H * D && history >= 3);
+  OFFER((c_tap == 1 && c_ch >= history) || (c_ch == 1 && c_tap >= conv.size(ch)));
+  OFFER(c_slot >= (conv.size(ch) - 1) * c_ch + (history - 1) * c_tap + 1);
+  OFFER(Q >= 1 && Q <= 32);
+  OFFER(shaped(rawv, {R, H, Q, D}, at::kBFloat16) && shaped(rawk, {R, H, Q, D}, at::kBFloat16) && shaped(rec_g, {R, H, Q, D}, at::kFloat) &&
+        shaped(rec_beta, {R, H, Q}, at::kFloat) && shaped(windows, {R, Q, 3 * H * D, 3}, at::kBFloat16));
+  for (const Tensor* t : {&rawv, &rawk, &rec_g, &rec_beta, &windows}) OFFER(t->device() == state.device() && t->is_contiguous());
+  for (const Tensor* t : {&rawv, &rawk, &rec_g, &rec_beta}) OFFER(at16(*t));
+  for (const Tensor* t : {&x, &raw_g, &raw_beta, &conv, &conv_weight, &A_log, &dt_bias, &out}) OFFER(t->device() == state.device());
+  OFFER(x.dim() == 2 && x.size(1) == 3 * H * D && x.stride(1) == 1 && x.stride(0) >= 3 * H * D && x.scalar_type() == at::kBFloat16);
+  const int64_t T = x.size(0);
+  OFFER(shaped(raw_g, {T, H * D}, at::kBFloat16) && raw_g.stride(1) == 1 && raw_g.stride(0) >= H * D);
+  OFFER(shaped(raw_beta, {T, H}, at::kBFloat16) && raw_beta.stride(1) == 1 && raw_beta.stride(0) >= H);
+  OFFER(shaped(conv_weight, {3 * H * D, 4}, at::kFloat) && conv_weight.is_contiguous());
+  OFFER(A_log.numel() == H && dt_bias.numel() == H * D && A_log.is_contiguous() && dt_bias.is_contiguous() &&
+        A_log.scalar_type() == at::kFloat && dt_bias.scalar_type() == at::kFloat);
+  OFFER(shaped(out, {T, H * D}, at::kBFloat16) && out.is_contiguous());
+  OFFER(std::isfinite(scale) && std::isfinite(lower_bound) && lower_bound < 0);
+  OFFER(index_vector(cu, state) && index_vector(src, state));
+  const int64_t N = src.numel();
+  OFFER(N > 0 && cu.numel() == N + 1 && N <= R);
+  const ByteSpan writes[] = {ByteSpan(out), ByteSpan(rawv), ByteSpan(rawk), ByteSpan(rec_g), ByteSpan(rec_beta), ByteSpan(windows)};
+  const ByteSpan reads[] = {ByteSpan(x), ByteSpan(raw_g), ByteSpan(raw_beta), ByteSpan(conv_weight), ByteSpan(conv), ByteSpan(state),
+                            ByteSpan(A_log), ByteSpan(dt_bias), ByteSpan(cu), ByteSpan(src)};
+  for (const ByteSpan& w : writes) {
+    for (const ByteSpan* other = writes; other != &w; ++other) OFFER(!w.meets(*other));
+    for (const ByteSpan& r : reads) OFFER(!w.meets(r));
+  }
+  int64_t strides[26] = {x.stride(0), x.stride(0), x.stride(0), raw_g.stride(0), raw_beta.stride(0)};
+  for (int i = 0; i < 3; ++i) {
+    const int64_t cs[3] = {c_slot, c_ch, c_tap};
+    for (int j = 0; j < 3; ++j) strides[5 + 3 * i + j] = cs[j];
+    for (int j = 0; j < 4; ++j) strides[14 + 4 * i + j] = windows.stride(j);
+  }
+  const int64_t segment = H * D;                                        // channels of q, of k and of v
+  const uint16_t* const xp = static_cast<const uint16_t*>(x.data_ptr());
+  const uint16_t* const cp = static_cast<const uint16_t*>(conv.data_ptr());
+  uint16_t* const wp = static_cast<uint16_t*>(windows.data_ptr());
+  const float* const wt = conv_weight.data_ptr<float>();
+  const c10::DeviceGuard guard(state.device());
+  launched(pla_kda_replay_verify_native_launch(
+      xp, xp + segment, xp + 2 * segment, raw_g.data_ptr(), raw_beta.data_ptr(), wt, wt + 4 * segment, wt + 8 * segment, cp,
+      cp + segment * c_ch, cp + 2 * segment * c_ch, A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), state.data_ptr<float>(),
+      out.data_ptr(), wp, wp + segment * windows.stride(2), wp + 2 * segment * windows.stride(2), rawv.data_ptr(), rawk.data_ptr(),
+      rec_g.data_ptr<float>(), rec_beta.data_ptr<float>(), src.data_ptr(), wide(src), cu.data_ptr(), wide(cu), (int)H, (int)N, (int)Q,
+      (float)scale, (float)lower_bound, strides, state.stride(0), (int)slots, (int)T, (int)null_block_id, stream_of(state)));
+  return true;
+}
+
+// Commit of the request-row records (facade: KDAReplayCommitContext.commit): plan, fold and conv windows of all layers.
+bool kda_replay_commit(const Tensor& sampled, const Tensor& source, const Tensor& cu, const OptTensor& mapping, const OptTensor& blocks,
+                       const OptTensor& computed, int64_t block_size, const Tensor& table, const Tensor& candidate, const Tensor& plan,
+                       int64_t heads, int64_t slots, int64_t Q, int64_t null_block_id, int64_t channels, int64_t rows,
+                       int64_t token_capacity) {
+  OFFER(token_capacity >= 0 && token_capacity <= 2147483647);
+  OFFER(index_vector(sampled, plan) && index_vector(source, plan) && index_vector(cu, plan) && source.scalar_type() == at::kInt);
+  const int64_t N = source.numel(), R = plan.size(1);
+  OFFER(N > 0 && N <= R && cu.numel() == N + 1);
+  if (mapping.has_value()) OFFER(index_vector(*mapping, plan) && mapping->numel() == N);
+  else OFFER(sampled.numel() >= N);
+  const bool align = blocks.has_value();
+  OFFER(align == computed.has_value());
+  if (align)
+    OFFER(index_vector(*computed, plan) && computed->numel() >= sampled.numel() && blocks->device() == plan.device() && blocks->dim() == 2 &&
+          blocks->size(1) > 0 && (blocks->scalar_type() == at::kInt || blocks->scalar_type() == at::kLong));
+  const c10::DeviceGuard guard(plan.device());
+  void* const stream = stream_of(plan);
+  launched(pla_kda_commit_plan_launch(
+      sampled.data_ptr(), wide(sampled), source.data_ptr(), wide(source), cu.data_ptr(), wide(cu), ptr(mapping), mapping ? wide(*mapping) : 0,
+      ptr(computed), computed ? wide(*computed) : 0, ptr(blocks), align ? wide(*blocks) : 0, (int)N, (int)R, (int)sampled.numel(),
+      align ? (int)blocks->size(0) : 0, align ? (int)blocks->size(1) : 0, (int)slots, (int)Q, (int)null_block_id, (int)token_capacity,
+      align ? blocks->stride(0) : 0, align ? blocks->stride(1) : 0, align ? block_size : 0, candidate.data_ptr<int32_t>(),
+      plan.data_ptr<int32_t>(), stream));
+  const int32_t* const lens = plan.data_ptr<int32_t>();
+  const int32_t *const final_slot = lens + R, *const boundary = lens + 2 * R, *const boundary_lens = lens + 3 * R;
+  const int layers = (int)table.size(0);
+  launched(pla_kda_fold_native_launch(table.data_ptr<int64_t>(), layers, source.data_ptr<int32_t>(), lens, final_slot, boundary,
+                                      boundary_lens, (int)N, (int)heads, (int)Q, (int)slots, (int)null_block_id, stream));
+  launched(pla_kda_conv_native_launch(table.data_ptr<int64_t>(), layers, lens, final_slot, boundary, boundary_lens, (int)N, (int)channels,
+                                      (int)Q, (int)rows, (int)slots, stream));
+  return true;
+}
+
+// Ring-mode verify (facade: fused_kda_decode_mtp_dspark).
+bool kda_verify_dspark(const Tensor& x_q, const Tensor& x_k, const Tensor& x_v, const Tensor& w_q, const Tensor& w_k, const Tensor& w_v,
+                       const Tensor& cs_q, const Tensor& cs_k, const Tensor& cs_v, const Tensor& g, const Tensor& beta, const Tensor& A_log,
+                       const Tensor& dt_bias, const Tensor& state, const Tensor& scratch, const Tensor& ic_q, const Tensor& ic_k,
+                       const Tensor& ic_v, const Tensor& indices, const Tensor& cu, double lower_bound, double scale, const Tensor& rawv,
+                       const Tensor& rawk, const Tensor& ring_g, const Tensor& ring_beta, const OptTensor& onorm_gate,
+                       const OptTensor& onorm_weight, double onorm_eps, const Tensor& out) {
+  constexpr int64_t D = 128, W = 4;
+  OFFER(x_q.dim() == 4 && x_q.size(0) == 1 && x_q.is_cuda() && x_q.size(3) == D && rawv.dim() == 4);
+  const int64_t T = x_q.size(1), H = x_q.size(2), N = cu.numel() - 1, L = rawv.size(2), slots = rawv.size(0);
+  OFFER(N > 0 && T > 0 && H > 0 && T % N == 0 && L >= T / N);
+  const int64_t window = T / N;
+  OFFER(shaped(state, {slots, H, D, D}, at::kFloat));
+  for (const Tensor* t : {&x_k, &x_v, &g, &beta, &w_q, &w_k, &w_v, &cs_q, &cs_k, &cs_v, &A_log, &dt_bias, &state, &out, &ic_q, &ic_k, &ic_v,
+                          &rawv, &rawk, &ring_g, &ring_beta})
+    OFFER(t->device() == x_q.device());
+  OFFER(shaped(rawv, {slots, H, L, D}, at::kBFloat16) && shaped(rawk, {slots, H, L, D}, at::kBFloat16) &&
+        shaped(ring_g, {slots, H, L, D}, at::kFloat) && shaped(ring_beta, {slots, H, L}, at::kFloat));
+  for (const Tensor* t : {&w_q, &w_k, &w_v}) OFFER(shaped(*t, {H * D, W}, at::kFloat) && t->is_contiguous());
+  OFFER(A_log.numel() == H && dt_bias.numel() == H * D && A_log.is_contiguous() && dt_bias.is_contiguous() &&
+        A_log.scalar_type() == at::kFloat && dt_bias.scalar_type() == at::kFloat);
+  OFFER(state.storage_offset() % 4 == 0);
+  OFFER(index_vector(indices, x_q) && index_vector(scratch, x_q) && index_vector(cu, x_q) && indices.numel() == N && scratch.numel() >= N);
+  int64_t strides[26];
+  int at = 0;
+  for (const Tensor* t : {&x_q, &x_k, &x_v, &g}) {
+    OFFER(t->sizes() == x_q.sizes() && t->scalar_type() == at::kBFloat16 && t->stride(3) == 1 && t->stride(2) == D && t->stride(1) >= H * D);
+    strides[at++] = t->stride(1);
+  }
+  OFFER(shaped(beta, {1, T, H}, at::kBFloat16) && beta.stride(2) == 1 && beta.stride(1) >= H);
+  strides[at++] = beta.stride(1);
+  for (const Tensor* t : {&cs_q, &cs_k, &cs_v}) {
+    OFFER(shaped(*t, {slots, H * D, W - 1}, at::kBFloat16));
+    for (int d = 0; d < 3; ++d) {
+      OFFER(t->stride(d) > 0);
+      strides[at++] = t->stride(d);
+    }
+  }
+  for (const Tensor* t : {&ic_q, &ic_k, &ic_v}) {
+    OFFER(t->dim() == 4 && t->size(1) >= window && t->size(2) == H * D && t->size(3) == W - 1 && t->scalar_type() == at::kBFloat16);
+    for (int d = 0; d < 4; ++d) {
+      OFFER(t->stride(d) > 0);
+      strides[at++] = t->stride(d);
+    }
+  }
+  OFFER(out.sizes() == x_q.sizes() && out.scalar_type() == at::kBFloat16);
+  for (const Tensor* t : {&out, &state, &rawv, &rawk, &ring_g, &ring_beta}) OFFER(t->is_contiguous());
+  const bool onorm = onorm_gate.has_value();
+  OFFER(onorm == onorm_weight.has_value());
+  if (onorm)
+    OFFER(onorm_gate->device() == x_q.device() && onorm_weight->device() == x_q.device() && onorm_gate->sizes() == x_q.sizes() &&
+          onorm_gate->scalar_type() == at::kBFloat16 && onorm_gate->stride(3) == 1 && onorm_gate->stride(2) == D &&
+          onorm_gate->stride(1) >= H * D && shaped(*onorm_weight, {D}, at::kFloat) && onorm_weight->is_contiguous() &&
+          std::isfinite(onorm_eps) && onorm_eps >= 0.0);
+  const c10::DeviceGuard guard(x_q.device());
+  launched(pla_kda_verify_dspark_launch(
+      x_q.data_ptr(), x_k.data_ptr(), x_v.data_ptr(), g.data_ptr(), beta.data_ptr(), w_q.data_ptr<float>(), w_k.data_ptr<float>(),
+      w_v.data_ptr<float>(), cs_q.data_ptr(), cs_k.data_ptr(), cs_v.data_ptr(), A_log.data_ptr<float>(), dt_bias.data_ptr<float>(),
+      state.data_ptr<float>(), out.data_ptr(), ic_q.data_ptr(), ic_k.data_ptr(), ic_v.data_ptr(), rawv.data_ptr(), rawk.data_ptr(),
+      ring_g.data_ptr<float>(), ring_beta.data_ptr<float>(), indices.data_ptr(), wide(indices), scratch.data_ptr(), wide(scratch),
+      cu.data_ptr(), wide(cu), (int)H, (int)N, (int)window, (int)L, (float)scale, (float)lower_bound, strides, ptr(onorm_gate),
+      onorm ? onorm_weight->data_ptr<float>() : nullptr, onorm ? onorm_gate->stride(1) : 0, onorm ? (float)onorm_eps : 0.f,
+      stream_of(x_q)));
+  return true;
+}
+
+// Commit of the ring records without track snapshots (facade: commit_kda_replayssm_after_verify): one fold for all
+// layers and the conv windows of every pool ([layers, slots, dim, width - 1]).
+bool kda_ring_commit(const Tensor& temporal, const Tensor& rawv, const Tensor& rawk, const Tensor& gk, const Tensor& beta,
+                     const Tensor& indices, const Tensor& accepted, const Tensor& last_step, const std::vector<Tensor>& conv,
+                     const std::vector<Tensor>& windows, int64_t null_block_id) {
+  constexpr int64_t D = 128;
+  OFFER(temporal.is_cuda() && temporal.dim() == 5 && rawk.dim() == 5);
+  const int64_t layers = temporal.size(0), slots = temporal.size(1), HV = temporal.size(2), H = rawk.size(2), L = rawk.size(3);
+  OFFER(layers > 0 && slots > 0 && shaped(temporal, {layers, slots, HV, D, D}, at::kFloat));
+  const auto act = rawk.scalar_type();
+  OFFER(act == at::kBFloat16 || act == at::kHalf);
+  OFFER(shaped(rawv, {layers, slots, HV, L, D}, act) && shaped(rawk, {layers, slots, H, L, D}, act) &&
+        shaped(gk, {layers, slots, HV, L, D}, at::kFloat) && shaped(beta, {layers, slots, HV, L}, at::kFloat));
+  // dense slots: every dimension behind the layer and the slot
+  auto dense_slot = [](const Tensor& t) {
+    int64_t expect = 1;
+    for (int64_t d = t.dim() - 1; d >= 2; --d) {
+      if (t.size(d) != 1 && t.stride(d) != expect) return false;
+      expect *= t.size(d);
+    }
+    return true;
+  };
+  for (const Tensor* t : {&temporal, &rawv, &rawk, &gk, &beta}) OFFER(t->device() == temporal.device() && dense_slot(*t));
+  OFFER(index_vector(indices, temporal) && index_vector(accepted, temporal) && index_vector(last_step, temporal));
+  OFFER(indices.scalar_type() == at::kInt && accepted.scalar_type() == at::kInt);
+  const int64_t B = indices.numel();
+  OFFER(B > 0 && accepted.numel() == B && last_step.numel() == B && conv.size() == windows.size());
+  for (size_t i = 0; i < conv.size(); ++i) {
+    const Tensor &dst = conv[i], &src = windows[i];
+    OFFER(dst.dim() == 4 && src.dim() == 5 && dst.device() == temporal.device() && src.device() == dst.device() &&
+          src.scalar_type() == dst.scalar_type() && (dst.scalar_type() == at::kBFloat16 || dst.scalar_type() == at::kFloat));
+    OFFER(src.size(0) == dst.size(0) && src.size(3) == dst.size(2) && src.size(4) == dst.size(3) && dst.size(3) >= 1 && dst.size(3) <= 4);
+    OFFER(dst.is_contiguous() || dst.transpose(-1, -2).is_contiguous());
+  }
+  const c10::DeviceGuard guard(temporal.device());
+  void* const stream = stream_of(temporal);
+  launched(pla_kda_fold_launch(
+      temporal.data_ptr<float>(), rawv.data_ptr(), rawk.data_ptr(), gk.data_ptr<float>(), beta.data_ptr<float>(), indices.data_ptr<int32_t>(),
+      accepted.data_ptr<int32_t>(), nullptr, nullptr, temporal.stride(1), rawv.stride(1), rawk.stride(1), gk.stride(1), beta.stride(1),
+      (int)layers, temporal.stride(0), rawv.stride(0), rawk.stride(0), gk.stride(0), beta.stride(0), (int)B, (int)H, (int)HV, (int)L,
+      (int)null_block_id, dtype_code(act), stream));
+  for (size_t i = 0; i < conv.size(); ++i) {
+    const Tensor &dst = conv[i], &src = windows[i];
+    launched(pla_conv_window_scatter_launch(
+        (int)dst.element_size(), (int)dst.size(3), src.data_ptr(), dst.data_ptr(), indices.data_ptr(), wide(indices), last_step.data_ptr(),
+        wide(last_step), (int)dst.size(0), (int)dst.size(2), (int)B, src.stride(0), src.stride(1), src.stride(2), src.stride(3), src.stride(4),
+        dst.stride(0), dst.stride(1), dst.stride(2), dst.stride(3), (int)src.size(1), (int)src.size(2), (int)dst.size(1), stream));
+  }
+  return true;
+}
+#undef OFFER
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -417,6 +658,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("lower_bound"), py::arg("initial_state"), py::arg("cu_seqlens"), py::arg("ssm_state_indices"),
         py::arg("num_accepted_tokens") = py::none(), py::arg("out") = py::none(), py::arg("fuse_gate") = py::none(),
         py::arg("is_sglang") = false);
+  m.def("_kda_replay_verify", &kda_replay_verify);
+  m.def("_kda_replay_commit", &kda_replay_commit);
+  m.def("_kda_verify_dspark", &kda_verify_dspark);
+  m.def("_kda_ring_commit", &kda_ring_commit);
   m.doc() = "pla.decode._C for MI355X: k-last gated delta-rule decode and MTP verify over libpla_gfx950.so";
   m.def(
       "fused_sigmoid_gating_delta_rule_forward_k_last",

@@ -20,6 +20,7 @@ import os
 import torch
 
 from ... import _lib
+from .. import _compiled, _sanity_enabled
 
 __all__ = ["fused_kda_decode_mtp_dspark", "commit_kda_replayssm_after_verify", "conv_window_scatter",
            "fold_accepted_prefix", "kda_mtp_verify"]
@@ -131,12 +132,22 @@ def commit_kda_replayssm_after_verify(*, spec_state, state_batch_indices, accept
     assert conv_state_layout in ("dim_width", "width_dim")
     if (mamba_track_indices is None) != (mamba_steps_to_track is None):
         raise ValueError("mamba_track_indices and mamba_steps_to_track must be given together")
+    conv = getattr(spec_state, "conv", None)
+    windows = getattr(spec_state, "intermediate_conv_window", None)
+    native = _compiled()
+    if (native and not _BYPASS and mamba_track_indices is None and conv_state_layout == "dim_width"
+            and conv is not None and windows is not None):
+        try:
+            if native._kda_ring_commit(spec_state.temporal, spec_state.replayssm_rawv, spec_state.replayssm_rawk,
+                                       spec_state.replayssm_g, spec_state.replayssm_beta, state_batch_indices,
+                                       accept_lens, last_correct_step_indices, conv, windows, int(null_block_id)):
+                return
+        except TypeError:                            # not the types the compiled layer takes: reported below
+            pass
     fold_accepted_prefix(spec_state.temporal, spec_state.replayssm_rawv, spec_state.replayssm_rawk,
                          spec_state.replayssm_g, spec_state.replayssm_beta,
                          state_batch_indices, accept_lens, null_block_id,
                          mamba_track_indices, mamba_steps_to_track)
-    conv = getattr(spec_state, "conv", None)
-    windows = getattr(spec_state, "intermediate_conv_window", None)
     if conv is None or windows is None:
         return
     if last_correct_step_indices is None:
@@ -182,6 +193,18 @@ def fused_kda_decode_mtp_dspark(*, x_q, x_k, x_v, w_q, w_k, w_v, cs_q, cs_k, cs_
         out = torch.empty_like(x_v, memory_format=torch.contiguous_format)
     if _BYPASS:
         return out
+
+    native = _compiled()
+    if native and not _sanity_enabled():             # the PLA_SANITY_CHECK diagnostics live below
+        try:
+            if native._kda_verify_dspark(x_q, x_k, x_v, w_q, w_k, w_v, cs_q, cs_k, cs_v, g, beta, A_log, dt_bias,
+                                         recurrent_state, intermediate_state_indices, intermediate_conv_q,
+                                         intermediate_conv_k, intermediate_conv_v, ssm_state_indices, cu_seqlens,
+                                         float(lower_bound), float(scale), *rings, onorm_gate, onorm_weight,
+                                         float(onorm_eps) if apply_onorm else 0.0, out):
+                return out
+        except TypeError:                            # not the types the compiled layer takes: reported below
+            pass
 
     def need(cond, msg):
         if not cond:

@@ -22,6 +22,7 @@ from typing import Optional
 import torch
 
 from ... import _lib
+from .. import _compiled
 
 __all__ = ["KDAReplayRecords", "KDAReplayCommitPlan", "KDAReplayCommitContext", "kda_replay_verify"]
 
@@ -136,6 +137,17 @@ def kda_replay_verify(*, mixed_qkv, raw_g, raw_beta, conv_weight, conv_state, ch
         out = torch.empty(mixed_qkv.size(0), H * D, dtype=torch.bfloat16, device=mixed_qkv.device)
     if _BYPASS:
         return out
+    scale = D ** -0.5 if scale is None else float(scale)
+    native = _compiled()
+    if native:
+        try:
+            if native._kda_replay_verify(mixed_qkv, raw_g, raw_beta, conv_weight, conv_state, state, A_log, dt_bias, out,
+                                         records.rawv, records.rawk, records.g, records.beta, records.conv,
+                                         query_start_loc, state_indices, conv_state_layout, float(lower_bound), scale,
+                                         int(null_block_id)):
+                return out
+        except TypeError:                            # not the types the compiled layer takes: reported below
+            pass
     _need(null_block_id in (-1, 0), "null_block_id must be -1 or 0")
     cs = _paged_cache(conv_state, state, conv_state_layout, H, slots)
     _check_records(records, state, H, Q, R)
@@ -154,7 +166,6 @@ def kda_replay_verify(*, mixed_qkv, raw_g, raw_beta, conv_weight, conv_state, ch
           and A_log.dtype == torch.float32 and dt_bias.dtype == torch.float32, "gate weights must be contiguous fp32")
     _need(out.dtype == torch.bfloat16 and tuple(out.shape) == (T, H * D) and out.is_contiguous(),
           "invalid replay tensor shape/dtype/contiguity")
-    scale = D ** -0.5 if scale is None else float(scale)
     _need(scale == scale and abs(scale) != float("inf") and lower_bound == lower_bound
           and abs(lower_bound) != float("inf") and lower_bound < 0, "scale/lower_bound must be finite fp32; bound < 0")
     cu, cu_wide = _index(query_start_loc, state)
@@ -330,6 +341,16 @@ class KDAReplayCommitContext:
             raise ValueError("align block_size must be >= spec_query_len")
         if _BYPASS:
             return self.plan
+        native = _compiled()
+        if native:
+            try:
+                if native._kda_replay_commit(num_sampled, state_indices, query_start_loc, request_indices, block_table,
+                                             num_computed_tokens, int(mamba_block_size or 0), self._table,
+                                             self._candidate, self._buffer, self._heads, self._slots, self._q,
+                                             self._null, self._channels, self._rows, int(token_capacity)):
+                    return self.plan
+            except TypeError:                        # not the types the compiled layer takes: reported below
+                pass
         _need(0 <= token_capacity <= 2 ** 31 - 1, "token_capacity must be between 0 and INT32_MAX")
         ref = self._buffer
         sampled, sampled_wide = _index(num_sampled, ref)
