@@ -297,6 +297,15 @@ int pla_conv_window_scatter_launch(
     int src_reqs, int src_steps, int dst_reqs, void* stream);
 
 /*
+ * The same rollback for `pools` (1..4) pools of one shape and element size in one launch; src, dst: `pools` base
+ * pointers each; strides: per pool src_s0..4, dst_s0..3.  Pools that a window is written to must not overlap.
+ */
+int pla_conv_windows_scatter_launch(
+    int elem_bytes, int km1, int pools, const void* const* src, void* const* dst, const int64_t* strides,
+    const void* dst_idx, int dst_idx_wide, const void* step_idx, int step_idx_wide,
+    int layers, int dim, int reqs, int src_reqs, int src_steps, int dst_reqs, void* stream);
+
+/*
  * Workspace size in bytes (256-byte aligned buffer) needed by pla_gdn_prefill_launch for T physical
  * tokens in N sequences.  Chunk metadata is sized for the worst case T/64 + N chunks so that no
  * host copy of cu_seqlens is needed.

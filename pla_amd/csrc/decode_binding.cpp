@@ -630,12 +630,32 @@ bool kda_ring_commit(const Tensor& temporal, const Tensor& rawv, const Tensor& r
       accepted.data_ptr<int32_t>(), nullptr, nullptr, temporal.stride(1), rawv.stride(1), rawk.stride(1), gk.stride(1), beta.stride(1),
       (int)layers, temporal.stride(0), rawv.stride(0), rawk.stride(0), gk.stride(0), beta.stride(0), (int)B, (int)H, (int)HV, (int)L,
       (int)null_block_id, dtype_code(act), stream));
-  for (size_t i = 0; i < conv.size(); ++i) {
-    const Tensor &dst = conv[i], &src = windows[i];
-    launched(pla_conv_window_scatter_launch(
-        (int)dst.element_size(), (int)dst.size(3), src.data_ptr(), dst.data_ptr(), indices.data_ptr(), wide(indices), last_step.data_ptr(),
-        wide(last_step), (int)dst.size(0), (int)dst.size(2), (int)B, src.stride(0), src.stride(1), src.stride(2), src.stride(3), src.stride(4),
-        dst.stride(0), dst.stride(1), dst.stride(2), dst.stride(3), (int)src.size(1), (int)src.size(2), (int)dst.size(1), stream));
+  // pools of one shape whose memory is disjoint roll back in one launch, others in one each
+  size_t together = conv.size() <= 4 ? conv.size() : 1;
+  for (size_t i = 0; i < together; ++i) {
+    bool same = conv[i].sizes() == conv[0].sizes() && windows[i].sizes() == windows[0].sizes() && conv[i].scalar_type() == conv[0].scalar_type();
+    for (size_t k = 0; k < conv.size() && same; ++k)
+      same = (k == i || !ByteSpan(conv[i]).meets(ByteSpan(conv[k]))) && !ByteSpan(conv[i]).meets(ByteSpan(windows[k]));
+    if (!same) {
+      together = 1;
+      break;
+    }
+  }
+  for (size_t first = 0; first < conv.size(); first += together) {
+    const void* src[4];
+    void* dst[4];
+    int64_t strides[4][9];
+    for (size_t x = 0; x < together; ++x) {
+      src[x] = windows[first + x].data_ptr();
+      dst[x] = conv[first + x].data_ptr();
+      for (int d = 0; d < 5; ++d) strides[x][d] = windows[first + x].stride(d);
+      for (int d = 0; d < 4; ++d) strides[x][5 + d] = conv[first + x].stride(d);
+    }
+    const Tensor &shape = conv[first], &rows = windows[first];
+    launched(pla_conv_windows_scatter_launch(
+        (int)shape.element_size(), (int)shape.size(3), (int)together, src, dst, strides[0], indices.data_ptr(), wide(indices),
+        last_step.data_ptr(), wide(last_step), (int)shape.size(0), (int)shape.size(2), (int)B, (int)rows.size(1), (int)rows.size(2),
+        (int)shape.size(1), stream));
   }
   return true;
 }

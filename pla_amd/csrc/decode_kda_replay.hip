@@ -386,22 +386,34 @@ __global__ __launch_bounds__(256, TMAX <= 4 ? 4 : 1) void kda_verify_dspark_kern
   }
 }
 
-// One thread per channel: copies the window of the selected step into the destination slot.
-template <typename T>
+// Windows of the selected steps into the destination slots, up to MAX_CONV_POOLS pools of one shape in a launch (the
+// grid's z index: pool x block of 256 threads).  DENSE: a window is one run of `items` 16-byte pieces on both sides,
+// copied by as many threads; otherwise one thread per channel copies its taps by stride.  Bound by launches and latency,
+// not by bytes: 64 requests x 4 layers of 4096 channels as three strided launches 3 x 8 us, as one dense launch 9 us.
+constexpr int MAX_CONV_POOLS = 4;
+struct ConvPools {
+  const void* src[MAX_CONV_POOLS]; void* dst[MAX_CONV_POOLS];
+  int64_t s[MAX_CONV_POOLS][5], d[MAX_CONV_POOLS][4];       // strides: layer, request, step, channel, tap; layer, slot, channel, tap
+};
+template <typename T, bool DENSE>
 __global__ __launch_bounds__(256) void conv_window_scatter_kernel(
-    const T* src, T* dst, const void* dst_idx, int dst_wide, const void* step_idx, int step_wide,
-    int dim, int km1, int64_t s_layer, int64_t s_req, int64_t s_step, int64_t s_dim, int64_t s_win,
-    int64_t d_layer, int64_t d_req, int64_t d_dim, int64_t d_win, int src_reqs, int src_steps, int dst_reqs) {
+    const ConvPools pools, const void* dst_idx, int dst_wide, const void* step_idx, int step_wide,
+    int items, int blocks, int km1, int src_reqs, int src_steps, int dst_reqs) {
   const int r = blockIdx.x;
   const int64_t layer = blockIdx.y;
+  const int x = blockIdx.z / blocks;
   const int64_t step = index_at(step_idx, step_wide, r);
   const int64_t d_i = index_at(dst_idx, dst_wide, r);
   if (step < 0 || d_i < 0 || d_i >= dst_reqs || r >= src_reqs || step >= src_steps) return;
-  const int d = blockIdx.z * 256 + threadIdx.x;
-  if (d >= dim) return;
-  const T* sp = src + layer * s_layer + (int64_t)r * s_req + step * s_step + (int64_t)d * s_dim;
-  T* dp = dst + layer * d_layer + d_i * d_req + (int64_t)d * d_dim;
-  for (int w = 0; w < km1; ++w) dp[w * d_win] = sp[w * s_win];
+  const int i = (blockIdx.z - x * blocks) * 256 + threadIdx.x;
+  if (i >= items) return;
+  const T* sp = static_cast<const T*>(pools.src[x]) + layer * pools.s[x][0] + (int64_t)r * pools.s[x][1] + step * pools.s[x][2];
+  T* dp = static_cast<T*>(pools.dst[x]) + layer * pools.d[x][0] + d_i * pools.d[x][1];
+  if constexpr (DENSE) {
+    reinterpret_cast<uint4*>(dp)[i] = reinterpret_cast<const uint4*>(sp)[i];
+  } else {
+    for (int w = 0; w < km1; ++w) dp[i * pools.d[x][2] + w * pools.d[x][3]] = sp[i * pools.s[x][3] + w * pools.s[x][4]];
+  }
 }
 
 // Conv windows of a commit plan into the paged conv histories of all layers: request r copies the window
@@ -550,6 +562,47 @@ extern "C" int pla_kda_replay_verify_native_launch(
   return launch_replay_verify(p, strides, Q, static_cast<hipStream_t>(stream));
 }
 
+extern "C" int pla_conv_windows_scatter_launch(
+    int elem_bytes, int km1, int pools, const void* const* src, void* const* dst, const int64_t* strides,
+    const void* dst_idx, int dst_idx_wide, const void* step_idx, int step_idx_wide,
+    int layers, int dim, int reqs, int src_reqs, int src_steps, int dst_reqs, void* stream) {
+  using namespace pla;
+  PLA_REQUIRE(elem_bytes == 2 || elem_bytes == 4, "conv scatter: element size must be 2 or 4 bytes, got %d", elem_bytes);
+  PLA_REQUIRE(km1 >= 1 && km1 <= 4, "conv scatter: unsupported conv window %d", km1);
+  PLA_REQUIRE(pools >= 1 && pools <= MAX_CONV_POOLS && src && dst && strides, "conv scatter: 1 to %d pools, got %d", MAX_CONV_POOLS, pools);
+  if (reqs == 0) return 0;
+  for (int x = 0; x < pools; ++x) PLA_REQUIRE(src[x] && dst[x], "null tensor pointer");
+  PLA_REQUIRE(dst_idx && step_idx, "null tensor pointer");
+  PLA_REQUIRE(layers > 0 && dim > 0 && reqs > 0 && layers <= 65535, "conv scatter: layers, dim and reqs must be positive");
+  // one run of 16-byte pieces per window: both sides channel-major or both tap-major without gaps, every window on a
+  // 16-byte boundary (all other layouts by channel)
+  ConvPools args{};
+  bool dense = (int64_t)dim * km1 * elem_bytes % 16 == 0;
+  for (int x = 0; x < pools; ++x) {
+    args.src[x] = src[x];
+    args.dst[x] = dst[x];
+    const int64_t* const s = strides + 9 * x;
+    const int64_t* const d = s + 5;
+    for (int i = 0; i < 5; ++i) args.s[x][i] = s[i];
+    for (int i = 0; i < 4; ++i) args.d[x][i] = d[i];
+    const bool channel_major = s[3] == km1 && s[4] == 1 && d[2] == km1 && d[3] == 1;
+    const bool tap_major = s[3] == 1 && s[4] == dim && d[2] == 1 && d[3] == dim;
+    dense = dense && (channel_major || tap_major) && aligned_at(src[x], 16) && aligned_at(dst[x], 16);
+    for (const int64_t pitch : {s[0], s[1], s[2], d[0], d[1]}) dense = dense && pitch * elem_bytes % 16 == 0;
+  }
+  const int items = dense ? (int)((int64_t)dim * km1 * elem_bytes / 16) : dim;
+  const int blocks = (items + 255) / 256;
+  PLA_REQUIRE((int64_t)blocks * pools <= 65535, "conv scatter: too many channels, got %d", dim);
+  const dim3 grid((unsigned)reqs, (unsigned)layers, (unsigned)(blocks * pools)), block(256);
+  auto run = [&](auto kernel) {
+    kernel<<<grid, block, 0, static_cast<hipStream_t>(stream)>>>(args, dst_idx, dst_idx_wide, step_idx, step_idx_wide, items, blocks, km1,
+                                                                 src_reqs, src_steps, dst_reqs);
+  };
+  if (elem_bytes == 2) dense ? run(conv_window_scatter_kernel<uint16_t, true>) : run(conv_window_scatter_kernel<uint16_t, false>);
+  else dense ? run(conv_window_scatter_kernel<uint32_t, true>) : run(conv_window_scatter_kernel<uint32_t, false>);
+  return check_launch("conv_window_scatter_kernel");
+}
+
 extern "C" int pla_conv_window_scatter_launch(
     int elem_bytes, int km1, const void* src, void* dst,
     const void* dst_idx, int dst_idx_wide, const void* step_idx, int step_idx_wide,
@@ -557,23 +610,9 @@ extern "C" int pla_conv_window_scatter_launch(
     int64_t src_s0, int64_t src_s1, int64_t src_s2, int64_t src_s3, int64_t src_s4,
     int64_t dst_s0, int64_t dst_s1, int64_t dst_s2, int64_t dst_s3,
     int src_reqs, int src_steps, int dst_reqs, void* stream) {
-  using namespace pla;
-  PLA_REQUIRE(elem_bytes == 2 || elem_bytes == 4, "conv scatter: element size must be 2 or 4 bytes, got %d", elem_bytes);
-  PLA_REQUIRE(km1 >= 1 && km1 <= 4, "conv scatter: unsupported conv window %d", km1);
-  if (reqs == 0) return 0;
-  PLA_REQUIRE(src && dst && dst_idx && step_idx, "null tensor pointer");
-  PLA_REQUIRE(layers > 0 && dim > 0 && reqs > 0 && layers <= 65535, "conv scatter: layers, dim and reqs must be positive");
-  const dim3 grid((unsigned)reqs, (unsigned)layers, (unsigned)((dim + 255) / 256)), block(256);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (elem_bytes == 2)
-    conv_window_scatter_kernel<uint16_t><<<grid, block, 0, s>>>(
-        (const uint16_t*)src, (uint16_t*)dst, dst_idx, dst_idx_wide, step_idx, step_idx_wide, dim, km1,
-        src_s0, src_s1, src_s2, src_s3, src_s4, dst_s0, dst_s1, dst_s2, dst_s3, src_reqs, src_steps, dst_reqs);
-  else
-    conv_window_scatter_kernel<uint32_t><<<grid, block, 0, s>>>(
-        (const uint32_t*)src, (uint32_t*)dst, dst_idx, dst_idx_wide, step_idx, step_idx_wide, dim, km1,
-        src_s0, src_s1, src_s2, src_s3, src_s4, dst_s0, dst_s1, dst_s2, dst_s3, src_reqs, src_steps, dst_reqs);
-  return check_launch("conv_window_scatter_kernel");
+  const int64_t strides[9] = {src_s0, src_s1, src_s2, src_s3, src_s4, dst_s0, dst_s1, dst_s2, dst_s3};
+  return pla_conv_windows_scatter_launch(elem_bytes, km1, 1, &src, &dst, strides, dst_idx, dst_idx_wide, step_idx, step_idx_wide, layers,
+                                         dim, reqs, src_reqs, src_steps, dst_reqs, stream);
 }
 
 extern "C" int pla_kda_conv_native_launch(

@@ -5,11 +5,13 @@ import types
 import pytest
 import torch
 
+from oracle import conv_window_scatter_reference
 from pla_amd.decode import _C, kda_replayssm_sglang as ring, kda_replayssm_vllm as paged
 from pla_amd.workloads import kda_replay_verify
 from test_replay_vllm_gpu import inputs, pages, records_filled, vector
 
 pytestmark = pytest.mark.gpu
+D = 128
 
 
 class _Counting:
@@ -72,3 +74,47 @@ def test_both_host_layers_leave_the_same_bits(monkeypatch, step, args, taken):
     torch.cuda.synchronize()
     for a, b in zip(got, want):
         assert torch.equal(a.cpu().view(torch.uint8) if a.is_contiguous() else a.cpu(), b.cpu().view(torch.uint8) if b.is_contiguous() else b.cpu())
+
+
+@pytest.mark.parametrize("layout", ["dense", "tap_major", "mixed", "interleaved", "shifted", "overlapping"])
+@pytest.mark.parametrize("heads,dtype,index_dtype", [(1, torch.bfloat16, torch.int32), (4, torch.bfloat16, torch.int64),
+                                                     (2, torch.float32, torch.int32)])
+def test_conv_rollback_of_three_pools(layout, heads, dtype, index_dtype):
+    """Pools that roll back in one launch of 16-byte pieces (dense, tap_major), in one launch by channel (mixed, shifted)
+    and in a launch each (interleaved, overlapping): every pool is the oracle's, bit for bit."""
+    layers, slots, rows, steps, dim = 2, 7, 5, 4, heads * D
+    g = torch.Generator().manual_seed(heads)
+
+    def filled(shape):
+        return torch.randn(*shape, generator=g).to(dtype).cuda()
+
+    if layout == "tap_major":
+        conv = [filled((layers, slots, 3, dim)).transpose(-1, -2) for _ in range(3)]
+    elif layout == "shifted":                            # bases off the 16-byte boundary
+        conv = [filled((layers * slots * dim * 3 + 1,))[1:].view(layers, slots, dim, 3) for _ in range(3)]
+    else:
+        conv = [filled((layers, slots, dim, 3)) for _ in range(3)]
+    if layout in ("tap_major", "mixed"):
+        windows = [filled((layers, rows, steps, 3, dim)).transpose(-1, -2) for _ in range(3)]
+    elif layout == "interleaved":                        # one tensor of all channels
+        windows = list(filled((layers, rows, steps, 3 * dim, 3)).split(dim, dim=3))
+    else:
+        windows = [filled((layers, rows, steps, dim, 3)) for _ in range(3)]
+    if layout == "overlapping":
+        conv[2] = conv[0]                                # the last pool's windows win
+    indices = torch.tensor([4, -1, 0, 6, 2], dtype=index_dtype)
+    last = torch.tensor([3, 2, -1, 0, 1], dtype=index_dtype)
+    want = [c.cpu().clone() for c in conv]
+    for i in range(3):
+        want[i] = conv_window_scatter_reference(want[i] if i < 2 or layout != "overlapping" else want[0], windows[i].cpu(), indices, last)
+    if layout == "overlapping":
+        want[0] = want[2]
+    state = torch.zeros(layers, slots, heads, D, D, device="cuda")
+    rec = torch.zeros(layers, slots, heads, 8, D, device="cuda")
+    spec = types.SimpleNamespace(temporal=state, replayssm_rawv=rec.bfloat16(), replayssm_rawk=rec.bfloat16(), replayssm_g=rec,
+                                 replayssm_beta=rec[..., 0].contiguous(), conv=conv, intermediate_conv_window=windows)
+    ring.commit_kda_replayssm_after_verify(spec_state=spec, state_batch_indices=indices.int().cuda(), accept_lens=last.int().cuda() + 1,
+                                           last_correct_step_indices=last.cuda())
+    torch.cuda.synchronize()
+    for c, expected in zip(conv, want):
+        assert torch.equal(c.cpu(), expected)
