@@ -582,7 +582,7 @@ __device__ __forceinline__ InlineSequences inline_sequences(const int32_t* cu_se
 // Chunk `index` of stage `stage` (all chunks in order when the call is not staged): its global chunk id, first token
 // and length, or id -1 when the stage holds fewer chunks.
 struct InlineTile { int cb, t0, len; };
-__device__ __forceinline__ InlineTile inline_tile(const InlineSequences& q, int stage, int index, int NC_max, int lane) {
+__device__ __forceinline__ InlineTile inline_tile(const InlineSequences& q, int stage, int index, int NC_max) {
   InlineTile t{-1, 0, 0};
   if (stage >= plan_stages(q.E)) return t;
   const int lo = stage_cut(q.nc, stage, q.E), hi = stage_cut(q.nc, stage + 1, q.E);

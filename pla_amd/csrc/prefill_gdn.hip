@@ -152,7 +152,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefill
   int cb, t0, len;
   if (p.inline_tables) {
     const InlineSequences seqs = inline_sequences(p.cu_seqlens, p.N, p.stg.stages, lane);
-    const InlineTile tile = inline_tile(seqs, p.stage, blockIdx.x / groups, p.NC_max, lane);
+    const InlineTile tile = inline_tile(seqs, p.stage, blockIdx.x / groups, p.NC_max);
     cb = tile.cb; t0 = tile.t0; len = tile.len;
     if (cb < 0) return;
   } else {

@@ -67,6 +67,8 @@ struct KdaPrefillParams {
   int pass;                                        // 0: whole sequences; 1, 2: the two sweeps over segments
   int stage;                                       // stage handled by this launch (prep kernel, passes 0 and 1)
   int H, NC_max;
+  int inline_tables;     // at most 64 sequences: kernels work the chunk tables out themselves (no table kernel)
+  int tail_blocks;       // workgroups appended to the preparation grid: segment tables, zeroing of the padded output rows
   // kda_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long) as
   // two halves, the others those of seq_order[n_long .. N) whole
   unsigned split_grid; int n_long;
@@ -121,11 +123,34 @@ __device__ __forceinline__ f32x4_t times4(const f32x4_t a, const f32x4_t b) {
 // fastest they read 256 bytes out of every row of the call).  Measured: 18 sequences of 121 to 999 tokens, 12 heads
 // 92 -> 85.6 us; 65 536 tokens, 32 heads 0.97-1.07 -> 0.88-0.91 ms (4.9 TB/s).
 __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillParams p) {
+  const int main_blocks = gridDim.x - p.tail_blocks;
+  if ((int)blockIdx.x >= main_blocks) {
+    // appended workgroups: the first of a call split into segments writes the tables its sweeps read, the others zero
+    // the padded rows of o
+    const int extra = blockIdx.x - main_blocks, builders = p.seg.seg_chunks > 0 ? 1 : 0;
+    if (extra < builders) {
+      chunk_map(p.cu_seqlens, p.N, p.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len);
+      __threadfence();
+      __syncthreads();
+      segment_map(p.seq_chunk_off, p.N, p.seg);
+    } else {
+      zero_tail(reinterpret_cast<uint16_t*>(p.o), p.cu_seqlens, p.N, p.T, p.H, extra - builders, p.tail_blocks - builders);
+    }
+    return;
+  }
   const int chunk = blockIdx.x / p.H, h = blockIdx.x - chunk * p.H;
-  const int cb = staged_chunk(p.stg, p.stage, chunk, p.seq_chunk_off[p.N]);
-  if (cb < 0) return;
-  const int t0 = p.chunk_tok[cb];
-  const int len = p.chunk_len[cb];
+  int cb, t0, len;
+  if (p.inline_tables) {
+    const InlineSequences seqs = inline_sequences(p.cu_seqlens, p.N, 0, threadIdx.x & 63);
+    const InlineTile t = inline_tile(seqs, 0, chunk, p.NC_max);
+    cb = t.cb; t0 = t.t0; len = t.len;
+    if (cb < 0) return;
+  } else {
+    cb = staged_chunk(p.stg, p.stage, chunk, p.seq_chunk_off[p.N]);
+    if (cb < 0) return;
+    t0 = p.chunk_tok[cb];
+    len = p.chunk_len[cb];
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kb = lane >> 4;
   const unsigned turn = blockIdx.x >> 3;             // the workgroup's place among those of its XCD
@@ -399,12 +424,30 @@ __device__ __forceinline__ void kda_sweep(const KdaPrefillParams& p, KdaSweepLds
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kb = lane >> 4;
   const int v_half = wide % HALVES;
+  // the chunks of the workgroup's sequence: worked out here (every wavefront for itself) or from the tables; segments are
+  // looked up in the segment table
+  int3 inline_chunks{-1, 0, 0};
+  int first_chunk = 0, first_token = 0, end_token = 0;
+  const bool inline_tables = p.inline_tables && p.pass == 0;
+  if (inline_tables) {
+    const InlineSequences seqs = inline_sequences(p.cu_seqlens, p.N, 0, lane);
+    const int n0 = __builtin_amdgcn_readfirstlane(wide / HALVES / p.H);
+    first_chunk = __builtin_amdgcn_readlane(seqs.off, n0);
+    first_token = __builtin_amdgcn_readlane(seqs.start, n0);
+    end_token = first_token + __builtin_amdgcn_readlane(seqs.len, n0);
+    inline_chunks = int3{first_chunk, min(first_chunk + __builtin_amdgcn_readlane(seqs.nc, n0), p.NC_max), seqs.E};
+  }
   const SweepRole role = select_sweep(p.pass, p.H, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
-                                      p.ht, p.ht_indices, p.ht_slot_stride, wide / HALVES);
+                                      p.ht, p.ht_indices, p.ht_slot_stride, wide / HALVES, inline_chunks);
   if (!role.active) return;
   const int n = role.n, h = role.head, c_begin = role.c_begin, c_end = role.c_end;
-  const int seq_start = p.cu_seqlens[n] + (c_begin - p.seq_chunk_off[n]) * CHUNK;
-  const int seq_len = min(p.cu_seqlens[n + 1] - seq_start, (c_end - c_begin) * CHUNK);
+  if (!inline_tables) {
+    first_chunk = p.seq_chunk_off[n];
+    first_token = p.cu_seqlens[n];
+    end_token = p.cu_seqlens[n + 1];
+  }
+  const int seq_start = first_token + (c_begin - first_chunk) * CHUNK;
+  const int seq_len = min(end_token - seq_start, (c_end - c_begin) * CHUNK);
   const int n_chunks = c_end - c_begin;
   auto chunk_len = [&](int c) { return min(CHUNK, seq_len - c * CHUNK); };
 
@@ -1180,11 +1223,16 @@ static int kda_prefill_run(
     p.stg.carry = segmented ? nullptr : reinterpret_cast<float*>(ws + L.carry);
     p.stg.stages = stages;
   }
-  launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.seg, p.stg,
-                segmented ? L.max_segments : N, o, H);
+  // At most 64 sequences: no table kernel runs ahead of the preparation (prefill_common.h), whose appended workgroups
+  // write the segment tables and zero the padded rows of o.
+  p.inline_tables = N <= INLINE_TABLE_SEQUENCES && stages == 0;
+  p.tail_blocks = p.inline_tables ? TABLE_WORKGROUPS - (segmented ? 0 : 1) : 0;
+  if (!p.inline_tables)
+    launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.seg, p.stg,
+                  segmented ? L.max_segments : N, o, H);
   const bool ok = launch_pipeline(
       s, stages, lease.get(), segmented, (unsigned)N * H, (unsigned)L.max_segments * H, &p.pass, &p.stage,
-      [&](hipStream_t ps) { hipLaunchKernelGGL(kda_prep_solve_kernel, dim3((unsigned)L.NC_max * H), dim3(256), 0, ps, p); },
+      [&](hipStream_t ps) { hipLaunchKernelGGL(kda_prep_solve_kernel, dim3((unsigned)L.NC_max * H + p.tail_blocks), dim3(256), 0, ps, p); },
       [&](unsigned grid) {
         // the first sweep over segments publishes no output: the lean variant, two workgroups per CU
         // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)

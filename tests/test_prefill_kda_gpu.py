@@ -466,3 +466,35 @@ def test_kda_prefill_correlated_keys_dense_triangular_system(lengths, noise):
     worst = max(rel_l2(final[n], exp_final[n]) for n in range(len(lengths)))
     print("KDA correlated keys", lengths, noise, "state rel-L2 %.3e" % worst)
     assert worst <= 1e-3, worst
+
+
+@pytest.mark.parametrize("longest,H", [(300, 1), (700, 5)])        # 64 chains (halves of a chain), 320 chains (longest first)
+@pytest.mark.parametrize("host_offsets", [False, True])
+def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, host_offsets):
+    """Calls of at most 64 sequences work their chunk tables out inside the kernels; with more sequences a table kernel
+    runs first.  64 ragged sequences (empty ones among them, a padded tail) against the oracle, then the same tokens with
+    one empty sequence appended must give the same bits."""
+    import random
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    rng = random.Random(longest)
+    lengths = [rng.choice((0, 1, 63, 64, 65, 130, longest // 3)) for _ in range(64)]
+    lengths[7], lengths[63] = longest, 77
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, longest, pad=9)
+    results = []
+    for extra in (0, 1):
+        offsets, start = offs + [offs[-1]] * extra, torch.cat([S0, S0[:extra]])
+        out = torch.full(v.shape, 7.0, dtype=torch.bfloat16, device="cuda")
+        final = torch.zeros_like(start).cuda()
+        flashkda_fwd(q.cuda(), k.cuda(), v.cuda(), raw.cuda(), beta.cuda(), A_log.cuda(), dt_bias.cuda(), out, scale=128 ** -0.5,
+                     lower_bound=-5.0, initial_state=start.cuda(), final_state=final,
+                     cu_seqlens=torch.tensor(offsets, dtype=torch.int32).cuda(), raw_cu_seqlens=tuple(offsets) if host_offsets else None)
+        torch.cuda.synchronize()
+        results.append((out, final[:64]))
+    want, want_final = _oracle(q, k, v, raw, beta, A_log, dt_bias, offs, S0, True)
+    total = offs[-1]
+    torch.testing.assert_close(results[0][0][:total].cpu().float(), want[:total].float(), atol=2e-2, rtol=2e-2)
+    assert torch.count_nonzero(results[0][0][total:]) == 0
+    assert rel_l2(results[0][1], want_final) <= 1e-3
+    for x, y in zip(*results):
+        nonempty = [n for n in range(64) if lengths[n]] if x.dim() == 4 else slice(None)
+        assert torch.equal(x[nonempty], y[nonempty])
