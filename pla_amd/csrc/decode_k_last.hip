@@ -601,6 +601,17 @@ struct FoldParams {
   const int64_t* layer_table;
 };
 
+// One token's record as it lies in memory: the lane's four channels of k and the log-decay, the wavefront's rows of v.
+template <int RPW>
+struct FoldRecord {
+  uint2 k; float4 g; uint32_t v[RPW / 2]; float beta;
+};
+
+// Bound by HBM on large commits and by the chain of tokens on small ones (8 or 16 rows per wavefront): a step is short
+// against a trip to memory, so there every token's record is requested one step ahead, the first one together with the
+// state tile (504 tiles, windows of eight tokens: 21.6 -> 20.4 us; what is left there are the vector instructions of the
+// row reductions).  With 32 rows that takes 142 registers, three wavefronts per SIMD instead of four, and the other
+// wavefronts cover the trips.
 template <typename act_t, int RPW>
 __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
   constexpr int R = RPW / 2;
@@ -643,8 +654,6 @@ __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
   }
   const Tile<float> h_tile(pool + (int64_t)slot * h0_slot_stride + (int64_t)i_hv * 16384);
   const int lane_off = ((rowbase + half) * 128 + 4 * c) * 4;
-  float s[R][4];
-  load_state<R>(h_tile, lane_off, s);
   const int64_t rec = p.records_by_request ? i_n : slot;
   const act_t* const kp = reinterpret_cast<const act_t*>(rawk) + layer * p.rawk_layer_stride + rec * p.rawk_slot_stride +
                           (int64_t)i_h * p.L * 128;
@@ -652,21 +661,38 @@ __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
                           (int64_t)i_hv * p.L * 128 + rowbase;
   const float* const gp = gk + layer * p.gk_layer_stride + rec * p.gk_slot_stride + (int64_t)i_hv * p.L * 128;
   const float* const bp = beta + layer * p.beta_layer_stride + rec * p.beta_slot_stride + (int64_t)i_hv * p.L;
+  auto request = [&](int t) {
+    FoldRecord<RPW> x;
+    x.k = *reinterpret_cast<const uint2*>(kp + t * 128 + 4 * c);
+    x.g = *reinterpret_cast<const float4*>(gp + t * 128 + 4 * c);
+    load_row_words<RPW>(vp + t * 128, x.v);
+    x.beta = bp[t];
+    return x;
+  };
+  constexpr bool AHEAD = RPW < 32;
+  FoldRecord<RPW> now, next;
+  if constexpr (AHEAD) next = request(0);
+  float s[R][4];
+  load_state<R>(h_tile, lane_off, s);
 
   for (int t = 0; t < n_acc; ++t) {
-    float kv[4], gv[4], dec[4], vv[R], unused[R];
-    load_k4(kp + t * 128, c, kv);
-    load_k4(gp + t * 128, c, gv);
-    uint32_t vw[R];
-    load_row_words<RPW>(vp + t * 128, vw);
-    row_scalars<act_t, RPW>(vw, half, vv);
+    if constexpr (AHEAD) {
+      now = next;
+      next = request(min(t + 1, n_acc - 1));
+    } else {
+      now = request(t);
+    }
+    float dec[4], vv[R], unused[R];
+    float kv[4] = {lo16<act_t>(now.k.x), hi16<act_t>(now.k.x), lo16<act_t>(now.k.y), hi16<act_t>(now.k.y)};
+    const float gv[4] = {now.g.x, now.g.y, now.g.z, now.g.w};
+    row_scalars<act_t, RPW>(now.v, half, vv);
     float ks = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ks = fmaf(kv[e], kv[e], ks);
     const float kn = 1.0f / sqrtf(row32_allreduce(ks) + 1e-6f);
 #pragma unroll
     for (int e = 0; e < 4; ++e) { kv[e] *= kn; dec[e] = __expf(gv[e]); }
-    delta_rows<R, true, false>(s, dec, 1.f, kv, kv, vv, bp[t], unused);
+    delta_rows<R, true, false>(s, dec, 1.f, kv, kv, vv, now.beta, unused);
     if (tracked && t == track_at)
       store_state<R>(Tile<float>(pool + (int64_t)track_slot * h0_slot_stride + (int64_t)i_hv * 16384), lane_off, s);
   }
