@@ -95,7 +95,6 @@ struct __align__(16) KdaPrepShared {
   };
   float B[CHUNK];
   float QI[CHUNK];         // 1 / |q_row|
-  float half_sum[128];     // per channel: sum of the gate over the first half of the rows
 };
 static_assert(sizeof(float[CHUNK][68]) <= sizeof(uint16_t[CHUNK][PITCH128]), "L must fit into Kn's storage");
 
@@ -114,10 +113,10 @@ __device__ __forceinline__ f32x4_t times4(const f32x4_t a, const f32x4_t b) {
 // Preparation of one (chunk, head).  What bounds it are its vector instructions (about 60 % of the SIMD cycles over the
 // launch, a further share in v_exp_f32; 12 wavefronts per CU by LDS), so the kernel counts them:
 //   G is kept in base 2 (scaled by log2 e where the gate is summed), so that a decay factor is one subtraction and
-//   one v_exp_f32; the gate's bound is applied in the scan's final addition; the masks of a chunk's missing rows are
+//   one v_exp_f32; the gate's bound is applied in the scan's additions; the masks of a chunk's missing rows are
 //   a branch that whole chunks skip; a thread owns the channels 32 s + 4 kb .. + 3 and the same + 16, both halves of one
-//   granule of the operand tiles, which it stores without an exchange; the scan runs over both halves of a chunk's rows
-//   in registers; the row blocks of phase 3 (1 to 4 blocks of work) rotate over the wavefronts.
+//   granule of the operand tiles, which it stores without an exchange; the scan runs over a chunk's rows in
+//   registers, the upper half after the lower; the row blocks of phase 3 (1 to 4 blocks of work) rotate over the wavefronts.
 // Where the call's tiles exceed the caches it is bound by memory (131 KiB read and written per tile), and the order of
 // the workgroups matters: heads vary fastest, so that the workgroups in flight read whole token rows (with the chunks
 // fastest they read 256 bytes out of every row of the call).  Measured: 18 sequences of 121 to 999 tokens, 12 heads
@@ -255,20 +254,24 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
   }
   __syncthreads();
   {
-    // inclusive sums per channel over the two halves of the rows, in registers; the second half starts from the first's sum
+    // Inclusive sums per channel, rows in registers, the upper half of the rows after the lower.  A chain of one fma a row:
+    // G_j - G_{j-1} is then off by one rounding of G_j.  Sums of the two halves formed side by side and scaled
+    // afterwards round both rows (and both sums) by themselves, two to three times that under strong decay.
     const float bound = p.lower_bound * LOG2E;
-    const int c = tid & 127, j0 = (CHUNK / 2) * (tid >> 7);
+    const int c = tid & 127;
+    const bool upper = wave >= 2;
+    float* const rows = &sh.G[upper ? CHUNK / 2 : 0][c];
     float x[CHUNK / 2];
 #pragma unroll
-    for (int j = 0; j < CHUNK / 2; ++j) x[j] = sh.G[j0 + j][c];
+    for (int j = 0; j < CHUNK / 2; ++j) x[j] = rows[j * 132];
+    auto scan = [&](float cum) {
 #pragma unroll
-    for (int j = 1; j < CHUNK / 2; ++j) x[j] += x[j - 1];
-    if (j0 == 0) sh.half_sum[c] = x[CHUNK / 2 - 1];
+      for (int j = 0; j < CHUNK / 2; ++j) rows[j * 132] = cum = fmaf(bound, x[j], cum);   // missing rows repeat G_last (their gate is zero)
+      return cum;
+    };
+    if (!upper) scan(0.f);
     __syncthreads();
-    const float base = j0 == 0 ? 0.f : bound * sh.half_sum[c];
-#pragma unroll
-    for (int j = 0; j < CHUNK / 2; ++j) sh.G[j0 + j][c] = fmaf(bound, x[j], base);   // missing rows repeat G_last (their gate is zero)
-    if (j0 != 0) p.eGlast[tile * 128 + c] = __builtin_amdgcn_exp2f(fmaf(bound, x[CHUNK / 2 - 1], base));
+    if (upper) p.eGlast[tile * 128 + c] = __builtin_amdgcn_exp2f(scan(sh.G[CHUNK / 2 - 1][c]));
   }
   __syncthreads();
 

@@ -498,3 +498,36 @@ def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, host_off
     for x, y in zip(*results):
         nonempty = [n for n in range(64) if lengths[n]] if x.dim() == 4 else slice(None)
         assert torch.equal(x[nonempty], y[nonempty])
+
+
+def test_kda_prefill_one_rounding_a_row_in_the_cumulative_decay():
+    """Sixty-two rows of the strongest decay, then a token with a value, then one that decays a little and writes nothing:
+    the final state is e^{g_last} k (x) beta v, and its error is that of G_last - G_{last - 1}.  |G| reaches 2^9 in base 2, so
+    one rounding of the cumulative decay a row leaves at most 2^-16 ln 2 = 1.06e-5; the 16-bit pairs, the reciprocal of
+    the gate and the norm add at most 5e-6.  With a rounding in either row, or in a sum scaled afterwards, some of the 1024
+    channels pass 1.6e-5."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    H, T = 8, 64
+    g = torch.Generator().manual_seed(5)
+    q, k = (torch.randn(T, H, 128, generator=g).bfloat16() for _ in range(2))
+    v = torch.zeros(T, H, 128, dtype=torch.bfloat16)
+    v[62] = 1.0 + torch.rand(H, 128, generator=g).bfloat16()
+    raw = (6.0 + torch.rand(T, H, 128, generator=g)).bfloat16()
+    raw[63] = (-4.0 + 0.5 * torch.randn(H, 128, generator=g)).bfloat16()
+    beta = torch.ones(T, H, dtype=torch.bfloat16)
+    beta[63] = -60.0                                     # sigmoid 1e-26
+    A_log, dt_bias = torch.zeros(H), torch.zeros(H, 128)
+    S0 = torch.zeros(1, H, 128, 128)
+    final = torch.empty_like(S0).cuda()
+    out = torch.empty_like(v).cuda()
+    flashkda_fwd(*(t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)), out, scale=128 ** -0.5, lower_bound=-5.0,
+                 initial_state=S0.cuda(), final_state=final, cu_seqlens=torch.tensor([0, T], dtype=torch.int32).cuda())
+    key = l2norm(k).to(k.dtype)[62].double() * torch.exp(-5.0 * torch.sigmoid(raw[63].double()))
+    value = torch.sigmoid(torch.ones((), dtype=torch.float64)) * v[62].double()
+    want = value[:, :, None] * key[:, None, :]
+    got = final[0].cpu().double()
+    heard = key.abs() > 0.02                             # the pairs are relative to the larger channels of a key
+    ratio = (got / want).mean(1)                         # over the 128 value rows, which share the factor
+    worst = (ratio - 1.0).abs()[heard].max().item()
+    print("cumulative decay: worst channel %.3e over %d channels" % (worst, int(heard.sum())))
+    assert worst <= 1.6e-5, worst
