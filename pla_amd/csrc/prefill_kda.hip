@@ -75,9 +75,11 @@ struct KdaPrefillParams {
   unsigned char seq_order[INLINE_TABLE_SEQUENCES];
 };
 
-// Operand tiles go out past the caches: the sweeps read them after the whole call's tiles were written.
-__device__ __forceinline__ void nt_store16(uint16_t* p, const uint4 v) {
-  __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t*>(p));
+// One 16-byte piece of an operand tile.  PAST_CACHES (tiles_past_caches): with the non-temporal hint.
+template <bool PAST_CACHES>
+__device__ __forceinline__ void store_tile16(uint16_t* p, const uint4 v) {
+  if constexpr (PAST_CACHES) __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4_t*>(p));
+  else *reinterpret_cast<uint4*>(p) = v;
 }
 
 constexpr float LOG2E = 1.4426950408889634f;
@@ -121,6 +123,7 @@ __device__ __forceinline__ f32x4_t times4(const f32x4_t a, const f32x4_t b) {
 // the workgroups matters: heads vary fastest, so that the workgroups in flight read whole token rows (with the chunks
 // fastest they read 256 bytes out of every row of the call).  Measured: 18 sequences of 121 to 999 tokens, 12 heads
 // 92 -> 85.6 us; 65 536 tokens, 32 heads 0.97-1.07 -> 0.88-0.91 ms (4.9 TB/s).
+template <bool PAST_CACHES>
 __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillParams p) {
   const int main_blocks = gridDim.x - p.tail_blocks;
   if ((int)blockIdx.x >= main_blocks) {
@@ -303,10 +306,10 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
       // holds channels 32 s + 4 kb .. + 3 and 32 s + 16 + 4 kb .. + 3, which are the thread's: one 16-byte store per
       // lane, whole rows per wavefront.
       const int64_t at = tile * 8192 + tile_offset(j, tid & 15), at2 = tile * 16384 + tile_offset(j, tid & 15);
-      nt_store16(p.Kg + at, make_uint4(kg[0], kg[1], kg[2], kg[3]));
-      nt_store16(p.Qg + at, make_uint4(qg[0], qg[1], qg[2], qg[3]));
-      nt_store16(p.Kt + at2, make_uint4(kt[0], kt[1], kt[2], kt[3]));
-      nt_store16(p.Kt + at2 + 8192, make_uint4(ktl[0], ktl[1], ktl[2], ktl[3]));
+      store_tile16<PAST_CACHES>(p.Kg + at, make_uint4(kg[0], kg[1], kg[2], kg[3]));
+      store_tile16<PAST_CACHES>(p.Qg + at, make_uint4(qg[0], qg[1], qg[2], qg[3]));
+      store_tile16<PAST_CACHES>(p.Kt + at2, make_uint4(kt[0], kt[1], kt[2], kt[3]));
+      store_tile16<PAST_CACHES>(p.Kt + at2 + 8192, make_uint4(ktl[0], ktl[1], ktl[2], ktl[3]));
     }
   }
 
@@ -1145,6 +1148,19 @@ extern "C" int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H) {
 // sequences of 32 810 tokens 0.997 / - / 0.948; twelve of 700 to 6000 tokens 0.757 / 0.712 / 0.676.
 constexpr double KDA_HALF_COST = 0.8, KDA_FILL_COST = 0.05;
 
+// Whether the preparation stores its operand tiles past the caches.  A call whose tiles stay in the 256 MB last-level cache
+// beside its inputs and outputs (64 KiB a tile more) sweeps them from there and loses by the hint, a larger one gains: the
+// tiles would push the inputs out and be gone themselves when the sweeps come to them.  us per call with / without the hint,
+// by MiB of tiles:
+//   41 (2 sequences, 950 tokens, 16 heads) 70.7 / 62.7      60 (6 of 270, 24 heads) 54.6 / 51.6      134 (4 of 768, 32 heads) 93.4 / 89.4
+//   151 (12 of 768, 12 heads) 115 / 112    168 (one of 4096, 32 heads) 192 / 185    175 (4 of 1024, 32 heads) 125 / 121-126
+//   197 (12 of 1024, 12 heads) 149.5 / 154.5    218 (18 of 740, 12 heads) 159.4 / 162.0    258 (4 of 1536, 32 heads) 178 / 183.5
+//   681 (8 of 2048, 32 heads) 445 / 458    2643 (one of 65 536, 32 heads) 2142 / 2167
+static bool tiles_past_caches(int NC_max, int H) {
+  constexpr int64_t tile_bytes = 4 * 16384 + 3 * TRI_BLOCKS * 1024 + 512;      // K e^G, scale Q e^G, the K e^{G_last-G} pair; W pair, P; e^{G_last}
+  return (int64_t)NC_max * H * tile_bytes > (int64_t)176 << 20;
+}
+
 static int kda_prefill_run(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
     int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_g, int64_t stride_beta,
@@ -1235,7 +1251,10 @@ static int kda_prefill_run(
                   segmented ? L.max_segments : N, o, H);
   const bool ok = launch_pipeline(
       s, stages, lease.get(), segmented, (unsigned)N * H, (unsigned)L.max_segments * H, &p.pass, &p.stage,
-      [&](hipStream_t ps) { hipLaunchKernelGGL(kda_prep_solve_kernel, dim3((unsigned)L.NC_max * H + p.tail_blocks), dim3(256), 0, ps, p); },
+      [&](hipStream_t ps) {
+        auto* const prepare = tiles_past_caches(L.NC_max, H) ? kda_prep_solve_kernel<true> : kda_prep_solve_kernel<false>;
+        hipLaunchKernelGGL(prepare, dim3((unsigned)L.NC_max * H + p.tail_blocks), dim3(256), 0, ps, p);
+      },
       [&](unsigned grid) {
         // the first sweep over segments publishes no output: the lean variant, two workgroups per CU
         // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)

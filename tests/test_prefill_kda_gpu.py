@@ -531,3 +531,24 @@ def test_kda_prefill_one_rounding_a_row_in_the_cumulative_decay():
     worst = (ratio - 1.0).abs()[heard].max().item()
     print("cumulative decay: worst channel %.3e over %d channels" % (worst, int(heard.sum())))
     assert worst <= 1.6e-5, worst
+
+
+def test_kda_prefill_same_bits_on_both_sides_of_the_store_rule():
+    """Twelve sequences of 12 heads hold 197 MiB of operand tiles, which are stored past the caches, six of them 99 MiB, which
+    are not: the same bits, sequence by sequence."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    lengths, H = [1024] * 5 + [1023, 1025] + [1024] * 5, 12
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = (t.cuda() if torch.is_tensor(t) else t for t in _inputs(lengths, H, 21))
+    whole, final = torch.empty_like(v), torch.empty_like(S0)
+
+    def call(first, end, out, state):
+        lo, hi = offs[first], offs[end]
+        flashkda_fwd(q[lo:hi], k[lo:hi], v[lo:hi], raw[lo:hi], beta[lo:hi], A_log, dt_bias, out, scale=128 ** -0.5, lower_bound=-5.0,
+                     initial_state=S0[first:end], final_state=state,
+                     cu_seqlens=torch.tensor([o - lo for o in offs[first:end + 1]], dtype=torch.int32).cuda())
+    call(0, 12, whole, final)
+    for first in (0, 6):
+        out, state = torch.empty_like(whole[offs[first]:offs[first + 6]]), torch.empty_like(final[:6])
+        call(first, first + 6, out, state)
+        assert torch.equal(out, whole[offs[first]:offs[first + 6]])
+        assert torch.equal(state, final[first:first + 6])
