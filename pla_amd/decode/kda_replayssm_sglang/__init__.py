@@ -68,6 +68,10 @@ def fold_accepted_prefix(temporal, rawv, rawk, gk, beta, state_batch_indices, ac
             raise RuntimeError("track indices and steps must have one entry per request")
     if not temporal[0, 0].is_contiguous():
         raise RuntimeError("temporal slots must be dense [HV, V, K]")
+    state_batch_indices, accept_lens = state_batch_indices.contiguous(), accept_lens.contiguous()
+    for t in (rawv, rawk, gk, beta, state_batch_indices, accept_lens, track_indices, track_steps):
+        if t is not None and t.device != temporal.device:
+            raise RuntimeError("fold tensors must share one device")
     stream = _lib.current_stream(temporal.device)
     act = _lib.dtype_code(rawk.dtype)
     if layers == 0 or B == 0:

@@ -194,3 +194,26 @@ def test_namespace_mirrors_the_reference_packages():
     a = importlib.import_module("pla_amd.decode.kda_mtp_sglang")
     b = importlib.import_module("pla_amd.decode.kda_replayssm_sglang")
     assert a.fused_kda_decode_mtp_dspark is b.fused_kda_decode_mtp_dspark
+
+
+def test_fold_reads_strided_index_vectors_and_refuses_another_device(monkeypatch):
+    """The kernel reads its index vectors as dense memory of the pool's device."""
+    from pla_amd import _lib
+    from pla_amd.decode.kda_replayssm_sglang import fold_accepted_prefix
+    seen = []
+    monkeypatch.setattr(_lib, "current_stream", lambda device: 0)
+    monkeypatch.setattr(_lib, "call", lambda name, *args: seen.append(
+        [list((ctypes.c_int32 * 3).from_address(args[i])) for i in (5, 6)]))
+    pool = torch.zeros(1, 4, 1, 128, 128)
+    rec = torch.zeros(1, 4, 1, 2, 128)
+    records = (rec.bfloat16(), rec.bfloat16(), rec, rec[..., 0].contiguous())
+    slots, lens = (torch.tensor(x, dtype=torch.int32)[::2] for x in ([3, 9, 1, 9, 2, 9], [2, 7, 1, 7, 2, 7]))
+    fold_accepted_prefix(pool, *records, slots, lens)
+    assert seen == [[[3, 1, 2], [2, 1, 2]]]
+    for elsewhere in range(6):                           # every tensor but the pool, one at a time
+        args = [t.to("meta") if i == elsewhere else t for i, t in enumerate((*records, slots, lens))]
+        with pytest.raises(RuntimeError, match="share one device"):
+            fold_accepted_prefix(pool, *args)
+    with pytest.raises(RuntimeError, match="share one device"):
+        fold_accepted_prefix(pool, *records, slots, lens, track_indices=slots.to("meta"), track_steps=lens)
+    assert len(seen) == 1
