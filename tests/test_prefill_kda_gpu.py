@@ -468,9 +468,11 @@ def test_kda_prefill_correlated_keys_dense_triangular_system(lengths, noise):
     assert worst <= 1e-3, worst
 
 
-@pytest.mark.parametrize("longest,H", [(300, 1), (700, 5)])        # 64 chains (halves of a chain), 320 chains (longest first)
+@pytest.mark.parametrize("longest,H,path", [(300, 1, "segments"),      # 64 chains: second sweep over one segment a sequence
+                                            (300, 2, "halves"),        # 128 chains: two workgroups a chain
+                                            (700, 5, "whole")])        # 320 chains: longest first with host offsets
 @pytest.mark.parametrize("host_offsets", [False, True])
-def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, host_offsets):
+def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, path, host_offsets):
     """Calls of at most 64 sequences work their chunk tables out inside the kernels; with more sequences a table kernel
     runs first.  64 ragged sequences (empty ones among them, a padded tail) against the oracle, then the same tokens with
     one empty sequence appended must give the same bits."""
@@ -479,6 +481,10 @@ def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, host_off
     rng = random.Random(longest)
     lengths = [rng.choice((0, 1, 63, 64, 65, 130, longest // 3)) for _ in range(64)]
     lengths[7], lengths[63] = longest, 77
+    # the rules of the call of 64 sequences (pick_segment_chunks and the choice of the sweep in prefill_kda.hip)
+    chains, chunks = 64 * H, (sum(lengths) + 9) // 64
+    segmented = chains <= 64 and 2 * max(16, -(-chunks * H // 256)) <= chunks
+    assert path == ("segments" if segmented else "halves" if chains <= 128 else "whole")
     q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, longest, pad=9)
     results = []
     for extra in (0, 1):
