@@ -63,9 +63,7 @@ struct KdaPrefillParams {
   uint16_t* P;                                     // [chunk, H, 6 blocks]: P in the same layout
   float* eGlast;                                   // [chunk, H, 128]: e^{G_last}
   SegmentTable seg;                                // split long sequences (seg.seg_chunks > 0)
-  StageTable stg;                                  // pipelined preparation and sweep (stg.stages > 0)
   int pass;                                        // 0: whole sequences; 1, 2: the two sweeps over segments
-  int stage;                                       // stage handled by this launch (prep kernel, passes 0 and 1)
   int H, NC_max;
   int inline_tables;     // at most 64 sequences: kernels work the chunk tables out themselves (no table kernel)
   int tail_blocks;       // workgroups appended to the preparation grid: segment tables, zeroing of the padded output rows
@@ -148,8 +146,8 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
     cb = t.cb; t0 = t.t0; len = t.len;
     if (cb < 0) return;
   } else {
-    cb = staged_chunk(p.stg, p.stage, chunk, p.seq_chunk_off[p.N]);
-    if (cb < 0) return;
+    if (chunk >= p.seq_chunk_off[p.N]) return;
+    cb = chunk;
     t0 = p.chunk_tok[cb];
     len = p.chunk_len[cb];
   }
@@ -443,7 +441,7 @@ __device__ __forceinline__ void kda_sweep(const KdaPrefillParams& p, KdaSweepLds
     end_token = first_token + __builtin_amdgcn_readlane(seqs.len, n0);
     inline_chunks = int3{first_chunk, min(first_chunk + __builtin_amdgcn_readlane(seqs.nc, n0), p.NC_max), seqs.E};
   }
-  const SweepRole role = select_sweep(p.pass, p.H, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
+  const SweepRole role = select_sweep(p.pass, p.H, p.N, p.seq_chunk_off, p.seg, StageTable{}, 0, p.h0, p.h0_indices, p.h0_slot_stride,
                                       p.ht, p.ht_indices, p.ht_slot_stride, wide / HALVES, inline_chunks);
   if (!role.active) return;
   const int n = role.n, h = role.head, c_begin = role.c_begin, c_end = role.c_end;
@@ -836,10 +834,10 @@ __global__ __launch_bounds__(512, 1) void kda_lean_sweep_kernel(const KdaPrefill
   const int vcol = 32 * cw + r16;
 
   // the two roles of this (segment, head): logical workgroups 2 i (zero state / real state) and 2 i + 1 (identity)
-  const SweepRole lead = select_sweep(1, p.H, p.N, p.seq_chunk_off, p.seg, p.stg, 0, p.h0, p.h0_indices, p.h0_slot_stride,
+  const SweepRole lead = select_sweep(1, p.H, p.N, p.seq_chunk_off, p.seg, StageTable{}, 0, p.h0, p.h0_indices, p.h0_slot_stride,
                                       p.ht, p.ht_indices, p.ht_slot_stride, 2 * (int)blockIdx.x);
   if (!lead.active) return;
-  const SweepRole mrole = select_sweep(1, p.H, p.N, p.seq_chunk_off, p.seg, p.stg, 0, p.h0, p.h0_indices, p.h0_slot_stride,
+  const SweepRole mrole = select_sweep(1, p.H, p.N, p.seq_chunk_off, p.seg, StageTable{}, 0, p.h0, p.h0_indices, p.h0_slot_stride,
                                        p.ht, p.ht_indices, p.ht_slot_stride, 2 * (int)blockIdx.x + 1);
   const SweepRole& role = m_side ? mrole : lead;
   const bool computing = role.active;                          // wave-uniform; false: wavefronts 4-7 of a first segment
@@ -1092,8 +1090,8 @@ __global__ __launch_bounds__(512, 1) void kda_lean_sweep_kernel(const KdaPrefill
 struct KdaWorkspaceLayout {
   size_t seq_chunk_off, chunk_seq, chunk_tok, chunk_len, Kg, Qg, Kt, W, P, eGlast;
   size_t seq_seg_off, seg_seq, seg_c0, seg_nc, segM, segB, segS, identity;
-  size_t order, stage_begin, carry, total;
-  int NC_max, seg_chunks, max_segments, stages;
+  size_t total;
+  int NC_max, seg_chunks, max_segments;
 };
 static KdaWorkspaceLayout kda_layout(int T, int N, int H) {
   KdaWorkspaceLayout L;
@@ -1118,16 +1116,6 @@ static KdaWorkspaceLayout kda_layout(int T, int N, int H) {
     const size_t states = (size_t)L.max_segments * H * 16384 * 4;
     L.segM = take(states); L.segB = take(states); L.segS = take(states);
     L.identity = take(16384 * 4);
-  }
-  // pipeline the preparation with the sweeps in stages where that pays
-  // Not staged: a sweep (104 KB of LDS) and a preparation workgroup (51 KB) fit a CU together and the staged call
-  // is correct (bit-identical per sequence), but the instruction-bound preparation slows the sweeps more than its
-  // overlap saves: 8 x 2048 tokens, 32 heads 0.50 -> 0.57 ms, 18 x 1100 tokens, 12 heads 0.24 -> 0.31 ms.
-  L.stages = 0;
-  if (L.stages > 0) {
-    L.order = take((size_t)L.NC_max * 4);
-    L.stage_begin = take((size_t)(MAX_STAGES + 2) * 4);
-    L.carry = L.seg_chunks > 0 ? 0 : take((size_t)N * H * 16384 * 4);
   }
   L.total = off;
   return L;
@@ -1223,9 +1211,9 @@ static int kda_prefill_run(
   }
   const bool v_halves = !segmented && (int64_t)N * H <= 128;
   // Ragged whole sequences whose offsets the host holds: the chains of the longest sequences run as two halves where
-  // that shortens the sweep (mixed_sweep_plan; the KDA path runs in one stage)
+  // that shortens the sweep (mixed_sweep_plan)
   bool mixed = false;
-  if (!segmented && !v_halves && raw_cu_seqlens != nullptr && N <= INLINE_TABLE_SEQUENCES && L.stages == 0) {
+  if (!segmented && !v_halves && raw_cu_seqlens != nullptr && N <= INLINE_TABLE_SEQUENCES) {
     int nc[INLINE_TABLE_SEQUENCES];
     for (int n = 0; n < N; ++n) nc[n] = (std::max(raw_cu_seqlens[n + 1] - raw_cu_seqlens[n], 0) + CHUNK - 1) / CHUNK;
     p.n_long = mixed_sweep_plan(nc, N, H, p.seq_order, KDA_HALF_COST, KDA_FILL_COST);
@@ -1234,48 +1222,40 @@ static int kda_prefill_run(
     mixed = p.n_long > 0 || (int64_t)N * H > CUS;
     p.split_grid = xcd_grouped_grid(2 * (unsigned)p.n_long * H, 2);
   }
-  const SideStreamLease lease(s, L.stages > 0);
-  const int stages = lease.get() != nullptr ? L.stages : 0;
-  if (stages > 0) {
-    p.stg.order = reinterpret_cast<int32_t*>(ws + L.order);
-    p.stg.stage_begin = reinterpret_cast<int32_t*>(ws + L.stage_begin);
-    p.stg.carry = segmented ? nullptr : reinterpret_cast<float*>(ws + L.carry);
-    p.stg.stages = stages;
-  }
   // At most 64 sequences: no table kernel runs ahead of the preparation (prefill_common.h), whose appended workgroups
   // write the segment tables and zero the padded rows of o.
-  p.inline_tables = N <= INLINE_TABLE_SEQUENCES && stages == 0;
+  p.inline_tables = N <= INLINE_TABLE_SEQUENCES;
   p.tail_blocks = p.inline_tables ? TABLE_WORKGROUPS - (segmented ? 0 : 1) : 0;
   if (!p.inline_tables)
-    launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.seg, p.stg,
-                  segmented ? L.max_segments : N, o, H);
-  const bool ok = launch_pipeline(
-      s, stages, lease.get(), segmented, (unsigned)N * H, (unsigned)L.max_segments * H, &p.pass, &p.stage,
-      [&](hipStream_t ps) {
-        auto* const prepare = tiles_past_caches(L.NC_max, H) ? kda_prep_solve_kernel<true> : kda_prep_solve_kernel<false>;
-        hipLaunchKernelGGL(prepare, dim3((unsigned)L.NC_max * H + p.tail_blocks), dim3(256), 0, ps, p);
-      },
-      [&](unsigned grid) {
-        // the first sweep over segments publishes no output: the lean variant, two workgroups per CU
-        // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)
-        if (p.pass == 1) hipLaunchKernelGGL(kda_lean_sweep_kernel, dim3(grid / 2), dim3(512), 0, s, p);
-        // Whole sequences that give at most 128 chains (few long ones are split into segments instead) leave half of the CUs idle: two
-        // workgroups then sweep a chain, 64 V columns each (the columns of V are independent: the same bits).
-        else if (mixed) hipLaunchKernelGGL(kda_sweep_mixed_kernel, dim3(p.split_grid + (unsigned)(N - p.n_long) * H), dim3(64 * (4 + KDA_SWEEP_COPIERS)), 0, s, p);
-        else if (v_halves) hipLaunchKernelGGL(kda_sweep_kernel<1>, dim3(xcd_grouped_grid(2 * grid, 2)), dim3(64 * (4 + KDA_SWEEP_COPIERS)), 0, s, p);
-        else hipLaunchKernelGGL(kda_sweep_kernel<2>, dim3(grid), dim3(64 * (4 + KDA_SWEEP_COPIERS)), 0, s, p);
-      });
-  PLA_REQUIRE(ok, "an event call of the staged prefill failed: %s", hipGetErrorString(hipGetLastError()));
+    launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.seg, StageTable{}, 0, o, H);
+  // Preparation, then the sweep, on one stream.  Not in stages as the GDN path: a sweep (104 KB of LDS) and a preparation
+  // workgroup (52 KB) fit a CU together, but the instruction-bound preparation slows the sweeps more than its overlap
+  // saves: 8 x 2048 tokens, 32 heads 0.50 -> 0.57 ms, 18 x 1100 tokens, 12 heads 0.24 -> 0.31 ms.
+  auto* const prepare = tiles_past_caches(L.NC_max, H) ? kda_prep_solve_kernel<true> : kda_prep_solve_kernel<false>;
+  hipLaunchKernelGGL(prepare, dim3((unsigned)L.NC_max * H + p.tail_blocks), dim3(256), 0, s, p);
+  const dim3 sweep_block(64 * (4 + KDA_SWEEP_COPIERS));
+  const unsigned chains = (unsigned)N * H, segment_chains = (unsigned)L.max_segments * H;
   if (segmented) {
-    hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid((unsigned)N * H * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, H,
+    // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)
+    p.pass = 1;
+    hipLaunchKernelGGL(kda_lean_sweep_kernel, dim3(segment_chains), dim3(512), 0, s, p);
+    hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, H,
                        N * H);
     p.pass = 2;
     // fewer (segment, head) pairs than half of the CUs (segments are at least 16 chunks long): two workgroups per pair
     // (an upper bound of their number from the token count alone: exact for a single sequence)
     if ((N == 1 ? ((T + CHUNK - 1) / CHUNK + L.seg_chunks - 1) / L.seg_chunks : (int64_t)(T / CHUNK + N) / L.seg_chunks + N) * H <= 128)
-      hipLaunchKernelGGL(kda_sweep_kernel<1>, dim3(xcd_grouped_grid(2 * (unsigned)L.max_segments * H, 2)), dim3(64 * (4 + KDA_SWEEP_COPIERS)), 0, s, p);
+      hipLaunchKernelGGL(kda_sweep_kernel<1>, dim3(xcd_grouped_grid(2 * segment_chains, 2)), sweep_block, 0, s, p);
     else
-      hipLaunchKernelGGL(kda_sweep_kernel<2>, dim3((unsigned)L.max_segments * H), dim3(64 * (4 + KDA_SWEEP_COPIERS)), 0, s, p);
+      hipLaunchKernelGGL(kda_sweep_kernel<2>, dim3(segment_chains), sweep_block, 0, s, p);
+  } else if (mixed) {
+    hipLaunchKernelGGL(kda_sweep_mixed_kernel, dim3(p.split_grid + (unsigned)(N - p.n_long) * H), sweep_block, 0, s, p);
+  } else if (v_halves) {
+    // Whole sequences that give at most 128 chains (few long ones are split into segments instead) leave half of the CUs idle: two
+    // workgroups then sweep a chain, 64 V columns each (the columns of V are independent: the same bits).
+    hipLaunchKernelGGL(kda_sweep_kernel<1>, dim3(xcd_grouped_grid(2 * chains, 2)), sweep_block, 0, s, p);
+  } else {
+    hipLaunchKernelGGL(kda_sweep_kernel<2>, dim3(chains), sweep_block, 0, s, p);
   }
   return check_launch("kda prefill launch");
 }
@@ -1311,7 +1291,7 @@ extern "C" int pla_kda_prefill_launch_raw(
 extern "C" int pla_kda_prefill_halved_sequences(const int32_t* raw_cu_seqlens, int N, int T, int H) {
   if (raw_cu_seqlens == nullptr || N <= 0 || N > INLINE_TABLE_SEQUENCES || T <= 0 || H <= 0) return 0;
   const KdaWorkspaceLayout L = kda_layout(T, N, H);
-  if (L.seg_chunks > 0 || L.stages > 0 || (int64_t)N * H <= 128) return 0;
+  if (L.seg_chunks > 0 || (int64_t)N * H <= 128) return 0;
   int nc[INLINE_TABLE_SEQUENCES];
   unsigned char order[INLINE_TABLE_SEQUENCES];
   for (int n = 0; n < N; ++n) nc[n] = (std::max(raw_cu_seqlens[n + 1] - raw_cu_seqlens[n], 0) + CHUNK - 1) / CHUNK;
