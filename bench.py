@@ -133,7 +133,7 @@ KDA_FLOP_PER_TOKEN = 5242880      # same with HV = H = 32 (one gram per head)
 # HBM bytes per call from rocprofv3 --pmc FETCH_SIZE (x2.00) and WRITE_SIZE (x1.00), summed over the kernels of
 # one call (profiles/gdn_prefill_kernels_32k.txt, profiles/kda_prefill_kernels_64k.txt)
 GDN_PREFILL_TRAFFIC_BYTES_PER_CALL = 1532000000
-KDA_PREFILL_TRAFFIC_BYTES_PER_CALL = 11129000000
+KDA_PREFILL_TRAFFIC_BYTES_PER_CALL = 10594000000
 
 
 def cpu_baseline_prefill(w):
@@ -650,7 +650,7 @@ def main():
         "ms_per_step": round(d["ms_per_step"], 5),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32", "data": "synthetic",
-        "config": {"workload": "configs[1]: GDN packed-QKV decode, 1 step, B=256 (243 active, 13 padded), "
+        "config": {"workload": "GDN packed-QKV decode, 1 step, B=256 (243 active, 13 padded), "
                                "H=16, HV=32, K=V=128, FP32 k-last pool of 4096 slots, bf16 activations",
                    "batch": 256, "n_active": d["n_active"], "pool_slots": 4096,
                    "slot_rotation": "16 disjoint slot sets, one per consecutive step"},

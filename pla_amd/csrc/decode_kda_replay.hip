@@ -72,8 +72,8 @@ __device__ __forceinline__ float conv_step(float (&taps)[3], float x, const floa
   return acc * fast_sigmoid(acc);
 }
 
-// (windows of up to four tokens: the compiler is held to 128 registers, four workgroups per CU instead of three - 124
-// without a spill, 42.3 -> 40.2 us for 64 requests of 32 heads; the eight-token kernel spills under that bound)
+// (windows of up to four tokens: the compiler is held to 128 registers, four workgroups per CU instead of three - 124,
+// with the fused norm 127, without a spill, 42.3 -> 40.2 us for 64 requests of 32 heads; the eight-token kernel spills under that bound)
 template <int TMAX, bool ONORM>
 __global__ __launch_bounds__(256, TMAX <= 4 ? 4 : 1) void kda_verify_dspark_kernel(const ReplayVerifyParams p) {
   const int tid = threadIdx.x;

@@ -17,7 +17,7 @@
 // FLA kernels (scripts/prefill/private/ref/chunk_intra.py:170-202); those operands are split into
 // bf16 hi + lo parts (bf16 has the range, the pair the precision).  The operands of the sequential
 // sweep (k e^{G}, q e^{G}, k e^{G_last - G}, W, P, S, X, U) all carry factors in (0, 1] and go to the
-// MFMA as fp16, rounded once.
+// MFMA as fp16, rounded once or (W, k e^{G_last - G}, U) as hi + lo pairs.
 //
 // Kernels:
 //   kda_prep_solve_kernel   one workgroup per (chunk, head): q/k L2 norm (rounded to bf16), lower-bound
@@ -110,17 +110,19 @@ __device__ __forceinline__ f32x4_t times4(const f32x4_t a, const f32x4_t b) {
   return f32x4_t{a[0] * b[0], a[1] * b[1], a[2] * b[2], a[3] * b[3]};
 }
 
-// Preparation of one (chunk, head).  What bounds it are its vector instructions (about 60 % of the SIMD cycles over the
-// launch, a further share in v_exp_f32; 12 wavefronts per CU by LDS), so the kernel counts them:
+// Preparation of one (chunk, head).  What bounds it are its vector instructions (10.4 k per workgroup; over 18 sequences of 121
+// to 999 tokens and 12 heads the SIMDs issue them in 54 % of the cycles, over 65 536 tokens and 32 heads in 74 %; 12 wavefronts
+// per CU by LDS), so the kernel counts them:
 //   G is kept in base 2 (scaled by log2 e where the gate is summed), so that a decay factor is one subtraction and
 //   one v_exp_f32; the gate's bound is applied in the scan's additions; the masks of a chunk's missing rows are
 //   a branch that whole chunks skip; a thread owns the channels 32 s + 4 kb .. + 3 and the same + 16, both halves of one
 //   granule of the operand tiles, which it stores without an exchange; the scan runs over a chunk's rows in
-//   registers, the upper half after the lower; the row blocks of phase 3 (1 to 4 blocks of work) rotate over the wavefronts.
-// Where the call's tiles exceed the caches it is bound by memory (131 KiB read and written per tile), and the order of
+//   registers, the upper half after the lower; the row blocks of phase 3 (1 to 4 blocks of work) rotate over the wavefronts
+//   (8 x 2048 tokens, 32 heads 446.8 -> 444.5 us a call).
+// Where the call's tiles exceed the caches its bytes take as long (131 KiB read and written per tile), and the order of
 // the workgroups matters: heads vary fastest, so that the workgroups in flight read whole token rows (with the chunks
-// fastest they read 256 bytes out of every row of the call).  Measured: 18 sequences of 121 to 999 tokens, 12 heads
-// 92 -> 85.6 us; 65 536 tokens, 32 heads 0.97-1.07 -> 0.88-0.91 ms (4.9 TB/s).
+// fastest they read 256 bytes out of every row of the call: 18 sequences 164.2 -> 159.2 us a call, one of 512 tokens, 32 heads
+// 49.3 -> 42.9).  All together: 18 sequences 92 -> 84-86 us, 65 536 tokens 0.97-1.07 -> 0.87-0.93 ms (4.7-5.0 TB/s).
 template <bool PAST_CACHES>
 __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillParams p) {
   const int main_blocks = gridDim.x - p.tail_blocks;
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(256) void kda_prep_solve_kernel(const KdaPrefillPar
     }
   }
 
-  // ---- phase 3: M and P, wavefront w owns row block w (reference row = first row of the block) --
+  // ---- phase 3: M and P, one row block per wavefront (bi; reference row = first row of the block) --
   {
     const float* const R = &sh.G[16 * bi][0];
     const int i_row = 16 * bi + r16;
