@@ -404,7 +404,7 @@ int pla_gdn_prefill_launch_static(
 int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H);
 
 /*
- * KDA chunk-64 prefill over packed variable-length sequences (per-channel lower-bound gate).
+ * KDA prefill over packed variable-length sequences, sub-chunks of 16 tokens (per-channel lower-bound gate).
  * Replaces _C.flashkda_fwd (pla/prefill/flashkdapro/ops.py:215-219) and the tc01 FLA stage
  * launchers fla_runtime::Launchers (src/prefill/flashkdapro/tc01/fla/launchers.h:38-78).
  *

@@ -32,10 +32,6 @@ __device__ __forceinline__ HiLo split8(f32x4_t a, f32x4_t b) {
   r.lo = __builtin_convertvector(x - back, bf16x8_t);
   return r;
 }
-__device__ __forceinline__ bf16x8_t round8(f32x4_t a, f32x4_t b) {
-  const f32x8_t x = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  return __builtin_convertvector(x, bf16x8_t);
-}
 
 // The same instruction shape with fp16 operands (v_mfma_f32_16x16x32_f16, same rate).  Operands travel as
 // eight 16-bit lanes in a bf16x8_t container (loads, LDS reads and transposing reads do not care what the

@@ -1,5 +1,5 @@
-// Pieces shared by the GDN and KDA chunk-64 prefill kernels: MFMA wrappers, bf16 hi/lo
-// splitting, operand access for v_mfma_f32_16x16x32_bf16 and the device-side chunk table.
+// Pieces of the GDN chunk-64 prefill kernels, some of them shared with KDA's: operand tiles, asynchronous copies, the
+// device-side chunk tables, the split of long sequences, the plans made on the host.
 #pragma once
 
 #include <mutex>
@@ -20,104 +20,6 @@ __device__ __forceinline__ uint2 read_tr4(const uint16_t* at) {
   return __builtin_bit_cast(uint2, v);
 }
 
-// Element r (0..3) of what read_tr4 returned, as FP32.
-template <typename T> __device__ __forceinline__ float quad_element(uint2 w, int r) {
-  const uint32_t pair = r < 2 ? w.x : w.y;
-  return (r & 1) ? hi16<T>(pair) : lo16<T>(pair);
-}
-
-// Pitch of a padded 128-wide LDS tile (16-bit elements): rows stay 16-byte aligned and consecutive rows start 4 banks
-// apart, which keeps the 8-byte reads of a wavefront conflict free.
-constexpr int PITCH128 = 136;
-
-// ---------------------------------------------------------------------------------------------
-// W = (I + L)^-1 diag(beta) for a strictly lower triangular 64 x 64 L (FP32, in LDS) on ONE wavefront, by
-// 16 x 16 blocks with the off-diagonal blocks on MFMA.  With N = (I + L)^-1: the diagonal blocks D_a = (I + L_aa)^-1 come from forward substitution over 16 rows
-// (lane 16 a + j owns column j of D_a), the others from N_ab = -D_a sum_{b <= c < a} L_ac N_cb in order of
-// a - b = 1, 2, 3 (13 products of 16 x 16 x 16 or 16 x 16 x 32).  FP32 values cross the MFMA as bf16
-// hi/lo pairs (hi.hi + hi.lo + lo.hi, error ~2^-16 per product).  L is used as workspace: D_a replaces
-// L_aa, D_b^T is parked in the unused block (b, b + 1) where lanes read it as a B operand, N_ab replaces
-// L_ab, and the fp16 tile leaves in 16-byte pieces (8 rows of 128 bytes per store instruction).  Only the
-// strictly lower triangle of L is read.
-__device__ __forceinline__ f32x4_t mfma_hilo(const HiLo& a, const HiLo& b, f32x4_t c) {
-  c = mfma16(a.lo, b.hi, c);
-  c = mfma16(a.hi, b.lo, c);
-  return mfma16(a.hi, b.hi, c);
-}
-
-// block_inverse_inplace leaves N = (I + L)^-1 in the lower triangle of L (the blocks above the diagonal hold
-// scratch); the two functions after it scale by beta and store W in one of two layouts.
-__device__ __forceinline__ void block_inverse_inplace(float (*L)[68], int lane) {
-  const int r16 = lane & 15, kb = lane >> 4;
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  {
-    // diagonal blocks: x_i = [i == j] - sum_{l < i} L_aa[i][l] x_l
-    const int a = kb, j = r16;
-    float x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-      for (int l4 = 0; l4 < i; l4 += 4) {
-        const float4 row = *reinterpret_cast<const float4*>(&L[16 * a + i][16 * a + l4]);
-        acc0 = fmaf(row.x, x[l4], acc0);
-        if (l4 + 1 < i) acc1 = fmaf(row.y, x[l4 + 1], acc1);
-        if (l4 + 2 < i) acc0 = fmaf(row.z, x[l4 + 2], acc0);
-        if (l4 + 3 < i) acc1 = fmaf(row.w, x[l4 + 3], acc1);
-      }
-      x[i] = (i == j ? 1.f : 0.f) - (acc0 + acc1);
-    }
-    // all reads of L_aa are done (one wavefront, LDS operations complete in order)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) L[16 * a + i][16 * a + j] = x[i];
-    if (a < 3) {
-#pragma unroll
-      for (int i4 = 0; i4 < 16; i4 += 4)
-        *reinterpret_cast<float4*>(&L[16 * a + j][16 * (a + 1) + i4]) = make_float4(x[i4], x[i4 + 1], x[i4 + 2], x[i4 + 3]);
-    }
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  // operands: A = rows of L (blocks c0 and, if c1 >= 0, c1 of block row a); lane (m, kb) holds columns 4 kb .. 4 kb + 3 of each
-  auto quad = [&](int row, int col) {
-    const float4 t = *reinterpret_cast<const float4*>(&L[row][col]);
-    return f32x4_t{t.x, t.y, t.z, t.w};
-  };
-  auto a_rows = [&](int a, int c0, int c1) {
-    return split8(quad(16 * a + r16, 16 * c0 + 4 * kb), c1 >= 0 ? quad(16 * a + r16, 16 * c1 + 4 * kb) : zero);
-  };
-  auto negate = [](f32x4_t t) { return f32x4_t{-t.x, -t.y, -t.z, -t.w}; };
-  // D_b as a B operand half: rows 4 kb .. 4 kb + 3 of column r16, read from the transposed copy
-  const f32x4_t D0 = quad(r16, 16 + 4 * kb), D1 = quad(16 + r16, 32 + 4 * kb), D2 = quad(32 + r16, 48 + 4 * kb);
-  const HiLo AD1 = a_rows(1, 1, -1), AD2 = a_rows(2, 2, -1), AD3 = a_rows(3, 3, -1);
-  const HiLo A32 = a_rows(3, 2, -1);
-  // a - b = 1
-  const f32x4_t Y10 = mfma_hilo(a_rows(1, 0, -1), split8(D0, zero), zero);
-  const f32x4_t Y21 = mfma_hilo(a_rows(2, 1, -1), split8(D1, zero), zero);
-  const f32x4_t Y32 = mfma_hilo(A32, split8(D2, zero), zero);
-  const f32x4_t X10 = negate(mfma_hilo(AD1, split8(Y10, zero), zero));
-  const f32x4_t X21 = negate(mfma_hilo(AD2, split8(Y21, zero), zero));
-  const f32x4_t X32 = negate(mfma_hilo(AD3, split8(Y32, zero), zero));
-  // a - b = 2
-  const HiLo B0 = split8(D0, X10);                        // [D_0; N_10], shared by N_20 and N_30
-  const f32x4_t Y20 = mfma_hilo(a_rows(2, 0, 1), B0, zero);
-  const f32x4_t Y31 = mfma_hilo(a_rows(3, 1, 2), split8(D1, X21), zero);
-  const f32x4_t X20 = negate(mfma_hilo(AD2, split8(Y20, zero), zero));
-  const f32x4_t X31 = negate(mfma_hilo(AD3, split8(Y31, zero), zero));
-  // a - b = 3
-  f32x4_t Y30 = mfma_hilo(a_rows(3, 0, 1), B0, zero);
-  Y30 = mfma_hilo(A32, split8(X20, zero), Y30);
-  const f32x4_t X30 = negate(mfma_hilo(AD3, split8(Y30, zero), zero));
-  // N_ab replaces L_ab (accumulator layout: lane (n, kb) holds rows 4 kb + r of column n)
-  auto put = [&](int a, int b, f32x4_t t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) L[16 * a + 4 * kb + r][16 * b + r16] = t[r];
-  };
-  put(1, 0, X10); put(2, 1, X21); put(3, 2, X32); put(2, 0, X20); put(3, 1, X31); put(3, 0, X30);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // A lower triangular 64 x 64 tile as the A (or B) operands of the products that contract over its columns: only six
 // of the eight 16 x 32 operand blocks hold anything (row block m, column half s: s = 0 for every m, s = 1 for
 // m = 2, 3).  Block b is 1 KiB: lane (r, kb) owns 16 bytes, columns 32 s + 4 kb .. + 3 and 32 s + 16 + 4 kb .. + 3 of
@@ -126,34 +28,10 @@ __device__ __forceinline__ void block_inverse_inplace(float (*L)[68], int lane) 
 constexpr int TRI_BLOCKS = 6;
 __device__ __forceinline__ constexpr int tri_block_m(int b) { return b < 4 ? b : b - 2; }
 __device__ __forceinline__ constexpr int tri_block_s(int b) { return b < 4 ? 0 : 1; }
-// W = N diag(beta) from the tile block_inverse_inplace leaves, as an fp16 hi + lo pair in that layout: hi blocks at
-// W, lo blocks at W + TRI_BLOCKS * 512 (halves).
-__device__ __forceinline__ void store_w_operand_blocks(float (*L)[68], const float* beta, int lane, uint16_t* W) {
-  const int r16 = lane & 15, kb = lane >> 4;
-#pragma unroll
-  for (int b = 0; b < TRI_BLOCKS; ++b) {
-    const int i = 16 * tri_block_m(b) + r16;
-    uint32_t hi[4], lo[4];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int j0 = 32 * tri_block_s(b) + 16 * half + 4 * kb;
-      const float4 n4 = *reinterpret_cast<const float4*>(&L[i][j0]);
-      const float4 b4 = *reinterpret_cast<const float4*>(&beta[j0]);
-      const float w0 = j0 <= i ? n4.x * b4.x : 0.f, w1 = j0 + 1 <= i ? n4.y * b4.y : 0.f;
-      const float w2 = j0 + 2 <= i ? n4.z * b4.z : 0.f, w3 = j0 + 3 <= i ? n4.w * b4.w : 0.f;
-      pack2_pair(w0, w1, hi[2 * half], lo[2 * half]);
-      pack2_pair(w2, w3, hi[2 * half + 1], lo[2 * half + 1]);
-    }
-    *reinterpret_cast<uint4*>(W + b * 512 + lane * 8) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-    *reinterpret_cast<uint4*>(W + (TRI_BLOCKS + b) * 512 + lane * 8) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-  }
-}
 
 // ---------------------------------------------------------------------------------------------
 // Asynchronous global -> LDS tile copies (global_load_lds_dwordx4: no registers, no LDS store
-// instructions).  Lane i of a wavefront writes its 16 bytes at (wave-uniform LDS base) + 16 i, so
-// a padded tile is filled as linear memory in 1 KiB pieces; a lane whose slot falls into a row's
-// padding re-reads the last 16 data bytes of that row (the padding is never read back).
+// instructions).  Lane i of a wavefront writes its 16 bytes at (wave-uniform LDS base) + 16 i.
 //
 // The copy is issued from inline assembly so that the compiler's wait-count bookkeeping does not
 // see it (it would drain every outstanding copy before each LDS read).  Kernels wait by hand with
@@ -186,45 +64,6 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ uint32_t lds_address(const void* ptr) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)ptr;
 }
-
-// Copy plan for one padded LDS tile: ROWS rows of PITCH_B bytes whose first VALID_B bytes are data,
-// filled from rows `row_pitch_b` apart in global memory by the WAVES wavefronts of a workgroup.
-// Each wavefront issues PIECES / WAVES copies, wavefront 0 also the PIECES % WAVES left over, so the copy
-// counts per wavefront are compile-time constants (EACH, FIRST).  The per-lane source offsets are
-// computed once; rows beyond `last_row` re-read that row.
-template <int ROWS, int PITCH_B, int VALID_B, int WAVES>
-struct TileCopy {
-  static constexpr int BYTES = ROWS * PITCH_B;
-  static_assert(BYTES % 1024 == 0 && PITCH_B % 16 == 0 && VALID_B % 16 == 0, "tiles are filled in 1 KiB pieces");
-  static constexpr int PIECES = BYTES / 1024;
-  static constexpr int EACH = PIECES / WAVES;
-  static constexpr int REST = PIECES % WAVES;
-  static constexpr int FIRST = EACH + REST;
-  uint32_t off[EACH > 0 ? EACH : 1];
-  uint32_t off_rest[REST > 0 ? REST : 1];
-
-  static __device__ __forceinline__ uint32_t source_offset(int piece, int lane, uint32_t row_pitch_b, int last_row) {
-    const int at = 1024 * piece + 16 * lane;
-    const int row = at / PITCH_B, cb = at - row * PITCH_B;
-    return (uint32_t)min(row, last_row) * row_pitch_b + (uint32_t)min(cb, VALID_B - 16);
-  }
-  __device__ __forceinline__ void plan(uint32_t row_pitch_b, int last_row, int wave, int lane) {
-#pragma unroll
-    for (int j0 = 0; j0 < EACH; ++j0) off[j0] = source_offset(WAVES * j0 + wave, lane, row_pitch_b, last_row);
-#pragma unroll
-    for (int j = 0; j < REST; ++j) off_rest[j] = source_offset(WAVES * EACH + j, lane, row_pitch_b, last_row);
-  }
-  // `gbase` (wave-uniform) addresses row 0 of the source tile.
-  __device__ __forceinline__ void issue(const void* tile, const char* gbase, int wave) const {
-    const uint32_t base = lds_address(tile) + 1024u * wave;
-#pragma unroll
-    for (int j0 = 0; j0 < EACH; ++j0) dma16(gbase, off[j0], base + 1024u * WAVES * j0);
-    if (wave == 0) {
-#pragma unroll
-      for (int j = 0; j < REST; ++j) dma16(gbase, off_rest[j], base + 1024u * (WAVES * EACH + j));
-    }
-  }
-};
 
 // ---------------------------------------------------------------------------------------------
 // Unpadded, swizzled 64 x 128 tiles of 16-bit values (16 KiB).  A row is sixteen 16-byte granules; granule g of row i
@@ -643,17 +482,20 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 // M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes), all 64 loads of a step requested before
 // the first product.
 constexpr int COMBINE_SPLIT = 8;
-static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, int heads, int chains) {
+static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int heads) {
   // the eight workgroups of a chain read the same M tiles: on one XCD they come from memory once (xcd_grouped_index)
-  const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, chains * COMBINE_SPLIT);
+  const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, N * heads * COMBINE_SPLIT);
   if (logical < 0) return;
   const int part = logical % COMBINE_SPLIT;
   const int chain = logical / COMBINE_SPLIT;
   const int n = chain / heads, h = chain - n * heads;
-  const int first = t.seq_seg_off[n], end = t.seq_seg_off[n + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // the sequence's segments, counted by every wavefront for itself (split calls have at most 64 sequences)
+  const int nc = (lane < N ? max(cu_seqlens[lane + 1] - cu_seqlens[lane], 0) : 0) + CHUNK - 1;
+  const int ns = (nc / CHUNK + t.seg_chunks - 1) / t.seg_chunks, before = wave_inclusive_scan(ns) - ns;
+  const int first = __builtin_amdgcn_readlane(before, n), end = first + __builtin_amdgcn_readlane(ns, n);
   if (end - first < 2) return;                 // a single segment starts from the caller's state
   __shared__ __align__(16) float S[16][132];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, kb = lane >> 4;
   const int col0 = 32 * wave + c;              // this lane's column of accumulator tile 0 (tile 1: + 16)
   // place of accumulator element (tile cb, row v) inside a [128, 128] tile

@@ -1,0 +1,259 @@
+// Pieces of the one-pass prefill sweeps over sub-chunks of 16 tokens: the operand layouts that producing and computing
+// wavefronts share through LDS, the inverse of a 16 x 16 unit triangle, the token range of a chain.
+//
+// Layout.  A token row of 128 channels is a row operand of the 16x16x32 MFMA in four contraction steps: lane (t, g) =
+// (lane % 16, lane / 16) holds channels 32 s + 8 g .. + 7 of token t, one 16-byte piece a step, which is also how the
+// rows lie in memory.  The state follows that order: accumulator block b = 2 s + h of S^T holds channel
+// 32 s + 8 (rho / 4) + 4 h + rho % 4 in row rho, so that blocks 2 s and 2 s + 1 of a lane, side by side, are its column
+// operand of step s.
+//   row tile      4 KiB, the pieces in the order (s, lane): written and read 16 bytes per lane at consecutive addresses
+//   turned tile   the same with token t ^ 4 g in the place of t: read through the transposing LDS read (tokens as
+//                 contraction), which then touches every bank once
+// Products go to the 16x16x32 MFMA alone.  (An accumulator that v_mfma_f32_16x16x16_f16 had written and 16x16x32 read one or two
+// instructions later was seen to lack the first product in half of its registers, depending on what else ran: the compiler
+// puts no wait between the two.)
+//   W             16 bytes per lane (i, g): W[i][4 g .. + 3] as fp16, hi then lo; against [X, X] one MFMA multiplies both
+//   P             8 bytes per lane (i, g): P[i][4 g .. + 3] as fp16
+#pragma once
+
+#include "prefill_common.h"
+
+namespace pla {
+
+constexpr int SUB = 16;                          // tokens of a sub-chunk
+
+__device__ __forceinline__ bf16x8_t pair_of(uint2 a, uint2 b) { return __builtin_bit_cast(bf16x8_t, make_uint4(a.x, a.y, b.x, b.y)); }
+__device__ __forceinline__ bf16x8_t lds_granule(const char* at) { return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(at)); }
+__device__ __forceinline__ uint2 lds_turned(const char* at) { return read_tr4(reinterpret_cast<const uint16_t*>(at)); }
+
+// Bytes from the start of a turned tile to what lane `lane` addresses for block (s = 0, h = 0); block (s, h): + 1024 s + 8 h.
+// Lane i of a group of sixteen addresses columns 4 (i % 4) .. + 3 of row i / 4 (read_tr4).
+__device__ __forceinline__ int turned_offset(int lane) {
+  const int g = lane >> 4, row = 4 * g + ((lane >> 2) & 3), quad = lane & 3;
+  return 16 * (16 * quad + (row ^ (4 * quad)));
+}
+// The place of lane (t, g)'s piece in a turned tile (step s: + 1024 s).
+__device__ __forceinline__ int turned_piece(int lane) {
+  const int t = lane & 15, g = lane >> 4;
+  return 16 * (16 * g + (t ^ (4 * g)));
+}
+
+// c + the products of two packed pairs (v_dot2_f32_bf16: exact products, FP32 sum).
+__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+}
+
+// Eight FP32 values as a bf16 pair each: hi to nearest, lo = bf16(x - hi); x is used up (v_dot2 forms x - hi in place).
+__device__ __forceinline__ bf16x8_t round_bf16(const float (&x)[8]) {
+  return __builtin_bit_cast(bf16x8_t, make_uint4(pack2<bf16_t>(x[0], x[1]), pack2<bf16_t>(x[2], x[3]), pack2<bf16_t>(x[4], x[5]),
+                                                 pack2<bf16_t>(x[6], x[7])));
+}
+__device__ __forceinline__ bf16x8_t rest_bf16(const float (&x)[8], bf16x8_t hi) {
+  const uint4 h = __builtin_bit_cast(uint4, hi);
+  // (-1, 0) and (0, -1), from registers: as an operand of this instruction the compiler writes 0x0000BF80 as the inline constant
+  // -1.0, whose 32 bits are the other pair
+  uint32_t LO, HI;
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(LO));
+  asm("s_mov_b32 %0, 0xbf800000" : "=s"(HI));
+  const float r[8] = {dot2_bf16(h.x, LO, x[0]), dot2_bf16(h.x, HI, x[1]), dot2_bf16(h.y, LO, x[2]), dot2_bf16(h.y, HI, x[3]),
+                      dot2_bf16(h.z, LO, x[4]), dot2_bf16(h.z, HI, x[5]), dot2_bf16(h.w, LO, x[6]), dot2_bf16(h.w, HI, x[7])};
+  return round_bf16(r);
+}
+
+// From here on this wavefront's conversions to fp16 round a finite value beyond the range to the largest finite fp16 (MODE bit
+// 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
+__device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
+
+// Four FP32 values as an fp16 pair each: hi to nearest after a clamp, the rest toward zero (as half8_pair).
+struct QuadPair { uint2 hi, lo; };
+__device__ __forceinline__ QuadPair quad_pair(f32x4_t x) {
+  QuadPair r;
+  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
+  auto two = [&](float a, float b, uint32_t& hi, uint32_t& lo) {
+    const f32x2_t v = {c(a), c(b)};
+    const f16x2_t h = __builtin_convertvector(v, f16x2_t);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = pack2_rtz(fmaf((float)h[0], -1.f, a), fmaf((float)h[1], -1.f, b));      // (one v_fma_mix_f32 each)
+  };
+  two(x[0], x[1], r.hi.x, r.lo.x);
+  two(x[2], x[3], r.hi.y, r.lo.y);
+  return r;
+}
+// Four FP32 values to fp16, to nearest after a clamp.
+__device__ __forceinline__ uint2 quad_sat(f32x4_t x) {
+  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
+  return make_uint2(pack2<f16_t>(c(x[0]), c(x[1])), pack2<f16_t>(c(x[2]), c(x[3])));
+}
+
+// Inclusive sum over the sixteen lanes of a DPP row (the tokens of a sub-chunk).
+__device__ __forceinline__ float row16_scan(float x) {
+  x += dpp_mov<0x111>(x);     // row_shr:1, 2, 4, 8; lanes outside the row count as zero
+  x += dpp_mov<0x112>(x);
+  x += dpp_mov<0x114>(x);
+  x += dpp_mov<0x118>(x);
+  return x;
+}
+// Lane 15 of the row, in every lane of it.
+__device__ __forceinline__ float row16_last(float x) { return dpp_mov<0x15F>(x); }      // row_newbcast:15
+// Sum over the four lanes (t, 0 .. 3) of a token.
+__device__ __forceinline__ float token_sum(float x) {
+  const LanePair a = swap_rows16(x);
+  const float y = a.lo + a.hi;
+  const LanePair b = swap_halves(y);
+  return b.lo + b.hi;
+}
+
+// Rows that a buffer access may reach: `rows` of them, `pitch` bytes apart, 256 bytes of each; reads beyond return zero, writes
+// are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_resource(const void* base, int rows, uint32_t pitch) {
+  const uint32_t bytes = rows > 0 ? (uint32_t)(min(rows, SUB) - 1) * pitch + 256u : 0u;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
+}
+
+// Order of this wavefront's own LDS accesses on both sides (the LDS serves one wavefront in order; this keeps the compiler
+// from moving them).
+__device__ __forceinline__ void own_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Lane `LANE` of the row, in every lane of it.
+template <int LANE>
+__device__ __forceinline__ float row16_lane(float x) { return dpp_mov<0x150 + LANE>(x); }   // row_newbcast
+
+// W = (I + L)^-1 diag(beta) of one sub-chunk on one wavefront.  `m`: lane (t, g) holds M[t][4 g + r], of which only j < t is
+// read; L_ij = beta_i M_ij, `beta` the lane's token's.  `scratch`: 1 KiB of LDS (W may replace it).  Every lane gathers row t of L
+// and solves for row t of N = (I + L)^-1 from N (I + L) = I, its last column first: with N[t][l] known, N[t][j] -= N[t][l] L[l][j]
+// for all j < l, where L[l][j] is lane l's register j, a DPP operand.  (With the columns of L read from LDS, one address a
+// read, the solve took 3000 of the 14 500 cycles of a producing wavefront.)
+// x[j] += row[j] of lane LANE * y for four j.  v_fmac_f32 with a DPP operand, which the compiler does not form; the s_nop
+// covers the wait states between a vector instruction that writes a register and a DPP operand that reads it.
+template <int LANE>
+__device__ __forceinline__ void fmac4_lane(float& a, float& b, float& c, float& d, float ra, float rb, float rc, float rd, float y) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %2, %6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(ra), "v"(rb), "v"(rc), "v"(rd), "v"(y), "n"(LANE));
+}
+template <int LANE>
+__device__ __forceinline__ void fmac_lane(float& a, float ra, float y) {
+  asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(ra), "v"(y), "n"(LANE));
+}
+template <int L>
+__device__ __forceinline__ void eliminate(const float (&row)[SUB], float (&x)[SUB]) {
+  if constexpr (L > 0) {
+    constexpr int REST = L % 4;                  // the highest ones first: x[L - 1] is needed next
+#pragma unroll
+    for (int j = L; j > REST; j -= 4)
+      fmac4_lane<L>(x[j - 1], x[j - 2], x[j - 3], x[j - 4], row[j - 1], row[j - 2], row[j - 3], row[j - 4], x[L]);
+#pragma unroll
+    for (int j = REST; j > 0; --j) fmac_lane<L>(x[j - 1], row[j - 1], x[L]);
+    eliminate<L - 1>(row, x);
+  }
+}
+template <int J>
+__device__ __forceinline__ void times_lane(float beta, float (&x)[SUB]) {
+  if constexpr (J < SUB) {
+    x[J] *= row16_lane<J>(beta);
+    times_lane<J + 1>(beta, x);
+  }
+}
+__device__ __forceinline__ void store_row(f32x4_t m, float beta, char* scratch, int lane) {
+  const int t = lane & 15, g = lane >> 4;
+  *reinterpret_cast<float4*>(scratch + 64 * t + 16 * g) = make_float4(-beta * m[0], -beta * m[1], -beta * m[2], -beta * m[3]);
+}
+__device__ __forceinline__ void solve_and_store_w(float beta, const char* scratch, char* w_tile, int lane) {
+  const int t = lane & 15, g = lane >> 4;
+  float row[SUB], x[SUB];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 c = *reinterpret_cast<const float4*>(scratch + 64 * t + 16 * q);
+    row[4 * q] = c.x; row[4 * q + 1] = c.y; row[4 * q + 2] = c.z; row[4 * q + 3] = c.w;
+  }
+#pragma unroll
+  for (int j = 0; j < SUB; ++j) x[j] = t == j ? 1.f : 0.f;
+  eliminate<SUB - 1>(row, x);
+  times_lane<0>(beta, x);
+  own_lds_order();
+  f32x4_t w;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) w[r] = g < 2 ? (g == 0 ? x[r] : x[4 + r]) : (g == 2 ? x[8 + r] : x[12 + r]);
+  const QuadPair pair = quad_pair(w);
+  *reinterpret_cast<uint4*>(w_tile + 16 * lane) = make_uint4(pair.hi.x, pair.hi.y, pair.lo.x, pair.lo.y);
+}
+
+// The ring of sub-chunks between producing and computing wavefronts.  Sub-chunk i lives in slot i % RING; full[slot] counts
+// its productions, done[slot] the computing wavefronts that have finished with it.  A wavefront's LDS operations happen in
+// order, so a count raised after the accesses it stands for needs no more than the compiler to keep the order.
+constexpr int RING = 8;
+struct RingFlags { uint32_t full[RING], done[RING]; };
+typedef __attribute__((address_space(3))) uint32_t lds_word_t;
+// (Through an LDS pointer: a generic one would be read as memory, behind every load and store in flight.)
+__device__ __forceinline__ uint32_t read_count(const uint32_t* count) {
+  return __hip_atomic_load((lds_word_t*)const_cast<uint32_t*>(count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ bool count_reached(uint32_t now, uint32_t target) {
+  return (int32_t)(__builtin_amdgcn_readfirstlane(now) - target) >= 0;
+}
+__device__ __forceinline__ void ring_reset(RingFlags* f) {      // by the whole workgroup, before any of it uses the ring
+  if (threadIdx.x < 2 * RING) reinterpret_cast<uint32_t*>(f)[threadIdx.x] = 0u;
+  __syncthreads();
+}
+__device__ __forceinline__ void wait_count(const uint32_t* count, uint32_t target) {
+  while (!count_reached(read_count(count), target)) __builtin_amdgcn_s_sleep(1);
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void slot_filled(RingFlags* f, int i, int lane) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (lane == 0)
+    __hip_atomic_store((lds_word_t*)&f->full[i % RING], (uint32_t)(i / RING) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void slot_done(RingFlags* f, int i, int lane) {
+  asm volatile("" ::: "memory");
+  if (lane == 0) __hip_atomic_fetch_add((lds_word_t*)&f->done[i % RING], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  asm volatile("" ::: "memory");
+}
+
+// Tokens and states of one chain: a (sequence, head), or a (segment, head) of a call whose sequences are split.
+struct Chain {
+  int64_t token;          // first token
+  int tokens, head;       // tokens (0: nothing to do)
+  int64_t slot;           // number of its first sub-chunk among prepared ones
+  const float* init;      // [V, K] tile the state starts from (nullptr: zero)
+  float* fin;             // [V, K] tile that receives the state at the end (nullptr: none)
+  float* keep;            // [V, K] tile that receives a copy of the start state (nullptr: none)
+  bool identity;          // the state starts from the identity and v is zero: the segment's transition matrix
+};
+// The tokens of sequence n, whatever the offsets hold, inside the call's T tokens.
+__device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n, int T) {
+  const int a = min(max(cu_seqlens[n], 0), T), b = min(max(cu_seqlens[n + 1], a), T);
+  return make_int2(a, b - a);
+}
+// Sub-chunk i of sequence n is number first_slot + i among the prepared ones of a call: sequences do not overlap in it, whatever
+// their lengths, and no table is needed.
+__device__ __forceinline__ int64_t first_slot(int n, int token) { return token / SUB + n; }
+// Segment s of a split call (at most 64 sequences), worked out by one wavefront: lane n counts the segments of sequence n.
+// sequence < 0: the call has fewer segments.
+struct Segment { int sequence, index, count, token, tokens; int64_t slot; };
+__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int s, int lane) {
+  const int2 range = lane < N ? sequence_tokens(cu_seqlens, lane, T) : make_int2(0, 0);
+  const int nc = (range.y + CHUNK - 1) / CHUNK, ns = (nc + seg_chunks - 1) / seg_chunks;
+  const int incl = wave_inclusive_scan(ns), before = incl - ns;
+  Segment r{-1, 0, 0, 0, 0, 0};
+  const unsigned long long owner = __ballot(s >= before && s < incl);
+  if (owner == 0) return r;
+  r.sequence = __builtin_amdgcn_readfirstlane(__ffsll((long long)owner) - 1);
+  r.index = s - __builtin_amdgcn_readlane(before, r.sequence);
+  r.count = __builtin_amdgcn_readlane(ns, r.sequence);
+  const int skipped = r.index * seg_chunks * CHUNK;
+  r.token = __builtin_amdgcn_readlane(range.x, r.sequence) + skipped;
+  r.slot = first_slot(r.sequence, r.token - skipped) + skipped / SUB;
+  r.tokens = min(seg_chunks * CHUNK, __builtin_amdgcn_readlane(range.y, r.sequence) - skipped);
+  return r;
+}
+
+}  // namespace pla

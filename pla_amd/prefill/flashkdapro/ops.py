@@ -5,9 +5,9 @@
 returns ``None``; ``g`` is the raw gate (the lower-bound gate is applied inside), ``beta`` raw
 logits; ``state_pool`` + ``state_indices`` update an indexed pool in place.
 
-Differences that follow from the gfx950 design: chunk size 64; states are FP32 only and are NOT
-rounded to bf16 at the read / publish boundary (the reference's tc01 backend rounds them); chunk
-metadata is built on the device, and ``raw_cu_seqlens`` is validated and used for one host-side
+Differences that follow from the gfx950 design: the recurrence goes in sub-chunks of 16 tokens (``CHUNK_SIZE``,
+the reference's, is the grain of segments); states are FP32 only and are NOT rounded to bf16 at the read / publish
+boundary (the reference's tc01 backend rounds them); the kernels take the offsets from the device, and ``raw_cu_seqlens`` is validated and used for one host-side
 decision that changes no bit of the results (``pla_kda_prefill_launch_raw``); there is
 one backend, so the ``PLA_FLASHKDA_*`` routing variables have no effect.
 """

@@ -558,3 +558,55 @@ def test_kda_prefill_same_bits_on_both_sides_of_the_store_rule():
         call(first, first + 6, out, state)
         assert torch.equal(out, whole[offs[first]:offs[first + 6]])
         assert torch.equal(state, final[first:first + 6])
+
+
+@pytest.mark.parametrize("lengths,H", [([1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 65, 129, 143, 720], 4),   # prepared: 56 chains, 98 tokens on average
+                                       ([300, 7], 2)])
+def test_kda_prefill_prepared_sub_chunks_give_the_bits_of_formed_ones(lengths, H):
+    """Calls of at most 128 chains take sub-chunks that a kernel prepared in memory, short ones and calls of more chains form
+    them in the sweep.  The same sequences (every remainder of 16 tokens) in both kinds of call, and against the oracle."""
+    from pla_amd import _lib
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=1600 + H)
+    copies = 140 // (H * len(lengths)) + 1                       # enough for a call of more than 128 chains
+    size = _lib.load().pla_kda_prefill_workspace_bytes
+    assert size(offs[-1], len(lengths), H) >= offs[-1] // 16 * H * 18432 > size(copies * offs[-1], copies * len(lengths), H)
+    exp_o, exp_final = _oracle(q, k, v, raw, beta, A_log, dt_bias, offs, S0, fast=True)
+    results = []
+    for times in (1, copies):
+        offsets = [i * offs[-1] + o for i in range(times) for o in offs[:-1]] + [times * offs[-1]]
+        args = [torch.cat([t] * times).cuda() for t in (q, k, v, raw, beta)] + [A_log.cuda(), dt_bias.cuda()]
+        out = torch.full((times * offs[-1], H, 128), 7.0, dtype=torch.bfloat16, device="cuda")
+        state = torch.cat([S0] * times).cuda()
+        final = torch.empty_like(state)
+        flashkda_fwd(*args, out, initial_state=state, final_state=final,
+                     cu_seqlens=torch.tensor(offsets, dtype=torch.int32).cuda())
+        torch.cuda.synchronize()
+        results += [(out[i * offs[-1]:(i + 1) * offs[-1]], final[i * len(lengths):(i + 1) * len(lengths)]) for i in range(times)]
+    out, final = results[0]
+    torch.testing.assert_close(out.cpu().float(), exp_o.float(), atol=2e-2, rtol=2e-2)
+    worst = max(rel_l2(final[n], exp_final[n]) for n in range(len(lengths)))
+    assert worst <= 1e-3, worst
+    for other in results[1:]:
+        assert torch.equal(other[0], out) and torch.equal(other[1], final)
+
+
+def test_kda_prefill_states_and_values_beyond_the_operand_range_saturate():
+    """|v| and |S| of 1e5 and more pass the range of the fp16 operands: the results degrade, no infinity or NaN appears, and a
+    head that holds ordinary values keeps its bits."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    lengths, H = [200, 33], 3
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=65504)
+    results = []
+    for factor in (1.0, 1e6):
+        vv, ss = v.clone(), S0.clone()
+        vv[:, 1] = (vv[:, 1].float() * factor).bfloat16()
+        ss[:, 2] *= factor * 10
+        out = torch.empty_like(v).cuda()
+        final = torch.empty_like(ss).cuda()
+        flashkda_fwd(*(t.cuda() for t in (q, k, vv, raw, beta, A_log, dt_bias)), out, initial_state=ss.cuda(), final_state=final,
+                     cu_seqlens=torch.tensor(offs, dtype=torch.int32).cuda())
+        torch.cuda.synchronize()
+        assert torch.isfinite(out.float()).all() and torch.isfinite(final).all()
+        results.append((out, final))
+    assert torch.equal(results[0][0][:, 0], results[1][0][:, 0]) and torch.equal(results[0][1][:, 0], results[1][1][:, 0])
