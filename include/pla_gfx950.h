@@ -281,6 +281,18 @@ int pla_kda_commit_plan_launch(
     int32_t* candidate, int32_t* plan, void* stream);
 
 /*
+ * The whole paged commit: the plan above, then pla_kda_fold_native_launch and pla_kda_conv_native_launch with it, in one
+ * launch or in three, whichever is the faster for the number of tiles.  Arguments as there; source is int32.
+ */
+int pla_kda_commit_launch(
+    const int64_t* layer_table, int layers, int heads, int channels, int rows,
+    const void* sampled, int sampled_wide, const int32_t* source, const void* offsets, int offsets_wide,
+    const void* mapping, int mapping_wide, const void* computed, int computed_wide, const void* blocks, int blocks_wide,
+    int batch, int capacity, int sampler_rows, int block_rows, int block_cols, int slots, int Q, int null_block_id,
+    int token_capacity, int64_t block_row_stride, int64_t block_col_stride, int64_t block_size,
+    int32_t* candidate, int32_t* plan, void* stream);
+
+/*
  * Conv-window rollback of the commit: dst[layer, dst_idx[r], :, :] = src[layer, r, step_idx[r], :, :]
  * for every request r with step_idx[r] >= 0, 0 <= dst_idx[r] < dst_reqs, r < src_reqs and
  * step_idx[r] < src_steps.  Replaces launch_conv_scatter

@@ -507,19 +507,13 @@ bool kda_replay_commit(const Tensor& sampled, const Tensor& source, const Tensor
           blocks->size(1) > 0 && (blocks->scalar_type() == at::kInt || blocks->scalar_type() == at::kLong));
   const c10::DeviceGuard guard(plan.device());
   void* const stream = stream_of(plan);
-  launched(pla_kda_commit_plan_launch(
-      sampled.data_ptr(), wide(sampled), source.data_ptr(), wide(source), cu.data_ptr(), wide(cu), ptr(mapping), mapping ? wide(*mapping) : 0,
-      ptr(computed), computed ? wide(*computed) : 0, ptr(blocks), align ? wide(*blocks) : 0, (int)N, (int)R, (int)sampled.numel(),
+  launched(pla_kda_commit_launch(
+      table.data_ptr<int64_t>(), (int)table.size(0), (int)heads, (int)channels, (int)rows, sampled.data_ptr(), wide(sampled),
+      source.data_ptr<int32_t>(), cu.data_ptr(), wide(cu), ptr(mapping), mapping ? wide(*mapping) : 0, ptr(computed),
+      computed ? wide(*computed) : 0, ptr(blocks), align ? wide(*blocks) : 0, (int)N, (int)R, (int)sampled.numel(),
       align ? (int)blocks->size(0) : 0, align ? (int)blocks->size(1) : 0, (int)slots, (int)Q, (int)null_block_id, (int)token_capacity,
       align ? blocks->stride(0) : 0, align ? blocks->stride(1) : 0, align ? block_size : 0, candidate.data_ptr<int32_t>(),
       plan.data_ptr<int32_t>(), stream));
-  const int32_t* const lens = plan.data_ptr<int32_t>();
-  const int32_t *const final_slot = lens + R, *const boundary = lens + 2 * R, *const boundary_lens = lens + 3 * R;
-  const int layers = (int)table.size(0);
-  launched(pla_kda_fold_native_launch(table.data_ptr<int64_t>(), layers, source.data_ptr<int32_t>(), lens, final_slot, boundary,
-                                      boundary_lens, (int)N, (int)heads, (int)Q, (int)slots, (int)null_block_id, stream));
-  launched(pla_kda_conv_native_launch(table.data_ptr<int64_t>(), layers, lens, final_slot, boundary, boundary_lens, (int)N, (int)channels,
-                                      (int)Q, (int)rows, (int)slots, stream));
   return true;
 }
 

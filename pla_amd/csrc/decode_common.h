@@ -97,6 +97,13 @@ __device__ __forceinline__ void store_row_scalars(act_t* p, int lane, const floa
   }
 }
 
+// A pointer that came out of a table in memory is one to any address space for the compiler, and such loads (FLAT) can only
+// be waited for all together, LDS reads included.  These are global.
+template <typename T>
+using global_ptr = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ global_ptr<T> as_global(T* p) { return (global_ptr<T>)p; }
+
 // State tiles are streamed exactly once per call, so they are moved with raw
 // buffer instructions carrying streaming cache hints: loads are non-temporal,
 // stores non-temporal with agent-scope write-through.  On MI355X this raises

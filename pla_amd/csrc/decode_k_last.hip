@@ -17,6 +17,7 @@
 // with one deliberate difference: corrupt cu_seqlens (negative start, length
 // above T_max) make the request a no-op instead of trapping the device.
 
+#include "commit_plan.h"
 #include "decode_common.h"
 #include "readonce_verify.h"
 #include "tuned_table.h"
@@ -612,31 +613,58 @@ struct FoldRecord {
 // state tile (504 tiles, windows of eight tokens: 21.6 -> 20.4 us; what is left there are the vector instructions of the
 // row reductions).  With 32 rows that takes 142 registers, three wavefronts per SIMD instead of four, and the other
 // wavefronts cover the trips.
-template <typename act_t, int RPW>
-__global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
+//
+// PLANNED: the paged commit in one launch.  A workgroup works out the plan of its own request (commit_plan.h) while its
+// state tile is on the way, and the workgroups behind the tiles copy the conv windows.  No workgroup reads what another
+// one writes, because the slots of a committing request are its own.
+struct CommitParams {
+  PlanInputs plan;
+  int32_t* plan_rows;              // [4, capacity]
+  int channels, layers;            // channels of the conv windows
+};
+
+// The plan row of request i_n from the first workgroup of its first tile; that of request 0 clears the rows behind the batch.
+__device__ inline void plan_row(const CommitParams& m, int i_n, bool first_tile, const Request& r) {
+  if (!first_tile || blockIdx.y != 0) return;
+  const int cap = m.plan.capacity;
+  if (threadIdx.x == 0) {
+    m.plan_rows[i_n] = r.tokens;
+    m.plan_rows[cap + i_n] = r.final_slot;
+    m.plan_rows[2 * cap + i_n] = r.boundary_slot;
+    m.plan_rows[3 * cap + i_n] = r.boundary_tokens;
+  }
+  if (i_n != 0) return;
+  for (int b = m.plan.batch + threadIdx.x; b < cap; b += 256)
+    for (int x = 0; x < 4; ++x) m.plan_rows[x * cap + b] = 0;
+}
+
+template <typename act_t, int RPW, bool PLANNED>
+__device__ __forceinline__ void fold_rows(const FoldParams p, const CommitParams& m, int tile, int64_t layer) {
   constexpr int R = RPW / 2;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int half = lane >> 5;
   const int c = lane & 31;
-  const int i_n = blockIdx.x / p.HV;
-  const int i_hv = blockIdx.x - i_n * p.HV;
+  const int i_n = tile / p.HV;
+  const int i_hv = tile - i_n * p.HV;
   const int i_h = i_hv / (p.HV / p.H);
   const int rowbase = (blockIdx.y * 4 + wave) * RPW;
 
   const int slot = p.slot_idx[i_n];
-  int n_acc = p.accept_lens[i_n];
-  const int final_slot = p.final_idx != nullptr ? p.final_idx[i_n] : slot;
-  const int track_slot = p.track_idx != nullptr ? p.track_idx[i_n] : p.null_block_id;
-  const int track_at = p.track_idx != nullptr ? p.track_step[i_n] - (p.track_is_len ? 1 : 0) : -1;
+  int n_acc = PLANNED ? 1 : p.accept_lens[i_n];
+  int final_slot = !PLANNED && p.final_idx != nullptr ? p.final_idx[i_n] : slot;
+  int track_slot = !PLANNED && p.track_idx != nullptr ? p.track_idx[i_n] : p.null_block_id;
+  int track_at = !PLANNED && p.track_idx != nullptr ? p.track_step[i_n] - (p.track_is_len ? 1 : 0) : -1;
   auto usable = [&](int id) { return id > p.null_block_id && (p.slots <= 0 || id < p.slots); };
-  if (!usable(slot) || !usable(final_slot) || n_acc <= 0) return;
+  if (!usable(slot) || !usable(final_slot) || n_acc <= 0) {
+    if constexpr (PLANNED) plan_row(m, i_n, i_hv == 0 && layer == 0, Request{NO_CLAIM, 0, 0, 0, 0});
+    return;
+  }
   if (n_acc > p.L) n_acc = p.L;
-  const bool tracked = track_at >= 0 && usable(track_slot);
+  bool tracked = track_at >= 0 && usable(track_slot);
 
   // Each wavefront reads its rows of the source tile before it writes any of them, so the destinations
   // may alias the source slot.
-  const int64_t layer = blockIdx.z;
   float* pool = p.h0 + layer * p.h0_layer_stride;
   int64_t h0_slot_stride = p.h0_slot_stride;
   const void* rawk = p.rawk;
@@ -674,6 +702,16 @@ __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
   if constexpr (AHEAD) next = request(0);
   float s[R][4];
   load_state<R>(h_tile, lane_off, s);
+  if constexpr (PLANNED) {
+    const Request r = commit_decision(m.plan, i_n);
+    plan_row(m, i_n, i_hv == 0 && layer == 0, r);
+    if (r.tokens == 0) return;
+    n_acc = r.tokens;
+    final_slot = r.final_slot;
+    track_slot = r.boundary_slot;
+    track_at = r.boundary_tokens - 1;
+    tracked = track_at >= 0;
+  }
 
   for (int t = 0; t < n_acc; ++t) {
     if constexpr (AHEAD) {
@@ -697,6 +735,29 @@ __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
       store_state<R>(Tile<float>(pool + (int64_t)track_slot * h0_slot_stride + (int64_t)i_hv * 16384), lane_off, s);
   }
   store_state<R>(Tile<float>(pool + (int64_t)final_slot * h0_slot_stride + (int64_t)i_hv * 16384), lane_off, s);
+}
+
+template <typename act_t, int RPW>
+__global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
+  fold_rows<act_t, RPW, false>(p, CommitParams{}, blockIdx.x, blockIdx.z);
+}
+
+template <int RPW>
+__global__ __launch_bounds__(256) void kda_commit_kernel(const FoldParams p, const CommitParams m) {
+  const int tiles = p.B * p.HV, folds = tiles * m.layers;
+  if ((int)blockIdx.x < folds) {
+    const int layer = blockIdx.x / tiles;
+    fold_rows<bf16_t, RPW, true>(p, m, blockIdx.x - layer * tiles, layer);
+    return;
+  }
+  const int groups = (m.channels + 255) / 256;                 // of 256 channels, of a request in a layer
+  const int g = (blockIdx.x - folds) * gridDim.y + blockIdx.y;
+  const int row = g / groups;
+  if (row >= p.B * m.layers) return;
+  const int layer = row / p.B, i_n = row - layer * p.B;
+  const Request r = commit_decision(m.plan, i_n);
+  const int channel = (g - row * groups) * 256 + threadIdx.x;
+  if (channel < m.channels) copy_conv_window(p.layer_table + layer * PLA_LAYER_TABLE_ENTRIES, i_n, channel, r);
 }
 
 // ---- host side ---------------------------------------------------------------
@@ -963,4 +1024,56 @@ extern "C" int pla_kda_fold_native_launch(
                (int64_t)heads * Q, batch, heads, heads, Q, null_block_id,
                final_indices, boundary_indices, boundary_lengths, 1, 1, slots, 0, 0, 0, 0, 0, layer_table};
   return launch_fold(p, PLA_BF16, stream, layers);
+}
+
+// Up to this many state tiles the paged commit is one launch.  There a workgroup's plan costs a trip to memory or two beside
+// the trip for its tile and saves two launches; with more tiles than the chip holds workgroups every round pays for it.
+// us at one / three launches (windows of 3-8 tokens; with a block table in brackets):
+//     8 tiles  6.8 / 9.1 (7.8 / 9.8)      240 tiles 11.6 / 13.9 (12.7 / 14.6)   480 tiles 24.9 / 23.4 (25.8 / 24.1)
+//    96 tiles 10.6 / 12.4 (11.6 / 13.0)   320 tiles 17.4 / 18.0 (18.4 / 18.5)   504 tiles 24.7 / 24.5 (26.7 / 25.0)
+constexpr int64_t COMMIT_ONE_LAUNCH_TILES = 320;
+
+extern "C" int pla_kda_commit_launch(
+    const int64_t* layer_table, int layers, int heads, int channels, int rows,
+    const void* sampled, int sampled_wide, const int32_t* source, const void* offsets, int offsets_wide,
+    const void* mapping, int mapping_wide, const void* computed, int computed_wide, const void* blocks, int blocks_wide,
+    int batch, int capacity, int sampler_rows, int block_rows, int block_cols, int slots, int Q, int null_block_id,
+    int token_capacity, int64_t block_row_stride, int64_t block_col_stride, int64_t block_size,
+    int32_t* candidate, int32_t* plan, void* stream) {
+  const PlanInputs in{sampled, source, offsets, mapping, computed, blocks,
+                      sampled_wide, 0, offsets_wide, mapping_wide, computed_wide, blocks_wide,
+                      batch, capacity, sampler_rows, block_rows, block_cols, slots, Q, null_block_id, token_capacity,
+                      block_row_stride, block_col_stride, block_size};
+  if (capacity == 0) return 0;
+  const int32_t *const final_slots = plan + capacity, *const boundary = final_slots + capacity, *const boundary_lens = boundary + capacity;
+  const bool fused = batch > 0 && (int64_t)batch * heads * layers <= COMMIT_ONE_LAUNCH_TILES && plan_apart(in, plan);
+  if (!fused) {
+    if (const int bad = pla_kda_commit_plan_launch(
+            sampled, sampled_wide, source, 0, offsets, offsets_wide, mapping, mapping_wide, computed, computed_wide, blocks, blocks_wide,
+            batch, capacity, sampler_rows, block_rows, block_cols, slots, Q, null_block_id, token_capacity, block_row_stride,
+            block_col_stride, block_size, candidate, plan, stream))
+      return bad;
+    if (const int bad = pla_kda_fold_native_launch(layer_table, layers, source, plan, final_slots, boundary, boundary_lens, batch, heads,
+                                                   Q, slots, null_block_id, stream))
+      return bad;
+    return pla_kda_conv_native_launch(layer_table, layers, plan, final_slots, boundary, boundary_lens, batch, channels, Q, rows, slots,
+                                      stream);
+  }
+  PLA_REQUIRE(layer_table && plan, "null table or plan pointer");
+  if (const int bad = check_plan_inputs(in)) return bad;
+  PLA_REQUIRE(layers >= 1 && layers <= 65535 && heads > 0 && channels > 0 && batch <= rows,
+              "commit requires 1..65535 layers, heads > 0, channels > 0 and batch <= record rows");
+  FoldParams p{nullptr, nullptr, nullptr, nullptr, nullptr, source, nullptr,
+               0, (int64_t)heads * Q * 128, (int64_t)heads * Q * 128, (int64_t)heads * Q * 128,
+               (int64_t)heads * Q, batch, heads, heads, Q, null_block_id,
+               nullptr, nullptr, nullptr, 1, 1, slots, 0, 0, 0, 0, 0, layer_table};
+  const int rpw = pick_rows_per_wave(batch * heads * layers);
+  const CommitParams m{in, plan, channels, layers};
+  const unsigned parts = 32 / rpw;
+  const unsigned conv_groups = (unsigned)(batch * layers) * (unsigned)((channels + 255) / 256);
+  const dim3 grid((unsigned)(batch * heads * layers) + (conv_groups + parts - 1) / parts, parts), block(256);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (rpw == 16) kda_commit_kernel<16><<<grid, block, 0, s>>>(p, m);
+  else kda_commit_kernel<8><<<grid, block, 0, s>>>(p, m);
+  return check_launch("kda_commit_kernel launch");
 }

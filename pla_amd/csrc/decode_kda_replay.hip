@@ -25,6 +25,7 @@
 // dst[layer, dst_idx[r], :, :] = src[layer, r, step_idx[r], :, :] for every request r with a
 // non-negative step and an in-range destination.
 
+#include "commit_plan.h"
 #include "decode_common.h"
 #include "readonce_verify.h"
 
@@ -449,21 +450,10 @@ __global__ __launch_bounds__(256) void conv_window_native_kernel(
   const int r = blockIdx.x;
   const int d = blockIdx.z * 256 + threadIdx.x;
   if (d >= channels || r >= rows) return;
-  const int64_t* const e = layer_table + (int64_t)blockIdx.y * PLA_LAYER_TABLE_ENTRIES;
-  uint16_t* const conv = reinterpret_cast<uint16_t*>(e[6]);
-  const uint16_t* const win = reinterpret_cast<const uint16_t*>(e[10]);
-  const int64_t c_slot = e[7], c_ch = e[8], c_tap = e[9], w_row = e[11], w_step = e[12], w_ch = e[13], w_tap = e[14];
-  const int count[2] = {boundary_lengths[r], lengths[r]};
-  const int dest[2] = {boundary_idx[r], final_idx[r]};
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int step = count[i] - 1;
-    if (step < 0 || step >= steps || dest[i] < 0 || dest[i] >= slots) continue;
-    const uint16_t* sp = win + r * w_row + step * w_step + d * w_ch;
-    uint16_t* dp = conv + dest[i] * c_slot + d * c_ch;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) dp[w * c_tap] = sp[w * w_tap];
-  }
+  Request todo{NO_CLAIM, lengths[r], final_idx[r], boundary_idx[r], boundary_lengths[r]};
+  if (todo.tokens > steps || todo.final_slot < 0 || todo.final_slot >= slots) todo.tokens = 0;
+  if (todo.boundary_tokens > steps || todo.boundary_slot < 0 || todo.boundary_slot >= slots) todo.boundary_tokens = 0;
+  copy_conv_window(layer_table + (int64_t)blockIdx.y * PLA_LAYER_TABLE_ENTRIES, r, d, todo);
 }
 
 static bool aligned_at(const void* ptr, size_t a) { return (reinterpret_cast<uintptr_t>(ptr) % a) == 0; }

@@ -1,0 +1,94 @@
+"""The paged commit in one launch against plan, fold and conv windows in three, bit for bit (the arithmetic of a tile is the
+same); and the plan of large batches, whose look-ups are spread over workgroups."""
+import pytest
+import torch
+
+from test_replay_vllm_gpu import inputs, pages, records_filled, vector
+
+pytestmark = pytest.mark.gpu
+BLOCK = 8
+
+
+def _context(requests, heads, q, n_layers, layout, capacity, seed):
+    from pla_amd.decode.kda_replayssm_vllm import KDAReplayCommitContext, kda_replay_verify
+    gen = torch.Generator().manual_seed(seed)
+    slots = requests + requests // 2 + 3
+    layers = [pages(slots, heads, q, layout, gen) for _ in range(n_layers)]
+    x = {k: v for k, v in inputs(heads, requests * q, gen).items() if k != "storage"}
+    source = (1 + torch.randperm(slots - 1, generator=gen)[:requests]).tolist()
+    offsets = list(range(0, requests * q + 1, q))
+    for layer in layers:
+        layer.replay_records = records_filled(capacity, heads, q)
+        layer.kv_cache = (layer.conv, layer.state)
+        kda_replay_verify(**x, conv_state=layer.conv, checkpoint_state=layer.state, records=layer.replay_records,
+                          query_start_loc=vector(offsets), state_indices=vector(source), conv_state_layout=layout, null_block_id=0)
+    return KDAReplayCommitContext.create(layers, q, capacity, layout, 0), layers, source, offsets, slots, gen
+
+
+def _three_launches(ctx, sampled, source, offsets, mapping, table, computed, tokens):
+    from pla_amd import _lib
+    N, R, layers = source.numel(), ctx._capacity, ctx._table.shape[0]
+    scratch, plan = torch.full((4, R), -9, dtype=torch.int32, device="cuda"), torch.full((4, R), -9, dtype=torch.int32, device="cuda")
+    stream, ptr = torch.cuda.current_stream().cuda_stream, lambda t: None if t is None else t.data_ptr()
+    rows, cols = (0, 0) if table is None else table.shape
+    _lib.call("pla_kda_commit_plan_launch", sampled.data_ptr(), 0, source.data_ptr(), 0, offsets.data_ptr(), 0, ptr(mapping), 0,
+              ptr(computed), 0, ptr(table), 0, N, R, sampled.numel(), rows, cols, ctx._slots, ctx._q, 0, tokens, cols,
+              0 if table is None else 1, 0 if table is None else BLOCK, scratch.data_ptr(), plan.data_ptr(), stream)
+    rows4 = [plan[c].data_ptr() for c in range(4)]
+    _lib.call("pla_kda_fold_native_launch", ctx._table.data_ptr(), layers, source.data_ptr(), *rows4, N, ctx._heads, ctx._q,
+              ctx._slots, 0, stream)
+    _lib.call("pla_kda_conv_native_launch", ctx._table.data_ptr(), layers, *rows4, N, ctx._channels, ctx._q, ctx._rows,
+              ctx._slots, stream)
+    return plan
+
+
+# one request; few tiles (8 rows per wavefront) and more (16 rows); more requests than threads of a workgroup; the largest
+# number of tiles of one launch, and one request more than that
+@pytest.mark.parametrize("requests,heads,q,n_layers,layout,capacity", [
+    (1, 1, 1, 1, "SD", 1), (5, 3, 4, 2, "DS", 9), (17, 6, 8, 2, "SD", 20), (260, 1, 2, 1, "DS", 300), (20, 8, 3, 2, "SD", 20),
+    (21, 8, 3, 2, "SD", 21)])
+@pytest.mark.parametrize("mode", ["plain", "mapping", "align"])
+def test_commit_in_one_launch_equals_three(requests, heads, q, n_layers, layout, capacity, mode):
+    ctx, layers, source, offsets, slots, gen = _context(requests, heads, q, n_layers, layout, capacity, 31 + requests)
+    ri = lambda lo, hi, n: torch.randint(lo, hi, (n,), generator=gen)
+    sampled = vector(ri(0, q + 2, requests + 2).tolist())
+    if requests > 16:                                            # no slot, a slot beyond the pool, two requests of one slot
+        source[1], source[2], source[4] = 0, slots + 5, source[3]
+    d_source, d_offsets = vector(source), vector(offsets)
+    mapping = vector(ri(-1, requests + 3, requests).tolist()) if mode == "mapping" else None
+    table = computed = None
+    kw = {}
+    if mode == "align":                                          # the blocks of a request: its source, then free or foreign slots
+        free = [s for s in range(1, slots) if s not in source]
+        cells = [[source[b] if 0 < source[b] < slots else 1, free[b % len(free)], (7 * b) % slots] for b in range(requests)]
+        table = torch.tensor(cells + [[1, 2, 3]] * 2, dtype=torch.int32, device="cuda")
+        computed = vector(ri(0, 2 * BLOCK, requests + 2).tolist())
+        kw = dict(block_table=table, num_computed_tokens=computed, mamba_block_size=BLOCK)
+    before = [(layer.state.clone(), layer.conv.clone()) for layer in layers]
+    want_plan = _three_launches(ctx, sampled, d_source, d_offsets, mapping, table, computed, offsets[-1])
+    want = [(layer.state.clone(), layer.conv.clone()) for layer in layers]
+    for layer, (state, conv) in zip(layers, before):
+        layer.state.copy_(state)
+        layer.conv.copy_(conv)
+    ctx._buffer.fill_(-9)
+    ctx.commit(sampled, d_source, d_offsets, request_indices=mapping, token_capacity=offsets[-1], **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(ctx._buffer, want_plan)
+    assert requests < 17 or (want_plan[0] > 0).any()
+    for layer, (state, conv) in zip(layers, want):
+        assert torch.equal(layer.state, state) and torch.equal(layer.conv, conv)
+
+
+def test_commit_takes_its_sources_from_its_own_plan():
+    """The final slots of a commit as the sources of the next: the plan is overwritten while it is an input."""
+    ctx, layers, source, offsets, slots, gen = _context(6, 2, 4, 1, "SD", 6, 77)
+    args = dict(num_sampled=vector([2, 1, 4, 3, 1, 2]), query_start_loc=vector(offsets), token_capacity=offsets[-1])
+    plan = ctx.commit(state_indices=vector(source), **args)
+    before = layers[0].state.clone(), layers[0].conv.clone()
+    ctx.commit(state_indices=plan.final_state_indices.clone(), **args)
+    want = layers[0].state.clone(), layers[0].conv.clone(), ctx._buffer.clone()
+    layers[0].state.copy_(before[0])
+    layers[0].conv.copy_(before[1])
+    ctx.commit(state_indices=plan.final_state_indices, **args)
+    assert torch.equal(layers[0].state, want[0]) and torch.equal(layers[0].conv, want[1]) and torch.equal(ctx._buffer, want[2])
+    assert plan.final_state_indices.tolist() == source
