@@ -29,7 +29,7 @@
 // against [U, U], sixteen tokens of each filling its contraction of 32.
 //
 // (A chunk of 64 tokens with its operands prepared in memory, 82 KB written and 76 and 98 KB read back per chunk and head, took 158
-// us for 18 ragged sequences of 12 heads and 2150 us for 65 536 tokens of 32 heads; this form takes 96 and 1740.)
+// us for 18 ragged sequences of 12 heads and 2150 us for 65 536 tokens of 32 heads; this form takes 95 and 1757.)
 //
 // Kernels:
 //   kda_prepare_kernel      calls of at most 128 chains: the operands of all sub-chunks, formed on every CU ahead of the sweep
@@ -664,9 +664,10 @@ extern "C" int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H) {
 }
 
 // The share of a KDA chain's chunk time that one of its two half workgroups takes, and how much longer a chunk takes
-// on a full chip than on an idle one (mixed_sweep_plan).  Measured, ms per call of 32 heads without / with the plan
-// at (0.9, 0.17) / at (0.8, 0.05): 8000 + 7000 + 1000 + 2000 + 3000 tokens 0.793 / 0.749 / 0.701; eight ragged
-// sequences of 32 810 tokens 0.997 / - / 0.948; twelve of 700 to 6000 tokens 0.757 / 0.712 / 0.676.
+// on a full chip than on an idle one (mixed_sweep_plan).  Measured, us per call without the plan / at (0.72, 0.05) / (0.8, 0.05)
+// / (0.9, 0.05): 8000 + 7000 + 1000 + 2000 + 3000 tokens of 32 heads 728 / 597 / 599 / 645; eight ragged sequences of 32 810
+// tokens 671 / 615 / 612 / 613; twelve of 700 to 6000 tokens 564 / 478 / 479 / 481; 18 of 121 to 999 tokens of 12 heads 105 / 95 /
+// 95 / 95.
 constexpr double KDA_HALF_COST = 0.8, KDA_FILL_COST = 0.05;
 
 static int kda_prefill_run(

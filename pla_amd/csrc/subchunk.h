@@ -9,11 +9,11 @@
 //   row tile      4 KiB, the pieces in the order (s, lane): written and read 16 bytes per lane at consecutive addresses
 //   turned tile   the same with token t ^ 4 g in the place of t: read through the transposing LDS read (tokens as
 //                 contraction), which then touches every bank once
+//   W             16 bytes per lane (i, g): W[i][4 g .. + 3] as fp16, hi then lo; against [X, X] one MFMA multiplies both
+//   P             8 bytes per lane (i, g): P[i][4 g .. + 3] as fp16
 // Products go to the 16x16x32 MFMA alone.  (An accumulator that v_mfma_f32_16x16x16_f16 had written and 16x16x32 read one or two
 // instructions later was seen to lack the first product in half of its registers, depending on what else ran: the compiler
 // puts no wait between the two.)
-//   W             16 bytes per lane (i, g): W[i][4 g .. + 3] as fp16, hi then lo; against [X, X] one MFMA multiplies both
-//   P             8 bytes per lane (i, g): P[i][4 g .. + 3] as fp16
 #pragma once
 
 #include "prefill_common.h"
@@ -122,66 +122,52 @@ __device__ __forceinline__ void own_lds_order() {
 template <int LANE>
 __device__ __forceinline__ float row16_lane(float x) { return dpp_mov<0x150 + LANE>(x); }   // row_newbcast
 
-// W = (I + L)^-1 diag(beta) of one sub-chunk on one wavefront.  `m`: lane (t, g) holds M[t][4 g + r], of which only j < t is
-// read; L_ij = beta_i M_ij, `beta` the lane's token's.  `scratch`: 1 KiB of LDS (W may replace it).  Every lane gathers row t of L
-// and solves for row t of N = (I + L)^-1 from N (I + L) = I, its last column first: with N[t][l] known, N[t][j] -= N[t][l] L[l][j]
-// for all j < l, where L[l][j] is lane l's register j, a DPP operand.  (With the columns of L read from LDS, one address a
-// read, the solve took 3000 of the 14 500 cycles of a producing wavefront.)
-// x[j] += row[j] of lane LANE * y for four j.  v_fmac_f32 with a DPP operand, which the compiler does not form; the s_nop
-// covers the wait states between a vector instruction that writes a register and a DPP operand that reads it.
-template <int LANE>
-__device__ __forceinline__ void fmac4_lane(float& a, float& b, float& c, float& d, float ra, float rb, float rc, float rd, float y) {
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
-      : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "v"(ra), "v"(rb), "v"(rc), "v"(rd), "v"(y), "n"(LANE));
-}
-template <int LANE>
-__device__ __forceinline__ void fmac_lane(float& a, float ra, float y) {
-  asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(ra), "v"(y), "n"(LANE));
-}
-template <int L>
-__device__ __forceinline__ void eliminate(const float (&row)[SUB], float (&x)[SUB]) {
-  if constexpr (L > 0) {
-    constexpr int REST = L % 4;                  // the highest ones first: x[L - 1] is needed next
-#pragma unroll
-    for (int j = L; j > REST; j -= 4)
-      fmac4_lane<L>(x[j - 1], x[j - 2], x[j - 3], x[j - 4], row[j - 1], row[j - 2], row[j - 3], row[j - 4], x[L]);
-#pragma unroll
-    for (int j = REST; j > 0; --j) fmac_lane<L>(x[j - 1], row[j - 1], x[L]);
-    eliminate<L - 1>(row, x);
-  }
-}
-template <int J>
-__device__ __forceinline__ void times_lane(float beta, float (&x)[SUB]) {
-  if constexpr (J < SUB) {
-    x[J] *= row16_lane<J>(beta);
-    times_lane<J + 1>(beta, x);
-  }
-}
+// W = (I + L)^-1 diag(beta) of one sub-chunk on one wavefront, from (I + L) W = diag(beta): lane (t, g) holds W[t][4 g .. + 3],
+// and with row l known every lane subtracts L[t][l] W[l][.], row l being lane l's registers, a DPP operand: four instructions
+// a step and no wait between them, as three others stand between a register's last write and its next use by DPP.
+// (Row t of the inverse solved in every group of sixteen lanes, last column first, took 120 such instructions for these 60, a
+// wait with every four, and 44 more for the factors beta and the choice of a group's columns: 18 ragged sequences of 12 heads
+// 98.4 -> 95.5 us, 65 536 tokens of 32 heads 1795 -> 1757, eight sequences of 2048 tokens 236.5 -> 231.4.)
+// `m`: lane (t, g) holds M[t][4 g + r], of which only j < t is read; L_ij = beta_i M_ij, `beta` the lane's token's.  `scratch`: 1
+// KiB of LDS (W may replace it).
 __device__ __forceinline__ void store_row(f32x4_t m, float beta, char* scratch, int lane) {
   const int t = lane & 15, g = lane >> 4;
-  *reinterpret_cast<float4*>(scratch + 64 * t + 16 * g) = make_float4(-beta * m[0], -beta * m[1], -beta * m[2], -beta * m[3]);
+  float4 x;                                        // row t of -L, zero from the diagonal on
+  x.x = 4 * g < t ? -beta * m[0] : 0.f;
+  x.y = 4 * g + 1 < t ? -beta * m[1] : 0.f;
+  x.z = 4 * g + 2 < t ? -beta * m[2] : 0.f;
+  x.w = 4 * g + 3 < t ? -beta * m[3] : 0.f;
+  *reinterpret_cast<float4*>(scratch + 64 * t + 16 * g) = x;
 }
+// x[c] += row[l] * x[c] of lane l, for l = 0 .. 14.  One block: nothing may come between a write and its use by DPP.  (v_fmac_f32
+// with a DPP operand is not formed by the compiler; the s_nop covers the wait states behind the last write before the block.)
+#define PLA_STEP(ROW, LANE)                                                             \
+  "v_fmac_f32_dpp %0, %0, " ROW " row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %1, %1, " ROW " row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %2, %2, " ROW " row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %3, %3, " ROW " row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void eliminate(const float (&row)[SUB], float (&x)[4]) {
+  asm("s_nop 1\n\t" PLA_STEP("%4", "0") PLA_STEP("%5", "1") PLA_STEP("%6", "2") PLA_STEP("%7", "3") PLA_STEP("%8", "4")
+      PLA_STEP("%9", "5") PLA_STEP("%10", "6") PLA_STEP("%11", "7") PLA_STEP("%12", "8") PLA_STEP("%13", "9")
+      PLA_STEP("%14", "10") PLA_STEP("%15", "11") PLA_STEP("%16", "12") PLA_STEP("%17", "13") PLA_STEP("%18", "14")
+      : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]), "+&v"(x[3])
+      : "v"(row[0]), "v"(row[1]), "v"(row[2]), "v"(row[3]), "v"(row[4]), "v"(row[5]), "v"(row[6]), "v"(row[7]), "v"(row[8]),
+        "v"(row[9]), "v"(row[10]), "v"(row[11]), "v"(row[12]), "v"(row[13]), "v"(row[14]));
+}
+#undef PLA_STEP
 __device__ __forceinline__ void solve_and_store_w(float beta, const char* scratch, char* w_tile, int lane) {
   const int t = lane & 15, g = lane >> 4;
-  float row[SUB], x[SUB];
+  float row[SUB], x[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const float4 c = *reinterpret_cast<const float4*>(scratch + 64 * t + 16 * q);
     row[4 * q] = c.x; row[4 * q + 1] = c.y; row[4 * q + 2] = c.z; row[4 * q + 3] = c.w;
   }
 #pragma unroll
-  for (int j = 0; j < SUB; ++j) x[j] = t == j ? 1.f : 0.f;
-  eliminate<SUB - 1>(row, x);
-  times_lane<0>(beta, x);
+  for (int r = 0; r < 4; ++r) x[r] = t == 4 * g + r ? beta : 0.f;
+  eliminate(row, x);
   own_lds_order();
-  f32x4_t w;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) w[r] = g < 2 ? (g == 0 ? x[r] : x[4 + r]) : (g == 2 ? x[8 + r] : x[12 + r]);
-  const QuadPair pair = quad_pair(w);
+  const QuadPair pair = quad_pair(f32x4_t{x[0], x[1], x[2], x[3]});
   *reinterpret_cast<uint4*>(w_tile + 16 * lane) = make_uint4(pair.hi.x, pair.hi.y, pair.lo.x, pair.lo.y);
 }
 
