@@ -15,12 +15,14 @@
 // others, one per SIMD beside them, form the operands of the next sub-chunks in LDS from the raw rows, each every fourth one.
 // A ring of eight slots with counters stands between them (subchunk.h); there is no barrier in the loop.
 // Nothing but the tokens, the outputs and the states crosses memory, and a call of many chains is one launch.  What bounds it is
-// issue: a sub-chunk costs a SIMD about 290 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 250
-// of its computing one, with 52 MFMAs that overlap little of it: 3600 cycles, of which each of the two alone takes 2440.  Eight
+// issue: a sub-chunk costs a SIMD about 255 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 250
+// of its computing one, with 56 MFMAs that overlap little of it: 3600 cycles with 290 producing instructions, of which each of the
+// two sides alone took 2440.  Eight
 // producing wavefronts instead of four gain nothing (168 registers: the computing ones spill), nor do eight computing ones of 16
 // columns (246 against 228 us, eight sequences of 2048 tokens, 32 heads: twice the LDS reads).  Sixteen tokens decay
-// by at most 16 x |lower_bound| <= 80, so e^{G} and e^{-G} are FP32 numbers and M and P are one product each, on the
-// FP32 MFMA; a longer chunk needs a reference row, and its exponentials again, for every block of 16 x 16.
+// by at most 16 x |lower_bound| <= 80, so e^{G} and e^{-G} are FP32 numbers and M and P one product each; a longer chunk needs
+// a reference row, and its exponentials again, for every block of 16 x 16.  M takes both factors as bf16 hi + lo pairs, P its key
+// factor: with that rounded once too the output is 1.14 x as far from 64 bits (44 calls), for the same time.
 //
 // The operands of the products with the state (k e^{G}, q e^{G}, k e^{G_last - G}, W, P, S, X, U) go to the MFMA as fp16,
 // rounded once or (W, k e^{G_last - G}, X, U) as hi + lo pairs: the pairs keep keys that repeat within a few tokens
@@ -29,7 +31,7 @@
 // against [U, U], sixteen tokens of each filling its contraction of 32.
 //
 // (A chunk of 64 tokens with its operands prepared in memory, 82 KB written and 76 and 98 KB read back per chunk and head, took 158
-// us for 18 ragged sequences of 12 heads and 2150 us for 65 536 tokens of 32 heads; this form takes 95 and 1757.)
+// us for 18 ragged sequences of 12 heads and 2150 us for 65 536 tokens of 32 heads; this form takes 96 and 1731.)
 //
 // Kernels:
 //   kda_prepare_kernel      calls of at most 128 chains: the operands of all sub-chunks, formed on every CU ahead of the sweep
@@ -204,14 +206,17 @@ __device__ __forceinline__ void kda_sub_chunk(const KdaGate& gate, KdaRows<OUT>&
     *reinterpret_cast<uint4*>(slot + Slot::TL + at) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
     const bf16x8_t ke_hi = round_bf16(ke), kn_hi = round_bf16(kn);
     m = mfma16(kn_hi, rest_bf16(ke, ke_hi), m);
-    m = mfma16(rest_bf16(kn, kn_hi), ke_hi, m);
+    const bf16x8_t kn_lo = rest_bf16(kn, kn_hi);
+    m = mfma16(kn_lo, ke_hi, m);
     m = mfma16(kn_hi, ke_hi, m);
     if constexpr (OUT) {
       float qe[8];
       normalised(rows.q[s], q_inv, qe);
 #pragma unroll
       for (int e = 0; e < 8; ++e) qe[e] *= ex[e];
-      pq = mfma16(kn_hi, round_bf16(qe), pq);
+      const bf16x8_t qe_hi = round_bf16(qe);
+      pq = mfma16(kn_lo, qe_hi, pq);
+      pq = mfma16(kn_hi, qe_hi, pq);
       *reinterpret_cast<uint4*>(slot + Slot::Q + 1024 * s + 16 * lane) = half_piece(qe);
     }
   }
