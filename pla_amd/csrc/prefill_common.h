@@ -731,9 +731,7 @@ inline int mixed_sweep_plan(const int* r, int N, int HV, unsigned char* order, d
 // costs about 25 us (two more launches, an event between two streams, the state through memory, a pipeline that
 // fills again), and the preparation only hides under a sweep on CUs that chains which ended early have left.
 // (Segmented calls already keep every CU busy with sweeps - staging them was measured for GDN: 0.57 -> 0.66 ms for
-// one sequence of 16 384 tokens -; and staging only pays where the preparation is bound by memory latency and leaves
-// the sweeps their issue slots, which holds for GDN and not for KDA, whose preparation is instruction bound: the KDA
-// path does not call this.)
+// one sequence of 16 384 tokens -; the KDA path has no stages: its sweeps form their operands themselves.)
 inline int pick_stages(int T, int N, int heads, int seg_chunks) {
   if (seg_chunks > 0) return 0;
   // (the stage map keeps (stages + 1) counters per sequence in LDS: at most 2048 sequences)
