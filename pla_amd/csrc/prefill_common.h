@@ -439,6 +439,23 @@ __device__ __forceinline__ InlineTile inline_tile(const InlineSequences& q, int 
   return t;
 }
 
+// The tokens of sequence n, whatever the offsets hold, inside the call's T tokens: (first token, tokens).
+__device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n, int T) {
+  const int a = min(max(cu_seqlens[n], 0), T), b = min(max(cu_seqlens[n + 1], a), T);
+  return make_int2(a, b - a);
+}
+// The segments of a split call (at most 64 sequences), counted by one wavefront: lane n counts those of sequence n.  The sweeps
+// and the combine step between them take the same counts from here, so that they agree on every tile whatever the offsets
+// hold.
+struct SegmentCounts { int2 tokens; int count, before; };      // of this lane's sequence; segments ahead of its first
+__device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int lane) {
+  SegmentCounts r;
+  r.tokens = lane < N ? sequence_tokens(cu_seqlens, lane, T) : make_int2(0, 0);
+  r.count = ((r.tokens.y + CHUNK - 1) / CHUNK + seg_chunks - 1) / seg_chunks;
+  r.before = wave_inclusive_scan(r.count) - r.count;
+  return r;
+}
+
 // Segments per sequence and the 128 x 128 identity.  Single workgroup, after chunk_map.
 __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N, SegmentTable t) {
   if (threadIdx.x < 64) {                     // exclusive scan of the segment counts, as in chunk_map
@@ -482,7 +499,7 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 // M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes), all 64 loads of a step requested before
 // the first product.
 constexpr int COMBINE_SPLIT = 8;
-static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int heads) {
+static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads) {
   // the eight workgroups of a chain read the same M tiles: on one XCD they come from memory once (xcd_grouped_index)
   const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, N * heads * COMBINE_SPLIT);
   if (logical < 0) return;
@@ -490,10 +507,9 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
   const int chain = logical / COMBINE_SPLIT;
   const int n = chain / heads, h = chain - n * heads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // the sequence's segments, counted by every wavefront for itself (split calls have at most 64 sequences)
-  const int nc = (lane < N ? max(cu_seqlens[lane + 1] - cu_seqlens[lane], 0) : 0) + CHUNK - 1;
-  const int ns = (nc / CHUNK + t.seg_chunks - 1) / t.seg_chunks, before = wave_inclusive_scan(ns) - ns;
-  const int first = __builtin_amdgcn_readlane(before, n), end = first + __builtin_amdgcn_readlane(ns, n);
+  // the sequence's segments, counted by every wavefront for itself; overlapping sequences may count more than there are tiles
+  const SegmentCounts s = count_segments(cu_seqlens, N, T, t.seg_chunks, lane);
+  const int first = __builtin_amdgcn_readlane(s.before, n), end = min(first + __builtin_amdgcn_readlane(s.count, n), t.max_segments);
   if (end - first < 2) return;                 // a single segment starts from the caller's state
   __shared__ __align__(16) float S[16][132];
   const int c = lane & 15, kb = lane >> 4;
@@ -562,7 +578,7 @@ inline int max_segments(int T, int N, int seg_chunks) { return seg_chunks > 0 ? 
 
 // Zero the rows of a dense [T, heads, 128] 16-bit output that lie beyond the last sequence (workgroup `block` of `blocks`).
 __device__ __forceinline__ void zero_tail(uint16_t* o, const int32_t* cu_seqlens, int N, int T, int heads, int block, int blocks) {
-  const int64_t first = (int64_t)cu_seqlens[N] * heads * 128;
+  const int64_t first = (int64_t)max(cu_seqlens[N], 0) * heads * 128;
   const int64_t total = (int64_t)T * heads * 128;
   for (int64_t i = first + (int64_t)block * blockDim.x + threadIdx.x; i < total; i += (int64_t)blocks * blockDim.x)
     o[i] = 0;

@@ -745,7 +745,7 @@ static int kda_prefill_run(
     p.pass = 1;
     hipLaunchKernelGGL(prepared ? kda_lean_sweep_kernel<true> : kda_lean_sweep_kernel<false>, dim3(segment_chains), lean_block, 0, s, p);
     hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
-                       N, H);
+                       N, T, H);
     p.pass = 2;
   }
   const unsigned sweeps = segmented ? segment_chains : chains;

@@ -214,31 +214,23 @@ struct Chain {
   float* keep;            // [V, K] tile that receives a copy of the start state (nullptr: none)
   bool identity;          // the state starts from the identity and v is zero: the segment's transition matrix
 };
-// The tokens of sequence n, whatever the offsets hold, inside the call's T tokens.
-__device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n, int T) {
-  const int a = min(max(cu_seqlens[n], 0), T), b = min(max(cu_seqlens[n + 1], a), T);
-  return make_int2(a, b - a);
-}
 // Sub-chunk i of sequence n is number first_slot + i among the prepared ones of a call: sequences do not overlap in it, whatever
 // their lengths, and no table is needed.
 __device__ __forceinline__ int64_t first_slot(int n, int token) { return token / SUB + n; }
-// Segment s of a split call (at most 64 sequences), worked out by one wavefront: lane n counts the segments of sequence n.
-// sequence < 0: the call has fewer segments.
+// Segment s of a split call (count_segments).  sequence < 0: the call has fewer segments.
 struct Segment { int sequence, index, count, token, tokens; int64_t slot; };
 __device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int s, int lane) {
-  const int2 range = lane < N ? sequence_tokens(cu_seqlens, lane, T) : make_int2(0, 0);
-  const int nc = (range.y + CHUNK - 1) / CHUNK, ns = (nc + seg_chunks - 1) / seg_chunks;
-  const int incl = wave_inclusive_scan(ns), before = incl - ns;
+  const SegmentCounts c = count_segments(cu_seqlens, N, T, seg_chunks, lane);
   Segment r{-1, 0, 0, 0, 0, 0};
-  const unsigned long long owner = __ballot(s >= before && s < incl);
+  const unsigned long long owner = __ballot(s >= c.before && s < c.before + c.count);
   if (owner == 0) return r;
   r.sequence = __builtin_amdgcn_readfirstlane(__ffsll((long long)owner) - 1);
-  r.index = s - __builtin_amdgcn_readlane(before, r.sequence);
-  r.count = __builtin_amdgcn_readlane(ns, r.sequence);
+  r.index = s - __builtin_amdgcn_readlane(c.before, r.sequence);
+  r.count = __builtin_amdgcn_readlane(c.count, r.sequence);
   const int skipped = r.index * seg_chunks * CHUNK;
-  r.token = __builtin_amdgcn_readlane(range.x, r.sequence) + skipped;
+  r.token = __builtin_amdgcn_readlane(c.tokens.x, r.sequence) + skipped;
   r.slot = first_slot(r.sequence, r.token - skipped) + skipped / SUB;
-  r.tokens = min(seg_chunks * CHUNK, __builtin_amdgcn_readlane(range.y, r.sequence) - skipped);
+  r.tokens = min(seg_chunks * CHUNK, __builtin_amdgcn_readlane(c.tokens.y, r.sequence) - skipped);
   return r;
 }
 

@@ -610,3 +610,34 @@ def test_kda_prefill_states_and_values_beyond_the_operand_range_saturate():
         assert torch.isfinite(out.float()).all() and torch.isfinite(final).all()
         results.append((out, final))
     assert torch.equal(results[0][0][:, 0], results[1][0][:, 0]) and torch.equal(results[0][1][:, 0], results[1][1][:, 0])
+
+
+@pytest.mark.parametrize("offsets", [(0, 1500, 9000), (-700, 1500, 4096), (0, 70000, 70001)])
+def test_kda_prefill_split_with_offsets_beyond_the_tokens(offsets, monkeypatch):
+    """Offsets on the device are not checked before the launch: every kernel of a split call takes the tokens of a sequence
+    inside [0, T], the step between the two sweeps included, so that nothing outside the call's buffers is written (these
+    offsets count more segments than there are tiles) and the results are those of the offsets held to that range."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd, ops
+    T, H, dev, guard = 4096, 2, "cuda", 1 << 20
+    q, k, v, raw, beta, A_log, dt_bias, _, S0 = _inputs([1500, 2596], H, seed=4096)
+    args = [t.to(dev) for t in (q, k, v, raw, beta, A_log, dt_bias)]
+    plain, guarded = ops._workspace, []
+
+    def workspace(*call):
+        ws, nbytes = plain(*call)
+        whole = torch.full((nbytes + 2 * guard,), 0xA5, dtype=torch.uint8, device=dev)
+        guarded.append((whole[:guard], whole[guard + nbytes:]))
+        whole[guard:guard + nbytes] = ws
+        return whole[guard:guard + nbytes], nbytes
+    monkeypatch.setattr(ops, "_workspace", workspace)
+    results = []
+    for offs in (offsets, [min(max(o, 0), T) for o in offsets]):
+        rows = torch.full((T + 128, H, 128), 7.0, dtype=torch.bfloat16, device=dev)
+        final = torch.full((4, H, 128, 128), 5.0, device=dev)
+        flashkda_fwd(*args, rows[64:64 + T], initial_state=S0.to(dev), final_state=final[1:3],
+                     cu_seqlens=torch.tensor(offs, dtype=torch.int32, device=dev))
+        torch.cuda.synchronize()
+        assert (rows[:64] == 7).all() and (rows[64 + T:] == 7).all() and (final[0] == 5).all() and (final[3] == 5).all()
+        results.append((rows, final))
+    assert all((part == 0xA5).all() for pair in guarded for part in pair)
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
