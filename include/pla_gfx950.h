@@ -426,6 +426,9 @@ int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H);
  *   q and k are L2-normalised (eps 1e-6 inside the root) and rounded to bf16 first.
  *   cu_seqlens [N+1] int32; rows of o at and beyond cu_seqlens[N] are zeroed.
  *   h0 / ht as in pla_gdn_prefill_launch (k-last FP32 [slots,H,128,128]).
+ *   o may be the very rows of q, k, v or g (same address, token pitch H * 128).  Any other overlap of o with an input is the
+ *   caller's to avoid: with v it is not looked for, with q, k, g, beta, A_log or dt_bias it is refused where the sweep reads
+ *   them beside its writes.
  */
 int pla_kda_prefill_launch(
     const void* q, const void* k, const void* v, const void* g, const void* beta,

@@ -220,6 +220,21 @@ py::object try_gdn_prefill_packed_qkv_fwd(
 
 #ifdef PLA_BIND_FLASHKDAPRO
 // ---------------------------------------------------------------------------------------------------------------
+// `t`, or a copy of it if it shares memory with `out` other than as its very rows (the kernels write rows of out while they read
+// others of their inputs; see pla_kda_prefill_launch).
+Tensor apart_from(const Tensor& t, const Tensor& out) {
+  auto range = [](const Tensor& x) {
+    int64_t last = 0;
+    for (int64_t d = 0; d < x.dim(); ++d) last += (x.size(d) - 1) * x.stride(d);
+    const uintptr_t begin = reinterpret_cast<uintptr_t>(x.data_ptr());
+    return std::pair<uintptr_t, uintptr_t>(begin, begin + (uintptr_t)((last + 1) * x.element_size()));
+  };
+  const auto a = range(t), b = range(out);
+  if (a.second <= b.first || a.first >= b.second) return t;
+  const bool same = a.first == b.first && t.scalar_type() == out.scalar_type() && t.sizes() == out.sizes() && t.strides() == out.strides();
+  return same ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
 // KDA chunk-64 prefill: flashkda_fwd with the 15 positional arguments of the reference's _C.flashkda_fwd
 // (pla/prefill/flashkdapro/ops.py:215-219).  True: launched; False: not in the plain form, nothing launched.
 bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& A_log,
@@ -249,6 +264,8 @@ bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const T
   for (const OptTensor* t : {&initial_state, &final_state})
     if (t->has_value() && (!plain_states(**t, q, H) || (!indexed && (*t)->size(0) < N))) return false;
   if (final_state && final_state->data_ptr() == out.data_ptr()) return false;
+  const Tensor q_in = apart_from(q, out), k_in = apart_from(k, out), g_in = apart_from(g, out), beta_in = apart_from(beta, out),
+               A_in = apart_from(A_log, out), bias_in = apart_from(dt_bias, out);
 
   const int64_t ws_bytes = pla_kda_prefill_workspace_bytes((int)T, (int)N, (int)H);
   Tensor ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
@@ -266,8 +283,8 @@ bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const T
   }
   const int32_t* idx = indexed ? state_indices->data_ptr<int32_t>() : nullptr;
   launched(pla_kda_prefill_launch_raw(
-      q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), q.stride(0), k.stride(0), v.stride(0), g.stride(0),
-      beta.stride(0), A_log.data_ptr<float>(), dt_bias.data_ptr<float>(), (float)lower_bound, (float)scale,
+      q_in.data_ptr(), k_in.data_ptr(), v.data_ptr(), g_in.data_ptr(), beta_in.data_ptr(), q_in.stride(0), k_in.stride(0), v.stride(0),
+      g_in.stride(0), beta_in.stride(0), A_in.data_ptr<float>(), bias_in.data_ptr<float>(), (float)lower_bound, (float)scale,
       cu_seqlens->data_ptr<int32_t>(), (int)N, (int)T,
       initial_state ? initial_state->data_ptr<float>() : nullptr, idx, initial_state ? initial_state->stride(0) : 0,
       final_state ? final_state->data_ptr<float>() : nullptr, idx, final_state ? final_state->stride(0) : 0,

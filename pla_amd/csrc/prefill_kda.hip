@@ -675,6 +675,29 @@ extern "C" int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H) {
 // 95 / 95.
 constexpr double KDA_HALF_COST = 0.8, KDA_FILL_COST = 0.05;
 
+// Whether the output shares memory with an input that the sweeps read where no kernel prepares their sub-chunks (q, k, g, beta and
+// the gate's parameters).  In place: every such input is the output's very rows, which a workgroup that sweeps all columns of a
+// chain has read before it writes them; two workgroups of one chain would each overwrite rows that the other has yet to read.
+enum class KdaOverlap { none, in_place, other };
+static KdaOverlap kda_overlap(const KdaPrefillParams& p) {
+  const uintptr_t o_begin = (uintptr_t)p.o, row = (uintptr_t)p.H * 256, o_end = o_begin + (uintptr_t)p.T * row;
+  KdaOverlap found = KdaOverlap::none;
+  auto look = [&](const void* base, int64_t pitch, uintptr_t bytes, bool rows_of_out) {
+    const uintptr_t begin = (uintptr_t)base, end = begin + (uintptr_t)((p.T - 1) * pitch) + bytes;
+    if (end <= o_begin || begin >= o_end) return;
+    const bool same = rows_of_out && begin == o_begin && (p.T == 1 || pitch == (int64_t)row);
+    if (!same) found = KdaOverlap::other;
+    else if (found == KdaOverlap::none) found = KdaOverlap::in_place;
+  };
+  look(p.q, 2 * p.stride_q, row, true);
+  look(p.k, 2 * p.stride_k, row, true);
+  look(p.g, 2 * p.stride_g, row, true);
+  look(p.beta, 2 * p.stride_beta, (uintptr_t)p.H * 2, false);
+  look(p.A_log, 0, (uintptr_t)p.H * 4, false);
+  look(p.dt_bias, 0, (uintptr_t)p.H * 512, false);
+  return found;
+}
+
 static int kda_prefill_run(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
     int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_g, int64_t stride_beta,
@@ -712,7 +735,10 @@ static int kda_prefill_run(
   p.H = H;
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const bool segmented = L.seg_chunks > 0;
+  const bool segmented = L.seg_chunks > 0, prepared = L.slots > 0;
+  const KdaOverlap overlap = prepared ? KdaOverlap::none : kda_overlap(p);     // (prepared: all read ahead of the sweep)
+  PLA_REQUIRE(overlap != KdaOverlap::other, "out shares memory with q, k, g, beta, A_log or dt_bias other than as the very rows of q, k or g");
+  const bool whole_chains = overlap == KdaOverlap::in_place, halves = L.halves && !whole_chains;
   if (segmented) {
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
     p.seg.M = reinterpret_cast<float*>(ws + L.segM);
@@ -724,7 +750,7 @@ static int kda_prefill_run(
   // Ragged whole sequences whose offsets the host holds: the chains of the longest sequences run as two halves where
   // that shortens the sweep (mixed_sweep_plan)
   bool mixed = false;
-  if (!segmented && !L.halves && raw_cu_seqlens != nullptr && N <= INLINE_TABLE_SEQUENCES) {
+  if (!segmented && !L.halves && !whole_chains && raw_cu_seqlens != nullptr && N <= INLINE_TABLE_SEQUENCES) {
     int nc[INLINE_TABLE_SEQUENCES];
     for (int n = 0; n < N; ++n) nc[n] = (std::max(raw_cu_seqlens[n + 1] - raw_cu_seqlens[n], 0) + CHUNK - 1) / CHUNK;
     p.n_long = mixed_sweep_plan(nc, N, H, p.seq_order, KDA_HALF_COST, KDA_FILL_COST);
@@ -735,7 +761,6 @@ static int kda_prefill_run(
   }
   const dim3 sweep_block(64 * (4 + FEEDERS)), lean_block(64 * (8 + FEEDERS));
   const unsigned chains = (unsigned)N * H, segment_chains = (unsigned)L.max_segments * H;
-  const bool prepared = L.slots > 0;
   if (prepared) {
     p.prepared = ws + L.prepared;
     hipLaunchKernelGGL(kda_prepare_kernel, dim3((unsigned)((L.slots * H + PREPARE_WAVES - 1) / PREPARE_WAVES)), dim3(64 * PREPARE_WAVES), 0, s, p);
@@ -750,7 +775,7 @@ static int kda_prefill_run(
   }
   const unsigned sweeps = segmented ? segment_chains : chains;
   if (mixed) hipLaunchKernelGGL(kda_sweep_mixed_kernel, dim3(p.split_grid + (unsigned)(N - p.n_long) * H), sweep_block, 0, s, p);
-  else if (L.halves) hipLaunchKernelGGL((prepared ? kda_sweep_kernel<1, true> : kda_sweep_kernel<1, false>), dim3(xcd_grouped_grid(2 * sweeps, 2)), sweep_block, 0, s, p);
+  else if (halves) hipLaunchKernelGGL((prepared ? kda_sweep_kernel<1, true> : kda_sweep_kernel<1, false>), dim3(xcd_grouped_grid(2 * sweeps, 2)), sweep_block, 0, s, p);
   else hipLaunchKernelGGL((kda_sweep_kernel<2, false>), dim3(sweeps), sweep_block, 0, s, p);
   return check_launch("kda prefill launch");
 }

@@ -35,6 +35,19 @@ def _token_rows(name, t, H, width):
     return t, t.stride(0)
 
 
+def _apart_from(t, out):
+    """``t``, or a copy of it if it shares memory with ``out`` other than as its very rows (the kernels write rows of
+    ``out`` while they read others of their inputs)."""
+    def span(x):
+        last = sum((n - 1) * s for n, s in zip(x.shape, x.stride()))
+        return x.data_ptr(), x.data_ptr() + (last + 1) * x.element_size()
+    (begin, end), (out_begin, out_end) = span(t), span(out)
+    if end <= out_begin or begin >= out_end:
+        return t
+    same = begin == out_begin and t.dtype == out.dtype and t.shape == out.shape and t.stride() == out.stride()
+    return t if same else t.clone(memory_format=torch.contiguous_format)
+
+
 # The compiled host layer (pla_amd/csrc/prefill_binding.cpp): see pla_amd/prefill/flashqla/ops.py.
 _native = None
 
@@ -129,6 +142,8 @@ def flashkda_fwd(
     dt_bias = dt_bias.to(torch.float32).reshape(H, DK).contiguous()
     if A_log.numel() != H:
         raise ValueError("A_log must be [H]")
+    q, k, g, beta, A_log, dt_bias = (_apart_from(t, out) for t in (q, k, g, beta, A_log, dt_bias))
+    sq, sk, sg = q.stride(0), k.stride(0), g.stride(0)
 
     _sanity.offsets(cu_seqlens, T, raw_cu_seqlens, reference=q)
     _sanity.operand_range(q, v=v, initial_state=initial_state)

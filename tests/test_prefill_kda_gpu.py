@@ -641,3 +641,51 @@ def test_kda_prefill_split_with_offsets_beyond_the_tokens(offsets, monkeypatch):
         results.append((rows, final))
     assert all((part == 0xA5).all() for pair in guarded for part in pair)
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("lengths,H", [([47, 40, 30], 24),                    # operands formed by two workgroups of a chain
+                                       ([1500, 200, 300, 400, 700], 32),      # the same for the longest sequences only
+                                       ([200, 33], 3), ([300] * 6, 24)])      # prepared ahead of the sweep; a workgroup a chain
+@pytest.mark.parametrize("shared", ["q", "k", "v", "g", "q shifted", "k shifted", "beta", "dt_bias"])
+def test_kda_prefill_out_in_the_memory_of_an_input(lengths, H, shared):
+    """`out` may lie in the memory of an input: as its very rows (the call then sweeps whole chains, so that no workgroup
+    overwrites what another one has yet to read) or elsewhere in it (the input is copied first; v is not among these).  The same
+    bits as with an output of its own, through both host layers; the C entry refuses what it cannot copy."""
+    from pla_amd import _lib
+    from pla_amd.prefill.flashkdapro import flashkda_fwd, ops
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=4040 + H, pad=5)
+    T, dev, names = q.shape[0], "cuda", ("q", "k", "v", "g", "beta", "A_log", "dt_bias")
+    cu = torch.tensor(offs, dtype=torch.int32, device=dev)
+    start = dict(zip(names, (t.to(dev) for t in (q, k, v, raw, beta, A_log, dt_bias))))
+
+    def run(x, out, native):
+        ops._native = None if native else False
+        final = torch.empty_like(S0, device=dev)
+        flashkda_fwd(*(x[n] for n in names), out, initial_state=S0.to(dev), final_state=final, cu_seqlens=cu, raw_cu_seqlens=tuple(offs))
+        torch.cuda.synchronize()
+        return out, final
+    want = run(start, torch.empty(T, H, 128, dtype=torch.bfloat16, device=dev), False)
+    for native in (False, True):
+        x = {n: t.clone() for n, t in start.items()}
+        memory = torch.zeros(T + 16, H, 128, dtype=torch.bfloat16, device=dev)
+        name, out = shared.split()[0], memory[:T]
+        if shared.endswith("shifted"):
+            x[name] = memory[16:].copy_(start[name])
+        elif name == "beta":
+            x[name] = memory.view(-1)[:T * H].view(T, H).copy_(start[name])
+        elif name == "dt_bias":
+            x[name] = memory.view(-1).view(torch.float32)[:H * 128].view(H, 128).copy_(start[name])
+        else:
+            x[name] = out.copy_(start[name])
+        got = run(x, out, native)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    ops._native = False
+    prepared = _lib.load().pla_kda_prefill_workspace_bytes(T, len(lengths), H) > 4096
+    if shared == "k shifted" and not prepared:
+        ws, nbytes = ops._workspace(T, len(lengths), H, torch.device(dev))
+        memory = torch.zeros(T + 16, H, 128, dtype=torch.bfloat16, device=dev)
+        with pytest.raises(Exception, match="shares memory"):
+            _lib.call("pla_kda_prefill_launch", start["q"].data_ptr(), memory[16:].data_ptr(), start["v"].data_ptr(), start["g"].data_ptr(),
+                      start["beta"].data_ptr(), *(H * 128,) * 4, H, start["A_log"].data_ptr(), start["dt_bias"].data_ptr(), -5.0,
+                      128 ** -0.5, cu.data_ptr(), len(lengths), T, None, None, 0, None, None, 0, memory.data_ptr(), ws.data_ptr(),
+                      nbytes, H, 128, 128, _lib.BF16, torch.cuda.current_stream().cuda_stream)
