@@ -85,14 +85,30 @@ __device__ __forceinline__ uint2 quad_sat(f32x4_t x) {
   return make_uint2(pack2<f16_t>(c(x[0]), c(x[1])), pack2<f16_t>(c(x[2]), c(x[3])));
 }
 
-// Inclusive sum over the sixteen lanes of a DPP row (the tokens of a sub-chunk).
-__device__ __forceinline__ float row16_scan(float x) {
-  x += dpp_mov<0x111>(x);     // row_shr:1, 2, 4, 8; lanes outside the row count as zero
-  x += dpp_mov<0x112>(x);
-  x += dpp_mov<0x114>(x);
-  x += dpp_mov<0x118>(x);
+// Sum over the lanes from this one to the last of a DPP row (the tokens of a sub-chunk).
+__device__ __forceinline__ float row16_suffix(float x) {
+  x += dpp_mov<0x101>(x);     // row_shl:1, 2, 4, 8; lanes outside the row count as zero
+  x += dpp_mov<0x102>(x);
+  x += dpp_mov<0x104>(x);
+  x += dpp_mov<0x108>(x);
   return x;
 }
+// The value of the next lane of the row, zero in its last lane.
+__device__ __forceinline__ float row16_next(float x) { return dpp_mov<0x101>(x); }
+// x[e] *= f[e] of the next lane of the row, unchanged in its last lane (a lane that a DPP operand leaves out is not written; the
+// compiler would form the factor 1 of that lane first), or of the row's first lane (the compiler would move it first where it
+// is used twice).  The s_nop covers the wait states behind the last write before the block.
+#define PLA_MUL(X, F, FROM) "v_mul_f32_dpp " X ", " F ", " X " " FROM " row_mask:0xf bank_mask:0xf\n\t"
+#define PLA_TIMES(FROM)                                                                                                   \
+  asm("s_nop 1\n\t" PLA_MUL("%0", "%8", FROM) PLA_MUL("%1", "%9", FROM) PLA_MUL("%2", "%10", FROM)                        \
+      PLA_MUL("%3", "%11", FROM) PLA_MUL("%4", "%12", FROM) PLA_MUL("%5", "%13", FROM) PLA_MUL("%6", "%14", FROM)         \
+      PLA_MUL("%7", "%15", FROM)                                                                                          \
+      : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]), "+&v"(x[3]), "+&v"(x[4]), "+&v"(x[5]), "+&v"(x[6]), "+&v"(x[7])            \
+      : "v"(f[0]), "v"(f[1]), "v"(f[2]), "v"(f[3]), "v"(f[4]), "v"(f[5]), "v"(f[6]), "v"(f[7]))
+__device__ __forceinline__ void times_next(float (&x)[8], const float (&f)[8]) { PLA_TIMES("row_shl:1"); }
+__device__ __forceinline__ void times_first(float (&x)[8], const float (&f)[8]) { PLA_TIMES("row_newbcast:0"); }
+#undef PLA_TIMES
+#undef PLA_MUL
 // Lane 15 of the row, in every lane of it.
 __device__ __forceinline__ float row16_last(float x) { return dpp_mov<0x15F>(x); }      // row_newbcast:15
 // Sum over the four lanes (t, 0 .. 3) of a token.
