@@ -174,8 +174,9 @@ __device__ __forceinline__ void kda_sub_chunk(const KdaGate& gate, KdaRows<OUT>&
   auto half_piece = [](const float (&x)[8]) {
     return make_uint4(pack2<f16_t>(x[0], x[1]), pack2<f16_t>(x[2], x[3]), pack2<f16_t>(x[4], x[5]), pack2<f16_t>(x[6], x[7]));
   };
-  // rows past the sequence: no decay, beta = 0
-  const float beta = valid ? fast_sigmoid(to_float(bf16_t{rows.beta})) : 0.f, ib = valid ? gate.inv_bound : 1e30f;
+  // rows past the sequence: no decay, beta = 0.  (The whole division and expf: v_exp_f32 of the scaled logit and v_rcp_f32 are 3e-7
+  // from the sigmoid above -4 and 9e-7 at -12, and a token's write is proportional to it.)
+  const float beta = valid ? 1.f / (1.f + expf(-to_float(bf16_t{rows.beta}))) : 0.f, ib = valid ? gate.inv_bound : 1e30f;
   const float k_inv = inverse_norm(rows.k);
   float q_inv = 0.f;
   if constexpr (OUT) q_inv = inverse_norm(rows.q);

@@ -720,3 +720,31 @@ def test_kda_prefill_out_in_the_memory_of_an_input(lengths, H, shared):
                       start["beta"].data_ptr(), *(H * 128,) * 4, H, start["A_log"].data_ptr(), start["dt_bias"].data_ptr(), -5.0,
                       128 ** -0.5, cu.data_ptr(), len(lengths), T, None, None, 0, None, None, 0, memory.data_ptr(), ws.data_ptr(),
                       nbytes, H, 128, 128, _lib.BF16, torch.cuda.current_stream().cuda_stream)
+
+
+def test_kda_prefill_beta_is_the_sigmoid_in_fp32():
+    """Sequences of one token with value 1 and a key of 64 entries of 1 (norm 8) from a zero state: the state is beta / 8, beta as
+    the fp16 pair of W.  Every bf16 logit of -8 to 4: the pair of an FP32 number within one unit (2^-23) of the sigmoid."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    N, H = 64, 64
+    logits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).float()
+    logits = logits[(logits >= -8) & (logits <= 4) & (logits.abs() > 1e-3)]
+    beta = logits.repeat(2)[:N * H].view(N, H).bfloat16()
+    k = torch.zeros(N, H, 128, dtype=torch.bfloat16)
+    k[..., ::2] = 1.0
+    one = torch.ones(N, H, 128, dtype=torch.bfloat16)
+    final, out = torch.empty(N, H, 128, 128, device="cuda"), torch.empty_like(one).cuda()
+    flashkda_fwd(*(t.cuda() for t in (k, k, one, one, beta, torch.zeros(H), torch.zeros(H, 128))), out, final_state=final,
+                 cu_seqlens=torch.arange(N + 1, dtype=torch.int32).cuda())
+
+    def pair(x):                                 # hi to nearest, the rest toward zero
+        x = x.float()
+        hi = x.half()
+        rest = x - hi.float()
+        lo = rest.half()
+        lo = torch.where(lo.float().abs() > rest.abs(), (lo.view(torch.int16) - 1).view(torch.float16), lo)
+        return hi.double() + lo.double()
+    want, got = torch.sigmoid(beta.double()), final[:, :, 0, 0].cpu().double() * 8
+    low, high = pair(want * (1 - 2.0 ** -23)), pair(want * (1 + 2.0 ** -23))
+    outside = (got < low) | (got > high)
+    assert not outside.any(), (int(outside.sum()), ((got - want).abs() / want)[outside].max())
