@@ -128,7 +128,7 @@ struct KdaGate {
   __device__ __forceinline__ KdaGate(const KdaPrefillParams& p, int head, float* lds_bias, int lane) : bias(lds_bias) {
     const float bound = p.lower_bound * LOG2E;
     slope = -expf(p.A_log[head]) * LOG2E;
-    inv_bound = bound < 0.f ? 1.f / bound : -1e30f;
+    inv_bound = bound < -1e-30f ? 1.f / bound : -1e30f;       // (nearer to zero it decays nothing; 0 x 1 / bound has to stay a number)
 #pragma unroll
     for (int i = 0; i < 2; ++i) lds_bias[lane + 64 * i] = slope * p.dt_bias[head * 128 + lane + 64 * i];
     own_lds_order();

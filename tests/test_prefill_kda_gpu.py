@@ -748,3 +748,23 @@ def test_kda_prefill_beta_is_the_sigmoid_in_fp32():
     low, high = pair(want * (1 - 2.0 ** -23)), pair(want * (1 + 2.0 ** -23))
     outside = (got < low) | (got > high)
     assert not outside.any(), (int(outside.sum()), ((got - want).abs() / want)[outside].max())
+
+
+@pytest.mark.parametrize("lower_bound", [0.0, -1e-45, -1e-39, -1.2e-38, -1e-30])
+def test_kda_prefill_bounds_near_zero_decay_nothing(lower_bound):
+    """Bounds whose reciprocal is beyond FP32 or nearly so, with raw gates at which the sigmoid is 0, 1 and between: no decay at
+    all, the same bits as a bound of zero."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    lengths, H = [70, 5], 2
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=39)
+    raw[::3], raw[1::3] = 1000.0, -1000.0
+    args = [t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)]
+    results = []
+    for bound in (lower_bound, 0.0):
+        out, final = torch.empty_like(v).cuda(), torch.empty_like(S0).cuda()
+        flashkda_fwd(*args, out, lower_bound=bound, initial_state=S0.cuda(), final_state=final,
+                     cu_seqlens=torch.tensor(offs, dtype=torch.int32).cuda())
+        results.append((out, final))
+    torch.cuda.synchronize()
+    assert torch.isfinite(results[0][0].float()).all() and torch.isfinite(results[0][1]).all()
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
