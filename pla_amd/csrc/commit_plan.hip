@@ -2,8 +2,9 @@
 // - the slot a request reads and the up to two slots it writes, -1 for none - and then decides on its share of them: a
 // wavefront per committing request, lanes striding over the other requests, looks its slots up among everybody else's
 // claims; the claims are never modified, so a clash cancels both sides whichever is examined first.  The claims live in
-// LDS, or in the caller's scratch rows (to which all workgroups write the same values) when the capacity exceeds
-// what LDS holds.
+// LDS, or in the caller's scratch rows (to which all workgroups write the same values) when the batch exceeds
+// what LDS holds.  Workgroups behind the batch only clear their plan rows (64 requests of a capacity of 16 384: 32.9 us
+// when they classified the batch as well, 4.6 now).
 //
 // Bound by latency: the trips to memory of a classification, then batch / 64 steps of look-up per request.  One workgroup
 // doing all look-ups takes the square of the batch: a commit of 768 requests (4 heads, 1 layer) took 235 us with it and
@@ -15,7 +16,9 @@ namespace pla {
 
 constexpr int PLAN_THREADS = 256;
 constexpr int PLAN_SHARE = 4;           // requests a workgroup decides on
-constexpr int PLAN_LDS_CAPACITY = 4096; // requests whose claims fit into 48 KB of LDS (3 x 4 bytes each)
+// Up to this many requests the claims lie in LDS: 36 KB, four workgroups a CU.  us of the plan, LDS / scratch: 64 requests 4.7 / 4.3,
+// 512 4.9 / 5.3, 1024 8.1 / 8.6, 2048 15.4 / 18.8, 3072 23.4 / 27.3; 4096 (three workgroups a CU, so a second round) 53.0 / 37.4.
+constexpr int PLAN_LDS_BATCH = 3072;
 
 template <bool IN_LDS>
 __global__ __launch_bounds__(PLAN_THREADS) void commit_plan_kernel(const PlanInputs in, int share, int32_t* spill, int32_t* plan) {
@@ -24,6 +27,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void commit_plan_kernel(const PlanInp
   int32_t* const writes_final = reads + in.batch;
   int32_t* const writes_boundary = writes_final + in.batch;
   const int cap = in.capacity, first = blockIdx.x * share, last = min(first + share, cap);
+  if (first >= in.batch) {
+    for (int i = threadIdx.x; i < 4 * (last - first); i += PLAN_THREADS) plan[(i & 3) * cap + first + (i >> 2)] = 0;
+    return;
+  }
 
   for (int b = threadIdx.x; b < max(in.batch, last); b += PLAN_THREADS) {
     const Request r = classify(in, b);
@@ -74,7 +81,7 @@ extern "C" int pla_kda_commit_plan_launch(
   const int share = plan_apart(in, plan) ? PLAN_SHARE : capacity;
   const dim3 grid((unsigned)((capacity + share - 1) / share)), block(PLAN_THREADS);
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (capacity <= PLAN_LDS_CAPACITY)
+  if (batch <= PLAN_LDS_BATCH)
     commit_plan_kernel<true><<<grid, block, (size_t)batch * 3 * sizeof(int32_t), s>>>(in, share, candidate, plan);
   else
     commit_plan_kernel<false><<<grid, block, 0, s>>>(in, share, candidate, plan);

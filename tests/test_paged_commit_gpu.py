@@ -92,3 +92,39 @@ def test_commit_takes_its_sources_from_its_own_plan():
     ctx.commit(state_indices=plan.final_state_indices, **args)
     assert torch.equal(layers[0].state, want[0]) and torch.equal(layers[0].conv, want[1]) and torch.equal(ctx._buffer, want[2])
     assert plan.final_state_indices.tolist() == source
+
+
+# every workgroup decides on four requests: batches of one share and of many, the largest whose claims LDS holds and the next
+# one, a capacity far above the batch (whose workgroups only clear rows), 64-bit inputs
+@pytest.mark.parametrize("batch,capacity,wide", [(1, 1, 0), (4, 5, 0), (5, 9, 1), (300, 5000, 0), (768, 768, 1), (3072, 3072, 0),
+                                                 (3073, 3073, 0), (3100, 5003, 1), (4096, 4097, 0)])
+@pytest.mark.parametrize("align", [False, True])
+def test_commit_plan_of_many_requests_matches_the_oracle(batch, capacity, wide, align):
+    from oracle import replay_commit_plan_reference
+    from pla_amd import _lib
+    gen = torch.Generator().manual_seed(batch + int(align))
+    ri = lambda lo, hi, n: torch.randint(lo, hi, (n,), generator=gen)
+    slots, q, rows, cols = 40 * batch + 2, 4, batch + 3, 5
+    offsets = [0] + ri(1, q + 1, batch).cumsum(0).tolist()
+    source = ri(1, slots, batch)
+    some = ri(0, batch, batch // 50 + 1)
+    source[some] = source[ri(0, batch, batch // 50 + 1)]              # clashes, and slots that do not exist
+    source[ri(0, batch, batch // 100)] = slots + 3
+    # (few requests commit in a large batch: the oracle compares each of them with every other one)
+    sampled = ri(0, q + 2, rows) * (torch.rand(rows, generator=gen) < max(0.02, min(1.0, 100 / batch)))
+    computed = ri(0, BLOCK * cols, rows)
+    table = ri(1, slots, rows * cols).reshape(rows, cols)
+    lists = [t.tolist() for t in (sampled, source, computed, table)]
+    want = replay_commit_plan_reference(lists[0], lists[1], offsets, slots=slots, Q=q, token_capacity=offsets[-1], null_block_id=0,
+                                        block_table=lists[3] if align else None, num_computed_tokens=lists[2] if align else None,
+                                        block_size=BLOCK if align else None, capacity=capacity)
+    dtype = torch.int64 if wide else torch.int32
+    d_sampled, d_source, d_offsets, d_computed, d_table = (torch.as_tensor(x).to(dtype).cuda() for x in (sampled, source, offsets, computed, table))
+    scratch, plan = (torch.full((4, capacity), -9, dtype=torch.int32, device="cuda") for _ in range(2))
+    _lib.call("pla_kda_commit_plan_launch", d_sampled.data_ptr(), wide, d_source.data_ptr(), wide, d_offsets.data_ptr(), wide, None, 0,
+              d_computed.data_ptr() if align else None, wide, d_table.data_ptr() if align else None, wide, batch, capacity, rows,
+              rows if align else 0, cols if align else 0, slots, q, 0, offsets[-1], cols if align else 0, 1 if align else 0,
+              BLOCK if align else 0, scratch.data_ptr(), plan.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert plan.cpu().tolist() == want
+    assert batch < 50 or sum(n > 0 for n in want[0]) >= 20
