@@ -292,6 +292,9 @@ int pla_kda_commit_launch(
     int token_capacity, int64_t block_row_stride, int64_t block_col_stride, int64_t block_size,
     int32_t* candidate, int32_t* plan, void* stream);
 
+/* Launches pla_kda_commit_launch takes for a batch whose plan shares no memory with its inputs (host arithmetic): 1 or 3. */
+int pla_kda_commit_launches(int batch, int heads, int layers);
+
 /*
  * Conv-window rollback of the commit: dst[layer, dst_idx[r], :, :] = src[layer, r, step_idx[r], :, :]
  * for every request r with step_idx[r] >= 0, 0 <= dst_idx[r] < dst_reqs, r < src_reqs and

@@ -1033,6 +1033,10 @@ extern "C" int pla_kda_fold_native_launch(
 //    96 tiles 10.6 / 12.4 (11.6 / 13.0)   320 tiles 17.4 / 18.0 (18.4 / 18.5)   504 tiles 24.7 / 24.5 (26.7 / 25.0)
 constexpr int64_t COMMIT_ONE_LAUNCH_TILES = 320;
 
+extern "C" int pla_kda_commit_launches(int batch, int heads, int layers) {
+  return batch > 0 && (int64_t)batch * heads * layers <= COMMIT_ONE_LAUNCH_TILES ? 1 : 3;
+}
+
 extern "C" int pla_kda_commit_launch(
     const int64_t* layer_table, int layers, int heads, int channels, int rows,
     const void* sampled, int sampled_wide, const int32_t* source, const void* offsets, int offsets_wide,
@@ -1046,7 +1050,7 @@ extern "C" int pla_kda_commit_launch(
                       block_row_stride, block_col_stride, block_size};
   if (capacity == 0) return 0;
   const int32_t *const final_slots = plan + capacity, *const boundary = final_slots + capacity, *const boundary_lens = boundary + capacity;
-  const bool fused = batch > 0 && (int64_t)batch * heads * layers <= COMMIT_ONE_LAUNCH_TILES && plan_apart(in, plan);
+  const bool fused = pla_kda_commit_launches(batch, heads, layers) == 1 && plan_apart(in, plan);
   if (!fused) {
     if (const int bad = pla_kda_commit_plan_launch(
             sampled, sampled_wide, source, 0, offsets, offsets_wide, mapping, mapping_wide, computed, computed_wide, blocks, blocks_wide,

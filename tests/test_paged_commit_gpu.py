@@ -1,5 +1,6 @@
 """The paged commit in one launch against plan, fold and conv windows in three, bit for bit (the arithmetic of a tile is the
-same); and the plan of large batches, whose look-ups are spread over workgroups."""
+same), on both sides of the line between them; and the plan of large batches, whose look-ups are spread over workgroups, against
+the oracle."""
 import pytest
 import torch
 
@@ -25,14 +26,19 @@ def _context(requests, heads, q, n_layers, layout, capacity, seed):
     return KDAReplayCommitContext.create(layers, q, capacity, layout, 0), layers, source, offsets, slots, gen
 
 
+def _wide(t):
+    return int(t is not None and t.dtype == torch.int64)
+
+
 def _three_launches(ctx, sampled, source, offsets, mapping, table, computed, tokens):
     from pla_amd import _lib
     N, R, layers = source.numel(), ctx._capacity, ctx._table.shape[0]
     scratch, plan = torch.full((4, R), -9, dtype=torch.int32, device="cuda"), torch.full((4, R), -9, dtype=torch.int32, device="cuda")
     stream, ptr = torch.cuda.current_stream().cuda_stream, lambda t: None if t is None else t.data_ptr()
     rows, cols = (0, 0) if table is None else table.shape
-    _lib.call("pla_kda_commit_plan_launch", sampled.data_ptr(), 0, source.data_ptr(), 0, offsets.data_ptr(), 0, ptr(mapping), 0,
-              ptr(computed), 0, ptr(table), 0, N, R, sampled.numel(), rows, cols, ctx._slots, ctx._q, 0, tokens, cols,
+    _lib.call("pla_kda_commit_plan_launch", sampled.data_ptr(), _wide(sampled), source.data_ptr(), 0, offsets.data_ptr(), _wide(offsets),
+              ptr(mapping), _wide(mapping), ptr(computed), _wide(computed), ptr(table), _wide(table), N, R, sampled.numel(),
+              rows, cols, ctx._slots, ctx._q, 0, tokens, cols,
               0 if table is None else 1, 0 if table is None else BLOCK, scratch.data_ptr(), plan.data_ptr(), stream)
     rows4 = [plan[c].data_ptr() for c in range(4)]
     _lib.call("pla_kda_fold_native_launch", ctx._table.data_ptr(), layers, source.data_ptr(), *rows4, N, ctx._heads, ctx._q,
@@ -47,36 +53,49 @@ def _three_launches(ctx, sampled, source, offsets, mapping, table, computed, tok
 @pytest.mark.parametrize("requests,heads,q,n_layers,layout,capacity", [
     (1, 1, 1, 1, "SD", 1), (5, 3, 4, 2, "DS", 9), (17, 6, 8, 2, "SD", 20), (260, 1, 2, 1, "DS", 300), (20, 8, 3, 2, "SD", 20),
     (21, 8, 3, 2, "SD", 21)])
-@pytest.mark.parametrize("mode", ["plain", "mapping", "align"])
+@pytest.mark.parametrize("mode", ["plain", "mapping", "align", "mapping 64 bits", "align 64 bits"])
 def test_commit_in_one_launch_equals_three(requests, heads, q, n_layers, layout, capacity, mode):
+    from pla_amd import _lib
+    assert _lib.load().pla_kda_commit_launches(requests, heads, n_layers) == (3 if requests == 21 else 1)
+    mode, dtype = mode.split()[0], torch.int64 if "64" in mode else torch.int32
     ctx, layers, source, offsets, slots, gen = _context(requests, heads, q, n_layers, layout, capacity, 31 + requests)
     ri = lambda lo, hi, n: torch.randint(lo, hi, (n,), generator=gen)
-    sampled = vector(ri(0, q + 2, requests + 2).tolist())
+    sampled = vector(ri(0, q + 2, requests + 2).tolist(), dtype)
     if requests > 16:                                            # no slot, a slot beyond the pool, two requests of one slot
         source[1], source[2], source[4] = 0, slots + 5, source[3]
-    d_source, d_offsets = vector(source), vector(offsets)
-    mapping = vector(ri(-1, requests + 3, requests).tolist()) if mode == "mapping" else None
+    d_source, d_offsets = vector(source), vector(offsets, dtype)
+    mapping = vector(ri(-1, requests + 3, requests).tolist(), dtype) if mode == "mapping" else None
     table = computed = None
     kw = {}
     if mode == "align":                                          # the blocks of a request: its source, then free or foreign slots
         free = [s for s in range(1, slots) if s not in source]
         cells = [[source[b] if 0 < source[b] < slots else 1, free[b % len(free)], (7 * b) % slots] for b in range(requests)]
-        table = torch.tensor(cells + [[1, 2, 3]] * 2, dtype=torch.int32, device="cuda")
-        computed = vector(ri(0, 2 * BLOCK, requests + 2).tolist())
+        table = torch.tensor(cells + [[1, 2, 3]] * 2, dtype=dtype, device="cuda")
+        computed = vector(ri(0, 2 * BLOCK, requests + 2).tolist(), dtype)
         kw = dict(block_table=table, num_computed_tokens=computed, mamba_block_size=BLOCK)
     before = [(layer.state.clone(), layer.conv.clone()) for layer in layers]
     want_plan = _three_launches(ctx, sampled, d_source, d_offsets, mapping, table, computed, offsets[-1])
     want = [(layer.state.clone(), layer.conv.clone()) for layer in layers]
-    for layer, (state, conv) in zip(layers, before):
-        layer.state.copy_(state)
-        layer.conv.copy_(conv)
-    ctx._buffer.fill_(-9)
-    ctx.commit(sampled, d_source, d_offsets, request_indices=mapping, token_capacity=offsets[-1], **kw)
-    torch.cuda.synchronize()
-    assert torch.equal(ctx._buffer, want_plan)
     assert requests < 17 or (want_plan[0] > 0).any()
-    for layer, (state, conv) in zip(layers, want):
-        assert torch.equal(layer.state, state) and torch.equal(layer.conv, conv)
+
+    def one_call():
+        ptr = lambda t: None if t is None else t.data_ptr()
+        grid, cols = (table.shape, table.shape[1]) if table is not None else ((0, 0), 0)
+        _lib.call("pla_kda_commit_launch", ctx._table.data_ptr(), n_layers, heads, ctx._channels, ctx._rows, sampled.data_ptr(),
+                  _wide(sampled), d_source.data_ptr(), d_offsets.data_ptr(), _wide(d_offsets), ptr(mapping), _wide(mapping),
+                  ptr(computed), _wide(computed), ptr(table), _wide(table), requests, capacity, sampled.numel(), *grid, slots, q, 0,
+                  offsets[-1], cols, 1 if cols else 0, BLOCK if cols else 0, ctx._candidate.data_ptr(), ctx._buffer.data_ptr(),
+                  torch.cuda.current_stream().cuda_stream)
+    for commit in (one_call, lambda: ctx.commit(sampled, d_source, d_offsets, request_indices=mapping, token_capacity=offsets[-1], **kw)):
+        for layer, (state, conv) in zip(layers, before):
+            layer.state.copy_(state)
+            layer.conv.copy_(conv)
+        ctx._buffer.fill_(-9)
+        commit()
+        torch.cuda.synchronize()
+        assert torch.equal(ctx._buffer, want_plan)
+        for layer, (state, conv) in zip(layers, want):
+            assert torch.equal(layer.state, state) and torch.equal(layer.conv, conv)
 
 
 def test_commit_takes_its_sources_from_its_own_plan():
