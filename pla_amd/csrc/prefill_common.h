@@ -180,6 +180,7 @@ struct SegmentTable {
   float* identity;        // [128, 128]
   int seg_chunks;         // chunks per segment (0: sequences are not split)
   int max_segments;
+  int split_from;         // chunks of the longest sequence from which on any is split (KDA; GDN splits whenever seg_chunks > 0)
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -447,11 +448,14 @@ __device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n
 // The segments of a split call (at most 64 sequences), counted by one wavefront: lane n counts those of sequence n.  The sweeps
 // and the combine step between them take the same counts from here, so that they agree on every tile whatever the offsets
 // hold.
-struct SegmentCounts { int2 tokens; int count, before; };      // of this lane's sequence; segments ahead of its first
-__device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int lane) {
+struct SegmentCounts { int2 tokens; int chunks, count, before; };      // chunks: of a segment; the others: of this lane's sequence
+__device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, const SegmentTable& t, int lane) {
   SegmentCounts r;
   r.tokens = lane < N ? sequence_tokens(cu_seqlens, lane, T) : make_int2(0, 0);
-  r.count = ((r.tokens.y + CHUNK - 1) / CHUNK + seg_chunks - 1) / seg_chunks;
+  const int nc = (r.tokens.y + CHUNK - 1) / CHUNK;
+  const int longest = __builtin_amdgcn_readlane(wave_scan(nc, 0, [](int a, int b) { return max(a, b); }), 63);
+  r.chunks = longest < t.split_from ? max(longest, 1) : t.seg_chunks;
+  r.count = (nc + r.chunks - 1) / r.chunks;
   r.before = wave_inclusive_scan(r.count) - r.count;
   return r;
 }
@@ -508,7 +512,7 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
   const int n = chain / heads, h = chain - n * heads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // the sequence's segments, counted by every wavefront for itself; overlapping sequences may count more than there are tiles
-  const SegmentCounts s = count_segments(cu_seqlens, N, T, t.seg_chunks, lane);
+  const SegmentCounts s = count_segments(cu_seqlens, N, T, t, lane);
   const int first = __builtin_amdgcn_readlane(s.before, n), end = min(first + __builtin_amdgcn_readlane(s.count, n), t.max_segments);
   if (end - first < 2) return;                 // a single segment starts from the caller's state
   __shared__ __align__(16) float S[16][132];

@@ -526,7 +526,7 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
     c.fin = kda_state_out(p, item, c.head);
     return c;
   }
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, item, lane);
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, item, lane);
   if (s.sequence < 0) return c;
   c.token = s.token;
   c.tokens = s.tokens;
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
   ring_reset(&lds.flags);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = blockIdx.x / p.H;
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, item, lane);
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, item, lane);
   if (s.sequence < 0 || s.index + 1 == s.count) return;
   const int64_t tile = (int64_t)blockIdx.x * 16384;
   Chain chain{};
@@ -623,11 +623,36 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
   }
 }
 
-// Segments of a split call: as long as gives every CU at most one (segment, head), with two thirds of a segment per sequence
-// allowed for what the lengths leave over (six sequences of 2000 to 7000 tokens, 8 heads: 264 pairs 267 us, 216 pairs 233), and
-// at least this many chunks (us per call at 16 / 8: one sequence of 2048 tokens, 32 heads 129.7 / 101.7; 4096, 32 heads 192.7 /
-// 140.0; 4096, 12 heads 148.5 / 102.8; 8192, 12 heads 172.7 / 149.1).
-constexpr int KDA_SEGMENT_CHUNKS = 8;
+// Segments of a split call (at most 64 chains).  A call is priced in us from its longest sequence (L chunks) and its (segment, head)
+// pairs: not split 13.5 + 2.84 L; split into segments of s chunks, 7.8 s for the two sweeps where the second one takes prepared
+// sub-chunks as halves (pairs on half of the CUs at most; preparing them takes 0.2 per thousand tokens and heads), 12.7 s otherwise, and
+// about 2 a segment for the combine step.  Segments are at
+// least as long as gives every CU one pair, with two thirds of a segment per sequence for what the lengths leave over (a second
+// round of pairs: six sequences of 2000 to 7000 tokens, 8 heads, 264 pairs 267 us, 216 pairs 233).  us per call, s = 3 / 4 / 8 / 16 / not
+// split: one of 2047 tokens, 4 heads 66.8 / 68.3 / 89.7 / 122 / 104; 4096, 8 heads 95 / 88 / 101 / 153 / 186; 3000, 16 heads 89 / 92 / 102 /
+// 154 / 145; 2047, 32 heads 129 / 90 / 106 / 135 / 112; two of 3000, 12 heads 137 / 148 / 129 / 162 / 152.
+// Splitting pays from sequences of about 13 + 0.28 chunks per chain on (us split / not: 870 tokens, 4 heads 51.9 / 52.1; 1020 54.4 / 58.6;
+// 1150, 24 heads 68.4 / 69.2; 1300, 32 heads 73.4 / 77.8; four of 1900, 12 heads 112 / 114).  The host knows the sum of several
+// sequences only: where their mean is below that line the kernels decide by the longest one (SegmentTable::split_from), which costs
+// 4 us where it turns out that nothing is split (six of 590 tokens, 4 heads 48.2 / 44.3, split 58.7; one of 3000 among
+// short ones 76.9 / 143), and calls of less than 32 chunks are not split.
+struct KdaSplit { int chunks, from; bool halves; };      // chunks of a segment (0: not split); SegmentTable::split_from; see KdaWorkspaceLayout
+static KdaSplit kda_split(int T, int N, int H, bool prepares) {
+  const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = 13 + 9 * chains / 32;
+  KdaSplit split{0, 0, false};
+  if (N == 1 ? chunks < line : T / CHUNK < 32) return split;
+  const int per_head = std::max(1, CUS / H - 2 * N / 3), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);
+  double best = 0.;
+  for (int s = least; s <= least + 16; ++s) {
+    const double pairs = (N == 1 ? (chunks + s - 1) / s : (double)chunks / s + 0.5 * N) * H;
+    const bool halves = prepares && pairs <= CUS / 2;
+    const double price = halves ? 18.5 + 7.8 * s + 2.3 * mean / s + 2e-4 * T * H : 24. + 12.7 * s + 1.8 * mean / s;
+    if (split.chunks == 0 || price < best) best = price, split = KdaSplit{s, 0, halves};
+  }
+  if (N > 1 && mean < line && (split.halves || 4 * mean < 3 * line))
+    split = prepares ? KdaSplit{split.halves ? split.chunks : least, line, true} : KdaSplit{std::max(8, least), 0, false};
+  return split;
+}
 // Calls of at most 128 chains leave half of the CUs without a sweep: kda_prepare_kernel forms their sub-chunks on all of them
 // and the sweeps copy them (a step of 16 tokens then takes 0.7 us instead of 1.3), unless the sequences are so short that the
 // second launch costs more than it saves (us per call, prepared / formed by the sweeps: 3 sequences of 47 tokens, 24 heads 19.0 /
@@ -638,7 +663,7 @@ constexpr int KDA_PREPARE_TOKENS = 96;
 constexpr int64_t KDA_PREPARE_BYTES = (int64_t)112 << 20;
 struct KdaWorkspaceLayout {
   size_t segM, segB, segS, prepared, total;
-  int seg_chunks, max_segments;
+  int seg_chunks, split_from, max_segments;
   int64_t slots;            // prepared sub-chunks (0: the sweeps form them)
   bool halves;              // two workgroups per chain
 };
@@ -646,19 +671,14 @@ static KdaWorkspaceLayout kda_layout(int T, int N, int H) {
   KdaWorkspaceLayout L{};
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t at = off; off = align_up256(off + bytes); return at; };
-  L.seg_chunks = pick_segment_chunks(T, N, H);
-  if (L.seg_chunks > 0) {
-    const int per_head = std::max(1, CUS / H - 2 * N / 3), chunks = T / CHUNK;
-    L.seg_chunks = std::max(KDA_SEGMENT_CHUNKS, (chunks + per_head - 1) / per_head);
-  }
+  const int64_t chains = (int64_t)N * H, slots = T / SUB + N + 1;
+  const bool prepares = slots * H * KdaSlot::BYTES <= KDA_PREPARE_BYTES;
+  const KdaSplit split = chains <= 64 ? kda_split(T, N, H, prepares) : KdaSplit{0, 0, false};
+  L.seg_chunks = split.chunks;
+  L.split_from = split.from;
   L.max_segments = max_segments(T, N, L.seg_chunks);
-  // chains that sweep with output at one time (segments: a bound from the token count, exact for one sequence)
-  const int64_t chains = L.seg_chunks == 0 ? (int64_t)N * H
-      : (N == 1 ? ((T + CHUNK - 1) / CHUNK + L.seg_chunks - 1) / L.seg_chunks : (int64_t)(T / CHUNK + N) / L.seg_chunks + N) * H;
-  L.halves = chains <= CUS / 2;
-  const int64_t slots = T / SUB + N + 1;
-  const bool prepare = L.halves && (L.seg_chunks > 0 || T > KDA_PREPARE_TOKENS * (int64_t)N) && slots * H * KdaSlot::BYTES <= KDA_PREPARE_BYTES;
-  L.slots = prepare ? slots : 0;
+  L.halves = L.seg_chunks > 0 ? split.halves : chains <= CUS / 2;
+  L.slots = L.halves && prepares && (L.seg_chunks > 0 || T > KDA_PREPARE_TOKENS * (int64_t)N) ? slots : 0;
   const size_t states = (size_t)L.max_segments * H * 16384 * 4;
   L.segM = take(states); L.segB = take(states); L.segS = take(states);
   L.prepared = take((size_t)L.slots * H * KdaSlot::BYTES);
@@ -753,6 +773,7 @@ static int kda_prefill_run(
     p.seg.S = reinterpret_cast<float*>(ws + L.segS);
     p.seg.seg_chunks = L.seg_chunks;
     p.seg.max_segments = L.max_segments;
+    p.seg.split_from = L.split_from;
   }
   // Ragged whole sequences whose offsets the host holds: the chains of the longest sequences run as two halves where
   // that shortens the sweep (mixed_sweep_plan)

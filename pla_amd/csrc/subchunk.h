@@ -235,18 +235,18 @@ struct Chain {
 __device__ __forceinline__ int64_t first_slot(int n, int token) { return token / SUB + n; }
 // Segment s of a split call (count_segments).  sequence < 0: the call has fewer segments.
 struct Segment { int sequence, index, count, token, tokens; int64_t slot; };
-__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int s, int lane) {
-  const SegmentCounts c = count_segments(cu_seqlens, N, T, seg_chunks, lane);
+__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, const SegmentTable& table, int s, int lane) {
+  const SegmentCounts c = count_segments(cu_seqlens, N, T, table, lane);
   Segment r{-1, 0, 0, 0, 0, 0};
   const unsigned long long owner = __ballot(s >= c.before && s < c.before + c.count);
   if (owner == 0) return r;
   r.sequence = __builtin_amdgcn_readfirstlane(__ffsll((long long)owner) - 1);
   r.index = s - __builtin_amdgcn_readlane(c.before, r.sequence);
   r.count = __builtin_amdgcn_readlane(c.count, r.sequence);
-  const int skipped = r.index * seg_chunks * CHUNK;
+  const int skipped = r.index * c.chunks * CHUNK;
   r.token = __builtin_amdgcn_readlane(c.tokens.x, r.sequence) + skipped;
   r.slot = first_slot(r.sequence, r.token - skipped) + skipped / SUB;
-  r.tokens = min(seg_chunks * CHUNK, __builtin_amdgcn_readlane(c.tokens.y, r.sequence) - skipped);
+  r.tokens = min(c.chunks * CHUNK, __builtin_amdgcn_readlane(c.tokens.y, r.sequence) - skipped);
   return r;
 }
 

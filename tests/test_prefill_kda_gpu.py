@@ -768,3 +768,33 @@ def test_kda_prefill_bounds_near_zero_decay_nothing(lower_bound):
     torch.cuda.synchronize()
     assert torch.isfinite(results[0][0].float()).all() and torch.isfinite(results[0][1]).all()
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("lengths,H,split", [([960], 1, True), ([1000], 8, True), ([765], 1, False),        # either side of the line
+                                             ([1300, 1290], 4, True), ([600, 590, 580, 200, 130], 4, False),
+                                             ([2000, 100, 64, 17, 0, 3], 4, True), ([1000, 500, 700, 64], 16, False),
+                                             ([1500, 900, 1100, 1290], 16, False), ([2112, 600, 1100, 700], 16, True)])
+def test_kda_prefill_split_by_the_longest_sequence(lengths, H, split):
+    """A single sequence is split from 13 + 0.28 chunks per chain on; several are if they hold 32 chunks, their longest one reaches that
+    line or their mean does.  Every call against the oracle; it has the bits of a call of more than 64 chains, which is never split,
+    exactly where nothing is split."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=len(lengths) + lengths[0], pad=3)
+    raw = (raw.float() - 7.0).bfloat16()                 # (a state that outlives a segment: sums in another order show)
+    args = [t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)]
+    cu = torch.tensor(offs, dtype=torch.int32).cuda()
+    out, final = torch.empty_like(v).cuda(), torch.empty_like(S0).cuda()
+    flashkda_fwd(*args, out, initial_state=S0.cuda(), final_state=final, cu_seqlens=cu)
+    torch.cuda.synchronize()
+    want, want_final = _oracle(q, k, v, raw, beta, A_log, dt_bias, offs, S0, fast=True)
+    torch.testing.assert_close(out[:offs[-1]].cpu().float(), want[:offs[-1]].float(), atol=2e-2, rtol=2e-2)
+    assert max(rel_l2(final[n], want_final[n]) for n in range(len(lengths))) <= 1e-3
+    # more than 64 chains are never split: the same tokens with copies of the heads beyond them
+    copies = 64 // (H * len(lengths)) + 1
+    wide = [t.repeat(1, copies, *(1,) * (t.dim() - 2)) for t in args[:5]] + [args[5].repeat(copies), args[6].repeat(copies, 1)]
+    o2 = torch.empty(q.shape[0], H * copies, 128, dtype=torch.bfloat16, device="cuda")
+    f2 = torch.empty(len(lengths), H * copies, 128, 128, device="cuda")
+    flashkda_fwd(*wide, o2, initial_state=S0.cuda().repeat(1, copies, 1, 1), final_state=f2, cu_seqlens=cu)
+    torch.cuda.synchronize()
+    same = torch.equal(o2[:, :H], out) and torch.equal(f2[:, :H], final)
+    assert same == (not split)
