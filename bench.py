@@ -257,7 +257,7 @@ def bench_prefill_reference_shapes(steps, device, only=None, host_offsets=True):
 
 
 def bench_prefill_kda(steps, device, cpu_leg=False):
-    """Config 4: KDA chunk-64 prefill of one 65 536-token sequence, 32 heads (32 independent chains)."""
+    """Config 4: KDA prefill of one 65 536-token sequence, 32 heads (32 independent chains)."""
     import torch
     from pla_amd.prefill.flashkdapro import flashkda_fwd
     from pla_amd.workloads import kda_prefill

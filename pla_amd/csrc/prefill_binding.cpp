@@ -235,7 +235,7 @@ Tensor apart_from(const Tensor& t, const Tensor& out) {
   return same ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
-// KDA chunk-64 prefill: flashkda_fwd with the 15 positional arguments of the reference's _C.flashkda_fwd
+// KDA prefill: flashkda_fwd with the 15 positional arguments of the reference's _C.flashkda_fwd
 // (pla/prefill/flashkdapro/ops.py:215-219).  True: launched; False: not in the plain form, nothing launched.
 bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta, const Tensor& A_log,
                       const Tensor& dt_bias, const Tensor& out, double scale, double lower_bound, const OptTensor& initial_state,
@@ -313,7 +313,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("raw_cu_seqlens"), py::arg("final_state_dtype"));
 #endif
 #ifdef PLA_BIND_FLASHKDAPRO
-  m.doc() = "Compiled host layer of pla.prefill.flashkdapro (KDA chunk-64 prefill on gfx950)";
+  m.doc() = "Compiled host layer of pla.prefill.flashkdapro (KDA prefill on gfx950, sub-chunks of 16 tokens)";
   m.def("try_flashkda_fwd", &try_flashkda_fwd,
         "flashkda_fwd for calls in the plain form: True when launched, False (nothing launched) for any other form",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("beta"), py::arg("A_log"), py::arg("dt_bias"),

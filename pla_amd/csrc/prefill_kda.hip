@@ -15,9 +15,8 @@
 // others, one per SIMD beside them, form the operands of the next sub-chunks in LDS from the raw rows, each every fourth one.
 // A ring of eight slots with counters stands between them (subchunk.h); there is no barrier in the loop.
 // Nothing but the tokens, the outputs and the states crosses memory, and a call of many chains is one launch.  What bounds it is
-// issue: a sub-chunk costs a SIMD about 255 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 250
-// of its computing one, with 56 MFMAs that overlap little of it: 3600 cycles with 290 producing instructions, of which each of the
-// two sides alone took 2440.  Eight
+// issue: a sub-chunk costs a SIMD about 300 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 245
+// of its computing one, with 59 MFMAs that overlap little of it: 3600 cycles, of which each of the two sides alone took 2440.  Eight
 // producing wavefronts instead of four gain nothing (168 registers: the computing ones spill), nor do eight computing ones of 16
 // columns (246 against 228 us, eight sequences of 2048 tokens, 32 heads: twice the LDS reads).  Sixteen tokens decay
 // by at most 16 x |lower_bound| <= 80, so a factor and its inverse are FP32 numbers and M and P one product each; a longer chunk needs
@@ -36,8 +35,10 @@
 // against 64 bits from 2.5e-4 to 1.1e-4 (ragged prompts of 121 to 999 tokens) for 1-2 % of the time.  One product takes [hi, lo]
 // against [U, U], sixteen tokens of each filling its contraction of 32.
 //
-// (A chunk of 64 tokens with its operands prepared in memory, 82 KB written and 76 and 98 KB read back per chunk and head, took 158
-// us for 18 ragged sequences of 12 heads and 2150 us for 65 536 tokens of 32 heads; this form takes 96 and 1731.)
+// (A chunk of 64 tokens with its operands prepared in memory, 82 KB written and 76 and 98 KB read back per chunk and head, took 160
+// us for 18 ragged sequences of 12 heads and 2160 us for 65 536 tokens of 32 heads; this form takes 102 and 1760.  Chains with a CU
+// to themselves are where the longer chunk was the faster: 2.0-2.2 us for its 64 tokens against 2.84 for four dependent steps here,
+// which one sequence of 500 to 1100 tokens still shows, 870 of 16 heads 51.3 and 55.5.)
 //
 // Kernels:
 //   kda_prepare_kernel      calls of at most 128 chains: the operands of all sub-chunks, formed on every CU ahead of the sweep
@@ -136,12 +137,12 @@ struct KdaGate {
 };
 
 // One sub-chunk on one wavefront, from its raw rows to `slot` (LDS or workspace); `scratch`: 1 KiB of LDS.  `loaded` runs when the
-// raw rows have been used.  What bounds it are its vector instructions, about 1100 with 128 exponentials and reciprocals
+// raw rows have been used.  What bounds it are its vector instructions, about 1200 with 128 exponentials and reciprocals
 // among them, so it counts those: eight channels at a time go through gate, sum over the tokens, norm and decay to
 // their places; the sum over the tokens, the broadcast of the last one and the rows of the triangular solve are DPP operands,
 // the gate's bound is folded into the reciprocal of its sigmoid.  M takes its operands as bf16 pairs (e^{-G} leaves the range
-// of fp16), P as bf16: the FP32 MFMA would take them as they are, but no vector instruction of the SIMD runs beside it
-// (64 of them a sub-chunk: 130 sequences-and-heads of 2048 tokens 224 -> 198 us without).
+// of fp16), P its key factor as such a pair: the FP32 MFMA would take them as they are, but no vector instruction of the SIMD
+// runs beside it (64 of them a sub-chunk: 130 sequences-and-heads of 2048 tokens 224 -> 198 us without).
 template <bool OUT, typename Loaded>
 __device__ __forceinline__ void kda_sub_chunk(const KdaGate& gate, KdaRows<OUT>& rows, bool valid, char* slot, char* scratch, int lane,
                                               Loaded loaded) {
@@ -589,7 +590,7 @@ __global__ __launch_bounds__(64 * (4 + FEEDERS), 1) void kda_sweep_mixed_kernel(
 // First sweep over segments, both roles in one workgroup.  A segment between the first and the last of its sequence is swept
 // twice without output - from a zero state (its B summary) and from the identity with v = 0 (its transition matrix M) -
 // and both sweeps multiply the same operands: wavefronts 0-3 carry the B columns (32 each), 4-7 the M columns, 8-11 form
-// the operands.  A first segment has no M role (its wavefronts 4-7 only pass the barriers); wavefronts 0-3 sweep it from
+// the operands.  A first segment has no M role (its wavefronts 4-7 return); wavefronts 0-3 sweep it from
 // its real start state, of which they keep a copy for the second sweep.
 template <bool PREPARED>
 __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(const KdaPrefillParams p) {
@@ -698,8 +699,8 @@ extern "C" int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H) {
 // The share of a KDA chain's chunk time that one of its two half workgroups takes, and how much longer a chunk takes
 // on a full chip than on an idle one (mixed_sweep_plan).  Measured, us per call without the plan / at (0.72, 0.05) / (0.8, 0.05)
 // / (0.9, 0.05): 8000 + 7000 + 1000 + 2000 + 3000 tokens of 32 heads 728 / 597 / 599 / 645; eight ragged sequences of 32 810
-// tokens 671 / 615 / 612 / 613; twelve of 700 to 6000 tokens 564 / 478 / 479 / 481; 18 of 121 to 999 tokens of 12 heads 105 / 95 /
-// 95 / 95.
+// tokens 671 / 615 / 612 / 613; twelve of 700 to 6000 tokens 564 / 478 / 479 / 481; 18 of 121 to 999 tokens of 12 heads 111 / 102 /
+// 102 / 102.
 constexpr double KDA_HALF_COST = 0.8, KDA_FILL_COST = 0.05;
 
 // Whether the output shares memory with an input that the sweeps read where no kernel prepares their sub-chunks (q, k, g, beta and

@@ -43,7 +43,8 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
-// Eight FP32 values as a bf16 pair each: hi to nearest, lo = bf16(x - hi); x is used up (v_dot2 forms x - hi in place).
+// Eight FP32 values as a bf16 pair each: round_bf16 is hi, to nearest, rest_bf16 is lo = bf16(x - hi) (v_dot2 forms x - hi in place:
+// x is used up).
 __device__ __forceinline__ bf16x8_t round_bf16(const float (&x)[8]) {
   return __builtin_bit_cast(bf16x8_t, make_uint4(pack2<bf16_t>(x[0], x[1]), pack2<bf16_t>(x[2], x[3]), pack2<bf16_t>(x[4], x[5]),
                                                  pack2<bf16_t>(x[6], x[7])));
@@ -73,16 +74,11 @@ __device__ __forceinline__ QuadPair quad_pair(f32x4_t x) {
     const f32x2_t v = {c(a), c(b)};
     const f16x2_t h = __builtin_convertvector(v, f16x2_t);
     hi = __builtin_bit_cast(uint32_t, h);
-    lo = pack2_rtz(fmaf((float)h[0], -1.f, a), fmaf((float)h[1], -1.f, b));      // (one v_fma_mix_f32 each)
+    lo = pack2_rtz(a - (float)h[0], b - (float)h[1]);
   };
   two(x[0], x[1], r.hi.x, r.lo.x);
   two(x[2], x[3], r.hi.y, r.lo.y);
   return r;
-}
-// Four FP32 values to fp16, to nearest after a clamp.
-__device__ __forceinline__ uint2 quad_sat(f32x4_t x) {
-  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
-  return make_uint2(pack2<f16_t>(c(x[0]), c(x[1])), pack2<f16_t>(c(x[2]), c(x[3])));
 }
 
 // Sum over the lanes from this one to the last of a DPP row (the tokens of a sub-chunk).
@@ -109,8 +105,6 @@ __device__ __forceinline__ void times_next(float (&x)[8], const float (&f)[8]) {
 __device__ __forceinline__ void times_first(float (&x)[8], const float (&f)[8]) { PLA_TIMES("row_newbcast:0"); }
 #undef PLA_TIMES
 #undef PLA_MUL
-// Lane 15 of the row, in every lane of it.
-__device__ __forceinline__ float row16_last(float x) { return dpp_mov<0x15F>(x); }      // row_newbcast:15
 // Sum over the four lanes (t, 0 .. 3) of a token.
 __device__ __forceinline__ float token_sum(float x) {
   const LanePair a = swap_rows16(x);

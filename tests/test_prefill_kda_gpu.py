@@ -1,4 +1,4 @@
-"""GPU parity of the KDA chunk-64 prefill against the CPU oracle, plus the reference's closed-form
+"""GPU parity of the KDA prefill against the CPU oracle, plus the reference's closed-form
 scenarios (tests/test_kda_prefill_flashkdapro.py:243-357) evaluated on the GPU path."""
 import pytest
 import torch
@@ -338,7 +338,7 @@ def test_kda_prefill_in_a_graph(lengths, H):
 
 @pytest.mark.parametrize("lengths,pad,H", [([2500, 0, 1111, 40], 5, 2), ([4096], 0, 1), ([1030, 2049], 0, 3)])
 def test_kda_prefill_split_sequences_match_oracle(lengths, pad, H):
-    """Few, long sequences are split into 16-chunk segments that are swept concurrently (zero-state
+    """Few, long sequences are split into segments that are swept concurrently (zero-state
     and identity sweeps, a combine step, a second sweep).  Ragged lengths, an empty sequence, a
     sequence shorter than one segment, initial and final states, against the float64 oracle."""
     from pla_amd.prefill.flashkdapro import flashkda_fwd
@@ -473,17 +473,17 @@ def test_kda_prefill_correlated_keys_dense_triangular_system(lengths, noise):
                                             (700, 5, "whole")])        # 320 chains: longest first with host offsets
 @pytest.mark.parametrize("host_offsets", [False, True])
 def test_kda_prefill_64_sequences_and_65_give_the_same_bits(longest, H, path, host_offsets):
-    """Calls of at most 64 sequences work their chunk tables out inside the kernels; with more sequences a table kernel
-    runs first.  64 ragged sequences (empty ones among them, a padded tail) against the oracle, then the same tokens with
-    one empty sequence appended must give the same bits."""
+    """Calls of at most 64 sequences may be split and, with host offsets, sweep their longest sequences first and as halves; with
+    more sequences every chain is swept whole in the order of the call.  64 ragged sequences (empty ones among them, a padded
+    tail) against the oracle, then the same tokens with one empty sequence appended must give the same bits."""
     import random
     from pla_amd.prefill.flashkdapro import flashkda_fwd
     rng = random.Random(longest)
     lengths = [rng.choice((0, 1, 63, 64, 65, 130, longest // 3)) for _ in range(64)]
     lengths[7], lengths[63] = longest, 77
-    # the rules of the call of 64 sequences (pick_segment_chunks and the choice of the sweep in prefill_kda.hip)
+    # the rules of the call of 64 sequences (kda_split and the choice of the sweep in prefill_kda.hip)
     chains, chunks = 64 * H, (sum(lengths) + 9) // 64
-    segmented = chains <= 64 and 2 * max(16, -(-chunks * H // 256)) <= chunks
+    segmented = chains <= 64 and chunks >= 32
     assert path == ("segments" if segmented else "halves" if chains <= 128 else "whole")
     q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, longest, pad=9)
     results = []
@@ -571,8 +571,8 @@ def test_kda_prefill_final_state_of_short_tails_under_a_strong_gate(mean, lower_
 
 
 def test_kda_prefill_same_bits_on_both_sides_of_the_store_rule():
-    """Twelve sequences of 12 heads hold 197 MiB of operand tiles, which are stored past the caches, six of them 99 MiB, which
-    are not: the same bits, sequence by sequence."""
+    """Twelve sequences of 12 heads form their sub-chunks in the sweep, six of them take prepared ones from memory: the same bits,
+    sequence by sequence."""
     from pla_amd.prefill.flashkdapro import flashkda_fwd
     lengths, H = [1024] * 5 + [1023, 1025] + [1024] * 5, 12
     q, k, v, raw, beta, A_log, dt_bias, offs, S0 = (t.cuda() if torch.is_tensor(t) else t for t in _inputs(lengths, H, 21))
@@ -623,8 +623,9 @@ def test_kda_prefill_prepared_sub_chunks_give_the_bits_of_formed_ones(lengths, H
 
 
 def test_kda_prefill_states_and_values_beyond_the_operand_range_saturate():
-    """|v| and |S| of 1e5 and more pass the range of the fp16 operands: the results degrade, no infinity or NaN appears, and a
-    head that holds ordinary values keeps its bits."""
+    """|v| and |S| of 1e5 and more pass the range of the fp16 operands: no infinity or NaN appears, a head that holds ordinary values
+    keeps its bits, and values beyond the range are held to it with their signs: the state and the output still point where those of
+    values in range point (the cosine of a normal variable and its sign is 0.80)."""
     from pla_amd.prefill.flashkdapro import flashkda_fwd
     lengths, H = [200, 33], 3
     q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=65504)
@@ -641,6 +642,10 @@ def test_kda_prefill_states_and_values_beyond_the_operand_range_saturate():
         assert torch.isfinite(out.float()).all() and torch.isfinite(final).all()
         results.append((out, final))
     assert torch.equal(results[0][0][:, 0], results[1][0][:, 0]) and torch.equal(results[0][1][:, 0], results[1][1][:, 0])
+    for x, y in ((results[0][0][:, 1], results[1][0][:, 1]), (results[0][1][:, 1], results[1][1][:, 1])):
+        cosine = torch.nn.functional.cosine_similarity(x.double().flatten(), y.double().flatten(), dim=0).item()
+        print("saturated against in range: cosine %.3f" % cosine)
+        assert cosine > 0.6 and y.abs().max() > 1e3 * x.abs().max()
 
 
 @pytest.mark.parametrize("offsets", [(0, 1500, 9000), (-700, 1500, 4096), (0, 70000, 70001)])
