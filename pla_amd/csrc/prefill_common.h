@@ -180,7 +180,6 @@ struct SegmentTable {
   float* identity;        // [128, 128]
   int seg_chunks;         // chunks per segment (0: sequences are not split)
   int max_segments;
-  int split_from;         // chunks of the longest sequence from which on any is split (KDA; GDN splits whenever seg_chunks > 0)
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -445,16 +444,17 @@ __device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n
   const int a = min(max(cu_seqlens[n], 0), T), b = min(max(cu_seqlens[n + 1], a), T);
   return make_int2(a, b - a);
 }
-// The segments of a split call (at most 64 sequences), counted by one wavefront: lane n counts those of sequence n.  The sweeps
+// The segments of a split call (at most 64 sequences), counted by one wavefront: lane n counts those of sequence n.  With a longest
+// sequence of less than `split_from` chunks none is split.  The sweeps
 // and the combine step between them take the same counts from here, so that they agree on every tile whatever the offsets
 // hold.
 struct SegmentCounts { int2 tokens; int chunks, count, before; };      // chunks: of a segment; the others: of this lane's sequence
-__device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, const SegmentTable& t, int lane) {
+__device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int split_from, int lane) {
   SegmentCounts r;
   r.tokens = lane < N ? sequence_tokens(cu_seqlens, lane, T) : make_int2(0, 0);
   const int nc = (r.tokens.y + CHUNK - 1) / CHUNK;
   const int longest = __builtin_amdgcn_readlane(wave_scan(nc, 0, [](int a, int b) { return max(a, b); }), 63);
-  r.chunks = longest < t.split_from ? max(longest, 1) : t.seg_chunks;
+  r.chunks = longest < split_from ? max(longest, 1) : seg_chunks;
   r.count = (nc + r.chunks - 1) / r.chunks;
   r.before = wave_inclusive_scan(r.count) - r.count;
   return r;
@@ -503,7 +503,7 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 // M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes), all 64 loads of a step requested before
 // the first product.
 constexpr int COMBINE_SPLIT = 8;
-static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads) {
+static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads, int split_from) {
   // the eight workgroups of a chain read the same M tiles: on one XCD they come from memory once (xcd_grouped_index)
   const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, N * heads * COMBINE_SPLIT);
   if (logical < 0) return;
@@ -512,7 +512,7 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
   const int n = chain / heads, h = chain - n * heads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // the sequence's segments, counted by every wavefront for itself; overlapping sequences may count more than there are tiles
-  const SegmentCounts s = count_segments(cu_seqlens, N, T, t, lane);
+  const SegmentCounts s = count_segments(cu_seqlens, N, T, t.seg_chunks, split_from, lane);
   const int first = __builtin_amdgcn_readlane(s.before, n), end = min(first + __builtin_amdgcn_readlane(s.count, n), t.max_segments);
   if (end - first < 2) return;                 // a single segment starts from the caller's state
   __shared__ __align__(16) float S[16][132];

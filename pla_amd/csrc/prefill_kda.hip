@@ -65,6 +65,7 @@ struct KdaPrefillParams {
   char* prepared;                                  // sub-chunks prepared by kda_prepare_kernel (null: the sweeps form them)
   SegmentTable seg;                                // split long sequences (seg.seg_chunks > 0)
   int pass;                                        // 0: whole sequences; 1, 2: the two sweeps over segments
+  int split_from;                                  // chunks of the longest sequence from which on any is split
   int H;
   // kda_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long) as
   // two halves, the others those of seq_order[n_long .. N) whole
@@ -527,7 +528,7 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
     c.fin = kda_state_out(p, item, c.head);
     return c;
   }
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, item, lane);
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
   if (s.sequence < 0) return c;
   c.token = s.token;
   c.tokens = s.tokens;
@@ -598,7 +599,7 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
   ring_reset(&lds.flags);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = blockIdx.x / p.H;
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, item, lane);
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
   if (s.sequence < 0 || s.index + 1 == s.count) return;
   const int64_t tile = (int64_t)blockIdx.x * 16384;
   Chain chain{};
@@ -634,10 +635,10 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
 // 154 / 145; 2047, 32 heads 129 / 90 / 106 / 135 / 112; two of 3000, 12 heads 137 / 148 / 129 / 162 / 152.
 // Splitting pays from sequences of about 13 + 0.28 chunks per chain on (us split / not: 870 tokens, 4 heads 51.9 / 52.1; 1020 54.4 / 58.6;
 // 1150, 24 heads 68.4 / 69.2; 1300, 32 heads 73.4 / 77.8; four of 1900, 12 heads 112 / 114).  The host knows the sum of several
-// sequences only: where their mean is below that line the kernels decide by the longest one (SegmentTable::split_from), which costs
+// sequences only: where their mean is below that line the kernels decide by the longest one (count_segments), which costs
 // 4 us where it turns out that nothing is split (six of 590 tokens, 4 heads 48.2 / 44.3, split 58.7; one of 3000 among
 // short ones 76.9 / 143), and calls of less than 32 chunks are not split.
-struct KdaSplit { int chunks, from; bool halves; };      // chunks of a segment (0: not split); SegmentTable::split_from; see KdaWorkspaceLayout
+struct KdaSplit { int chunks, from; bool halves; };      // chunks of a segment (0: not split); KdaPrefillParams::split_from; see KdaWorkspaceLayout
 static KdaSplit kda_split(int T, int N, int H, bool prepares) {
   const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = 13 + 9 * chains / 32;
   KdaSplit split{0, 0, false};
@@ -774,7 +775,7 @@ static int kda_prefill_run(
     p.seg.S = reinterpret_cast<float*>(ws + L.segS);
     p.seg.seg_chunks = L.seg_chunks;
     p.seg.max_segments = L.max_segments;
-    p.seg.split_from = L.split_from;
+    p.split_from = L.split_from;
   }
   // Ragged whole sequences whose offsets the host holds: the chains of the longest sequences run as two halves where
   // that shortens the sweep (mixed_sweep_plan)
@@ -799,7 +800,7 @@ static int kda_prefill_run(
     p.pass = 1;
     hipLaunchKernelGGL(prepared ? kda_lean_sweep_kernel<true> : kda_lean_sweep_kernel<false>, dim3(segment_chains), lean_block, 0, s, p);
     hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
-                       N, T, H);
+                       N, T, H, p.split_from);
     p.pass = 2;
   }
   const unsigned sweeps = segmented ? segment_chains : chains;

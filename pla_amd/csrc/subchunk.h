@@ -229,8 +229,8 @@ struct Chain {
 __device__ __forceinline__ int64_t first_slot(int n, int token) { return token / SUB + n; }
 // Segment s of a split call (count_segments).  sequence < 0: the call has fewer segments.
 struct Segment { int sequence, index, count, token, tokens; int64_t slot; };
-__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, const SegmentTable& table, int s, int lane) {
-  const SegmentCounts c = count_segments(cu_seqlens, N, T, table, lane);
+__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int split_from, int s, int lane) {
+  const SegmentCounts c = count_segments(cu_seqlens, N, T, seg_chunks, split_from, lane);
   Segment r{-1, 0, 0, 0, 0, 0};
   const unsigned long long owner = __ballot(s >= c.before && s < c.before + c.count);
   if (owner == 0) return r;
