@@ -170,7 +170,7 @@ __device__ __forceinline__ void chunk_map(const int32_t* cu_seqlens, int N, int 
 //   pass 2   every segment runs from its true S_in and writes o; the last one delivers the final state
 // which costs three sweeps over a middle segment instead of one but runs them all concurrently.
 struct SegmentTable {
-  int32_t* seq_seg_off;   // [N + 1] first segment of each sequence
+  int32_t* seq_seg_off;   // [N + 1] first segment of each sequence (KDA's kernels count them: count_segments)
   int32_t* seg_seq;       // [segments] sequence of a segment
   int32_t* seg_c0;        // first chunk (global chunk index)
   int32_t* seg_nc;        // number of chunks
@@ -445,9 +445,8 @@ __device__ __forceinline__ int2 sequence_tokens(const int32_t* cu_seqlens, int n
   return make_int2(a, b - a);
 }
 // The segments of a split call (at most 64 sequences), counted by one wavefront: lane n counts those of sequence n.  With a longest
-// sequence of less than `split_from` chunks none is split.  The sweeps
-// and the combine step between them take the same counts from here, so that they agree on every tile whatever the offsets
-// hold.
+// sequence of less than `split_from` chunks none is split.  The sweeps and the combine step between them take the same counts from
+// here, so that they agree on every tile whatever the offsets hold.
 struct SegmentCounts { int2 tokens; int chunks, count, before; };      // chunks: of a segment; the others: of this lane's sequence
 __device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int split_from, int lane) {
   SegmentCounts r;
@@ -503,6 +502,7 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 // M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes), all 64 loads of a step requested before
 // the first product.
 constexpr int COMBINE_SPLIT = 8;
+template <bool TABLE>
 static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads, int split_from) {
   // the eight workgroups of a chain read the same M tiles: on one XCD they come from memory once (xcd_grouped_index)
   const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, N * heads * COMBINE_SPLIT);
@@ -511,9 +511,19 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
   const int chain = logical / COMBINE_SPLIT;
   const int n = chain / heads, h = chain - n * heads;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // the sequence's segments, counted by every wavefront for itself; overlapping sequences may count more than there are tiles
-  const SegmentCounts s = count_segments(cu_seqlens, N, T, t.seg_chunks, split_from, lane);
-  const int first = __builtin_amdgcn_readlane(s.before, n), end = min(first + __builtin_amdgcn_readlane(s.count, n), t.max_segments);
+  // the sequence's segments as the sweeps have them: from the table (GDN), or counted by every wavefront for itself; offsets
+  // of overlapping sequences may give more of them than there are tiles.  (Counting them for GDN too: 2915 tokens of 16 heads 110.3 ->
+  // 110.9 us, 8192 of 8 122.1 -> 123.2.)
+  int first, end;
+  if constexpr (TABLE) {
+    first = t.seq_seg_off[n];
+    end = t.seq_seg_off[n + 1];
+  } else {
+    const SegmentCounts s = count_segments(cu_seqlens, N, T, t.seg_chunks, split_from, lane);
+    first = __builtin_amdgcn_readlane(s.before, n);
+    end = first + __builtin_amdgcn_readlane(s.count, n);
+  }
+  end = min(end, t.max_segments);
   if (end - first < 2) return;                 // a single segment starts from the caller's state
   __shared__ __align__(16) float S[16][132];
   const int c = lane & 15, kb = lane >> 4;

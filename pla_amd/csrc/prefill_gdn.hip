@@ -1626,7 +1626,7 @@ static int gdn_prefill_run(
       });
   PLA_REQUIRE(ok, "an event call of the staged prefill failed: %s", hipGetErrorString(hipGetLastError()));
   if (segmented) {
-    hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid((unsigned)N * HV * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
+    hipLaunchKernelGGL(segment_combine_kernel<true>, dim3(xcd_grouped_grid((unsigned)N * HV * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
                        N, T, HV, 0);
     p.pass = 2;
     // Segments are at least 16 chunks long, so short calls and calls of few heads give fewer (segment, head) pairs than

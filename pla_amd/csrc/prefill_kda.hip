@@ -799,7 +799,7 @@ static int kda_prefill_run(
     // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)
     p.pass = 1;
     hipLaunchKernelGGL(prepared ? kda_lean_sweep_kernel<true> : kda_lean_sweep_kernel<false>, dim3(segment_chains), lean_block, 0, s, p);
-    hipLaunchKernelGGL(segment_combine_kernel, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
+    hipLaunchKernelGGL(segment_combine_kernel<false>, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
                        N, T, H, p.split_from);
     p.pass = 2;
   }
