@@ -431,7 +431,7 @@ int64_t pla_kda_prefill_workspace_bytes(int T, int N, int H);
  *   h0 / ht as in pla_gdn_prefill_launch (k-last FP32 [slots,H,128,128]).
  *   o may be the very rows of q, k, v or g (same address, token pitch H * 128).  Any other overlap of o with an input is the
  *   caller's to avoid: with v it is not looked for, with q, k, g, beta, A_log or dt_bias it is refused where the sweep reads
- *   them beside its writes.
+ *   them beside its writes.  ht shares memory with no input but h0: a chain stores its state while others read theirs.
  */
 int pla_kda_prefill_launch(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
