@@ -15,8 +15,10 @@
 // others, one per SIMD beside them, form the operands of the next sub-chunks in LDS from the raw rows, each every fourth one.
 // A ring of eight slots with counters stands between them (subchunk.h); there is no barrier in the loop.
 // Nothing but the tokens, the outputs and the states crosses memory, and a call of many chains is one launch.  What bounds it is
-// issue: a sub-chunk costs a SIMD about 300 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 245
-// of its computing one, with 59 MFMAs that overlap little of it: 3600 cycles, of which each of the two sides alone took 2440.  Eight
+// issue: a sub-chunk costs a SIMD about 300 vector instructions of its producing wavefront (a quarter of a sub-chunk) and 210
+// of its computing one, with 59 MFMAs that overlap little of it (with 245: 3600 cycles, of which each of the two sides alone took 2440; the
+// 35 were clamps that the saturating conversions repeat and the subtractions of quad_pair: 18 ragged sequences of 12 heads 102.3 ->
+// 99.3 us, 65 536 tokens of 32 heads 1737 -> 1684).  Eight
 // producing wavefronts instead of four gain nothing (168 registers: the computing ones spill), nor do eight computing ones of 16
 // columns (246 against 228 us, eight sequences of 2048 tokens, 32 heads: twice the LDS reads).  Sixteen tokens decay
 // by at most 16 x |lower_bound| <= 80, so a factor and its inverse are FP32 numbers and M and P one product each; a longer chunk needs
@@ -36,9 +38,9 @@
 // against [U, U], sixteen tokens of each filling its contraction of 32.
 //
 // (A chunk of 64 tokens with its operands prepared in memory, 82 KB written and 76 and 98 KB read back per chunk and head, took 160
-// us for 18 ragged sequences of 12 heads and 2160 us for 65 536 tokens of 32 heads; this form takes 102 and 1760.  Chains with a CU
-// to themselves are where the longer chunk was the faster: 2.0-2.2 us for its 64 tokens against 2.84 for four dependent steps here,
-// which one sequence of 500 to 1100 tokens still shows, 870 of 16 heads 51.3 and 55.5.)
+// us for 18 ragged sequences of 12 heads and 2160 us for 65 536 tokens of 32 heads; this form takes 99 and 1690.  Chains with a CU
+// to themselves are where the longer chunk was the faster: 2.0-2.2 us for its 64 tokens against 2.45-2.7 for four dependent steps here,
+// which one sequence of 700 to 1000 tokens of 8 to 16 heads still shows, 870 of 16 heads 51.5 and 53.0.)
 //
 // Kernels:
 //   kda_prepare_kernel      calls of at most 128 chains: the operands of all sub-chunks, formed on every CU ahead of the sweep
@@ -435,8 +437,8 @@ __device__ __forceinline__ void kda_compute(const KdaPrefillParams& p, KdaLds<OU
       f32x4_t x;
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = (nb == 0 ? lo16<bf16_t>(vraw[r]) : hi16<bf16_t>(vraw[r])) - KS[nb][r];
-      const QuadPair xp = quad_pair(x);
-      u[nb] = quad_pair(mfma16h(w, pair_of(xp.hi, xp.hi), mfma16h(w, pair_of(xp.lo, xp.lo), zero)));
+      const QuadPair xp = quad_pair<true>(x);
+      u[nb] = quad_pair<true>(mfma16h(w, pair_of(xp.hi, xp.hi), mfma16h(w, pair_of(xp.lo, xp.lo), zero)));
       uh[nb] = pair_of(u[nb].hi, u[nb].hi);
       ul[nb] = pair_of(u[nb].lo, u[nb].lo);
     }
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
   }
 }
 
-// Segments of a split call (at most 64 chains).  A call is priced in us from its longest sequence (L chunks) and its (segment, head)
+// Segments of a split call (at most 64 chains).  A call is priced in us (of steps 4 % longer than they are now) from its longest sequence (L chunks) and its (segment, head)
 // pairs: not split 13.5 + 2.84 L; split into segments of s chunks, 7.8 s for the two sweeps where the second one takes prepared
 // sub-chunks as halves (pairs on half of the CUs at most; preparing them takes 0.2 per thousand tokens and heads), 12.7 s otherwise, and
 // about 2 a segment for the combine step.  Segments are at

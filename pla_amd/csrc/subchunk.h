@@ -65,16 +65,21 @@ __device__ __forceinline__ bf16x8_t rest_bf16(const float (&x)[8], bf16x8_t hi) 
 // 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
 __device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
 
-// Four FP32 values as an fp16 pair each: hi to nearest after a clamp, the rest toward zero (as half8_pair).
+// Four FP32 values as an fp16 pair each: hi to nearest after a clamp (SATURATES: of a wavefront whose conversions do that, see
+// fp16_saturates), the rest toward zero (as half8_pair).  x - hi is one v_fma_mix_f32, which takes a half of hi as it is; the compiler
+// forms a conversion and a subtraction.  Both halves of hi come from x, so that an MFMA that wrote x has been waited for.
 struct QuadPair { uint2 hi, lo; };
+template <bool SATURATES>
 __device__ __forceinline__ QuadPair quad_pair(f32x4_t x) {
   QuadPair r;
-  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
+  auto c = [](float v) { return SATURATES ? v : __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
   auto two = [&](float a, float b, uint32_t& hi, uint32_t& lo) {
     const f32x2_t v = {c(a), c(b)};
-    const f16x2_t h = __builtin_convertvector(v, f16x2_t);
-    hi = __builtin_bit_cast(uint32_t, h);
-    lo = pack2_rtz(a - (float)h[0], b - (float)h[1]);
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+    float rest_a, rest_b;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(rest_a) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rest_b) : "v"(hi), "v"(b));
+    lo = pack2_rtz(rest_a, rest_b);
   };
   two(x[0], x[1], r.hi.x, r.lo.x);
   two(x[2], x[3], r.hi.y, r.lo.y);
@@ -177,7 +182,7 @@ __device__ __forceinline__ void solve_and_store_w(float beta, const char* scratc
   for (int r = 0; r < 4; ++r) x[r] = t == 4 * g + r ? beta : 0.f;
   eliminate(row, x);
   own_lds_order();
-  const QuadPair pair = quad_pair(f32x4_t{x[0], x[1], x[2], x[3]});
+  const QuadPair pair = quad_pair<false>(f32x4_t{x[0], x[1], x[2], x[3]});
   *reinterpret_cast<uint4*>(w_tile + 16 * lane) = make_uint4(pair.hi.x, pair.hi.y, pair.lo.x, pair.lo.y);
 }
 
