@@ -635,14 +635,15 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(c
 // round of pairs: six sequences of 2000 to 7000 tokens, 8 heads, 264 pairs 267 us, 216 pairs 233).  us per call, s = 3 / 4 / 8 / 16 / not
 // split: one of 2047 tokens, 4 heads 66.8 / 68.3 / 89.7 / 122 / 104; 4096, 8 heads 95 / 88 / 101 / 153 / 186; 3000, 16 heads 89 / 92 / 102 /
 // 154 / 145; 2047, 32 heads 129 / 90 / 106 / 135 / 112; two of 3000, 12 heads 137 / 148 / 129 / 162 / 152.
-// Splitting pays from sequences of about 13 + 0.28 chunks per chain on (us split / not: 870 tokens, 4 heads 51.9 / 52.1; 1020 54.4 / 58.6;
-// 1150, 24 heads 68.4 / 69.2; 1300, 32 heads 73.4 / 77.8; four of 1900, 12 heads 112 / 114).  The host knows the sum of several
-// sequences only: where their mean is below that line the kernels decide by the longest one (count_segments), which costs
+// Splitting pays from sequences of about 15 + 0.13 chunks per chain on, 13 + 0.28 from 13 chains on (us split / not: 770 tokens, 1 head
+// 48.5 / 42.9; 890 48.5 / 47.1; 960 49.4 / 49.6; 870, 4 heads 50.6 / 49.2; 960 51.3 / 52.3; 960, 8 heads 53.7 / 52.9; 1020 55.1 / 55.6; 870,
+// 16 heads 56.7 / 53.2; 1150 62.8 / 65.3; 1150, 24 heads 66.9 / 65.3; 1250 67.3 / 69.0; 1300, 32 heads 72.1 / 73.4; 1400 75.7 / 77.4).
+// The host knows the sum of several sequences only: where their mean is below that line the kernels decide by the longest one (count_segments), which costs
 // 4 us where it turns out that nothing is split (six of 590 tokens, 4 heads 48.2 / 44.3, split 58.7; one of 3000 among
 // short ones 76.9 / 143), and calls of less than 32 chunks are not split.
 struct KdaSplit { int chunks, from; bool halves; };      // chunks of a segment (0: not split); KdaPrefillParams::split_from; see KdaWorkspaceLayout
 static KdaSplit kda_split(int T, int N, int H, bool prepares) {
-  const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = 13 + 9 * chains / 32;
+  const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = std::max(15 + chains / 8, 13 + 9 * chains / 32);
   KdaSplit split{0, 0, false};
   if (N == 1 ? chunks < line : T / CHUNK < 32) return split;
   const int per_head = std::max(1, CUS / H - 2 * N / 3), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);

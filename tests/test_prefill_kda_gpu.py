@@ -775,12 +775,12 @@ def test_kda_prefill_bounds_near_zero_decay_nothing(lower_bound):
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
 
 
-@pytest.mark.parametrize("lengths,H,split", [([960], 1, True), ([1000], 8, True), ([765], 1, False),        # either side of the line
+@pytest.mark.parametrize("lengths,H,split", [([960], 1, True), ([1000], 8, True), ([765], 1, False), ([890], 1, False),        # either side of the line
                                              ([1300, 1290], 4, True), ([600, 590, 580, 200, 130], 4, False),
                                              ([2000, 100, 64, 17, 0, 3], 4, True), ([1000, 500, 700, 64], 16, False),
                                              ([1500, 900, 1100, 1290], 16, False), ([2112, 600, 1100, 700], 16, True)])
 def test_kda_prefill_split_by_the_longest_sequence(lengths, H, split):
-    """A single sequence is split from 13 + 0.28 chunks per chain on; several are if they hold 32 chunks, their longest one reaches that
+    """A single sequence is split from 15 + 0.13 chunks per chain on, 13 + 0.28 from 13 chains on; several are if they hold 32 chunks, their longest one reaches that
     line or their mean does.  Every call against the oracle; it has the bits of a call of more than 64 chains, which is never split,
     exactly where nothing is split."""
     from pla_amd.prefill.flashkdapro import flashkda_fwd
