@@ -66,8 +66,9 @@ __device__ __forceinline__ bf16x8_t rest_bf16(const float (&x)[8], bf16x8_t hi) 
 __device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
 
 // Four FP32 values as an fp16 pair each: hi to nearest after a clamp (SATURATES: of a wavefront whose conversions do that, see
-// fp16_saturates), the rest toward zero (as half8_pair).  x - hi is one v_fma_mix_f32, which takes a half of hi as it is; the compiler
-// forms a conversion and a subtraction.  Both halves of hi come from x, so that an MFMA that wrote x has been waited for.
+// fp16_saturates), the rest toward zero (as half8_pair).  x - hi is one v_fma_mix_f32, which takes a half of hi as it is, in the
+// place of x (in registers of its own the mixed sweep spills eight more); the compiler forms a conversion and a subtraction.  Both
+// halves of hi come from x, so that an MFMA that wrote x has been waited for.
 struct QuadPair { uint2 hi, lo; };
 template <bool SATURATES>
 __device__ __forceinline__ QuadPair quad_pair(f32x4_t x) {
@@ -76,10 +77,9 @@ __device__ __forceinline__ QuadPair quad_pair(f32x4_t x) {
   auto two = [&](float a, float b, uint32_t& hi, uint32_t& lo) {
     const f32x2_t v = {c(a), c(b)};
     hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-    float rest_a, rest_b;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(rest_a) : "v"(hi), "v"(a));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rest_b) : "v"(hi), "v"(b));
-    lo = pack2_rtz(rest_a, rest_b);
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(a) : "v"(hi));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(b) : "v"(hi));
+    lo = pack2_rtz(a, b);
   };
   two(x[0], x[1], r.hi.x, r.lo.x);
   two(x[2], x[3], r.hi.y, r.lo.y);
