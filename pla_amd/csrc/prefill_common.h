@@ -163,20 +163,22 @@ __device__ __forceinline__ void chunk_map(const int32_t* cu_seqlens, int N, int 
 // chip.  The per-token recurrence is affine in the state, S_out = S_in M + B, where for one segment
 // B is the state the segment produces from a zero state and M (K x K) is what it produces from the
 // identity with all values v = 0 (rows of the k-last state transform independently).  So:
-//   pass 1   no output.  A first segment runs from the caller's state, keeps a copy of it and delivers the state it
-//            ends in (its B); every segment between the first and the last of its sequence runs twice, from zero
-//            (-> B) and from the identity with v = 0 (-> M); the last segment does not run: nothing needs its summary
-//   combine  per (sequence, head): S_in of every later segment, S <- S M + B in FP32
-//   pass 2   every segment runs from its true S_in and writes o; the last one delivers the final state
-// which costs three sweeps over a middle segment instead of one but runs them all concurrently.
+//   pass 1   A first segment runs from the caller's state, with output: it is done with, and the state it ends in is
+//            its B (or, where it is the whole sequence, the final state); every segment between the first and the last
+//            of its sequence runs twice without output, from zero (-> B) and from the identity with v = 0 (-> M); the
+//            last segment does not run: nothing needs its summary
+//   combine  per (sequence, head): the state each middle segment ends in, S <- S M + B in FP32, in the place of its B
+//   pass 2   every later segment runs from the state its predecessor ends in and writes o; the last one delivers the
+//            final state
+// which costs three sweeps over a middle segment instead of one but runs them all concurrently.  Both passes run
+// one workgroup less per sequence and head than there are segments: a chip of 256 CUs takes nine segments of 32 heads.
 struct SegmentTable {
   int32_t* seq_seg_off;   // [N + 1] first segment of each sequence (KDA's kernels count them: count_segments)
   int32_t* seg_seq;       // [segments] sequence of a segment
   int32_t* seg_c0;        // first chunk (global chunk index)
   int32_t* seg_nc;        // number of chunks
   float* M;               // [segment, head, 128, 128] transition matrices
-  float* B;               // [segment, head, V, K] zero-state results (first segments: the state they end in)
-  float* S;               // [segment, head, V, K] state entering the segment
+  float* B;               // [segment, head, V, K] zero-state results, then the state the segment ends in (first segments: at once)
   float* identity;        // [128, 128]
   int seg_chunks;         // chunks per segment (0: sequences are not split)
   int max_segments;
@@ -297,8 +299,7 @@ struct SweepRole {
   int n, head, c_begin, c_end;
   const float* init;      // [V, K] tile the state starts from (nullptr: zero)
   float* fin;             // [V, K] tile that receives the state at the end (nullptr: none)
-  float* keep_init;       // [V, K] tile that receives a copy of the start state (nullptr: none)
-  bool zero_v, active;
+  bool zero_v, output, active;
 };
 __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, const int32_t* seq_chunk_off,
                                                   const SegmentTable& seg, const StageTable& stg, int stage,
@@ -309,10 +310,9 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
   // inline_chunks (pass 0 only, x >= 0): (first chunk, end chunk, stages in effect) of the workgroup's sequence worked
   // out by the caller (inline_sequences) instead of read from the tables
   // block: the logical workgroup index when the caller remaps blockIdx (see xcd_grouped_index), else blockIdx.x
-  // Segments: the first sweep publishes no output at all (a first segment keeps a copy of its start state and only
-  // delivers the state it ends in), the second sweep runs every segment with output.  The LAST segment of a sequence
-  // has no part in the first sweep - nothing needs its summary -: the second sweep takes it from the state the combine
-  // step (or, for a sequence of one segment, the caller) provides and delivers the final state itself.
+  // Segments: the first sweep runs a FIRST segment with output from the caller's state and those between the first and
+  // the last for their summaries; the second sweep runs every later segment with output, from the state the combine
+  // step left in its predecessor's B, and the last one delivers the final state.
   SweepRole r{};
   auto state_in = [&](int n, int head) -> const float* {
     const int slot = (h0 != nullptr) ? (h0_indices ? h0_indices[n] : n) : -1;
@@ -330,6 +330,7 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
     r.c_begin = inline_chunks.x >= 0 ? inline_chunks.x : seq_chunk_off[r.n];
     r.c_end = inline_chunks.x >= 0 ? inline_chunks.y : seq_chunk_off[r.n + 1];
     if (r.c_begin >= r.c_end) return r;              // empty sequence: state untouched, no output
+    r.output = true;
     r.init = state_in(r.n, r.head);
     r.fin = state_out(r.n, r.head);
     if (stg.stages > 0) carry = stg.carry + ((int64_t)r.n * heads + r.head) * 16384;
@@ -346,22 +347,20 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
     r.c_end = r.c_begin + seg.seg_nc[s];
     const int64_t tile = ((int64_t)s * heads + r.head) * 16384;
     if (pass == 1) {
-      if (last) return r;
       if (first) {
         if (from_identity) return r;
+        r.output = true;
         r.init = state_in(r.n, r.head);
-        r.fin = seg.B + tile;                           // B of a first segment: the state entering the second
-        carry = seg.B + tile;
-        r.keep_init = seg.S + tile;
+        r.fin = last ? state_out(r.n, r.head) : seg.B + tile;
       } else {
+        if (last) return r;
         if (from_identity) { r.init = seg.identity; r.zero_v = true; r.fin = seg.M + tile; }
         else r.fin = seg.B + tile;
-        carry = r.fin;
       }
     } else {
-      // the state entering the segment: the caller's for a sequence of one segment, else the copy its first segment
-      // kept or what the combine step stored
-      r.init = (first && last) ? state_in(r.n, r.head) : seg.S + tile;
+      if (first) return r;
+      r.output = true;
+      r.init = seg.B + tile - (int64_t)heads * 16384;
       if (last) r.fin = state_out(r.n, r.head);
     }
   }
@@ -371,7 +370,7 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
     const int nc = r.c_end - r.c_begin, c0 = r.c_begin;
     r.c_begin = c0 + stage_cut(nc, stage, E);
     r.c_end = c0 + stage_cut(nc, stage + 1, E);
-    if (stage > 0) { r.init = carry; r.keep_init = nullptr; }      // the start state is kept by stage 0 only
+    if (stage > 0) r.init = carry;
     if (stage < plan_stages(E) - 1) r.fin = carry;
   }
   r.active = true;
@@ -494,16 +493,16 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 }
 
 // Eight workgroups of 256 threads per (sequence, head), each owning 16 rows of the state (rows transform
-// independently): walks the sequence's segments and stores the state entering every later segment (the last one
-// included: the second sweep carries it to the final state).  A step S <- S M + B is a 16 x 128 x 128 product per workgroup on the FP32 MFMA
+// independently): walks the sequence's middle segments and leaves the state each of them ends in - the one that enters
+// the next - in the place of its B.  A step S <- S M + B is a 16 x 128 x 128 product per workgroup on the FP32 MFMA
 // (v_mfma_f32_16x16x4_f32, exact products, FP32 accumulation): wavefront w owns columns 32 w .. 32 w + 31 as two
 // accumulator tiles that start from B; the A operand is the workgroup's 16 rows of S from LDS (lane (r, kb) takes
 // S[r][16 s + 4 kb + e] for step (s, e)), the B operand the matching row of M straight from memory (lane (c, kb):
-// M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes), all 64 loads of a step requested before
-// the first product.
+// M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes).  M and B do not depend on the state, so those
+// of the next segment are requested before the products of this one: a step then waits for its products, not for memory.
 constexpr int COMBINE_SPLIT = 8;
 template <bool TABLE>
-static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads, int split_from) {
+static __global__ __launch_bounds__(256, 1) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads, int split_from) {
   // the eight workgroups of a chain read the same M tiles: on one XCD they come from memory once (xcd_grouped_index)
   const int logical = xcd_grouped_index(blockIdx.x, COMBINE_SPLIT, N * heads * COMBINE_SPLIT);
   if (logical < 0) return;
@@ -524,48 +523,50 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
     end = first + __builtin_amdgcn_readlane(s.count, n);
   }
   end = min(end, t.max_segments);
-  if (end - first < 2) return;                 // a single segment starts from the caller's state
-  __shared__ __align__(16) float S[16][132];
+  if (end - first < 3) return;                 // no middle segment: the second one starts from the first one's B
+  __shared__ __align__(16) float S[2][16][132];
   const int c = lane & 15, kb = lane >> 4;
   const int col0 = 32 * wave + c;              // this lane's column of accumulator tile 0 (tile 1: + 16)
   // place of accumulator element (tile cb, row v) inside a [128, 128] tile
   auto at = [&](int cb, int v) { return (int64_t)(16 * part + 4 * kb + v) * 128 + col0 + 16 * cb; };
-  f32x4_t acc[2];
-  {
-    const float* src = t.B + ((int64_t)first * heads + h) * 16384;
+  auto tile_of = [&](int seg) { return ((int64_t)seg * heads + h) * 16384; };
+  struct Operands { float m[2][32]; f32x4_t b[2]; };
+  auto request = [&](int seg, Operands& x) {
+    const float* const Mt = t.M + tile_of(seg);
+    const float* const Bt = t.B + tile_of(seg);
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[cb][v] = src[at(cb, v)];
-  }
-  for (int seg = first + 1; seg < end; ++seg) {
-    const int64_t tile = ((int64_t)seg * heads + h) * 16384;
-    // the state entering this segment: to memory for the second sweep, to LDS as the A operand of this step
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        t.S[tile + at(cb, v)] = acc[cb][v];
-        S[4 * kb + v][col0 + 16 * cb] = acc[cb][v];
-      }
-    if (seg + 1 == end) break;                 // the last segment: nothing follows it
-    // M rows and the B tile of this segment, requested before the barrier
-    const float* Mt = t.M + tile;
-    float m[2][32];
+      for (int v = 0; v < 4; ++v) x.b[cb][v] = Bt[at(cb, v)];
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb) m[cb][4 * s8 + e] = Mt[(int64_t)(16 * s8 + 4 * kb + e) * 128 + col0 + 16 * cb];
+        for (int cb = 0; cb < 2; ++cb) x.m[cb][4 * s8 + e] = Mt[(int64_t)(16 * s8 + 4 * kb + e) * 128 + col0 + 16 * cb];
+  };
+  f32x4_t acc[2];
+  {
+    const float* src = t.B + tile_of(first);
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[cb][v] = t.B[tile + at(cb, v)];
-    __syncthreads();
+      for (int v = 0; v < 4; ++v) acc[cb][v] = src[at(cb, v)];
+  }
+  const int last = end - 1;                    // the last segment has no summary
+  // S in LDS is double buffered by the parity of the step: one barrier a step
+  auto step = [&](int seg, const Operands& x, float (&Sp)[16][132]) {
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        Sp[4 * kb + v][col0 + 16 * cb] = acc[cb][v];
+        acc[cb][v] = x.b[cb][v];
+      }
+    lds_barrier();
     float4 a[8];
 #pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) a[s8] = *reinterpret_cast<const float4*>(&S[c][16 * s8 + 4 * kb]);
+    for (int s8 = 0; s8 < 8; ++s8) a[s8] = *reinterpret_cast<const float4*>(&Sp[c][16 * s8 + 4 * kb]);
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8)
 #pragma unroll
@@ -573,22 +574,27 @@ static __global__ __launch_bounds__(256) void segment_combine_kernel(SegmentTabl
         const float av = e == 0 ? a[s8].x : e == 1 ? a[s8].y : e == 2 ? a[s8].z : a[s8].w;
 #pragma unroll
         for (int cb = 0; cb < 2; ++cb)
-          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, m[cb][4 * s8 + e], acc[cb], 0, 0, 0);
+          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x.m[cb][4 * s8 + e], acc[cb], 0, 0, 0);
       }
-    __syncthreads();                           // every wavefront has read S before the next step overwrites it
+    float* const dst = t.B + tile_of(seg);
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dst[at(cb, v)] = acc[cb][v];
+  };
+  Operands even, odd;
+  request(first + 1, even);
+  for (int seg = first + 1; seg < last; seg += 2) {
+    if (seg + 1 < last) request(seg + 1, odd);
+    step(seg, even, S[0]);
+    if (seg + 1 < last) {
+      if (seg + 2 < last) request(seg + 2, even);
+      step(seg + 1, odd, S[1]);
+    }
   }
 }
 
-// Chunks per segment for a call of T tokens, N sequences and `heads` value heads: 0 (no split) unless
-// the call has at most 64 chains and the segments would be at least 16 chunks long and at least two.
-inline int pick_segment_chunks(int T, int N, int heads) {
-  if ((int64_t)N * heads > 64) return 0;
-  const int nc = T / CHUNK;
-  int seg = (int)(((int64_t)nc * heads + 255) / 256);
-  if (seg < 16) seg = 16;
-  return 2 * seg > nc ? 0 : seg;
-}
-inline int max_segments(int T, int N, int seg_chunks) { return seg_chunks > 0 ? T / CHUNK / seg_chunks + N + 1 : 0; }
+constexpr int CUS = 256;
 
 // Zero the rows of a dense [T, heads, 128] 16-bit output that lie beyond the last sequence (workgroup `block` of `blocks`).
 __device__ __forceinline__ void zero_tail(uint16_t* o, const int32_t* cu_seqlens, int N, int T, int heads, int block, int blocks) {
@@ -724,7 +730,6 @@ class SideStreamLease {
 // halves leave them, or as all the work needs on all CUs), and a chunk takes up to `fill_cost` (17 % for GDN) longer as the chip fills (3.0
 // us with a third of the CUs busy, 3.5 us with all of them: the sweeps share the memory system).  The split is taken
 // where the price falls by 5 % or more.
-constexpr int CUS = 256;
 inline int mixed_sweep_plan(const int* r, int N, int HV, unsigned char* order, double half_cost = 0.9, double fill_cost = 0.17) {
   for (int n = 0; n < N; ++n) {
     int at = n;

@@ -38,8 +38,9 @@
 //                            of at most 128 chains)
 //   gdn_fused_sweep_mixed_kernel  the same sweep for ragged whole sequences: the chains of the longest sequences as
 //                            two halves, the others whole, in one launch (plan from the host offsets)
-//   gdn_lean_sweep_kernel    first sweep over segments (no output): the zero-state and the identity sweep of a
-//                            segment side by side in one workgroup of eight wavefronts that share every tile
+//   gdn_first_sweep_kernel   first sweep over segments: first segments with output (the fused sweep), of every other but
+//                            the last one the zero-state and the identity sweep side by side in one workgroup of eight
+//                            wavefronts that share every tile
 
 #include <algorithm>
 #include <type_traits>
@@ -433,18 +434,19 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefill
 }
 
 // ---------------------------------------------------------------------------------------------
-// First sweep over segments, both roles in one workgroup.  A later segment is swept twice without output - from a
-// zero state (its B summary) and from the identity with v = 0 (its transition matrix M) - and both sweeps multiply
+// First sweep over segments, a segment between the first and the last of its sequence: swept twice without output - from
+// a zero state (its B summary) and from the identity with v = 0 (its transition matrix M) -, and both sweeps multiply
 // the same K and W tiles.  One workgroup of eight wavefronts per (segment, value head) runs them side by side:
 // wavefronts 0-3 carry the B columns (32 each), wavefronts 4-7 the M columns and, having no values to subtract,
 // also issue every global -> LDS copy, so each tile crosses memory and LDS once for the two sweeps and two
-// wavefronts share a SIMD.  A first segment has no M role: its wavefronts 4-7 only copy, wavefronts 0-3 sweep it
-// from its real start state (of which they keep a copy for the second sweep).  All tiles are double buffered by
+// wavefronts share a SIMD.  All tiles are double buffered by
 // chunk parity (90 KB of LDS: K and V in swizzled unpadded tiles, 134 us -> 124 us per sweep of 32 chunks against rows
 // padded to 272 bytes) and there is one barrier per chunk: at the barrier that opens chunk c its tiles have landed (every
 // wavefront waited for its own copies) and the buffers of chunk c - 1 are free for the copies of chunk c + 1.
+constexpr int LEAN_OFF_W = 0, LEAN_OFF_G = LEAN_OFF_W + 2 * 2 * TRI_BLOCKS * 1024, LEAN_OFF_K = LEAN_OFF_G + 2 * 1024;
+constexpr int LEAN_OFF_V = LEAN_OFF_K + 2 * TILE128_HALVES * 2, LEAN_LDS_BYTES = LEAN_OFF_V + 2 * TILE128_HALVES * 2;
 template <typename act_t>
-__global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefillParams p) {
+__device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int pair) {
   constexpr int NB = 2;
   // what gdn_wsolve_kernel left per (chunk, value head): W (six blocks hi, six lo) and the tile of decay factors
   constexpr int W_BYTES = 2 * TRI_BLOCKS * 1024, G_BYTES = GTILE_FLOATS * 4;
@@ -460,17 +462,13 @@ __global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefill
   const int cw = wave & 3;                                     // position among the four wavefronts of a role
   const int vcol = 32 * cw + r16;
 
-  // the two roles of this (segment, head): logical workgroups 2 i (zero state / real state) and 2 i + 1 (identity)
-  // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
-  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, p.seg.max_segments * p.HV);
-  if (pair < 0) return;
+  // the two roles of this (segment, head): logical workgroups 2 i (zero state) and 2 i + 1 (identity)
   const SweepRole lead = select_sweep(1, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
                                       p.ht, p.ht_indices, p.ht_slot_stride, 2 * pair);
   if (!lead.active) return;
   const SweepRole mrole = select_sweep(1, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
                                        p.ht, p.ht_indices, p.ht_slot_stride, 2 * pair + 1);
   const SweepRole& role = m_side ? mrole : lead;
-  const bool computing = role.active;                          // wave-uniform; false: wavefronts 4-7 of a first segment
   const int n = lead.n, hv = lead.head, c_begin = lead.c_begin, c_end = lead.c_end;
   const int h = hv / (p.HV / p.H);
   const int seq_start = p.cu_seqlens[n] + (c_begin - p.seq_chunk_off[n]) * CHUNK;
@@ -478,18 +476,18 @@ __global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefill
   const int n_chunks = c_end - c_begin;
   auto chunk_len = [&](int c) { return min(CHUNK, seq_len - c * CHUNK); };
 
-  __shared__ __align__(1024) uint16_t tK[2][KV_HALVES];
-  __shared__ __align__(1024) uint16_t tV[2][KV_HALVES];
   // W [parity]: the six-block operand layout (hi blocks, then lo blocks)
-  __shared__ __align__(16) uint16_t tW[2][2 * TRI_BLOCKS * 512];
+  uint16_t (*const tW)[2 * TRI_BLOCKS * 512] = reinterpret_cast<uint16_t (*)[2 * TRI_BLOCKS * 512]>(lds_all + LEAN_OFF_W);
   // decay factors: [64,128) e^{G}, [128,192) e^{G_last - G}, [192] e^{G_last}
-  __shared__ __align__(16) float tG[2][256];
+  float (*const tG)[256] = reinterpret_cast<float (*)[256]>(lds_all + LEAN_OFF_G);
+  uint16_t (*const tK)[KV_HALVES] = reinterpret_cast<uint16_t (*)[KV_HALVES]>(lds_all + LEAN_OFF_K);
+  uint16_t (*const tV)[KV_HALVES] = reinterpret_cast<uint16_t (*)[KV_HALVES]>(lds_all + LEAN_OFF_V);
 
   // S^T slices in accumulator layout: St[nb][mc][r] = S[v = vcol + 16 nb][c = 16 mc + 4 kb + r]
   f32x4_t St[NB][8];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
-    if (computing && role.init != nullptr) {
+    if (role.init != nullptr) {
       const float* src = role.init + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc) {
@@ -500,16 +498,7 @@ __global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefill
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc) St[nb][mc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-  if (computing && role.keep_init != nullptr) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      float* dst = role.keep_init + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
-#pragma unroll
-      for (int mc = 0; mc < 8; ++mc)
-        *reinterpret_cast<float4*>(dst + 16 * mc) = make_float4(St[nb][mc].x, St[nb][mc].y, St[nb][mc].z, St[nb][mc].w);
-    }
-  }
-  const bool use_v = computing && !role.zero_v;                // the identity sweep runs with v = 0
+  const bool use_v = !role.zero_v;                // the identity sweep runs with v = 0
   // LDS reads.  K operand of contraction step s for row block mi; the lane's V values of rows 16 mi + 4 kb .. + 3, column
   // vcol + 16 nb, by one transposing read: lane t of a group of 16 addresses columns 32 cw + 16 nb + 4 (t % 4) .. + 3 of
   // row 16 mi + 4 kb + t / 4, which in a swizzled tile is half (t % 2) of granule 4 cw + 2 nb + (t % 4) / 2; the
@@ -565,7 +554,6 @@ __global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefill
     wait_vmcnt<0>();                                 // this wavefront's copies for chunk ci have landed
     __syncthreads();                                 // ... and chunk ci - 1 is finished: its buffers are free
     if (m_side && ci + 1 < n_chunks) issue(ci + 1);
-    if (!computing) continue;
     const uint16_t* const K = tK[par];
     const uint16_t* const V = tV[par];
     const float* const G = tG[par];
@@ -701,7 +689,7 @@ __global__ __launch_bounds__(512, 1) void gdn_lean_sweep_kernel(const GdnPrefill
     }
   }
 
-  if (computing && role.fin != nullptr) {
+  if (role.fin != nullptr) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       float* dst = role.fin + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
@@ -769,7 +757,7 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
     inline_chunks = int3{seq_first_chunk, min(seq_first_chunk + __builtin_amdgcn_readlane(seqs.nc, n0), p.NC_max), seqs.E};
   }
   const SweepRole role = select_sweep(p.pass, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
-                                      p.ht, p.ht_indices, p.ht_slot_stride, block, inline_chunks);
+                                      p.ht, p.ht_indices, p.ht_slot_stride, p.pass == 1 ? 2 * block : block, inline_chunks);
   if (!role.active) return;
   const int n = role.n, hv = role.head, c_begin = role.c_begin, c_end = role.c_end;
   const int h = hv / (p.HV / p.H);
@@ -1005,15 +993,6 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc) St[nb][mc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-  if (role.keep_init != nullptr) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      float* dst = role.keep_init + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
-#pragma unroll
-      for (int mc = 0; mc < 8; ++mc)
-        *reinterpret_cast<float4*>(dst + 16 * mc) = make_float4(St[nb][mc].x, St[nb][mc].y, St[nb][mc].z, St[nb][mc].w);
-    }
-  }
   uint16_t* const o_lane = reinterpret_cast<uint16_t*>(p.o) + ((int64_t)(seq_start + r16) * p.HV + hv) * 128 + vbase + 4 * kb;
   // V through the transposing read: lane t of a group addresses columns vbase + 16 nb + 4 (t % 4) .. + 3 of row
   // 16 mi + 4 kb + t / 4, i.e. half (t % 2) of granule 4 wave + 2 nb + (t % 4) / 2; the swizzle 8 (kb & 1) + 2 (t / 4)
@@ -1351,9 +1330,24 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
   }
 }
 
+// First sweep over segments: first segments for good, with output, from their real start states (which takes as long per
+// chunk as the two roles of the others), those behind them for their summaries.
+template <typename act_t>
+__global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefillParams p) {
+  static_assert(LEAN_LDS_BYTES <= FUSED_LDS_BYTES, "one array serves both sweeps");
+  __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
+  // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
+  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, p.seg.max_segments * p.HV);
+  if (pair < 0) return;
+  const int s = pair / p.HV;
+  if (s >= p.seg.seq_seg_off[p.N]) return;
+  if (s == p.seg.seq_seg_off[p.seg.seg_seq[s]]) fused_sweep<act_t, 2>(p, lds_all, pair);
+  else lean_sweep<act_t>(p, lds_all, pair);
+}
+
 struct GdnWorkspaceLayout {
   size_t seq_chunk_off, chunk_seq, chunk_tok, chunk_len, q_rows, k_rows, kn, kinv, gtile, W;
-  size_t seq_seg_off, seg_seq, seg_c0, seg_nc, segM, segB, segS, identity;
+  size_t seq_seg_off, seg_seq, seg_c0, seg_nc, segM, segB, identity;
   size_t order, stage_begin, carry, total;
   int NC_max, seg_chunks, max_segments, stages;
 };
@@ -1375,7 +1369,31 @@ static int mixed_sweep_from_offsets(const int32_t* raw_cu_seqlens, int N, int HV
   return mixed_sweep_plan(r, N, HV, order);
 }
 
-static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_stages = true) {
+// Chunks per segment for a call of at most 64 (sequence, value head) chains and at least 32 chunks, 0: not split.  A length of s
+// chunks is priced in us from the call's longest sequence (of several the host has the mean only, which random lengths exceed by
+// about half): 4.4 s for the two sweeps where the second one runs as halves ((segment, head) pairs on half of the CUs at most),
+// 6.5 s otherwise, and 1.2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep,
+// which runs one segment less per sequence than there are (of N sequences it counts a third of that).  us per call, s = 3 / 4 / 5 / 6 / 8
+// / 10 / 16 / not split: one of 2048 tokens, 16 value heads 71 / 65.5 / 66.6 / 68.9 / 74.3 / 83 / 107 / 82.2; 32 heads 100 / 78.2 / 76.2 / 78.3 /
+// 80.0 / 86.6 / 110 / 85.5; 64 heads - / 120 / 122 / 120 / 92.5 / 101 / 112 / 87.5; 4096, 16 heads - / - / 88.0 / 87.3 / 88.5 / 92.0 / 115.6 / 152; 32
+// heads - / - / 132 / 136 / 103.5 / 106.8 / 120.7 / 153.6; 8192, 8 heads - / - / - / - / - / 104.7 / 122.8 / 284.  (Segments of 16 chunks
+// at least, as before: the column of 16.)
+static int gdn_segment_chunks(int T, int N, int HV) {
+  if ((int64_t)N * HV > 64 || T / CHUNK < 32) return 0;
+  const int chunks = N == 1 ? (T - 1) / CHUNK + 1 : T / CHUNK, pairs = CUS + HV * (N == 1 ? 1 : N / 3);
+  const double longest = N == 1 ? chunks : std::min<double>(chunks, 1.5 * chunks / N);
+  const int least = std::max(3, (int)(((int64_t)chunks * HV + pairs - 1) / pairs));
+  int best = 0;
+  double best_price = 0.;
+  for (int s = least; s <= least + 16; ++s) {
+    const double swept = (N == 1 ? (chunks - 1) / s : std::max(0., (double)chunks / s - 0.5 * N)) * HV;
+    const double price = (swept <= CUS / 2 ? 4.4 : 6.5) * s + 1.2 * longest / s;
+    if (best == 0 || price < best_price) best_price = price, best = s;
+  }
+  return best;
+}
+
+static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chunks, bool allow_stages) {
   GdnWorkspaceLayout L;
   L.NC_max = T / CHUNK + N;
   size_t off = 0;
@@ -1390,15 +1408,15 @@ static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_sta
   L.kinv = take((size_t)T * H * 4);
   L.gtile = take((size_t)L.NC_max * HV * GTILE_FLOATS * 4);
   L.W = take((size_t)L.NC_max * HV * 2 * TRI_BLOCKS * 1024);
-  L.seg_chunks = pick_segment_chunks(T, N, HV);
-  L.max_segments = max_segments(T, N, L.seg_chunks);
+  L.seg_chunks = seg_chunks;
+  L.max_segments = seg_chunks == 0 ? 0 : N == 1 ? (T - 1) / CHUNK / seg_chunks + 1 : (T / CHUNK + N) / seg_chunks + N;
   if (L.seg_chunks > 0) {
     L.seq_seg_off = take((size_t)(N + 1) * 4);
     L.seg_seq = take((size_t)L.max_segments * 4);
     L.seg_c0 = take((size_t)L.max_segments * 4);
     L.seg_nc = take((size_t)L.max_segments * 4);
     const size_t states = (size_t)L.max_segments * HV * 16384 * 4;
-    L.segM = take(states); L.segB = take(states); L.segS = take(states);
+    L.segM = take(states); L.segB = take(states);
     L.identity = take(16384 * 4);
   }
   // pipeline the preparation with the sweeps in stages where that pays
@@ -1411,7 +1429,18 @@ static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_sta
   L.total = off;
   return L;
 }
-
+// The plan of a call is one for all entry points, so where segments as short as that would outgrow the library's own array, calls
+// small enough for it with segments of 16 chunks (of three tiles each, which it has always taken) get the shortest that fit.
+static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_stages = true) {
+  const int best = gdn_segment_chunks(T, N, HV);
+  const size_t tile = (size_t)HV * 16384 * 4, before = 3 * (size_t)(T / CHUNK / 16 + N + 1) * tile;
+  if (best > 0 && gdn_layout_of(T, N, H, HV, 0, false).total + before <= PLA_GDN_PREFILL_STATIC_BYTES)
+    for (int s = best; s <= 4 * best; ++s) {
+      const GdnWorkspaceLayout L = gdn_layout_of(T, N, H, HV, s, allow_stages);
+      if (L.total <= PLA_GDN_PREFILL_STATIC_BYTES) return L;
+    }
+  return gdn_layout_of(T, N, H, HV, best, allow_stages);
+}
 
 // Workspace of pla_gdn_prefill_launch_static: one array per GPU, held until the process ends.  In host code the
 // array's name is only a handle for the runtime, not a device address; the address on the current device comes from
@@ -1533,7 +1562,6 @@ static int gdn_prefill_run(
     p.seg.seg_nc = reinterpret_cast<int32_t*>(ws + L.seg_nc);
     p.seg.M = reinterpret_cast<float*>(ws + L.segM);
     p.seg.B = reinterpret_cast<float*>(ws + L.segB);
-    p.seg.S = reinterpret_cast<float*>(ws + L.segS);
     p.seg.identity = reinterpret_cast<float*>(ws + L.identity);
     p.seg.seg_chunks = L.seg_chunks;
     p.seg.max_segments = L.max_segments;
@@ -1598,10 +1626,10 @@ static int gdn_prefill_run(
         }
       },
       [&](unsigned grid) {
-        if (p.pass == 1) {        // first sweep over segments: no output, both roles in one workgroup per (segment, head)
+        if (p.pass == 1) {        // first sweep over segments
           const unsigned g = xcd_grouped_grid(grid / 2, (unsigned)(HV / H));
-          if (half_act) hipLaunchKernelGGL(gdn_lean_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
-          else hipLaunchKernelGGL(gdn_lean_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
+          if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
+          else hipLaunchKernelGGL(gdn_first_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
         } else {
           // Whole sequences that give at most 128 chains (few long ones are split into segments instead) leave half of the CUs idle: two
           // workgroups then sweep a chain, 64 V columns each - the columns of V are independent, so the results are the
@@ -1629,15 +1657,15 @@ static int gdn_prefill_run(
     hipLaunchKernelGGL(segment_combine_kernel<true>, dim3(xcd_grouped_grid((unsigned)N * HV * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
                        N, T, HV, 0);
     p.pass = 2;
-    // Segments are at least 16 chunks long, so short calls and calls of few heads give fewer (segment, head) pairs than
-    // half of the CUs: the second sweep then runs two workgroups per pair, 64 V columns each, as above.  The number of
-    // segments is known exactly where the caller passed the offsets on the host, else from the tokens alone.
-    int64_t segments = N == 1 ? ((T + CHUNK - 1) / CHUNK + L.seg_chunks - 1) / L.seg_chunks : (int64_t)(T / CHUNK + N) / L.seg_chunks + N;
+    // Short calls and calls of few heads give fewer (segment, head) pairs than half of the CUs: the second sweep then runs
+    // two workgroups per pair, 64 V columns each, as above.  The number of segments that it sweeps is known exactly where
+    // the caller passed the offsets on the host, else from the tokens alone.
+    int64_t segments = N == 1 ? L.max_segments - 1 : (int64_t)(T / CHUNK + N) / L.seg_chunks;
     if (raw_cu_seqlens != nullptr) {
       segments = 0;
       for (int n = 0; n < N; ++n) {
         const int nc = (std::max(raw_cu_seqlens[n + 1] - raw_cu_seqlens[n], 0) + CHUNK - 1) / CHUNK;
-        segments += (nc + L.seg_chunks - 1) / L.seg_chunks;
+        segments += std::max(0, nc - 1) / L.seg_chunks;
       }
     }
     if (segments * HV <= 128) {

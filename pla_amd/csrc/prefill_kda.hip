@@ -48,8 +48,8 @@
 //                           columns each (calls of at most 128 chains)
 //   kda_sweep_mixed_kernel  ragged whole sequences: the chains of the longest sequences as two halves, the others whole, in one
 //                           launch (plan from the host offsets)
-//   kda_lean_sweep_kernel   first sweep over segments: the zero-state sweep and the transition-matrix sweep of a segment
-//                           in one workgroup that forms the operands once for both, no output
+//   kda_first_sweep_kernel  first sweep over segments: first segments with output, of every other but the last one the zero-state
+//                           sweep and the transition-matrix sweep in one workgroup that forms the operands once for both
 
 #include "subchunk.h"
 
@@ -362,7 +362,6 @@ __device__ __forceinline__ void kda_compute(const KdaPrefillParams& p, KdaLds<OU
         *reinterpret_cast<float4*>(tile + (int64_t)(vcol + nb) * 128 + 32 * (b >> 1) + 8 * g + 4 * (b & 1)) =
             make_float4(St[nb][b][0], St[nb][b][1], St[nb][b][2], St[nb][b][3]);
   };
-  if (chain.keep != nullptr) store_state(chain.keep);
 
   // V: NB adjacent values of rows 4 g + r of a sub-chunk, requested AHEAD sub-chunks ahead; o likewise.  Both through buffers that
   // end with the chain (rows beyond read as zero and are not written), so that a step has no branch for them.
@@ -531,13 +530,11 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
     return c;
   }
   const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0) return c;
+  if (s.sequence < 0 || s.index == 0) return c;      // (the first sweep was done with the first segments)
   c.token = s.token;
   c.tokens = s.tokens;
   c.slot = s.slot;
-  // the state entering the segment: the caller's for a sequence of one segment, else the copy its first segment kept or
-  // what the combine step stored
-  c.init = s.count == 1 ? kda_state_in(p, s.sequence, c.head) : p.seg.S + (int64_t)index * 16384;
+  c.init = p.seg.B + (int64_t)(index - p.H) * 16384;  // the state its predecessor ends in
   if (s.index + 1 == s.count) c.fin = kda_state_out(p, s.sequence, c.head);
   return c;
 }
@@ -590,40 +587,41 @@ __global__ __launch_bounds__(64 * (4 + FEEDERS), 1) void kda_sweep_mixed_kernel(
   }
 }
 
-// First sweep over segments, both roles in one workgroup.  A segment between the first and the last of its sequence is swept
-// twice without output - from a zero state (its B summary) and from the identity with v = 0 (its transition matrix M) -
-// and both sweeps multiply the same operands: wavefronts 0-3 carry the B columns (32 each), 4-7 the M columns, 8-11 form
-// the operands.  A first segment has no M role (its wavefronts 4-7 return); wavefronts 0-3 sweep it from
-// its real start state, of which they keep a copy for the second sweep.
+// First sweep over segments.  A segment between the first and the last of its sequence is swept twice without
+// output - from a zero state (its B summary) and from the identity with v = 0 (its transition matrix M) - and both sweeps
+// multiply the same operands: wavefronts 0-3 carry the B columns (32 each), 4-7 the M columns, 8-11 form the operands.  A
+// first segment is swept from its real start state and for good, with output: wavefronts 0-7 carry 16 columns each (with 32
+// they need more registers than twelve wavefronts leave them), which takes about as long as the two roles of the others.
 template <bool PREPARED>
-__global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_lean_sweep_kernel(const KdaPrefillParams p) {
-  __shared__ KdaLds<false> lds;
-  ring_reset(&lds.flags);
+__global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_first_sweep_kernel(const KdaPrefillParams p) {
+  __shared__ union { KdaLds<true> out; KdaLds<false> lean; } lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = blockIdx.x / p.H;
   const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0 || s.index + 1 == s.count) return;
+  if (s.sequence < 0 || (s.index > 0 && s.index + 1 == s.count)) return;
   const int64_t tile = (int64_t)blockIdx.x * 16384;
   Chain chain{};
   chain.token = s.token;
   chain.tokens = s.tokens;
   chain.slot = s.slot;
   chain.head = blockIdx.x - item * p.H;
+  if (s.index == 0) {
+    ring_reset(&lds.out.flags);
+    chain.init = kda_state_in(p, s.sequence, chain.head);
+    chain.fin = s.count == 1 ? kda_state_out(p, s.sequence, chain.head) : p.seg.B + tile;
+    if (wave < 8) kda_compute<1, true>(p, lds.out, chain, lane, 16 * wave);
+    else if (PREPARED) kda_copy<true, FEEDERS>(p, lds.out, chain, lane, wave - 8, 8);
+    else kda_produce<true, FEEDERS>(p, lds.out, chain, lane, wave - 8, 8);
+    return;
+  }
+  ring_reset(&lds.lean.flags);
   if (wave >= 8) {
-    const uint32_t readers = s.index == 0 ? 4 : 8;
-    if (PREPARED) kda_copy<false, FEEDERS>(p, lds, chain, lane, wave - 8, readers);
-    else kda_produce<false, FEEDERS>(p, lds, chain, lane, wave - 8, readers);
-  } else if (wave < 4) {
-    if (s.index == 0) {
-      chain.init = kda_state_in(p, s.sequence, chain.head);
-      chain.keep = p.seg.S + tile;
-    }
-    chain.fin = p.seg.B + tile;
-    kda_compute<2, false>(p, lds, chain, lane, 32 * wave);
-  } else if (s.index > 0) {
-    chain.identity = true;
-    chain.fin = p.seg.M + tile;
-    kda_compute<2, false>(p, lds, chain, lane, 32 * (wave - 4));
+    if (PREPARED) kda_copy<false, FEEDERS>(p, lds.lean, chain, lane, wave - 8, 8);
+    else kda_produce<false, FEEDERS>(p, lds.lean, chain, lane, wave - 8, 8);
+  } else {
+    chain.identity = wave >= 4;
+    chain.fin = (chain.identity ? p.seg.M : p.seg.B) + tile;
+    kda_compute<2, false>(p, lds.lean, chain, lane, 32 * (wave & 3));
   }
 }
 
@@ -646,10 +644,10 @@ static KdaSplit kda_split(int T, int N, int H, bool prepares) {
   const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = std::max(15 + chains / 8, 13 + 9 * chains / 32);
   KdaSplit split{0, 0, false};
   if (N == 1 ? chunks < line : T / CHUNK < 32) return split;
-  const int per_head = std::max(1, CUS / H - 2 * N / 3), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);
+  const int per_head = std::max(1, CUS / H + (N == 1 ? 1 : N / 3)), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);
   double best = 0.;
   for (int s = least; s <= least + 16; ++s) {
-    const double pairs = (N == 1 ? (chunks + s - 1) / s : (double)chunks / s + 0.5 * N) * H;
+    const double pairs = (N == 1 ? (chunks - 1) / s : (double)chunks / s - 0.5 * N) * H;
     const bool halves = prepares && pairs <= CUS / 2;
     const double price = halves ? 18.5 + 7.8 * s + 2.3 * mean / s + 2e-4 * T * H : 24. + 12.7 * s + 1.8 * mean / s;
     if (split.chunks == 0 || price < best) best = price, split = KdaSplit{s, 0, halves};
@@ -667,7 +665,7 @@ static KdaSplit kda_split(int T, int N, int H, bool prepares) {
 constexpr int KDA_PREPARE_TOKENS = 96;
 constexpr int64_t KDA_PREPARE_BYTES = (int64_t)112 << 20;
 struct KdaWorkspaceLayout {
-  size_t segM, segB, segS, prepared, total;
+  size_t segM, segB, prepared, total;
   int seg_chunks, split_from, max_segments;
   int64_t slots;            // prepared sub-chunks (0: the sweeps form them)
   bool halves;              // two workgroups per chain
@@ -681,11 +679,11 @@ static KdaWorkspaceLayout kda_layout(int T, int N, int H) {
   const KdaSplit split = chains <= 64 ? kda_split(T, N, H, prepares) : KdaSplit{0, 0, false};
   L.seg_chunks = split.chunks;
   L.split_from = split.from;
-  L.max_segments = max_segments(T, N, L.seg_chunks);
+  L.max_segments = L.seg_chunks > 0 ? T / CHUNK / L.seg_chunks + N + 1 : 0;
   L.halves = L.seg_chunks > 0 ? split.halves : chains <= CUS / 2;
   L.slots = L.halves && prepares && (L.seg_chunks > 0 || T > KDA_PREPARE_TOKENS * (int64_t)N) ? slots : 0;
   const size_t states = (size_t)L.max_segments * H * 16384 * 4;
-  L.segM = take(states); L.segB = take(states); L.segS = take(states);
+  L.segM = take(states); L.segB = take(states);
   L.prepared = take((size_t)L.slots * H * KdaSlot::BYTES);
   L.total = off > 0 ? off : 256;                 // (never empty: a null workspace is refused)
   return L;
@@ -775,7 +773,6 @@ static int kda_prefill_run(
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
     p.seg.M = reinterpret_cast<float*>(ws + L.segM);
     p.seg.B = reinterpret_cast<float*>(ws + L.segB);
-    p.seg.S = reinterpret_cast<float*>(ws + L.segS);
     p.seg.seg_chunks = L.seg_chunks;
     p.seg.max_segments = L.max_segments;
     p.split_from = L.split_from;
@@ -792,16 +789,15 @@ static int kda_prefill_run(
     mixed = p.n_long > 0 || (int64_t)N * H > CUS;
     p.split_grid = xcd_grouped_grid(2 * (unsigned)p.n_long * H, 2);
   }
-  const dim3 sweep_block(64 * (4 + FEEDERS)), lean_block(64 * (8 + FEEDERS));
+  const dim3 sweep_block(64 * (4 + FEEDERS)), first_block(64 * (8 + FEEDERS));
   const unsigned chains = (unsigned)N * H, segment_chains = (unsigned)L.max_segments * H;
   if (prepared) {
     p.prepared = ws + L.prepared;
     hipLaunchKernelGGL(kda_prepare_kernel, dim3((unsigned)((L.slots * H + PREPARE_WAVES - 1) / PREPARE_WAVES)), dim3(64 * PREPARE_WAVES), 0, s, p);
   }
   if (segmented) {
-    // the first sweep over segments publishes no output: both of its roles in one workgroup per (segment, head)
     p.pass = 1;
-    hipLaunchKernelGGL(prepared ? kda_lean_sweep_kernel<true> : kda_lean_sweep_kernel<false>, dim3(segment_chains), lean_block, 0, s, p);
+    hipLaunchKernelGGL(prepared ? kda_first_sweep_kernel<true> : kda_first_sweep_kernel<false>, dim3(segment_chains), first_block, 0, s, p);
     hipLaunchKernelGGL(segment_combine_kernel<false>, dim3(xcd_grouped_grid(chains * COMBINE_SPLIT, COMBINE_SPLIT)), dim3(256), 0, s, p.seg, cu_seqlens,
                        N, T, H, p.split_from);
     p.pass = 2;

@@ -226,7 +226,6 @@ struct Chain {
   int64_t slot;           // number of its first sub-chunk among prepared ones
   const float* init;      // [V, K] tile the state starts from (nullptr: zero)
   float* fin;             // [V, K] tile that receives the state at the end (nullptr: none)
-  float* keep;            // [V, K] tile that receives a copy of the start state (nullptr: none)
   bool identity;          // the state starts from the identity and v is zero: the segment's transition matrix
 };
 // Sub-chunk i of sequence n is number first_slot + i among the prepared ones of a call: sequences do not overlap in it, whatever

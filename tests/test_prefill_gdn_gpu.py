@@ -272,6 +272,19 @@ def test_gdn_prefill_split_sequences_match_oracle(lengths, tail_pad, H, HV):
     _check(w, fast=True)
 
 
+@pytest.mark.parametrize("lengths,tail_pad,H,HV", [
+    ([2048], 0, 1, 4), ([2049], 3, 2, 4),                              # segments of three chunks; a last one of one token
+    ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2),                  # one, two, three and more segments a sequence
+    ([3000, 5], 0, 8, 32), ([2111], 0, 16, 64)])                       # second sweep over whole pairs; few, long segments
+def test_gdn_prefill_segments_at_their_edges(lengths, tail_pad, H, HV):
+    """A first segment of a split sequence is swept once, with output; the combine step only concerns the segments between
+    the first and the last: sequences of one, of two and of many segments, ends one token beyond a segment's and one short of
+    it.  Against the oracle, at the bounds of the whole file."""
+    from pla_amd.workloads import gdn_prefill_packed
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 3, seed=50 + sum(lengths), tail_pad=tail_pad)
+    _check(w, fast=True)
+
+
 def test_gdn_prefill_staged_pipeline_matches_oracle_and_unstaged_bits():
     """With at least 128 chains and 16 chunks per sequence on average the preparation and the sweep
     are pipelined in stages on two streams.  Ragged lengths with an empty sequence and sequences

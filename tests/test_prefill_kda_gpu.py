@@ -367,6 +367,25 @@ def test_kda_prefill_split_sequences_match_oracle(lengths, pad, H):
                 assert rel_l2(final[n, head], exp_final[n, head]) <= 1e-3, (n, head)
 
 
+@pytest.mark.parametrize("lengths,H", [([1025], 1), ([2048], 2), ([191, 192, 193, 0, 1, 384, 385, 1300], 2),    # prepared sub-chunks
+                                       ([4500], 32)])                                                          # formed by the sweeps
+def test_kda_prefill_segments_at_their_edges(lengths, H):
+    """A first segment of a split sequence is swept once, with output, by eight wavefronts of sixteen columns; the combine step
+    only concerns the segments between the first and the last: sequences of one, two and many segments, ends one token beyond
+    a segment's and one short of it, against the float64 oracle at the bounds of the whole file."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=616)
+    dev = "cuda"
+    out = torch.full((q.shape[0], H, 128), float("nan"), dtype=torch.bfloat16, device=dev)
+    final = torch.full((len(lengths), H, 128, 128), float("nan"), device=dev)
+    flashkda_fwd(q.to(dev), k.to(dev), v.to(dev), raw.to(dev), beta.to(dev), A_log.to(dev), dt_bias.to(dev), out,
+                 initial_state=S0.to(dev), final_state=final, cu_seqlens=torch.tensor(offs, dtype=torch.int32, device=dev))
+    torch.cuda.synchronize()
+    exp_o, exp_final = _oracle(q, k, v, raw, beta, A_log, dt_bias, offs, S0, fast=True)
+    torch.testing.assert_close(out.cpu().float(), exp_o.float(), atol=2e-2, rtol=2e-2)
+    assert all(rel_l2(final[n, head], exp_final[n, head]) <= 1e-3 for n in range(len(lengths)) for head in range(H))
+
+
 @pytest.mark.parametrize("lengths,H,halved", [([1500, 1300, 300, 64, 0, 777, 500, 200, 900], 16, 2),
                                               ([900, 800, 100, 64, 0, 300, 200, 150, 400, 130, 77, 60], 12, 2),
                                               ([1500, 200, 300, 400, 700], 32, 1),
