@@ -978,12 +978,16 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 
   // ---- the computing wavefronts ----
   const int vbase = 64 * v_half + 16 * NB * wave;
-  const int vcol = vbase + r16;
+  // The lane's V column of block nb: with NB = 2 the two blocks take turns every four columns, so that a lane's outputs of
+  // both (four adjacent columns of each) are sixteen bytes of a row, stored in one piece past the caches: with 8 bytes a
+  // lane the stores alone were a sixth of a sweep on a full chip (16 384 tokens of 32 value heads, second sweep 124 -> 113 us;
+  // through an LDS tile and the feeding wavefronts as whole rows of 256 bytes: 119).
+  auto v_row = [&](int nb) { return NB == 2 ? vbase + 8 * (r16 >> 2) + (r16 & 3) + 4 * nb : vbase + r16; };
   f32x4_t St[NB][8];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
     if (role.init != nullptr) {
-      const float* src = role.init + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
+      const float* src = role.init + (int64_t)v_row(nb) * 128 + 4 * kb;
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc) {
         const float4 t4 = *reinterpret_cast<const float4*>(src + 16 * mc);
@@ -993,12 +997,13 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc) St[nb][mc] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-  uint16_t* const o_lane = reinterpret_cast<uint16_t*>(p.o) + ((int64_t)(seq_start + r16) * p.HV + hv) * 128 + vbase + 4 * kb;
-  // V through the transposing read: lane t of a group addresses columns vbase + 16 nb + 4 (t % 4) .. + 3 of row
-  // 16 mi + 4 kb + t / 4, i.e. half (t % 2) of granule 4 wave + 2 nb + (t % 4) / 2; the swizzle 8 (kb & 1) + 2 (t / 4)
-  // of that row does not depend on mi, and block nb = 1 differs from nb = 0 in one bit of the granule index
-  const int trV = (4 * kb + (r16 >> 2)) * 128 + 8 * ((vbase / 8 + ((r16 & 3) >> 1)) ^ (8 * (kb & 1) + 2 * (r16 >> 2))) + 4 * (r16 & 1);
-  auto v_at = [&](const uint16_t* V, int mi, int nb) { return V + ((trV + 16 * 128 * mi) ^ (16 * nb)); };
+  uint16_t* const o_lane = reinterpret_cast<uint16_t*>(p.o) + ((int64_t)(seq_start + r16) * p.HV + hv) * 128 + vbase + 4 * NB * kb;
+  // V through the transposing read: lane t of a group addresses four adjacent columns of row 16 mi + 4 kb + t / 4, whose
+  // swizzle 8 (kb & 1) + 2 (t / 4) does not depend on mi: half nb of granule vbase / 8 + t % 4, or (NB = 1) half t % 2 of
+  // granule vbase / 8 + (t % 4) / 2
+  const int trV = (4 * kb + (r16 >> 2)) * 128 + (NB == 2 ? 0 : 4 * (r16 & 1)) +
+                  8 * ((vbase / 8 + (NB == 2 ? r16 & 3 : (r16 & 3) >> 1)) ^ (8 * (kb & 1) + 2 * (r16 >> 2)));
+  auto v_at = [&](const uint16_t* V, int mi, int nb) { return V + trV + 16 * 128 * mi + 4 * nb; };
   // Byte offsets of this lane's operand reads inside an operand tile.  The granule index enters the address in bits 4-7
   // and the swizzle is an exclusive or, so a step (or a group of 32 columns) further is one exclusive or of the WHOLE
   // address with 64 s (tile bases are multiples of 256); row blocks and halves are constant offsets of the read.
@@ -1268,11 +1273,15 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
         // output rows of token block ni = k - 8
         const int ni = k - 8;
         if (FULL || 16 * ni + r16 < len) {
+          uint32_t w[2 * NB];
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
-            const uint2 packed = make_uint2(pack2<act_t>(OT[nb][ni][0], OT[nb][ni][1]), pack2<act_t>(OT[nb][ni][2], OT[nb][ni][3]));
-            *reinterpret_cast<uint2*>(dst + (int64_t)16 * ni * p.HV * 128 + 16 * nb) = packed;
+            w[2 * nb] = pack2<act_t>(OT[nb][ni][0], OT[nb][ni][1]);
+            w[2 * nb + 1] = pack2<act_t>(OT[nb][ni][2], OT[nb][ni][3]);
           }
+          uint16_t* const at = dst + (int64_t)16 * ni * p.HV * 128;
+          if constexpr (NB == 2) __builtin_nontemporal_store(u32x4_t{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4_t*>(at));
+          else *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
         }
       }
       SB();
@@ -1290,7 +1299,7 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   if (role.fin != nullptr) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      float* dst = role.fin + (int64_t)(vcol + 16 * nb) * 128 + 4 * kb;
+      float* dst = role.fin + (int64_t)v_row(nb) * 128 + 4 * kb;
 #pragma unroll
       for (int mc = 0; mc < 8; ++mc)
         *reinterpret_cast<float4*>(dst + 16 * mc) = make_float4(St[nb][mc].x, St[nb][mc].y, St[nb][mc].z, St[nb][mc].w);
