@@ -46,18 +46,14 @@ __device__ __forceinline__ bf16x8_t half8(f32x4_t a, f32x4_t b) {
 }
 // Saturating roundings: a magnitude beyond the fp16 range becomes the largest finite fp16 (65504), never an
 // infinity, so that out-of-range operands degrade the result instead of turning it into NaN.
-//   half8_sat   round to nearest even after a clamp to +-65504 (one v_med3_f32 per element)
+//   half8       round to nearest even, in a wavefront whose conversions saturate (fp16_saturates)
 //   half8_rtz   round toward zero (v_cvt_pkrtz_f16_f32 saturates by itself); the error is one-sided, up to one
 //               unit in the last place, which is fine where many roundings average (the state slices) or where
 //               a low part follows
-//   half8_pair  hi = nearest after the clamp, lo = the rest rounded toward zero: x to about 22 bits, hi + lo
+//   half8_pair  hi = nearest (saturating as half8), lo = the rest rounded toward zero: x to about 22 bits, hi + lo
 //               saturating at 2 x 65504.  (hi is rounded to nearest so that values in fp16's subnormal range,
 //               where lo underflows to zero, keep an unbiased error.)
 typedef __fp16 fp16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ bf16x8_t half8_sat(f32x4_t a, f32x4_t b) {
-  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
-  return half8(f32x4_t{c(a.x), c(a.y), c(a.z), c(a.w)}, f32x4_t{c(b.x), c(b.y), c(b.z), c(b.w)});
-}
 __device__ __forceinline__ bf16x8_t half8_rtz(f32x4_t a, f32x4_t b) {
   const u32x4_t w = {__builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a.x, a.y)),
                      __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a.z, a.w)),
@@ -65,10 +61,14 @@ __device__ __forceinline__ bf16x8_t half8_rtz(f32x4_t a, f32x4_t b) {
                      __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(b.z, b.w))};
   return __builtin_bit_cast(bf16x8_t, w);
 }
+// From here on this wavefront's conversions to fp16 round a finite value beyond the range to the largest finite fp16 (MODE bit
+// 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
+__device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
+
 struct HalfPair { bf16x8_t hi, lo; };
 __device__ __forceinline__ HalfPair half8_pair(f32x4_t a, f32x4_t b) {
   HalfPair r;
-  r.hi = half8_sat(a, b);
+  r.hi = half8(a, b);
   const f32x8_t back = __builtin_convertvector(__builtin_bit_cast(f16x8_t, r.hi), f32x8_t);
   r.lo = half8_rtz(f32x4_t{a.x - back[0], a.y - back[1], a.z - back[2], a.w - back[3]},
                    f32x4_t{b.x - back[4], b.y - back[5], b.z - back[6], b.w - back[7]});
@@ -91,6 +91,19 @@ __device__ __forceinline__ void pack2_pair_small(float x, float y, uint32_t& hi,
   const f16x2_t h = __builtin_convertvector(c, f16x2_t);
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x - (float)h[0], y - (float)h[1]));
+}
+
+// c + the products of two packed pairs: v_dot2_f32_bf16 (exact products, FP32 sum); fp16 pairs through two multiply-adds,
+// which keep subnormal values.
+template <typename act_t>
+__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c);
+template <>
+__device__ __forceinline__ float dot2<bf16_t>(uint32_t a, uint32_t b, float c) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
+}
+template <>
+__device__ __forceinline__ float dot2<f16_t>(uint32_t a, uint32_t b, float c) {
+  return fmaf(hi16<f16_t>(a), hi16<f16_t>(b), fmaf(lo16<f16_t>(a), lo16<f16_t>(b), c));
 }
 
 }  // namespace pla

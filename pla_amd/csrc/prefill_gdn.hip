@@ -27,14 +27,14 @@
 //   gdn_align_rows_kernel    q / k rows that start on 4-byte boundaries only are copied into dense buffers first
 //   gdn_wsolve_kernel        preparation, one wavefront per (chunk, value head): gate, beta and their chunk-local
 //                            cumsum, the decay-factor tile, normalised K, K K^T on MFMA, the inverse of I + L by
-//                            16 x 16 blocks, W (hi, lo) in the six-block operand layout; for calls split into
-//                            segments also the normalised K rows and (one appended workgroup) the tables
+//                            16 x 16 blocks, W (hi, lo) in the six-block operand layout; the normalised K rows where
+//                            the sweeps copy them, and for calls split into segments (one appended workgroup) the tables
 //   gdn_fused_sweep_kernel   sequential kernel with output, over whole sequences or (second sweep) over segments: one
 //                            workgroup per (sequence or segment, value head) of four computing wavefronts (32 V
 //                            columns of S^T each, in MFMA accumulator layout, the chain K S^T -> X -> U -> S^T in
-//                            registers) and four feeding wavefronts that normalise the raw q / k rows into LDS
-//                            tiles, form P and issue the global -> LDS copies of V, W and the decay factors; two
-//                            barriers per chunk; with NB = 1 two workgroups per chain, 64 V columns each (calls
+//                            registers) and four feeding wavefronts that bring the raw q rows (and k rows, or copies of
+//                            normalised ones) into LDS tiles, form P and issue the global -> LDS copies of V, W and the
+//                            decay factors; two barriers per chunk; with NB = 1 two workgroups per chain, 64 V columns each (calls
 //                            of at most 128 chains)
 //   gdn_fused_sweep_mixed_kernel  the same sweep for ragged whole sequences: the chains of the longest sequences as
 //                            two halves, the others whole, in one launch (plan from the host offsets)
@@ -68,8 +68,8 @@ struct GdnPrefillParams {
   void* o;                                            // [T, HV, 128] dense
   // workspace
   int32_t* seq_chunk_off; int32_t* chunk_seq; int32_t* chunk_tok; int32_t* chunk_len;
-  uint16_t* kn;                                       // [T, H, 128] normalised K rows in operand column order (calls split into segments)
-  float* kinv;                                        // [H, T] 1 / |k| per row (a head's tokens are contiguous)
+  uint16_t* kn;                                       // [T, H, 128] normalised K rows in operand column order (store_kn)
+  float* kinv;                                        // [H, T] 1 / |k| per row (a head's tokens are contiguous; calls without kn)
   float* gcum; float* beta;
   uint16_t* W;                                        // fp16 [chunk, HV, 12 blocks of 1 KiB]: W = hi + lo, six-block operand layout
   float* gtile;          // [chunk, HV, 320]: scale e^{G} | e^{G} | e^{G_last - G} | e^{G_last} | G
@@ -80,7 +80,7 @@ struct GdnPrefillParams {
   int H, HV, NC_max;
   int inline_tables;     // at most 64 whole sequences: kernels work the chunk tables out themselves (no table kernel)
   int tail_blocks;       // workgroups appended to the preparation grid that zero the output rows beyond the last sequence
-  int store_kn;          // gdn_wsolve_kernel also stores the normalised K rows (kn): the first sweep over segments copies them
+  int store_kn;          // gdn_wsolve_kernel stores the normalised K rows (kn) for the sweeps to copy, else 1 / |k|
   // gdn_fused_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long)
   // as two halves, the others those of seq_order[n_long .. N) whole
   unsigned split_grid; int n_long;
@@ -126,9 +126,8 @@ __device__ __forceinline__ uint32_t from_other_half(uint32_t x) {
 // of a workgroup (the value heads of one q/k head) share the loading and normalising of the keys through LDS: a
 // quarter fewer vector instructions per tile and half the registers for raw rows, which brings three wavefronts
 // to a SIMD without spills (config 3 0.450 -> 0.440 ms, 8 x 2048 tokens 0.233 -> 0.224 ms; four per SIMD by a launch
-// bound measure the same: the kernel is bound by its vector instructions now, not by latency).  For a call split
-// into segments (store_kn) the wavefront that normalised a row block also stores it: the first sweep over segments
-// copies its K tiles from those rows.
+// bound measure the same: the kernel is bound by its vector instructions now, not by latency).  The wavefront that
+// normalised a row block also stores it where the sweeps copy their K tiles from those rows (store_kn).
 template <typename act_t, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefillParams p) {
   const int groups = p.HV / WAVES;
@@ -269,7 +268,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefill
         const LanePair r2 = swap_halves(r1.lo + r1.hi);
         inv = rsqrtf(r2.lo + r2.hi + 1e-6f);
         // the sweep scales the raw rows by the same factor, so both kernels hold the same rounded keys
-        if (ok && kb == 0 && first_group) p.kinv[(int64_t)h * p.T + t0 + 16 * mb + r16] = inv;
+        if (ok && kb == 0 && first_group && !p.store_kn) p.kinv[(int64_t)h * p.T + t0 + 16 * mb + r16] = inv;
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
@@ -454,6 +453,7 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
   // of an operand tile, V with its columns in order)
   using CopyWide = SwizzledTileCopy<4>;
   constexpr int KV_HALVES = TILE128_HALVES;
+  fp16_saturates();
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -639,7 +639,7 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
       for (int s = 0; s < 2; ++s) {
         bf16x8_t xb[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) xb[nb] = half8_sat(X[nb][2 * s], X[nb][2 * s + 1]);
+        for (int nb = 0; nb < NB; ++nb) xb[nb] = half8(X[nb][2 * s], X[nb][2 * s + 1]);      // (saturating: fp16_saturates)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -712,15 +712,15 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
 // Wavefronts 0-3 compute, each on its own 32 V columns of S^T, nothing crossing wavefronts (the chain K S^T -> X -> U
 // -> S^T stays in registers; the query product is formed after U, so its accumulators and those of K S^T never live
 // together).
-// Wavefronts 4-7 feed them, so that neither the normalised rows nor P cross memory:
-//   rows   wavefronts 4, 5 take the raw K rows of the next chunk (32 rows each), 6, 7 the raw Q rows: loaded one
-//          chunk ahead into registers (16 lanes per row, 16 bytes per lane).  K rows are scaled by the row's 1 / |k|
-//          (from the preparation kernel, so that both kernels round the very same normalised keys), rounded to the
-//          activation dtype and written to the LDS tile as fp16.  Q only enters the output, so its rows are written
-//          unscaled and 1 / |q| (summed here) joins the row factors of the output and of P instead
+// Wavefronts 4-7 feed them, so that P does not cross memory:
+//   Q      each takes sixteen raw rows of the next chunk, loaded one chunk ahead into registers (16 lanes per row, 16
+//          bytes per lane).  Q only enters the output, so its rows are written unscaled and 1 / |q| (summed here) joins
+//          the row factors of the output and of P
 //   P      scale tril(q_i . k_j e^{G_i - G_j}) of the current chunk from those tiles: the products are formed
 //          transposed (A = K rows, B = Q rows), which leaves a lane with four consecutive j of one token i, i.e. with
 //          8 of the 16 bytes it owns in the six-block operand layout (prefill_common.h) that phase 3 reads
+//   K      copied (KN: normalised rows in the column order of an operand tile, from the preparation), or sixteen raw rows as
+//          for Q, scaled by 1 / |k| (from the preparation, so that both kernels round the very same normalised keys)
 //   copies V, W (12 KiB, six-block layout, hi then lo) and the decay-factor tile by global -> LDS copies
 // Two barriers per chunk: A opens the chunk (all tiles of it are complete, those of the chunk before are free),
 // B precedes the product with P (P is complete).  The computing wavefronts run a hand-ordered schedule: every LDS
@@ -736,11 +736,11 @@ constexpr int FUSED_LDS_BYTES = FUSED_OFF_V + 2 * TILE128_HALVES * 2;
 
 // The sweep of one workgroup.  `wide`: 2 / NB x the chain's logical index (sequence x HV + value head, or segment x
 // HV + value head in the second sweep over segments) plus, for NB = 1, the half of the V columns it takes.
-template <typename act_t, int NB>
+template <typename act_t, int NB, bool KN>
 __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int wide) {
   constexpr int CW = 4, AUX = 4;
   constexpr int HALVES = 2 / NB;             // workgroups per chain: NB = 1 sweeps 64 of the 128 V columns
-  using CopyV = SwizzledTileCopy<AUX>;
+  using CopyTile = SwizzledTileCopy<AUX>;
   const int block = wide / HALVES, v_half = wide % HALVES;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -793,28 +793,48 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
     // ---- the feeding wavefronts: one instance of this code per wavefront (its role is a compile-time constant) ----
     auto feed = [&](auto role_tag) __attribute__((always_inline)) {
       constexpr int a = decltype(role_tag)::value;
-      constexpr bool q_side = a >= 2;
-      constexpr int row0 = 32 * (a & 1);                  // this wavefront's rows of a chunk: row0 .. row0 + 31
+      constexpr int row0 = 16 * a;                        // this wavefront's Q rows of a chunk: row0 .. row0 + 15
       const int lr = lane >> 4, lc = lane & 15;           // piece j: row row0 + 4 j + lr, columns 8 lc .. 8 lc + 7
-      const int64_t row_pitch = q_side ? p.stride_q : p.stride_k;
+      // the lane's 16 bytes of a row are columns 8 lc .. 8 lc + 7: the first 8 bytes belong to granule 4 (lc / 4) + 2 (lc % 2),
+      // half (lc / 2) % 2, the other 8 to the granule after it (same half).  The row's swizzle 2 (row & 7) = 2 lr + 8 (j & 1) is
+      // even, so the second granule lies 16 bytes after the first.
+      const int g0 = 4 * (lc >> 2) + 2 * (lc & 1), half = (lc >> 1) & 1;
+      const int at_even = (row0 + lr) * 128 + 8 * (g0 ^ (2 * lr)) + 4 * half;            // j even
+      const int at_odd = (row0 + lr) * 128 + 8 * (g0 ^ (2 * lr + 8)) + 4 * half;         // j odd
+      auto put = [&](uint16_t* tile, int j, const uint32_t (&w)[4]) {
+        uint16_t* const at = tile + ((j & 1) ? at_odd : at_even) + 4 * j * 128;
+        *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
+        *reinterpret_cast<uint2*>(at + 8) = make_uint2(w[2], w[3]);
+      };
       // bases of the sequence part (wave-uniform, 64-bit) and offsets inside a chunk (per lane, 32-bit)
-      const char* const rows_b = reinterpret_cast<const char*>(q_side ? p.q : p.k) + ((int64_t)seq_start * row_pitch + h * 128) * 2;
+      const char* const q_b = reinterpret_cast<const char*>(p.q) + ((int64_t)seq_start * p.stride_q + h * 128) * 2;
+      const uint32_t k_row_b = KN ? (uint32_t)p.H * 256u : (uint32_t)(p.stride_k * 2);
+      const char* const k_b = KN ? reinterpret_cast<const char*>(p.kn) + ((int64_t)seq_start * p.H + h) * 256
+                                 : reinterpret_cast<const char*>(p.k) + ((int64_t)seq_start * p.stride_k + h * 128) * 2;
       const char* const kinv_b = reinterpret_cast<const char*>(p.kinv + (int64_t)h * p.T + seq_start);
-      const int64_t chunk_pitch_b = (int64_t)CHUNK * row_pitch * 2;
+      const int64_t q_pitch_b = (int64_t)CHUNK * p.stride_q * 2, k_pitch_b = (int64_t)CHUNK * k_row_b;      // of a chunk
       const char* const v_b = reinterpret_cast<const char*>(p.v) + ((int64_t)seq_start * p.stride_v + hv * 128) * 2;
       const char* const w_b = reinterpret_cast<const char*>(p.W) + ((int64_t)c_begin * p.HV + hv) * (2 * TRI_BLOCKS * 1024);
       const char* const gt_b = reinterpret_cast<const char*>(p.gtile) + ((int64_t)c_begin * p.HV + hv) * (GTILE_FLOATS * 4);
-      CopyV plan_v;
+      CopyTile plan_k, plan_v;
+      if constexpr (KN) plan_k.plan(k_row_b, CHUNK - 1, a, lane);
       plan_v.plan((uint32_t)(p.stride_v * 2), CHUNK - 1, a, lane);
 
-      // global -> LDS copies of chunk c (its buffers are free): V, W and the decay-factor tile
+      // global -> LDS copies of chunk c (its buffers are free): K, V, W and the decay-factor tile
       auto issue_copies = [&](int c) {
         const int par = c & 1;
+        const char* ks = k_b + c * k_pitch_b;
         const char* vs = v_b + (int64_t)c * CHUNK * p.stride_v * 2;
         const int len = chunk_len(c);
-        if (len == CHUNK) plan_v.issue(tV[par], vs, a);
-        else {                                           // rows past the sequence end re-read its last row
-          CopyV tail;
+        if (len == CHUNK) {
+          if constexpr (KN) plan_k.issue(tK[par], ks, a);
+          plan_v.issue(tV[par], vs, a);
+        } else {                                         // rows past the sequence end re-read its last row (their U is zero)
+          CopyTile tail;
+          if constexpr (KN) {
+            tail.plan(k_row_b, len - 1, a, lane);
+            tail.issue(tK[par], ks, a);
+          }
           tail.plan((uint32_t)(p.stride_v * 2), len - 1, a, lane);
           tail.issue(tV[par], vs, a);
         }
@@ -823,78 +843,66 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
         for (int j = 0; j < 2 * TRI_BLOCKS / AUX; ++j)
           dma16(ws, 1024u * (AUX * j + a) + 16u * lane, lds_address(&tW[par][0]) + 1024u * (AUX * j + a));
         const char* gs = gt_b + (int64_t)c * p.HV * (GTILE_FLOATS * 4);
-        if (a == 1) dma16(gs, 16u * lane, lds_address(&tG[par][0]));
-        if (a == 2) dma16(gs, 1024u + 16u * (lane & 15), lds_address(&tG[par][256]));   // 64 floats; lanes 16-63 repeat them
+        if (a == 0) dma16(gs, 16u * lane, lds_address(&tG[par][0]));
+        if (a == 1) dma16(gs, 1024u + 16u * (lane & 15), lds_address(&tG[par][256]));   // 64 floats; lanes 16-63 repeat them
       };
-      // raw rows of chunk c into registers (rows past the end of the sequence part re-read its last row)
-      auto load_rows = [&](int c, uint4 (&raw)[8], float (&inv)[8]) {
-        const char* const cb = rows_b + (int64_t)c * chunk_pitch_b;
-        const char* const ib = kinv_b + (int64_t)c * CHUNK * 4;
+      // raw Q rows (and K rows) of chunk c into registers (rows past the end of the sequence part re-read its last row)
+      struct Rows { uint4 q[4], k[KN ? 1 : 4]; float inv[KN ? 1 : 4]; };
+      auto load_rows = [&](int c, Rows& raw) {
+        const char* const qs = q_b + c * q_pitch_b;
         const int last = seq_len - 1 - c * CHUNK;          // last valid row of this chunk (>= 63 for a full one)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < 4; ++j) {
           const uint32_t row = (uint32_t)min(row0 + 4 * j + lr, last);
-          raw[j] = *reinterpret_cast<const uint4*>(cb + row * (uint32_t)(row_pitch * 2) + 16u * lc);
-          // without normalisation the preparation never writes 1 / |k|: the workspace words are not read at all
-          inv[j] = (q_side || !p.normalize_qk) ? 1.f : *reinterpret_cast<const float*>(ib + row * 4u);
+          raw.q[j] = *reinterpret_cast<const uint4*>(qs + row * (uint32_t)(p.stride_q * 2) + 16u * lc);
+          if constexpr (!KN) {
+            raw.k[j] = *reinterpret_cast<const uint4*>(k_b + c * k_pitch_b + row * k_row_b + 16u * lc);
+            // without normalisation the preparation never writes 1 / |k|: the workspace words are not read at all
+            raw.inv[j] = p.normalize_qk ? *reinterpret_cast<const float*>(kinv_b + (int64_t)c * CHUNK * 4 + row * 4u) : 1.f;
+          }
         }
       };
-      // K rows: scaled by 1 / |k|, rounded to the activation dtype (the operand of the reference), written as fp16,
-      // which holds those values exactly; rows past the end of the sequence are zero.  Q rows feed the output only:
-      // they are written as they are (fp16 of the raw value) and 1 / |q| goes to tRq, from where it enters the
-      // output through the row factor scale e^G and P through its row factor.
-      auto write_rows = [&](int c, const uint4 (&raw)[8], const float (&inv_in)[8]) {
-        // The lane's 16 bytes are columns 8 lc .. 8 lc + 7 of row row0 + lr + 4 j: the first 8 bytes belong to granule
-        // 4 (lc / 4) + 2 (lc % 2), half (lc / 2) % 2, the other 8 to the granule after it (same half).  The row's swizzle
-        // 2 (row & 7) = 2 lr + 8 (j & 1) is even, so the second granule lies 16 bytes after the first.
-        uint16_t* const tile = q_side ? tQ[c & 1] : tK[c & 1];
-        const int g0 = 4 * (lc >> 2) + 2 * (lc & 1), half = (lc >> 1) & 1;
-        uint16_t* const T_even = tile + (row0 + lr) * 128 + 8 * (g0 ^ (2 * lr)) + 4 * half;        // j even
-        uint16_t* const T_odd = tile + (row0 + lr) * 128 + 8 * (g0 ^ (2 * lr + 8)) + 4 * half;     // j odd
-        auto put = [&](int j, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
-          uint16_t* const at = ((j & 1) ? T_odd : T_even) + 4 * j * 128;
-          *reinterpret_cast<uint2*>(at) = make_uint2(w0, w1);
-          *reinterpret_cast<uint2*>(at + 8) = make_uint2(w2, w3);
-        };
-        const int len = chunk_len(c);
-        if constexpr (q_side) {
-          float ss[8];
+      // K rows: scaled by 1 / |k|, rounded to the activation dtype (the operand of the reference), written as fp16, which holds
+      // those values exactly.  Q rows feed the output only: they are written as they are (fp16 of the raw value) and 1 / |q|
+      // goes to tRq, from where it enters the output through the row factor scale e^G and P through its row factor.
+      auto write_rows = [&](int c, const Rows& raw) {
+        if constexpr (!KN) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const uint32_t in[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-            uint32_t w[4];
-            float acc = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float a0 = lo16<act_t>(in[e]), a1 = hi16<act_t>(in[e]);
-              acc += a0 * a0 + a1 * a1;
-              w[e] = pack2_rtz(a0, a1);
-            }
-            ss[j] = acc;
-            put(j, w[0], w[1], w[2], w[3]);
-          }
-#pragma unroll
-          for (int j = 0; j < 8; ++j) ss[j] = row16_allreduce(ss[j]);
-          float* const rq = &tRq[c & 1][row0 + lr];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float r = rsqrtf(ss[j] + 1e-6f);
-            if (lc == 0) rq[4 * j] = p.normalize_qk ? r : 1.f;
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const uint32_t in[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-            const float inv = row0 + 4 * j + lr < len ? inv_in[j] : 0.f;
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t in[4] = {raw.k[j].x, raw.k[j].y, raw.k[j].z, raw.k[j].w};
             uint32_t w[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              const uint32_t r = pack2<act_t>(lo16<act_t>(in[e]) * inv, hi16<act_t>(in[e]) * inv);
+              const uint32_t r = pack2<act_t>(lo16<act_t>(in[e]) * raw.inv[j], hi16<act_t>(in[e]) * raw.inv[j]);
               w[e] = pack2_rtz(lo16<act_t>(r), hi16<act_t>(r));
             }
-            put(j, w[0], w[1], w[2], w[3]);
+            put(tK[c & 1], j, w);
           }
         }
+        float ss[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t in[4] = {raw.q[j].x, raw.q[j].y, raw.q[j].z, raw.q[j].w};
+          uint32_t w[4];
+          float acc = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc = dot2<act_t>(in[e], in[e], acc);
+            if constexpr (std::is_same<act_t, f16_t>::value) w[e] = in[e];
+            else w[e] = pack2_rtz(lo16<act_t>(in[e]), hi16<act_t>(in[e]));
+          }
+          ss[j] = acc;
+          put(tQ[c & 1], j, w);
+        }
+        // The four rows' sums over the sixteen lanes of a row, together: a lane pair exchanges one of two sums, a pair of
+        // pairs one of the two that are left, and lane lc ends up with that of row lc % 4
+        const bool b0 = lc & 1, b1 = lc & 2;
+        const float s01 = (b0 ? ss[1] : ss[0]) + dpp_mov<0xB1>(b0 ? ss[0] : ss[1]);
+        const float s23 = (b0 ? ss[3] : ss[2]) + dpp_mov<0xB1>(b0 ? ss[2] : ss[3]);
+        float sum = (b1 ? s23 : s01) + dpp_mov<0x4E>(b1 ? s01 : s23);
+        sum += dpp_mov<0x124>(sum);                        // row_ror:4
+        sum += dpp_mov<0x128>(sum);                        // row_ror:8
+        if (lc < 4) tRq[c & 1][row0 + lr + 4 * lc] = p.normalize_qk ? fast_rsqrt(sum + 1e-6f) : 1.f;
       };
       // P of chunk c from its K and Q tiles: this wavefront's blocks of the six
       auto form_p = [&](int c) {
@@ -938,7 +946,7 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
           }
           *reinterpret_cast<uint4*>(tP + b * 512 + lane * 8) = make_uint4(w[0], w[1], w[2], w[3]);
         };
-        // three (nj, ni) products on each wavefront of the Q side, two on each of the K side (whose rows cost more)
+        // three (nj, ni) products on two of the wavefronts, two on those that copy the decay factors
         if constexpr (a == 0) block(std::integral_constant<int, 1>{});
         else if constexpr (a == 1) block(std::integral_constant<int, 5>{});
         else if constexpr (a == 2) { block(std::integral_constant<int, 0>{}); block(std::integral_constant<int, 3>{}); }
@@ -947,26 +955,22 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 
       // `raw` holds the rows of the chunk that is written next; the rows after those are requested right after
       // barrier A (behind the copies) into `ahead` and change over at the end of the iteration.
-      uint4 raw[8], ahead[8];
-      float inv[8], inv_ahead[8];
+      Rows raw, ahead;
       if (n_chunks > 0) {
         issue_copies(0);
-        load_rows(0, raw, inv);
-        write_rows(0, raw, inv);
-        if (n_chunks > 1) load_rows(1, raw, inv);
+        load_rows(0, raw);
+        write_rows(0, raw);
+        if (n_chunks > 1) load_rows(1, raw);
       }
       for (int ci = 0; ci < n_chunks; ++ci) {
         wait_vmcnt<0>();                               // this wavefront's copies for chunk ci have landed
         lds_barrier();                                 // barrier A (the rows this wavefront wrote are in LDS)
         if (ci + 1 < n_chunks) issue_copies(ci + 1);
-        if (ci + 2 < n_chunks) load_rows(ci + 2, ahead, inv_ahead);
+        if (ci + 2 < n_chunks) load_rows(ci + 2, ahead);
         form_p(ci);
         lds_barrier();                                 // barrier B (P is in LDS; copies and loads stay in flight)
-        if (ci + 1 < n_chunks) write_rows(ci + 1, raw, inv);
-        if (ci + 2 < n_chunks) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) { raw[j] = ahead[j]; inv[j] = inv_ahead[j]; }
-        }
+        if (ci + 1 < n_chunks) write_rows(ci + 1, raw);
+        if (ci + 2 < n_chunks) raw = ahead;
       }
     };
     if (wave == CW) feed(std::integral_constant<int, 0>{});
@@ -977,6 +981,7 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   }
 
   // ---- the computing wavefronts ----
+  fp16_saturates();
   const int vbase = 64 * v_half + 16 * NB * wave;
   // The lane's V column of block nb: with NB = 2 the two blocks take turns every four columns, so that a lane's outputs of
   // both (four adjacent columns of each) are sixteen bytes of a row, stored in one piece past the caches: with 8 bytes a
@@ -1030,8 +1035,8 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 
   auto pk = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y)); };
-  auto pk_sat = [](float x, float y) {
-    const f32x2_t c = {__builtin_amdgcn_fmed3f(x, -65504.f, 65504.f), __builtin_amdgcn_fmed3f(y, -65504.f, 65504.f)};
+  auto pk_sat = [](float x, float y) {             // (saturating: fp16_saturates)
+    const f32x2_t c = {x, y};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(c, f16x2_t));
   };
   // hi = x rounded toward zero (which saturates at the largest finite fp16 value by itself), lo = the rest,
@@ -1310,19 +1315,19 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 
 // One workgroup per (sequence, value head), or per (segment, value head) in the second sweep over segments (NB = 2);
 // NB = 1: two per chain, 64 V columns each (the columns of V are independent: same bits).
-template <typename act_t, int NB>
+template <typename act_t, int NB, bool KN>
 __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_kernel(const GdnPrefillParams p) {
   constexpr int HALVES = 2 / NB;
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   const int wide = xcd_grouped_index(blockIdx.x, HALVES * (p.HV / p.H), HALVES * (p.pass == 2 ? p.seg.max_segments : p.N) * p.HV);
   if (wide < 0) return;
-  fused_sweep<act_t, NB>(p, lds_all, wide);
+  fused_sweep<act_t, NB, KN>(p, lds_all, wide);
 }
 
 // Whole sequences of unequal length, swept in one launch whose longest chains decide how long it lasts while the CUs
 // of chains that have ended stand idle: the chains of the longest sequences are swept as two halves (which start
 // first: workgroups are dispatched in index order), those of the others whole, longest first.
-template <typename act_t>
+template <typename act_t, bool KN>
 __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const GdnPrefillParams p) {
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   const int ratio = p.HV / p.H;
@@ -1330,12 +1335,12 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
     const int wide = xcd_grouped_index(blockIdx.x, 2 * ratio, 2 * p.n_long * p.HV);
     if (wide < 0) return;
     const int chain = wide >> 1, k = chain / p.HV;
-    fused_sweep<act_t, 1>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
+    fused_sweep<act_t, 1, KN>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
   } else {
     const int chain = xcd_grouped_index(blockIdx.x - p.split_grid, ratio, (p.N - p.n_long) * p.HV);
     if (chain < 0) return;
     const int k = chain / p.HV;
-    fused_sweep<act_t, 2>(p, lds_all, p.seq_order[p.n_long + k] * p.HV + chain - k * p.HV);
+    fused_sweep<act_t, 2, KN>(p, lds_all, p.seq_order[p.n_long + k] * p.HV + chain - k * p.HV);
   }
 }
 
@@ -1350,7 +1355,7 @@ __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefil
   if (pair < 0) return;
   const int s = pair / p.HV;
   if (s >= p.seg.seq_seg_off[p.N]) return;
-  if (s == p.seg.seq_seg_off[p.seg.seg_seq[s]]) fused_sweep<act_t, 2>(p, lds_all, pair);
+  if (s == p.seg.seq_seg_off[p.seg.seg_seq[s]]) fused_sweep<act_t, 2, true>(p, lds_all, pair);
   else lean_sweep<act_t>(p, lds_all, pair);
 }
 
@@ -1560,9 +1565,14 @@ static int gdn_prefill_run(
     p.q = q_rows; p.k = k_rows;
     p.stride_q = p.stride_k = (int64_t)H * 128;
   }
-  // a call split into segments: the preparation also stores the normalised K rows, which the first sweep copies
-  p.store_kn = segmented;
   const bool v_halves = !segmented && (int64_t)N * HV <= 128;
+  // Normalised K rows in memory take the scaling of the keys from the sweeps of every value head and cost the preparation a
+  // tile per q/k head and chunk.  They pay where the chip is not full (128 chains at most: 3 short prompts 24.0 -> 22.6 us, one of
+  // 1100 tokens, 32 value heads 56.2 -> 51.0) and from three value heads a q/k head on (six ragged prompts, 48 of 16 heads 177 ->
+  // 171; eight of 512, 24 of 8 48.8 -> 47.3); of two the write shows (eight of 2048, 32 of 16 170 -> 184).  The sweeps over
+  // segments read them anyway.
+  const bool kn = segmented || v_halves || HV >= 3 * H;
+  p.store_kn = kn;
   if (segmented) {
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
     p.seg.seq_seg_off = reinterpret_cast<int32_t*>(ws + L.seq_seg_off);
@@ -1648,16 +1658,16 @@ static int gdn_prefill_run(
             p.n_long = p.stage == mixed_stage ? halved : 0;
             p.split_grid = xcd_grouped_grid(2 * (unsigned)p.n_long * HV, 2 * (unsigned)(HV / H));
             const unsigned g = p.split_grid + xcd_grouped_grid((unsigned)(N - p.n_long) * HV, (unsigned)(HV / H));
-            if (half_act) hipLaunchKernelGGL(gdn_fused_sweep_mixed_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
-            else hipLaunchKernelGGL(gdn_fused_sweep_mixed_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
+            if (half_act) hipLaunchKernelGGL((kn ? gdn_fused_sweep_mixed_kernel<f16_t, true> : gdn_fused_sweep_mixed_kernel<f16_t, false>), dim3(g), dim3(512), 0, s, p);
+            else hipLaunchKernelGGL((kn ? gdn_fused_sweep_mixed_kernel<bf16_t, true> : gdn_fused_sweep_mixed_kernel<bf16_t, false>), dim3(g), dim3(512), 0, s, p);
           } else if (v_halves) {
             const unsigned g = xcd_grouped_grid(2 * grid, 2 * (unsigned)(HV / H));
-            if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1>), dim3(g), dim3(512), 0, s, p);
-            else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1>), dim3(g), dim3(512), 0, s, p);
+            if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
+            else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
           } else {
             const unsigned g = xcd_grouped_grid(grid, (unsigned)(HV / H));
-            if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 2>), dim3(g), dim3(512), 0, s, p);
-            else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 2>), dim3(g), dim3(512), 0, s, p);
+            if (half_act) hipLaunchKernelGGL((kn ? gdn_fused_sweep_kernel<f16_t, 2, true> : gdn_fused_sweep_kernel<f16_t, 2, false>), dim3(g), dim3(512), 0, s, p);
+            else hipLaunchKernelGGL((kn ? gdn_fused_sweep_kernel<bf16_t, 2, true> : gdn_fused_sweep_kernel<bf16_t, 2, false>), dim3(g), dim3(512), 0, s, p);
           }
         }
       });
@@ -1679,12 +1689,12 @@ static int gdn_prefill_run(
     }
     if (segments * HV <= 128) {
       const unsigned g = xcd_grouped_grid(2 * (unsigned)L.max_segments * HV, 2 * (unsigned)(HV / H));
-      if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1>), dim3(g), dim3(512), 0, s, p);
-      else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1>), dim3(g), dim3(512), 0, s, p);
+      if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
+      else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
     } else {
       const unsigned g = xcd_grouped_grid((unsigned)L.max_segments * HV, (unsigned)(HV / H));
-      if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 2>), dim3(g), dim3(512), 0, s, p);
-      else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 2>), dim3(g), dim3(512), 0, s, p);
+      if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 2, true>), dim3(g), dim3(512), 0, s, p);
+      else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 2, true>), dim3(g), dim3(512), 0, s, p);
     }
   }
   return check_launch("gdn prefill launch");

@@ -160,10 +160,10 @@ __device__ __forceinline__ void kda_sub_chunk(const KdaGate& gate, KdaRows<OUT>&
     float a = 0.f, b = 0.f;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      a = dot2_bf16(w[s].x, w[s].x, a);
-      b = dot2_bf16(w[s].y, w[s].y, b);
-      a = dot2_bf16(w[s].z, w[s].z, a);
-      b = dot2_bf16(w[s].w, w[s].w, b);
+      a = dot2<bf16_t>(w[s].x, w[s].x, a);
+      b = dot2<bf16_t>(w[s].y, w[s].y, b);
+      a = dot2<bf16_t>(w[s].z, w[s].z, a);
+      b = dot2<bf16_t>(w[s].w, w[s].w, b);
     }
     return fast_rsqrt(token_sum(a + b) + 1e-6f);
   };

@@ -38,11 +38,6 @@ __device__ __forceinline__ int turned_piece(int lane) {
   return 16 * (16 * g + (t ^ (4 * g)));
 }
 
-// c + the products of two packed pairs (v_dot2_f32_bf16: exact products, FP32 sum).
-__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
-}
-
 // Eight FP32 values as a bf16 pair each: round_bf16 is hi, to nearest, rest_bf16 is lo = bf16(x - hi) (v_dot2 forms x - hi in place:
 // x is used up).
 __device__ __forceinline__ bf16x8_t round_bf16(const float (&x)[8]) {
@@ -56,14 +51,10 @@ __device__ __forceinline__ bf16x8_t rest_bf16(const float (&x)[8], bf16x8_t hi) 
   uint32_t LO, HI;
   asm("s_mov_b32 %0, 0xbf80" : "=s"(LO));
   asm("s_mov_b32 %0, 0xbf800000" : "=s"(HI));
-  const float r[8] = {dot2_bf16(h.x, LO, x[0]), dot2_bf16(h.x, HI, x[1]), dot2_bf16(h.y, LO, x[2]), dot2_bf16(h.y, HI, x[3]),
-                      dot2_bf16(h.z, LO, x[4]), dot2_bf16(h.z, HI, x[5]), dot2_bf16(h.w, LO, x[6]), dot2_bf16(h.w, HI, x[7])};
+  const float r[8] = {dot2<bf16_t>(h.x, LO, x[0]), dot2<bf16_t>(h.x, HI, x[1]), dot2<bf16_t>(h.y, LO, x[2]), dot2<bf16_t>(h.y, HI, x[3]),
+                      dot2<bf16_t>(h.z, LO, x[4]), dot2<bf16_t>(h.z, HI, x[5]), dot2<bf16_t>(h.w, LO, x[6]), dot2<bf16_t>(h.w, HI, x[7])};
   return round_bf16(r);
 }
-
-// From here on this wavefront's conversions to fp16 round a finite value beyond the range to the largest finite fp16 (MODE bit
-// 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
-__device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
 
 // Four FP32 values as an fp16 pair each: hi to nearest after a clamp (SATURATES: of a wavefront whose conversions do that, see
 // fp16_saturates), the rest toward zero (as half8_pair).  x - hi is one v_fma_mix_f32, which takes a half of hi as it is, in the

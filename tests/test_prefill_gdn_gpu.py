@@ -272,6 +272,32 @@ def test_gdn_prefill_split_sequences_match_oracle(lengths, tail_pad, H, HV):
     _check(w, fast=True)
 
 
+@pytest.mark.parametrize("H,HV", [(8, 24), (12, 24), (24, 24)])
+def test_gdn_prefill_keys_copied_or_formed_by_the_sweep(H, HV):
+    """More than 128 chains of whole sequences: from three value heads a q/k head on the sweeps copy the normalised keys that
+    the preparation stored, else their feeding wavefronts form them.  Tail chunks of 1, 63 and 64 rows, an empty sequence;
+    against the oracle, and the same bits as each sequence alone (few chains: always copied)."""
+    from pla_amd.prefill.flashqla import gdn_prefill_packed_qkv_fwd
+    from pla_amd.workloads import gdn_prefill_packed
+    lengths = [65, 127, 0, 64, 200, 1]
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 3, seed=300 + H, tail_pad=2)
+    pool0 = w["initial_state"].clone()
+    _check(w, fast=True)
+    w["initial_state"].copy_(pool0)
+    _, _, o, _, _ = _run_workload(w)
+    pool = w["initial_state"].clone()
+    offs, idx = w["_meta"]["offsets"], w["initial_state_indices"]
+    for n in (0, 1, 4):
+        w["initial_state"].copy_(pool0)
+        lo, hi = offs[n], offs[n + 1]
+        r = gdn_prefill_packed_qkv_fwd(w["packed_qkv"][lo:hi], w["raw_gate_a"][lo:hi], w["raw_beta_b"][lo:hi], w["A_log"],
+                                       w["dt_bias"], torch.tensor([0, hi - lo], dtype=torch.int32, device="cuda"), num_qk_heads=H,
+                                       num_v_heads=HV, scale=w["scale"], initial_state=w["initial_state"],
+                                       initial_state_indices=idx[n:n + 1])
+        torch.cuda.synchronize()
+        assert torch.equal(r[2][0], o[0, lo:hi]) and torch.equal(w["initial_state"][int(idx[n])], pool[int(idx[n])]), n
+
+
 @pytest.mark.parametrize("lengths,tail_pad,H,HV", [
     ([2048], 0, 1, 4), ([2049], 3, 2, 4),                              # segments of three chunks; a last one of one token
     ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2),                  # one, two, three and more segments a sequence
