@@ -200,8 +200,11 @@ def flashkda_fwd(
         return None
 
     ws, nbytes = _workspace(T, N, H, q.device)
-    if final_state is not None and not (initial_state is not None and final_state.data_ptr() == initial_state.data_ptr()):
-        # sequences of length zero keep their incoming (or zero) state
+    # sequences of length zero keep their incoming (or zero) state: copied ahead of the launch, which writes every other final
+    # state itself, unless the host's offsets show that there is none
+    empty = raw_host is None or any(raw_host[n] == raw_host[n + 1] for n in range(N))
+    if empty and final_state is not None and not (initial_state is not None
+                                                  and final_state.data_ptr() == initial_state.data_ptr()):
         if initial_state is not None:
             if indexed:
                 final_state[state_indices.long()] = initial_state[state_indices.long()]

@@ -367,6 +367,31 @@ def test_kda_prefill_split_sequences_match_oracle(lengths, pad, H):
                 assert rel_l2(final[n, head], exp_final[n, head]) <= 1e-3, (n, head)
 
 
+@pytest.mark.parametrize("lengths", [[5, 70], [5, 0, 70], [0, 1], [40, 2100]])
+@pytest.mark.parametrize("start", [False, True])
+@pytest.mark.parametrize("native", [False, True])
+def test_kda_prefill_final_states_with_host_offsets(lengths, start, native):
+    """The host copies the start states ahead of the launch for sequences of length zero only, where its offsets tell: every
+    final state is written either way (the buffer holds NaN), with the bits of the call without host offsets."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd, ops
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, 2, seed=717)
+    args = [t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)]
+    results = []
+    ops._native = None if native else False
+    for host in (None, tuple(offs)):
+        out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device="cuda")
+        final = torch.full(S0.shape, float("nan"), device="cuda")
+        flashkda_fwd(*args, out, initial_state=S0.cuda() if start else None, final_state=final,
+                     cu_seqlens=torch.tensor(offs, dtype=torch.int32, device="cuda"), raw_cu_seqlens=host)
+        torch.cuda.synchronize()
+        results.append((out, final))
+    assert torch.isfinite(results[0][1]).all()
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    for n, length in enumerate(lengths):
+        if length == 0:
+            assert torch.equal(results[1][1][n].cpu(), S0[n] if start else torch.zeros_like(S0[n]))
+
+
 @pytest.mark.parametrize("lengths,H", [([1025], 1), ([2048], 2), ([191, 192, 193, 0, 1, 384, 385, 1300], 2),    # prepared sub-chunks
                                        ([4500], 32)])                                                          # formed by the sweeps
 def test_kda_prefill_segments_at_their_edges(lengths, H):
