@@ -281,8 +281,8 @@ int pla_kda_commit_plan_launch(
     int32_t* candidate, int32_t* plan, void* stream);
 
 /*
- * The whole paged commit: the plan above, then pla_kda_fold_native_launch and pla_kda_conv_native_launch with it, in one
- * launch or in three, whichever is the faster for the number of tiles.  Arguments as there; source is int32.
+ * The whole paged commit: the plan above, then what pla_kda_fold_native_launch and pla_kda_conv_native_launch do with it, in
+ * one launch or with the plan in a launch of its own, whichever is the faster for the number of tiles.  Arguments as there; source is int32.
  */
 int pla_kda_commit_launch(
     const int64_t* layer_table, int layers, int heads, int channels, int rows,
@@ -292,7 +292,8 @@ int pla_kda_commit_launch(
     int token_capacity, int64_t block_row_stride, int64_t block_col_stride, int64_t block_size,
     int32_t* candidate, int32_t* plan, void* stream);
 
-/* Launches pla_kda_commit_launch takes for a batch whose plan shares no memory with its inputs (host arithmetic): 1 or 3. */
+/* The form pla_kda_commit_launch takes for a batch whose plan shares no memory with its inputs (host arithmetic): 1 for one
+ * launch, 3 for plan, fold and conv windows as parts of their own (of which the latter two share a launch). */
 int pla_kda_commit_launches(int batch, int heads, int layers);
 
 /*

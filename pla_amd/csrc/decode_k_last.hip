@@ -742,6 +742,26 @@ __global__ __launch_bounds__(256) void kda_fold_kernel(const FoldParams p) {
   fold_rows<act_t, RPW, false>(p, CommitParams{}, blockIdx.x, blockIdx.z);
 }
 
+// The fold of a commit plan, and behind its tiles the conv windows of the same layer (as conv_window_native_kernel copies them):
+// they share no memory and the windows hide under the fold, a launch less (504 tiles, windows of eight tokens, with both verify
+// calls ahead 49.3 -> 47.0 us; 2400 tiles, windows of four 126.4 -> 121.3).
+template <int RPW>
+__global__ __launch_bounds__(256) void kda_fold_windows_kernel(const FoldParams p, int channels) {
+  const int tiles = p.B * p.HV;
+  if ((int)blockIdx.x < tiles) {
+    fold_rows<bf16_t, RPW, false>(p, CommitParams{}, blockIdx.x, blockIdx.z);
+    return;
+  }
+  const int groups = (channels + 255) / 256;                   // of 256 channels, of a request
+  const int g = (blockIdx.x - tiles) * gridDim.y + blockIdx.y;
+  const int row = g / groups, channel = (g - row * groups) * 256 + threadIdx.x;
+  if (row >= p.B || channel >= channels) return;
+  Request todo{NO_CLAIM, p.accept_lens[row], p.final_idx[row], p.track_idx[row], p.track_step[row]};
+  if (todo.tokens > p.L || todo.final_slot < 0 || todo.final_slot >= p.slots) todo.tokens = 0;
+  if (todo.boundary_tokens > p.L || todo.boundary_slot < 0 || todo.boundary_slot >= p.slots) todo.boundary_tokens = 0;
+  copy_conv_window(p.layer_table + blockIdx.z * PLA_LAYER_TABLE_ENTRIES, row, channel, todo);
+}
+
 template <int RPW>
 __global__ __launch_bounds__(256) void kda_commit_kernel(const FoldParams p, const CommitParams m) {
   const int tiles = p.B * p.HV, folds = tiles * m.layers;
@@ -1027,8 +1047,8 @@ extern "C" int pla_kda_fold_native_launch(
 }
 
 // Up to this many state tiles the paged commit is one launch.  There a workgroup's plan costs a trip to memory or two beside
-// the trip for its tile and saves two launches; with more tiles than the chip holds workgroups every round pays for it.
-// us at one / three launches (windows of 3-8 tokens; with a block table in brackets):
+// the trip for its tile and saves a launch; with more tiles than the chip holds workgroups every round pays for it.
+// us at one launch / at three, the conv windows apart from the fold (windows of 3-8 tokens; with a block table in brackets):
 //     8 tiles  6.8 / 9.1 (7.8 / 9.8)      240 tiles 11.6 / 13.9 (12.7 / 14.6)   480 tiles 24.9 / 23.4 (25.8 / 24.1)
 //    96 tiles 10.6 / 12.4 (11.6 / 13.0)   320 tiles 17.4 / 18.0 (18.4 / 18.5)   504 tiles 24.7 / 24.5 (26.7 / 25.0)
 constexpr int64_t COMMIT_ONE_LAUNCH_TILES = 320;
@@ -1057,20 +1077,27 @@ extern "C" int pla_kda_commit_launch(
             batch, capacity, sampler_rows, block_rows, block_cols, slots, Q, null_block_id, token_capacity, block_row_stride,
             block_col_stride, block_size, candidate, plan, stream))
       return bad;
-    if (const int bad = pla_kda_fold_native_launch(layer_table, layers, source, plan, final_slots, boundary, boundary_lens, batch, heads,
-                                                   Q, slots, null_block_id, stream))
-      return bad;
-    return pla_kda_conv_native_launch(layer_table, layers, plan, final_slots, boundary, boundary_lens, batch, channels, Q, rows, slots,
-                                      stream);
   }
   PLA_REQUIRE(layer_table && plan, "null table or plan pointer");
   if (const int bad = check_plan_inputs(in)) return bad;
+  if (batch == 0) return 0;
   PLA_REQUIRE(layers >= 1 && layers <= 65535 && heads > 0 && channels > 0 && batch <= rows,
               "commit requires 1..65535 layers, heads > 0, channels > 0 and batch <= record rows");
   FoldParams p{nullptr, nullptr, nullptr, nullptr, nullptr, source, nullptr,
                0, (int64_t)heads * Q * 128, (int64_t)heads * Q * 128, (int64_t)heads * Q * 128,
                (int64_t)heads * Q, batch, heads, heads, Q, null_block_id,
                nullptr, nullptr, nullptr, 1, 1, slots, 0, 0, 0, 0, 0, layer_table};
+  if (!fused) {
+    p.accept_lens = plan; p.final_idx = final_slots; p.track_idx = boundary; p.track_step = boundary_lens;
+    const int rpw = pick_rows_per_wave(batch * heads * layers);
+    const unsigned parts = 32 / rpw, conv_groups = (unsigned)batch * (unsigned)((channels + 255) / 256);
+    const dim3 grid((unsigned)(batch * heads) + (conv_groups + parts - 1) / parts, parts, (unsigned)layers), block(256);
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (rpw == 32) kda_fold_windows_kernel<32><<<grid, block, 0, s>>>(p, channels);
+    else if (rpw == 16) kda_fold_windows_kernel<16><<<grid, block, 0, s>>>(p, channels);
+    else kda_fold_windows_kernel<8><<<grid, block, 0, s>>>(p, channels);
+    return check_launch("kda_fold_windows_kernel launch");
+  }
   const int rpw = pick_rows_per_wave(batch * heads * layers);
   const CommitParams m{in, plan, channels, layers};
   const unsigned parts = 32 / rpw;
