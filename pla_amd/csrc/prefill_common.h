@@ -181,6 +181,7 @@ struct SegmentTable {
   float* B;               // [segment, head, V, K] zero-state results, then the state the segment ends in (first segments: at once)
   float* identity;        // [128, 128]
   int seg_chunks;         // chunks per segment (0: sequences are not split)
+  int split_from;         // GDN: with a longest sequence of fewer chunks none is split (KDA's kernels: count_segments)
   int max_segments;
 };
 
@@ -460,6 +461,13 @@ __device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlen
 
 // Segments per sequence and the 128 x 128 identity.  Single workgroup, after chunk_map.
 __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N, SegmentTable t) {
+  int longest = 0;                            // every wavefront for itself
+  for (int base = 0; base < N; base += 64) {
+    const int n = base + (threadIdx.x & 63);
+    longest = max(longest, n < N ? seq_chunk_off[n + 1] - seq_chunk_off[n] : 0);
+  }
+  longest = __builtin_amdgcn_readlane(wave_scan(longest, 0, [](int a, int b) { return max(a, b); }), 63);
+  if (longest < t.split_from) t.seg_chunks = max(longest, 1);
   if (threadIdx.x < 64) {                     // exclusive scan of the segment counts, as in chunk_map
     const int lane0 = threadIdx.x;
     int carry = 0;

@@ -1345,17 +1345,24 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
 }
 
 // First sweep over segments: first segments for good, with output, from their real start states (which takes as long per
-// chunk as the two roles of the others), those behind them for their summaries.
+// chunk as the two roles of the others), those behind them for their summaries.  Two workgroups a (segment, value head): where
+// all of them together leave CUs for it both sweep a first segment, 64 V columns each, else the first one does it alone, as it
+// does with the summaries.
 template <typename act_t>
 __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefillParams p) {
   static_assert(LEAN_LDS_BYTES <= FUSED_LDS_BYTES, "one array serves both sweeps");
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
-  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, p.seg.max_segments * p.HV);
+  const int pairs = p.seg.max_segments * p.HV, grid = gridDim.x / 2;
+  const bool second = (int)blockIdx.x >= grid;             // (behind all others in the grid)
+  const int pair = xcd_grouped_index(second ? blockIdx.x - grid : blockIdx.x, p.HV / p.H, pairs);
   if (pair < 0) return;
-  const int s = pair / p.HV;
-  if (s >= p.seg.seq_seg_off[p.N]) return;
-  if (s == p.seg.seq_seg_off[p.seg.seg_seq[s]]) fused_sweep<act_t, 2, true>(p, lds_all, pair);
+  const int s = pair / p.HV, segments = p.seg.seq_seg_off[p.N];
+  if (s >= segments) return;
+  const bool first = s == p.seg.seq_seg_off[p.seg.seg_seq[s]], halves = segments * p.HV <= CUS;
+  if (first && halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * pair + (second ? 1 : 0));
+  else if (second) return;
+  else if (first) fused_sweep<act_t, 2, true>(p, lds_all, pair);
   else lean_sweep<act_t>(p, lds_all, pair);
 }
 
@@ -1363,7 +1370,7 @@ struct GdnWorkspaceLayout {
   size_t seq_chunk_off, chunk_seq, chunk_tok, chunk_len, q_rows, k_rows, kn, kinv, gtile, W;
   size_t seq_seg_off, seg_seq, seg_c0, seg_nc, segM, segB, identity;
   size_t order, stage_begin, carry, total;
-  int NC_max, seg_chunks, max_segments, stages;
+  int NC_max, seg_chunks, max_segments, split_from, stages;
 };
 // The plan for a call of N <= INLINE_TABLE_SEQUENCES whole sequences run in `stages` stages (0: unstaged): *stage
 // receives the stage whose sweep is the last one.
@@ -1384,31 +1391,38 @@ static int mixed_sweep_from_offsets(const int32_t* raw_cu_seqlens, int N, int HV
 }
 
 // Chunks per segment for a call of at most 64 (sequence, value head) chains and at least 32 chunks, 0: not split.  A length of s
-// chunks is priced in us from the call's longest sequence (of several the host has the mean only, which random lengths exceed by
-// about half): 4.4 s for the two sweeps where the second one runs as halves ((segment, head) pairs on half of the CUs at most),
-// 6.5 s otherwise, and 1.2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep,
-// which runs one segment less per sequence than there are (of N sequences it counts a third of that).  us per call, s = 3 / 4 / 5 / 6 / 8
-// / 10 / 16 / not split: one of 2048 tokens, 16 value heads 71 / 65.5 / 66.6 / 68.9 / 74.3 / 83 / 107 / 82.2; 32 heads 100 / 78.2 / 76.2 / 78.3 /
-// 80.0 / 86.6 / 110 / 85.5; 64 heads - / 120 / 122 / 120 / 92.5 / 101 / 112 / 87.5; 4096, 16 heads - / - / 88.0 / 87.3 / 88.5 / 92.0 / 115.6 / 152; 32
-// heads - / - / 132 / 136 / 103.5 / 106.8 / 120.7 / 153.6; 8192, 8 heads - / - / - / - / - / 104.7 / 122.8 / 284.  (Segments of 16 chunks
-// at least, as before: the column of 16.)
-static int gdn_segment_chunks(int T, int N, int HV) {
-  if ((int64_t)N * HV > 64 || T / CHUNK < 32) return 0;
-  const int chunks = N == 1 ? (T - 1) / CHUNK + 1 : T / CHUNK, pairs = CUS + HV * (N == 1 ? 1 : N / 3);
+// chunks is priced in us from the call's longest sequence (L chunks; of several the host has the mean only, which random lengths
+// exceed by about half): 3.8 s for the two sweeps where the second one runs as halves ((segment, head) pairs on half of the CUs at
+// most), 5 s otherwise, 2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep,
+// which runs one segment less per sequence than there are (of N sequences it counts a third of that).  One sequence is split where
+// that is below 16 + 1.75 L, with 33 for the launches and 0.06 per thousand tokens and heads for the keys it stores.  us per call,
+// s = 4 / 5 / 6 / 8 / 10 / 12 / 16 / not split: one of 2048 tokens, 16 value heads 67.8 / 68.9 / - / - / - / - / - / 72.7; 32 heads 78.8 / 76.6 / 78.5 /
+// 78.5 / 85.9 / - / - / 76.1; 64 heads - / - / - / 90.1 / 97.3 / - / - / 76.6; 3000, 48 heads - / - / - / 107.5 / 112.0 / 117.6 / - / 113.5; 4096, 16
+// heads 94.0 / 87.2 / 88.1 / 86.7 / 91.8 / - / - / 133; 32 heads - / - / - / 102 / 105 / 111 / 116 / 134; 8192, 8 heads - / - / - / 102.7 / 104.0
+// / - / - / 242; 16 384, 24 heads with 22 and 24 chunks (264 pairs and 240) 323 and 233.
+// Of several sequences the device has the lengths: where the longest is below the line at which splitting it pays, none is split
+// (segment_map) and the first sweep takes them all: us split / not, 1000 + 1050 tokens of 16 heads 62.5 / 53.5; three of 700, 12 heads
+// 68.5 / 48.0; four of 400 to 600, 16 heads 58.1 / 43.6.
+struct GdnSplit { int chunks, from; };      // SegmentTable::seg_chunks (0: not split), split_from
+static GdnSplit gdn_split(int T, int N, int HV) {
+  if ((int64_t)N * HV > 64 || T / CHUNK < 32) return GdnSplit{0, 0};
+  const int chunks = N == 1 ? (T - 1) / CHUNK + 1 : T / CHUNK, per_head = CUS / HV + (N == 1 ? 1 : N / 3);
   const double longest = N == 1 ? chunks : std::min<double>(chunks, 1.5 * chunks / N);
-  const int least = std::max(3, (int)(((int64_t)chunks * HV + pairs - 1) / pairs));
+  const int least = std::max(3, (chunks + per_head - 1) / per_head);
   int best = 0;
   double best_price = 0.;
   for (int s = least; s <= least + 16; ++s) {
     const double swept = (N == 1 ? (chunks - 1) / s : std::max(0., (double)chunks / s - 0.5 * N)) * HV;
-    const double price = (swept <= CUS / 2 ? 4.4 : 6.5) * s + 1.2 * longest / s;
+    const double price = (swept <= CUS / 2 ? 3.8 : 5.) * s + 2. * longest / s;
     if (best == 0 || price < best_price) best_price = price, best = s;
   }
-  return best;
+  const double fixed = 17. + 6e-5 * T * HV, sweeps = best_price - 2. * longest / best;
+  const int from = (int)((fixed + sweeps) / (1.75 - 2. / best)) + 1;
+  return N > 1 ? GdnSplit{best, from} : chunks < from ? GdnSplit{0, 0} : GdnSplit{best, 0};
 }
 
 static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chunks, bool allow_stages) {
-  GdnWorkspaceLayout L;
+  GdnWorkspaceLayout L{};
   L.NC_max = T / CHUNK + N;
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t at = off; off = align_up256(off + bytes); return at; };
@@ -1446,15 +1460,18 @@ static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chu
 // The plan of a call is one for all entry points, so where segments as short as that would outgrow the library's own array, calls
 // small enough for it with segments of 16 chunks (of three tiles each, which it has always taken) get the shortest that fit.
 static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_stages = true) {
-  const int best = gdn_segment_chunks(T, N, HV);
+  const GdnSplit split = gdn_split(T, N, HV);
   const size_t tile = (size_t)HV * 16384 * 4, before = 3 * (size_t)(T / CHUNK / 16 + N + 1) * tile;
-  if (best > 0 && gdn_layout_of(T, N, H, HV, 0, false).total + before <= PLA_GDN_PREFILL_STATIC_BYTES)
-    for (int s = best; s <= 4 * best; ++s) {
-      const GdnWorkspaceLayout L = gdn_layout_of(T, N, H, HV, s, allow_stages);
-      if (L.total <= PLA_GDN_PREFILL_STATIC_BYTES) return L;
+  GdnWorkspaceLayout L = gdn_layout_of(T, N, H, HV, split.chunks, allow_stages);
+  if (split.chunks > 0 && gdn_layout_of(T, N, H, HV, 0, false).total + before <= PLA_GDN_PREFILL_STATIC_BYTES)
+    for (int s = split.chunks + 1; s <= 4 * split.chunks && L.total > PLA_GDN_PREFILL_STATIC_BYTES; ++s) {
+      const GdnWorkspaceLayout longer = gdn_layout_of(T, N, H, HV, s, allow_stages);
+      if (longer.total <= PLA_GDN_PREFILL_STATIC_BYTES) L = longer;
     }
-  return gdn_layout_of(T, N, H, HV, best, allow_stages);
+  L.split_from = split.from;
+  return L;
 }
+
 
 // Workspace of pla_gdn_prefill_launch_static: one array per GPU, held until the process ends.  In host code the
 // array's name is only a handle for the runtime, not a device address; the address on the current device comes from
@@ -1584,6 +1601,7 @@ static int gdn_prefill_run(
     p.seg.identity = reinterpret_cast<float*>(ws + L.identity);
     p.seg.seg_chunks = L.seg_chunks;
     p.seg.max_segments = L.max_segments;
+    p.seg.split_from = L.split_from;
   }
   // the staged pipeline needs a side stream: without one (pool exhausted) the call runs unstaged, decided before
   // anything is launched
@@ -1646,7 +1664,7 @@ static int gdn_prefill_run(
       },
       [&](unsigned grid) {
         if (p.pass == 1) {        // first sweep over segments
-          const unsigned g = xcd_grouped_grid(grid / 2, (unsigned)(HV / H));
+          const unsigned g = 2 * xcd_grouped_grid(grid / 2, (unsigned)(HV / H));
           if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
           else hipLaunchKernelGGL(gdn_first_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
         } else {

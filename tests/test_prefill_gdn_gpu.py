@@ -301,7 +301,8 @@ def test_gdn_prefill_keys_copied_or_formed_by_the_sweep(H, HV):
 @pytest.mark.parametrize("lengths,tail_pad,H,HV", [
     ([2048], 0, 1, 4), ([2049], 3, 2, 4),                              # segments of three chunks; a last one of one token
     ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2),                  # one, two, three and more segments a sequence
-    ([3000, 5], 0, 8, 32), ([2111], 0, 16, 64)])                       # second sweep over whole pairs; few, long segments
+    ([3000, 5], 0, 8, 32), ([4159], 0, 16, 64),                        # second sweep over whole pairs; few, long segments
+    ([700, 760, 650], 2, 4, 12), ([2000, 1, 129], 0, 12, 12)])         # none split by the device; one on the line
 def test_gdn_prefill_segments_at_their_edges(lengths, tail_pad, H, HV):
     """A first segment of a split sequence is swept once, with output; the combine step only concerns the segments between
     the first and the last: sequences of one, of two and of many segments, ends one token beyond a segment's and one short of
