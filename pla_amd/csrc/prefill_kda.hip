@@ -530,11 +530,12 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
     return c;
   }
   const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0 || s.index == 0) return c;      // (the first sweep was done with the first segments)
+  if (s.sequence < 0 || (s.index == 0 && s.count > 1)) return c;      // (the first sweep was done with it)
   c.token = s.token;
   c.tokens = s.tokens;
   c.slot = s.slot;
-  c.init = p.seg.B + (int64_t)(index - p.H) * 16384;  // the state its predecessor ends in
+  // the caller's state for a sequence of one segment, else what its predecessor ends in
+  c.init = s.count == 1 ? kda_state_in(p, s.sequence, c.head) : p.seg.B + (int64_t)(index - p.H) * 16384;
   if (s.index + 1 == s.count) c.fin = kda_state_out(p, s.sequence, c.head);
   return c;
 }
@@ -591,14 +592,16 @@ __global__ __launch_bounds__(64 * (4 + FEEDERS), 1) void kda_sweep_mixed_kernel(
 // output - from a zero state (its B summary) and from the identity with v = 0 (its transition matrix M) - and both sweeps
 // multiply the same operands: wavefronts 0-3 carry the B columns (32 each), 4-7 the M columns, 8-11 form the operands.  A
 // first segment is swept from its real start state and for good, with output: wavefronts 0-7 carry 16 columns each (with 32
-// they need more registers than twelve wavefronts leave them), which takes about as long as the two roles of the others.
+// they need more registers than twelve wavefronts leave them), which takes about as long as the two roles of the others.  A
+// sequence of one segment is left to the second sweep, which may run it as two halves (four of 400 to 600 tokens, 16 heads, that
+// the kernels do not split: 51.9 us, swept here 62.5).
 template <bool PREPARED>
 __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_first_sweep_kernel(const KdaPrefillParams p) {
   __shared__ union { KdaLds<true> out; KdaLds<false> lean; } lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = blockIdx.x / p.H;
   const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0 || (s.index > 0 && s.index + 1 == s.count)) return;
+  if (s.sequence < 0 || s.index + 1 == s.count) return;
   const int64_t tile = (int64_t)blockIdx.x * 16384;
   Chain chain{};
   chain.token = s.token;
@@ -608,7 +611,7 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_first_sweep_kernel(
   if (s.index == 0) {
     ring_reset(&lds.out.flags);
     chain.init = kda_state_in(p, s.sequence, chain.head);
-    chain.fin = s.count == 1 ? kda_state_out(p, s.sequence, chain.head) : p.seg.B + tile;
+    chain.fin = p.seg.B + tile;
     if (wave < 8) kda_compute<1, true>(p, lds.out, chain, lane, 16 * wave);
     else if (PREPARED) kda_copy<true, FEEDERS>(p, lds.out, chain, lane, wave - 8, 8);
     else kda_produce<true, FEEDERS>(p, lds.out, chain, lane, wave - 8, 8);
@@ -628,11 +631,11 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_first_sweep_kernel(
 // Segments of a split call (at most 64 chains).  A call is priced in us (of steps 4 % longer than they are now) from its longest sequence (L chunks) and its (segment, head)
 // pairs: not split 13.5 + 2.84 L; split into segments of s chunks, 7.8 s for the two sweeps where the second one takes prepared
 // sub-chunks as halves (pairs on half of the CUs at most; preparing them takes 0.2 per thousand tokens and heads), 12.7 s otherwise, and
-// about 2 a segment for the combine step.  Segments are at
-// least as long as gives every CU one pair, with two thirds of a segment per sequence for what the lengths leave over (a second
-// round of pairs: six sequences of 2000 to 7000 tokens, 8 heads, 264 pairs 267 us, 216 pairs 233).  us per call, s = 3 / 4 / 8 / 16 / not
-// split: one of 2047 tokens, 4 heads 66.8 / 68.3 / 89.7 / 122 / 104; 4096, 8 heads 95 / 88 / 101 / 153 / 186; 3000, 16 heads 89 / 92 / 102 /
-// 154 / 145; 2047, 32 heads 129 / 90 / 106 / 135 / 112; two of 3000, 12 heads 137 / 148 / 129 / 162 / 152.
+// about 2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep, which runs one
+// segment less per split sequence than there are.  us per call, s = 3 / 4 / 8 / 16 / not split: one of 2048 tokens, 4 heads 63.4 / 64.4 /
+// 83.2 / - / 94.6; 4096, 8 heads 94.5 / 83.8 / 94.9 / 141 / 168; 3000, 16 heads 88.3 / 88.3 / 94.7 / 142 / 132; 2048, 32 heads 125 / 84.6 / 97.0 / - /
+// 101.  (The prices are from before first segments were swept once, for good; over fifty shapes their choice is 0-3 % from the best
+// length, 5 % for one of 3000 tokens, 32 heads.)
 // Splitting pays from sequences of about 15 + 0.13 chunks per chain on, 13 + 0.28 from 13 chains on (us split / not: 770 tokens, 1 head
 // 48.5 / 42.9; 890 48.5 / 47.1; 960 49.4 / 49.6; 870, 4 heads 50.6 / 49.2; 960 51.3 / 52.3; 960, 8 heads 53.7 / 52.9; 1020 55.1 / 55.6; 870,
 // 16 heads 56.7 / 53.2; 1150 62.8 / 65.3; 1150, 24 heads 66.9 / 65.3; 1250 67.3 / 69.0; 1300, 32 heads 72.1 / 73.4; 1400 75.7 / 77.4).
@@ -644,7 +647,7 @@ static KdaSplit kda_split(int T, int N, int H, bool prepares) {
   const int chains = N * H, chunks = (T - 1) / CHUNK + 1, mean = (chunks + N - 1) / N, line = std::max(15 + chains / 8, 13 + 9 * chains / 32);
   KdaSplit split{0, 0, false};
   if (N == 1 ? chunks < line : T / CHUNK < 32) return split;
-  const int per_head = std::max(1, CUS / H + (N == 1 ? 1 : N / 3)), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);
+  const int per_head = std::max(1, CUS / H + (N == 1 ? 1 : 0)), least = std::max(3, ((N == 1 ? chunks : T / CHUNK) + per_head - 1) / per_head);
   double best = 0.;
   for (int s = least; s <= least + 16; ++s) {
     const double pairs = (N == 1 ? (chunks - 1) / s : (double)chunks / s - 0.5 * N) * H;
