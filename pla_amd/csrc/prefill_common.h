@@ -300,7 +300,7 @@ struct SweepRole {
   int n, head, c_begin, c_end;
   const float* init;      // [V, K] tile the state starts from (nullptr: zero)
   float* fin;             // [V, K] tile that receives the state at the end (nullptr: none)
-  bool zero_v, output, active;
+  bool zero_v, active;
 };
 __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, const int32_t* seq_chunk_off,
                                                   const SegmentTable& seg, const StageTable& stg, int stage,
@@ -331,7 +331,6 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
     r.c_begin = inline_chunks.x >= 0 ? inline_chunks.x : seq_chunk_off[r.n];
     r.c_end = inline_chunks.x >= 0 ? inline_chunks.y : seq_chunk_off[r.n + 1];
     if (r.c_begin >= r.c_end) return r;              // empty sequence: state untouched, no output
-    r.output = true;
     r.init = state_in(r.n, r.head);
     r.fin = state_out(r.n, r.head);
     if (stg.stages > 0) carry = stg.carry + ((int64_t)r.n * heads + r.head) * 16384;
@@ -350,7 +349,6 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
     if (pass == 1) {
       if (first) {
         if (from_identity) return r;
-        r.output = true;
         r.init = state_in(r.n, r.head);
         r.fin = last ? state_out(r.n, r.head) : seg.B + tile;
       } else {
@@ -360,7 +358,6 @@ __device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, co
       }
     } else {
       if (first) return r;
-      r.output = true;
       r.init = seg.B + tile - (int64_t)heads * 16384;
       if (last) r.fin = state_out(r.n, r.head);
     }
