@@ -46,14 +46,19 @@ __device__ __forceinline__ bf16x8_t half8(f32x4_t a, f32x4_t b) {
 }
 // Saturating roundings: a magnitude beyond the fp16 range becomes the largest finite fp16 (65504), never an
 // infinity, so that out-of-range operands degrade the result instead of turning it into NaN.
-//   half8       round to nearest even, in a wavefront whose conversions saturate (fp16_saturates)
+//   half8_sat   round to nearest even after a clamp to +-65504 (one v_med3_f32 per element, which also turns an infinity or a
+//               NaN into a finite operand: 0 x inf in a triangular product would reach rows that do not depend on it)
 //   half8_rtz   round toward zero (v_cvt_pkrtz_f16_f32 saturates by itself); the error is one-sided, up to one
 //               unit in the last place, which is fine where many roundings average (the state slices) or where
 //               a low part follows
-//   half8_pair  hi = nearest (saturating as half8), lo = the rest rounded toward zero: x to about 22 bits, hi + lo
+//   half8_pair  hi = nearest after the clamp, lo = the rest rounded toward zero: x to about 22 bits, hi + lo
 //               saturating at 2 x 65504.  (hi is rounded to nearest so that values in fp16's subnormal range,
 //               where lo underflows to zero, keep an unbiased error.)
 typedef __fp16 fp16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ bf16x8_t half8_sat(f32x4_t a, f32x4_t b) {
+  auto c = [](float v) { return __builtin_amdgcn_fmed3f(v, -65504.f, 65504.f); };
+  return half8(f32x4_t{c(a.x), c(a.y), c(a.z), c(a.w)}, f32x4_t{c(b.x), c(b.y), c(b.z), c(b.w)});
+}
 __device__ __forceinline__ bf16x8_t half8_rtz(f32x4_t a, f32x4_t b) {
   const u32x4_t w = {__builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a.x, a.y)),
                      __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(a.z, a.w)),
@@ -68,7 +73,7 @@ __device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 |
 struct HalfPair { bf16x8_t hi, lo; };
 __device__ __forceinline__ HalfPair half8_pair(f32x4_t a, f32x4_t b) {
   HalfPair r;
-  r.hi = half8(a, b);
+  r.hi = half8_sat(a, b);
   const f32x8_t back = __builtin_convertvector(__builtin_bit_cast(f16x8_t, r.hi), f32x8_t);
   r.lo = half8_rtz(f32x4_t{a.x - back[0], a.y - back[1], a.z - back[2], a.w - back[3]},
                    f32x4_t{b.x - back[4], b.y - back[5], b.z - back[6], b.w - back[7]});

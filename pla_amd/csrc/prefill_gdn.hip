@@ -453,7 +453,6 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
   // of an operand tile, V with its columns in order)
   using CopyWide = SwizzledTileCopy<4>;
   constexpr int KV_HALVES = TILE128_HALVES;
-  fp16_saturates();
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -639,7 +638,7 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
       for (int s = 0; s < 2; ++s) {
         bf16x8_t xb[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) xb[nb] = half8(X[nb][2 * s], X[nb][2 * s + 1]);      // (saturating: fp16_saturates)
+        for (int nb = 0; nb < NB; ++nb) xb[nb] = half8_sat(X[nb][2 * s], X[nb][2 * s + 1]);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -1035,8 +1034,8 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 
   auto pk = [](float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, y)); };
-  auto pk_sat = [](float x, float y) {             // (saturating: fp16_saturates)
-    const f32x2_t c = {x, y};
+  auto pk_sat = [](float x, float y) {
+    const f32x2_t c = {__builtin_amdgcn_fmed3f(x, -65504.f, 65504.f), __builtin_amdgcn_fmed3f(y, -65504.f, 65504.f)};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(c, f16x2_t));
   };
   // hi = x rounded toward zero (which saturates at the largest finite fp16 value by itself), lo = the rest,

@@ -586,6 +586,38 @@ def test_gdn_prefill_operands_beyond_the_fp16_range_stay_finite():
     assert rel_l2(final[1], exp_final[1]) <= 1e-3
 
 
+@pytest.mark.parametrize("lengths,at,H,HV", [([150, 90], 37, 2, 4),                       # few chains: two workgroups each
+                                             ([100, 140, 70, 90, 65], 30, 16, 32),        # many chains, keys formed by the sweep
+                                             ([100, 140, 70, 90, 65], 130, 8, 32),        # many chains, keys copied
+                                             ([3000, 70], 1415, 2, 4)])                   # a segment that is swept for its summary
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_gdn_prefill_value_that_is_not_finite_stays_behind_its_token(lengths, at, H, HV, value):
+    """One infinite or NaN element of v in the middle of a chunk: the roundings to fp16 make it finite, so that the exact zeros
+    above the diagonal of the chunk's triangular operands keep it from the tokens before it.  Everything that does not depend
+    on it (those tokens, the other columns, heads and sequences, the states' other rows) has the bits of the call without it,
+    and nothing becomes infinite or NaN."""
+    from pla_amd.workloads import gdn_prefill_packed
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 2, seed=91 + at)
+    pool0 = w["initial_state"].clone()
+    offs, hv, col = w["_meta"]["offsets"], HV - 1, 77
+    hit = max(n for n in range(len(lengths)) if offs[n] <= at)
+    w["packed_qkv"] = w["packed_qkv"].clone()
+    results = []
+    for x in (1.0, value):
+        w["packed_qkv"][at, 2 * H * 128 + hv * 128 + col] = x
+        w["initial_state"].copy_(pool0)
+        _, _, o, _, final = _run_workload(w)
+        torch.cuda.synchronize()
+        results.append((o[0].clone(), final.clone()))
+    (o, final), (o_x, final_x) = results
+    assert torch.isfinite(o_x.float()).all() and torch.isfinite(final_x).all()
+    o[at:offs[hit + 1], hv, col] = 0
+    o_x[at:offs[hit + 1], hv, col] = 0
+    final[hit, hv, col] = 0
+    final_x[hit, hv, col] = 0
+    assert torch.equal(o, o_x) and torch.equal(final, final_x)
+
+
 def test_gdn_prefill_staged_calls_from_two_threads_on_two_streams():
     """Two host threads, each on a stream of its own, enqueue staged calls (fork to a side stream, join again) at
     the same time: every call takes a side stream and events of its own for the time it enqueues, so neither waits
