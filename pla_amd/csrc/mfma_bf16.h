@@ -66,10 +66,6 @@ __device__ __forceinline__ bf16x8_t half8_rtz(f32x4_t a, f32x4_t b) {
                      __builtin_bit_cast(unsigned, __builtin_amdgcn_cvt_pkrtz(b.z, b.w))};
   return __builtin_bit_cast(bf16x8_t, w);
 }
-// From here on this wavefront's conversions to fp16 round a finite value beyond the range to the largest finite fp16 (MODE bit
-// 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
-__device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
-
 struct HalfPair { bf16x8_t hi, lo; };
 __device__ __forceinline__ HalfPair half8_pair(f32x4_t a, f32x4_t b) {
   HalfPair r;

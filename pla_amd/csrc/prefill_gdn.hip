@@ -980,7 +980,6 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   }
 
   // ---- the computing wavefronts ----
-  fp16_saturates();
   const int vbase = 64 * v_half + 16 * NB * wave;
   // The lane's V column of block nb: with NB = 2 the two blocks take turns every four columns, so that a lane's outputs of
   // both (four adjacent columns of each) are sixteen bytes of a row, stored in one piece past the caches: with 8 bytes a

@@ -56,6 +56,10 @@ __device__ __forceinline__ bf16x8_t rest_bf16(const float (&x)[8], bf16x8_t hi) 
   return round_bf16(r);
 }
 
+// From here on this wavefront's conversions to fp16 round a finite value beyond the range to the largest finite fp16 (MODE bit
+// 23, FP16_OVFL; infinities stay): to nearest with the saturation that otherwise only rounding toward zero gives.
+__device__ __forceinline__ void fp16_saturates() { __builtin_amdgcn_s_setreg(1 | (23 << 6), 1); }
+
 // Four FP32 values as an fp16 pair each: hi to nearest after a clamp (SATURATES: of a wavefront whose conversions do that, see
 // fp16_saturates), the rest toward zero (as half8_pair).  x - hi is one v_fma_mix_f32, which takes a half of hi as it is, in the
 // place of x (in registers of its own the mixed sweep spills eight more); the compiler forms a conversion and a subtraction.  Both

@@ -618,6 +618,27 @@ def test_gdn_prefill_value_that_is_not_finite_stays_behind_its_token(lengths, at
     assert torch.equal(o, o_x) and torch.equal(final, final_x)
 
 
+@pytest.mark.parametrize("lengths,H,HV", [([100], 2, 4), ([100, 140, 70, 90, 65], 16, 32), ([2500], 2, 4)])
+def test_gdn_prefill_fp16_outputs_beyond_the_range_are_infinite(lengths, H, HV):
+    """fp16 activations: an output beyond the range is stored as an infinity of its sign, as a conversion to fp16 gives it (only
+    the roundings of operands saturate), so that a caller's check for overflow sees it.  Values of 2^12 and a scale of 1024
+    head-dimension scales keep every operand inside the range; outputs within 1.5 % of its end may fall on either side.  Few
+    chains, many chains, a call split into segments."""
+    from pla_amd.workloads import gdn_prefill_packed
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 2, seed=17, dtype=torch.float16)
+    w["packed_qkv"] = w["packed_qkv"].clone()
+    w["packed_qkv"][:, 2 * H * 128:] *= 4096
+    w["scale"] = 1024 * 128 ** -0.5
+    exp_o, _ = _oracle_workload(w, fast=True)
+    _, _, o, _, _ = _run_workload(w)
+    torch.cuda.synchronize()
+    o = o[0].cpu().double()
+    beyond, inside = exp_o.abs() > 1.015 * 65520, exp_o.abs() < 0.985 * 65504
+    assert beyond.sum() > 100 and inside.sum() > 100
+    assert torch.isinf(o[beyond]).all() and torch.equal(torch.sign(o[beyond]), torch.sign(exp_o[beyond]))
+    assert torch.isfinite(o[inside]).all()
+
+
 def test_gdn_prefill_staged_calls_from_two_threads_on_two_streams():
     """Two host threads, each on a stream of its own, enqueue staged calls (fork to a side stream, join again) at
     the same time: every call takes a side stream and events of its own for the time it enqueues, so neither waits
