@@ -463,6 +463,21 @@ int pla_kda_prefill_launch_raw(
     void* o, void* workspace, int64_t workspace_bytes,
     int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens);
 
+/*
+ * pla_kda_prefill_launch_raw for final states apart from the start states (ht shares no memory with h0): the final state
+ * of an empty sequence, which the other two calls leave as it is, is written as well, with its start state (or zero).
+ * What is empty is decided by cu_seqlens on the device.
+ */
+int pla_kda_prefill_launch_states(
+    const void* q, const void* k, const void* v, const void* g, const void* beta,
+    int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_g, int64_t stride_beta,
+    const float* A_log, const float* dt_bias, float lower_bound, float scale,
+    const int32_t* cu_seqlens, int N, int T,
+    const float* h0, const int32_t* h0_indices, int64_t h0_slot_stride,
+    float* ht, const int32_t* ht_indices, int64_t ht_slot_stride,
+    void* o, void* workspace, int64_t workspace_bytes,
+    int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens);
+
 /* As pla_gdn_prefill_halved_sequences, for pla_kda_prefill_launch_raw.  Host arithmetic only. */
 int pla_kda_prefill_halved_sequences(const int32_t* raw_cu_seqlens, int N, int T, int H);
 

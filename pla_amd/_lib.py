@@ -111,6 +111,14 @@ SIGNATURES = {
         _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64,
         _c_p, _c_p, _c_i64,
         _c_int, _c_int, _c_int, _c_int, _c_p, _c_p],
+    "pla_kda_prefill_launch_states": [
+        _c_p, _c_p, _c_p, _c_p, _c_p,
+        _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+        _c_p, _c_p, _c_f, _c_f,
+        _c_p, _c_int, _c_int,
+        _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64,
+        _c_p, _c_p, _c_i64,
+        _c_int, _c_int, _c_int, _c_int, _c_p, _c_p],
 }
 
 _lib = None

@@ -220,18 +220,22 @@ py::object try_gdn_prefill_packed_qkv_fwd(
 
 #ifdef PLA_BIND_FLASHKDAPRO
 // ---------------------------------------------------------------------------------------------------------------
+// Whether the bytes between the first and the last element of two tensors overlap.
+bool shares_memory(const Tensor& x, const Tensor& y) {
+  auto range = [](const Tensor& t) {
+    int64_t last = 0;
+    for (int64_t d = 0; d < t.dim(); ++d) last += (t.size(d) - 1) * t.stride(d);
+    const uintptr_t begin = reinterpret_cast<uintptr_t>(t.data_ptr());
+    return std::pair<uintptr_t, uintptr_t>(begin, begin + (uintptr_t)((last + 1) * t.element_size()));
+  };
+  const auto a = range(x), b = range(y);
+  return a.second > b.first && a.first < b.second;
+}
 // `t`, or a copy of it if it shares memory with `out` other than as its very rows (the kernels write rows of out while they read
 // others of their inputs; see pla_kda_prefill_launch).
 Tensor apart_from(const Tensor& t, const Tensor& out) {
-  auto range = [](const Tensor& x) {
-    int64_t last = 0;
-    for (int64_t d = 0; d < x.dim(); ++d) last += (x.size(d) - 1) * x.stride(d);
-    const uintptr_t begin = reinterpret_cast<uintptr_t>(x.data_ptr());
-    return std::pair<uintptr_t, uintptr_t>(begin, begin + (uintptr_t)((last + 1) * x.element_size()));
-  };
-  const auto a = range(t), b = range(out);
-  if (a.second <= b.first || a.first >= b.second) return t;
-  const bool same = a.first == b.first && t.scalar_type() == out.scalar_type() && t.sizes() == out.sizes() && t.strides() == out.strides();
+  if (!shares_memory(t, out)) return t;
+  const bool same = t.data_ptr() == out.data_ptr() && t.scalar_type() == out.scalar_type() && t.sizes() == out.sizes() && t.strides() == out.strides();
   return same ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
@@ -269,11 +273,11 @@ bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const T
 
   const int64_t ws_bytes = pla_kda_prefill_workspace_bytes((int)T, (int)N, (int)H);
   Tensor ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
-  // Sequences of length zero keep their incoming (or zero) state.  The launch writes every other final state itself, so where the
-  // host's offsets show that there is none, nothing is copied ahead of it (18 sequences of 12 heads: 28 MB, 6.7 us of 98.6).
-  bool empty = host_offsets.empty();
-  for (size_t n = 1; n < host_offsets.size(); ++n) empty = empty || host_offsets[n] == host_offsets[n - 1];
-  if (empty && final_state && !(initial_state && final_state->data_ptr() == initial_state->data_ptr())) {
+  // Sequences of length zero keep their incoming (or zero) state: in dense states apart from the incoming ones the launch writes
+  // it, else it is copied ahead of the launch.
+  const bool in_place = final_state && initial_state && final_state->data_ptr() == initial_state->data_ptr();
+  const bool by_launch = final_state && !indexed && !(initial_state && shares_memory(*initial_state, *final_state));
+  if (final_state && !in_place && !by_launch) {
     if (indexed) {
       const Tensor rows = state_indices->to(at::kLong);
       if (initial_state) final_state->index_copy_(0, rows, initial_state->index_select(0, rows));
@@ -285,7 +289,7 @@ bool try_flashkda_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const T
     }
   }
   const int32_t* idx = indexed ? state_indices->data_ptr<int32_t>() : nullptr;
-  launched(pla_kda_prefill_launch_raw(
+  launched((by_launch ? pla_kda_prefill_launch_states : pla_kda_prefill_launch_raw)(
       q_in.data_ptr(), k_in.data_ptr(), v.data_ptr(), g_in.data_ptr(), beta_in.data_ptr(), q_in.stride(0), k_in.stride(0), v.stride(0),
       g_in.stride(0), beta_in.stride(0), A_in.data_ptr<float>(), bias_in.data_ptr<float>(), (float)lower_bound, (float)scale,
       cu_seqlens->data_ptr<int32_t>(), (int)N, (int)T,

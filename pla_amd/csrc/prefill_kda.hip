@@ -69,6 +69,7 @@ struct KdaPrefillParams {
   int pass;                                        // 0: whole sequences; 1, 2: the two sweeps over segments
   int split_from;                                  // chunks of the longest sequence from which on any is split
   int H;
+  int empty_states;                                // also write the final states of empty sequences
   // kda_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long) as
   // two halves, the others those of seq_order[n_long .. N) whole
   unsigned split_grid; int n_long;
@@ -540,11 +541,26 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
   return c;
 }
 
+// The final state of an empty sequence, which no chain reaches: the one it starts from (or zero), by the workgroups that sweep
+// (sequence, head) `index`, or that segment and head, last.  (Copied ahead of the launch, for every sequence, it is a launch and up to 7 us: 18
+// sequences of 12 heads, 28 MB.)
+template <int NB>
+__device__ __forceinline__ void kda_empty_state(const KdaPrefillParams& p, int index, int half) {
+  const int n = index / p.H, head = index - n * p.H;
+  if (n >= p.N || sequence_tokens(p.cu_seqlens, n, p.T).y > 0) return;
+  const float* const src = kda_state_in(p, n, head);
+  float* const dst = kda_state_out(p, n, head);
+  if (dst == nullptr) return;
+  for (int i = 64 * 128 * half + 4 * threadIdx.x; i < 64 * 128 * (half + NB); i += 4 * blockDim.x)
+    *reinterpret_cast<float4*>(dst + i) = src != nullptr ? *reinterpret_cast<const float4*>(src + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
 constexpr int FEEDERS = 4;                         // producing or copying wavefronts of a workgroup
 template <int NB, bool PREPARED>
 __device__ __forceinline__ void kda_sweep(const KdaPrefillParams& p, KdaLds<true>& lds, int index, int half) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Chain chain = kda_chain(p, index, lane);
+  if (p.empty_states && (p.pass == 2 || chain.tokens == 0)) kda_empty_state<NB>(p, index, half);
   if (chain.tokens == 0) return;
   if (wave < 4) kda_compute<NB, true>(p, lds, chain, lane, 64 * half + 16 * NB * wave);
   else if (PREPARED) kda_copy<true, FEEDERS>(p, lds, chain, lane, wave - 4, 4);
@@ -739,7 +755,7 @@ static int kda_prefill_run(
     const float* h0, const int32_t* h0_indices, int64_t h0_slot_stride,
     float* ht, const int32_t* ht_indices, int64_t ht_slot_stride,
     void* o, void* workspace, int64_t workspace_bytes,
-    int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens) {
+    int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens, bool empty_states) {
   PLA_REQUIRE(K == 128 && V == 128, "KDA prefill requires head_dim K == V == 128, got K=%d, V=%d", K, V);
   PLA_REQUIRE(T > 0 && N > 0 && H > 0, "KDA prefill needs at least one token, sequence and head");
   PLA_REQUIRE(act_dtype == PLA_BF16, "KDA prefill takes bf16 activations");
@@ -766,6 +782,7 @@ static int kda_prefill_run(
   p.ht = ht; p.ht_indices = ht_indices; p.ht_slot_stride = ht_slot_stride;
   p.o = o;
   p.H = H;
+  p.empty_states = empty_states;
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool segmented = L.seg_chunks > 0, prepared = L.slots > 0;
@@ -823,7 +840,7 @@ extern "C" int pla_kda_prefill_launch(
     int H, int K, int V, int act_dtype, void* stream) {
   return kda_prefill_run(q, k, v, g, beta, stride_q, stride_k, stride_v, stride_g, stride_beta, A_log, dt_bias, lower_bound, scale,
                          cu_seqlens, N, T, h0, h0_indices, h0_slot_stride, ht, ht_indices, ht_slot_stride, o, workspace,
-                         workspace_bytes, H, K, V, act_dtype, stream, nullptr);
+                         workspace_bytes, H, K, V, act_dtype, stream, nullptr, false);
 }
 
 extern "C" int pla_kda_prefill_launch_raw(
@@ -837,7 +854,21 @@ extern "C" int pla_kda_prefill_launch_raw(
     int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens) {
   return kda_prefill_run(q, k, v, g, beta, stride_q, stride_k, stride_v, stride_g, stride_beta, A_log, dt_bias, lower_bound, scale,
                          cu_seqlens, N, T, h0, h0_indices, h0_slot_stride, ht, ht_indices, ht_slot_stride, o, workspace,
-                         workspace_bytes, H, K, V, act_dtype, stream, raw_cu_seqlens);
+                         workspace_bytes, H, K, V, act_dtype, stream, raw_cu_seqlens, false);
+}
+
+extern "C" int pla_kda_prefill_launch_states(
+    const void* q, const void* k, const void* v, const void* g, const void* beta,
+    int64_t stride_q, int64_t stride_k, int64_t stride_v, int64_t stride_g, int64_t stride_beta,
+    const float* A_log, const float* dt_bias, float lower_bound, float scale,
+    const int32_t* cu_seqlens, int N, int T,
+    const float* h0, const int32_t* h0_indices, int64_t h0_slot_stride,
+    float* ht, const int32_t* ht_indices, int64_t ht_slot_stride,
+    void* o, void* workspace, int64_t workspace_bytes,
+    int H, int K, int V, int act_dtype, void* stream, const int32_t* raw_cu_seqlens) {
+  return kda_prefill_run(q, k, v, g, beta, stride_q, stride_k, stride_v, stride_g, stride_beta, A_log, dt_bias, lower_bound, scale,
+                         cu_seqlens, N, T, h0, h0_indices, h0_slot_stride, ht, ht_indices, ht_slot_stride, o, workspace,
+                         workspace_bytes, H, K, V, act_dtype, stream, raw_cu_seqlens, true);
 }
 
 extern "C" int pla_kda_prefill_halved_sequences(const int32_t* raw_cu_seqlens, int N, int T, int H) {

@@ -35,16 +35,21 @@ def _token_rows(name, t, H, width):
     return t, t.stride(0)
 
 
+def _share_memory(x, y):
+    """Whether the bytes between the first and the last element of two tensors overlap."""
+    def span(t):
+        last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+        return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+    (begin, end), (other_begin, other_end) = span(x), span(y)
+    return end > other_begin and begin < other_end
+
+
 def _apart_from(t, out):
     """``t``, or a copy of it if it shares memory with ``out`` other than as its very rows (the kernels write rows of
     ``out`` while they read others of their inputs)."""
-    def span(x):
-        last = sum((n - 1) * s for n, s in zip(x.shape, x.stride()))
-        return x.data_ptr(), x.data_ptr() + (last + 1) * x.element_size()
-    (begin, end), (out_begin, out_end) = span(t), span(out)
-    if end <= out_begin or begin >= out_end:
+    if not _share_memory(t, out):
         return t
-    same = begin == out_begin and t.dtype == out.dtype and t.shape == out.shape and t.stride() == out.stride()
+    same = t.data_ptr() == out.data_ptr() and t.dtype == out.dtype and t.shape == out.shape and t.stride() == out.stride()
     return t if same else t.clone(memory_format=torch.contiguous_format)
 
 
@@ -200,11 +205,12 @@ def flashkda_fwd(
         return None
 
     ws, nbytes = _workspace(T, N, H, q.device)
-    # sequences of length zero keep their incoming (or zero) state: copied ahead of the launch, which writes every other final
-    # state itself, unless the host's offsets show that there is none
-    empty = raw_host is None or any(raw_host[n] == raw_host[n + 1] for n in range(N))
-    if empty and final_state is not None and not (initial_state is not None
-                                                  and final_state.data_ptr() == initial_state.data_ptr()):
+    # sequences of length zero keep their incoming (or zero) state: in dense states apart from the incoming ones the launch
+    # writes it, else it is copied ahead of the launch
+    in_place = final_state is not None and initial_state is not None and final_state.data_ptr() == initial_state.data_ptr()
+    by_launch = (final_state is not None and not indexed
+                 and not (initial_state is not None and _share_memory(initial_state, final_state)))
+    if final_state is not None and not in_place and not by_launch:
         if initial_state is not None:
             if indexed:
                 final_state[state_indices.long()] = initial_state[state_indices.long()]
@@ -217,7 +223,7 @@ def flashkda_fwd(
                 final_state[:N].zero_()
     idx_ptr = _lib.ptr(state_indices) if indexed else None
     _lib.call(
-        "pla_kda_prefill_launch_raw",
+        "pla_kda_prefill_launch_states" if by_launch else "pla_kda_prefill_launch_raw",
         q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(),
         sq, sk, sv, sg, beta.stride(0),
         A_log.data_ptr(), dt_bias.data_ptr(), float(lower_bound), float(scale),

@@ -336,6 +336,51 @@ def test_kda_prefill_in_a_graph(lengths, H):
         assert torch.equal(f_graph.view(torch.int32), f_eager.view(torch.int32)), replay
 
 
+@pytest.mark.parametrize("lengths,H", [([40, 70, 90], 4),                        # few chains: two workgroups each
+                                       ([64, 300, 100, 200], 40),                # many chains
+                                       ([1500, 200, 300, 400, 700], 32),         # the longest sequence as halves
+                                       ([2100, 700, 600], 2)])                   # split into segments
+@pytest.mark.parametrize("start", [False, True])
+@pytest.mark.parametrize("native", [False, True])
+def test_kda_prefill_sequence_that_is_empty_in_a_replay_only(lengths, H, start, native):
+    """A call captured with host offsets that show no empty sequence, replayed with device offsets that give the second one's
+    tokens to the first: the results are those of an eager call with the new offsets, final states of the empty sequence (its
+    start state, or zero) among them.  The host offsets change no bit."""
+    from pla_amd.prefill.flashkdapro import flashkda_fwd, ops
+    q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, H, seed=818)
+    args = [t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)]
+    ops._native = None if native else False
+    later = list(offs)
+    later[1] = offs[2]
+    cu = torch.tensor(offs, dtype=torch.int32, device="cuda")
+    new = torch.tensor(later, dtype=torch.int32, device="cuda")
+    S = S0.cuda() if start else None
+
+    def run(out, final, offsets, host):
+        flashkda_fwd(*args, out, initial_state=S, final_state=final, cu_seqlens=offsets, raw_cu_seqlens=host)
+
+    expected = torch.empty(q.shape, dtype=torch.bfloat16, device="cuda"), torch.full(S0.shape, float("nan"), device="cuda")
+    run(*expected, new, None)
+    got = torch.empty_like(expected[0]), torch.empty_like(expected[1])
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        run(*got, cu, tuple(offs))                             # warm-up on the capture stream
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        run(*got, cu, tuple(offs))
+    cu.copy_(new)
+    for _ in range(2):
+        got[0].fill_(float("nan"))
+        got[1].fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got[1][1], S[1] if start else torch.zeros_like(got[1][1]))
+        assert torch.equal(got[0], expected[0]) and torch.equal(got[1], expected[1])
+
+
 @pytest.mark.parametrize("lengths,pad,H", [([2500, 0, 1111, 40], 5, 2), ([4096], 0, 1), ([1030, 2049], 0, 3)])
 def test_kda_prefill_split_sequences_match_oracle(lengths, pad, H):
     """Few, long sequences are split into segments that are swept concurrently (zero-state
@@ -371,8 +416,8 @@ def test_kda_prefill_split_sequences_match_oracle(lengths, pad, H):
 @pytest.mark.parametrize("start", [False, True])
 @pytest.mark.parametrize("native", [False, True])
 def test_kda_prefill_final_states_with_host_offsets(lengths, start, native):
-    """The host copies the start states ahead of the launch for sequences of length zero only, where its offsets tell: every
-    final state is written either way (the buffer holds NaN), with the bits of the call without host offsets."""
+    """Every final state is written (the buffer holds NaN), those of sequences of length zero too, with and without host offsets
+    and with the same bits."""
     from pla_amd.prefill.flashkdapro import flashkda_fwd, ops
     q, k, v, raw, beta, A_log, dt_bias, offs, S0 = _inputs(lengths, 2, seed=717)
     args = [t.cuda() for t in (q, k, v, raw, beta, A_log, dt_bias)]
