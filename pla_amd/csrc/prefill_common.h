@@ -292,79 +292,40 @@ __device__ __forceinline__ int xcd_grouped_index(int hw_index, int group, int to
   return logical < total ? logical : -1;
 }
 
-// What one workgroup of a sequential kernel sweeps: a whole sequence (pass 0, blockIdx = (sequence,
-// head)) or one segment in one of the roles above (pass 1: blockIdx = (segment, head, from-identity
-// flag); pass 2: (segment, head)); with stages (passes 0 and 1) only the part of it that belongs to
-// `stage`, which may hold no chunk at all, the state being carried from stage to stage in a tile.
+// What one workgroup of a GDN sweep runs through: a whole sequence (with stages only the part of it that belongs to
+// `stage`, which may hold no chunk at all, the state being carried from stage to stage in a tile), or one segment of a split
+// call in one of the roles above.
 struct SweepRole {
   int n, head, c_begin, c_end;
   const float* init;      // [V, K] tile the state starts from (nullptr: zero)
   float* fin;             // [V, K] tile that receives the state at the end (nullptr: none)
   bool zero_v, active;
 };
-__device__ __forceinline__ SweepRole select_sweep(int pass, int heads, int N, const int32_t* seq_chunk_off,
-                                                  const SegmentTable& seg, const StageTable& stg, int stage,
-                                                  const float* h0, const int32_t* h0_indices,
-                                                  int64_t h0_slot_stride, float* ht, const int32_t* ht_indices,
-                                                  int64_t ht_slot_stride, int block = -1,
-                                                  const int3 inline_chunks = int3{-1, 0, 0}) {
-  // inline_chunks (pass 0 only, x >= 0): (first chunk, end chunk, stages in effect) of the workgroup's sequence worked
-  // out by the caller (inline_sequences) instead of read from the tables
-  // block: the logical workgroup index when the caller remaps blockIdx (see xcd_grouped_index), else blockIdx.x
-  // Segments: the first sweep runs a FIRST segment with output from the caller's state and those between the first and
-  // the last for their summaries; the second sweep runs every later segment with output, from the state the combine
-  // step left in its predecessor's B, and the last one delivers the final state.
+struct SweepStates { const float* h0; const int32_t* h0_indices; int64_t h0_slot_stride; float* ht; const int32_t* ht_indices; int64_t ht_slot_stride; };
+__device__ __forceinline__ const float* state_in(const SweepStates& x, int n, int head) {
+  const int slot = (x.h0 != nullptr) ? (x.h0_indices ? x.h0_indices[n] : n) : -1;
+  return slot >= 0 ? x.h0 + (int64_t)slot * x.h0_slot_stride + (int64_t)head * 16384 : nullptr;
+}
+__device__ __forceinline__ float* state_out(const SweepStates& x, int n, int head) {
+  const int slot = (x.ht != nullptr) ? (x.ht_indices ? x.ht_indices[n] : n) : -1;
+  return slot >= 0 ? x.ht + (int64_t)slot * x.ht_slot_stride + (int64_t)head * 16384 : nullptr;
+}
+// block: logical index of the (sequence, head).  inline_chunks (x >= 0): (first chunk, end chunk, stages in effect) of its sequence
+// worked out by the caller (inline_sequences) instead of read from the tables.
+__device__ __forceinline__ SweepRole sequence_role(int block, int heads, const int32_t* seq_chunk_off, const StageTable& stg, int stage,
+                                                   const SweepStates& states, const int3 inline_chunks) {
   SweepRole r{};
-  auto state_in = [&](int n, int head) -> const float* {
-    const int slot = (h0 != nullptr) ? (h0_indices ? h0_indices[n] : n) : -1;
-    return slot >= 0 ? h0 + (int64_t)slot * h0_slot_stride + (int64_t)head * 16384 : nullptr;
-  };
-  auto state_out = [&](int n, int head) -> float* {
-    const int slot = (ht != nullptr) ? (ht_indices ? ht_indices[n] : n) : -1;
-    return slot >= 0 ? ht + (int64_t)slot * ht_slot_stride + (int64_t)head * 16384 : nullptr;
-  };
-  float* carry = nullptr;
-  if (pass == 0) {
-    const int logical = block >= 0 ? block : (int)blockIdx.x;
-    r.n = logical / heads;
-    r.head = logical - r.n * heads;
-    r.c_begin = inline_chunks.x >= 0 ? inline_chunks.x : seq_chunk_off[r.n];
-    r.c_end = inline_chunks.x >= 0 ? inline_chunks.y : seq_chunk_off[r.n + 1];
-    if (r.c_begin >= r.c_end) return r;              // empty sequence: state untouched, no output
-    r.init = state_in(r.n, r.head);
-    r.fin = state_out(r.n, r.head);
-    if (stg.stages > 0) carry = stg.carry + ((int64_t)r.n * heads + r.head) * 16384;
-  } else {
-    const int logical = block >= 0 ? block : (int)blockIdx.x;
-    const int item = pass == 1 ? (logical >> 1) : logical;
-    const bool from_identity = pass == 1 && (logical & 1);
-    const int s = item / heads;
-    r.head = item - s * heads;
-    if (s >= seg.seq_seg_off[N]) return r;
-    r.n = seg.seg_seq[s];
-    const bool first = s == seg.seq_seg_off[r.n], last = s + 1 == seg.seq_seg_off[r.n + 1];
-    r.c_begin = seg.seg_c0[s];
-    r.c_end = r.c_begin + seg.seg_nc[s];
-    const int64_t tile = ((int64_t)s * heads + r.head) * 16384;
-    if (pass == 1) {
-      if (first) {
-        if (from_identity) return r;
-        r.init = state_in(r.n, r.head);
-        r.fin = last ? state_out(r.n, r.head) : seg.B + tile;
-      } else {
-        if (last) return r;
-        if (from_identity) { r.init = seg.identity; r.zero_v = true; r.fin = seg.M + tile; }
-        else r.fin = seg.B + tile;
-      }
-    } else {
-      if (first) return r;
-      r.init = seg.B + tile - (int64_t)heads * 16384;
-      if (last) r.fin = state_out(r.n, r.head);
-    }
-  }
-  if (carry != nullptr && stg.stages > 0) {
+  r.n = block / heads;
+  r.head = block - r.n * heads;
+  r.c_begin = inline_chunks.x >= 0 ? inline_chunks.x : seq_chunk_off[r.n];
+  r.c_end = inline_chunks.x >= 0 ? inline_chunks.y : seq_chunk_off[r.n + 1];
+  if (r.c_begin >= r.c_end) return r;              // empty sequence: state untouched, no output
+  r.init = state_in(states, r.n, r.head);
+  r.fin = state_out(states, r.n, r.head);
+  if (stg.stages > 0) {
     const int E = inline_chunks.x >= 0 ? inline_chunks.z : stg.stage_begin[MAX_STAGES + 1];   // the plan word (stage_plan)
     if (stage >= plan_stages(E)) return r;                                      // an empty stage: the one before it delivered the state
+    float* const carry = stg.carry + ((int64_t)r.n * heads + r.head) * 16384;
     const int nc = r.c_end - r.c_begin, c0 = r.c_begin;
     r.c_begin = c0 + stage_cut(nc, stage, E);
     r.c_end = c0 + stage_cut(nc, stage + 1, E);
@@ -453,6 +414,56 @@ __device__ __forceinline__ SegmentCounts count_segments(const int32_t* cu_seqlen
   r.chunks = longest < split_from ? max(longest, 1) : seg_chunks;
   r.count = (nc + r.chunks - 1) / r.chunks;
   r.before = wave_inclusive_scan(r.count) - r.count;
+  return r;
+}
+
+// Segment `i` of those that one of the sweeps over segments runs: the first one all but the last of each sequence (`second`: all
+// but the first), a sequence of one segment belonging to the sweep that names it (`singles`).  `count` is that of the lane's sequence.
+// Counted like this, the workgroups of segments that a sweep does not run are all behind the others in its grid.  Among them each
+// takes its turn on a CU, and as workgroups go to the XCDs and their engines in turn, full or not, 228 that swept could take two rounds
+// on 256 CUs (first sweep, us, among them / behind: KDA, 2245 + 1173 + 1657 + 1355 tokens of 12 heads 84.0 / 48.6; GDN, three of 4200 to
+// 4500 tokens, 16 value heads 87.0 / 53.8; 16 384 tokens, 32 value heads, where it is the last 32 of 288, 128 / 105.6).
+struct SweptSegment { int sequence, index, count, number; };      // sequence < 0: none; number: among all segments of the call
+struct SweptSegments { int before, swept; unsigned long long left_out; };
+__device__ __forceinline__ SweptSegments swept_segments(int count, bool singles) {      // lane n: of sequence n
+  SweptSegments r;
+  r.swept = count > 1 ? count - 1 : singles ? count : 0;
+  r.before = wave_inclusive_scan(r.swept) - r.swept;
+  r.left_out = __ballot(count > r.swept);
+  return r;
+}
+__device__ __forceinline__ SweptSegment swept_segment(const SweptSegments& s, int count, bool second, int i) {
+  const unsigned long long owner = __ballot(i >= s.before && i < s.before + s.swept);
+  if (owner == 0) return SweptSegment{-1, 0, 0, 0};
+  SweptSegment r;
+  r.sequence = __builtin_amdgcn_readfirstlane(__ffsll((long long)owner) - 1);
+  r.count = __builtin_amdgcn_readlane(count, r.sequence);
+  const int before = __builtin_amdgcn_readlane(s.before, r.sequence);
+  r.index = i - before + (second && r.count > 1 ? 1 : 0);
+  r.number = before + __popcll(s.left_out & ((1ull << r.sequence) - 1)) + r.index;
+  return r;
+}
+// The role of (segment, head) in a sweep of a GDN call.
+//   FIRST_OUT  first sweep, a first segment: with output from the caller's state
+//   ZERO, IDENTITY  first sweep, a segment between the first and the last: for its summaries B and M
+//   LATER      second sweep: with output from the state that the combine step left in its predecessor's B
+enum class SegmentSweep { FIRST_OUT, ZERO, IDENTITY, LATER };
+__device__ __forceinline__ SweepRole segment_role(SegmentSweep sweep, const SweptSegment& s, int head, int heads, const SegmentTable& seg,
+                                                  const SweepStates& states) {
+  SweepRole r{};
+  if (s.sequence < 0 || s.number >= seg.max_segments) return r;      // (number: offsets that do not fit the workspace)
+  r.active = true;
+  r.n = s.sequence;
+  r.head = head;
+  r.c_begin = seg.seg_c0[s.number];
+  r.c_end = r.c_begin + seg.seg_nc[s.number];
+  const int64_t tile = ((int64_t)s.number * heads + head) * 16384;
+  if (sweep == SegmentSweep::FIRST_OUT) r.init = state_in(states, r.n, head);
+  if (sweep == SegmentSweep::IDENTITY) { r.init = seg.identity; r.zero_v = true; }
+  if (sweep == SegmentSweep::LATER) r.init = seg.B + tile - (int64_t)heads * 16384;
+  if (sweep == SegmentSweep::IDENTITY) r.fin = seg.M + tile;
+  else if (s.index + 1 == s.count) r.fin = state_out(states, r.n, head);
+  else if (sweep != SegmentSweep::LATER) r.fin = seg.B + tile;
   return r;
 }
 
@@ -786,7 +797,7 @@ template <typename Prepare, typename Sweep>
 inline bool launch_pipeline(hipStream_t s, int stages, SideStream* side, bool segmented, unsigned grid_whole,
                             unsigned grid_segments, int* pass_field, int* stage_field, Prepare prepare, Sweep sweep) {
   *pass_field = segmented ? 1 : 0;
-  const unsigned grid = segmented ? 2 * grid_segments : grid_whole;
+  const unsigned grid = segmented ? grid_segments : grid_whole;
   if (stages == 0) {
     *stage_field = 0;
     prepare(s);

@@ -62,9 +62,7 @@ struct GdnPrefillParams {
   const int32_t* cu_seqlens; int N; int T;            // packed offsets, sequences, physical tokens
   float scale; int normalize_qk;
   // state
-  const float* h0; const int32_t* h0_indices; int64_t h0_slot_stride;   // read (may be null)
-  float* ht; const int32_t* ht_indices; int64_t ht_slot_stride;         // written (may be null)
-  // output
+  SweepStates states;                                 // h0 read, ht written (either may be null)
   void* o;                                            // [T, HV, 128] dense
   // workspace
   int32_t* seq_chunk_off; int32_t* chunk_seq; int32_t* chunk_tok; int32_t* chunk_len;
@@ -81,6 +79,7 @@ struct GdnPrefillParams {
   int inline_tables;     // at most 64 whole sequences: kernels work the chunk tables out themselves (no table kernel)
   int tail_blocks;       // workgroups appended to the preparation grid that zero the output rows beyond the last sequence
   int store_kn;          // gdn_wsolve_kernel stores the normalised K rows (kn) for the sweeps to copy, else 1 / |k|
+  // gdn_first_sweep_kernel: the workgroups from `split_grid` on take the second halves of first segments
   // gdn_fused_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long)
   // as two halves, the others those of seq_order[n_long .. N) whole
   unsigned split_grid; int n_long;
@@ -445,7 +444,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefill
 constexpr int LEAN_OFF_W = 0, LEAN_OFF_G = LEAN_OFF_W + 2 * 2 * TRI_BLOCKS * 1024, LEAN_OFF_K = LEAN_OFF_G + 2 * 1024;
 constexpr int LEAN_OFF_V = LEAN_OFF_K + 2 * TILE128_HALVES * 2, LEAN_LDS_BYTES = LEAN_OFF_V + 2 * TILE128_HALVES * 2;
 template <typename act_t>
-__device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int pair) {
+__device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const SweptSegment& segment, const int hv) {
   constexpr int NB = 2;
   // what gdn_wsolve_kernel left per (chunk, value head): W (six blocks hi, six lo) and the tile of decay factors
   constexpr int W_BYTES = 2 * TRI_BLOCKS * 1024, G_BYTES = GTILE_FLOATS * 4;
@@ -461,14 +460,9 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
   const int cw = wave & 3;                                     // position among the four wavefronts of a role
   const int vcol = 32 * cw + r16;
 
-  // the two roles of this (segment, head): logical workgroups 2 i (zero state) and 2 i + 1 (identity)
-  const SweepRole lead = select_sweep(1, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
-                                      p.ht, p.ht_indices, p.ht_slot_stride, 2 * pair);
-  if (!lead.active) return;
-  const SweepRole mrole = select_sweep(1, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
-                                       p.ht, p.ht_indices, p.ht_slot_stride, 2 * pair + 1);
-  const SweepRole& role = m_side ? mrole : lead;
-  const int n = lead.n, hv = lead.head, c_begin = lead.c_begin, c_end = lead.c_end;
+  const SweepRole role = segment_role(m_side ? SegmentSweep::IDENTITY : SegmentSweep::ZERO, segment, hv, p.HV, p.seg, p.states);
+  if (!role.active) return;
+  const int n = role.n, c_begin = role.c_begin, c_end = role.c_end;
   const int h = hv / (p.HV / p.H);
   const int seq_start = p.cu_seqlens[n] + (c_begin - p.seq_chunk_off[n]) * CHUNK;
   const int seq_len = min(p.cu_seqlens[n + 1] - seq_start, (c_end - c_begin) * CHUNK);
@@ -733,10 +727,11 @@ constexpr int FUSED_OFF_W = (FUSED_OFF_RQ + 2 * CHUNK * 4 + 1023) / 1024 * 1024,
 constexpr int FUSED_OFF_K = FUSED_OFF_Q + 2 * TILE128_HALVES * 2, FUSED_OFF_V = FUSED_OFF_K + 2 * TILE128_HALVES * 2;
 constexpr int FUSED_LDS_BYTES = FUSED_OFF_V + 2 * TILE128_HALVES * 2;
 
-// The sweep of one workgroup.  `wide`: 2 / NB x the chain's logical index (sequence x HV + value head, or segment x
-// HV + value head in the second sweep over segments) plus, for NB = 1, the half of the V columns it takes.
+// The sweep of one workgroup.  `wide`: 2 / NB x the chain's logical index (sequence x HV + value head, or that of `segment` among
+// those of a sweep over segments) plus, for NB = 1, the half of the V columns it takes.
 template <typename act_t, int NB, bool KN>
-__device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int wide) {
+__device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int wide,
+                                            const SweptSegment& segment = SweptSegment{-1, 0, 0, 0}) {
   constexpr int CW = 4, AUX = 4;
   constexpr int HALVES = 2 / NB;             // workgroups per chain: NB = 1 sweeps 64 of the 128 V columns
   using CopyTile = SwizzledTileCopy<AUX>;
@@ -755,8 +750,9 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
     seq_end_token = seq_first_token + __builtin_amdgcn_readlane(seqs.len, n0);
     inline_chunks = int3{seq_first_chunk, min(seq_first_chunk + __builtin_amdgcn_readlane(seqs.nc, n0), p.NC_max), seqs.E};
   }
-  const SweepRole role = select_sweep(p.pass, p.HV, p.N, p.seq_chunk_off, p.seg, p.stg, p.stage, p.h0, p.h0_indices, p.h0_slot_stride,
-                                      p.ht, p.ht_indices, p.ht_slot_stride, p.pass == 1 ? 2 * block : block, inline_chunks);
+  const SweepRole role = p.pass == 0 ? sequence_role(block, p.HV, p.seq_chunk_off, p.stg, p.stage, p.states, inline_chunks)
+                                     : segment_role(p.pass == 1 ? SegmentSweep::FIRST_OUT : SegmentSweep::LATER, segment, block % p.HV,
+                                                    p.HV, p.seg, p.states);
   if (!role.active) return;
   const int n = role.n, hv = role.head, c_begin = role.c_begin, c_end = role.c_end;
   const int h = hv / (p.HV / p.H);
@@ -1311,6 +1307,12 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
 }
 #undef SB
 
+// Segments of the lane's sequence in a split call (at most 64 sequences).
+__device__ __forceinline__ int segment_count(const GdnPrefillParams& p) {
+  const int lane = threadIdx.x & 63;
+  return lane < p.N ? p.seg.seq_seg_off[lane + 1] - p.seg.seq_seg_off[lane] : 0;
+}
+
 // One workgroup per (sequence, value head), or per (segment, value head) in the second sweep over segments (NB = 2);
 // NB = 1: two per chain, 64 V columns each (the columns of V are independent: same bits).
 template <typename act_t, int NB, bool KN>
@@ -1319,7 +1321,12 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_kernel(const GdnPrefil
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   const int wide = xcd_grouped_index(blockIdx.x, HALVES * (p.HV / p.H), HALVES * (p.pass == 2 ? p.seg.max_segments : p.N) * p.HV);
   if (wide < 0) return;
-  fused_sweep<act_t, NB, KN>(p, lds_all, wide);
+  SweptSegment segment{-1, 0, 0, 0};
+  if (KN && p.pass == 2) {
+    const int count = segment_count(p);
+    segment = swept_segment(swept_segments(count, false), count, true, wide / HALVES / p.HV);
+  }
+  fused_sweep<act_t, NB, KN>(p, lds_all, wide, segment);
 }
 
 // Whole sequences of unequal length, swept in one launch whose longest chains decide how long it lasts while the CUs
@@ -1343,25 +1350,31 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
 }
 
 // First sweep over segments: first segments for good, with output, from their real start states (which takes as long per
-// chunk as the two roles of the others), those behind them for their summaries.  Two workgroups a (segment, value head): where
-// all of them together leave CUs for it both sweep a first segment, 64 V columns each, else the first one does it alone, as it
-// does with the summaries.
+// chunk as the two roles of the others), those behind them for their summaries.  Where all of them together leave CUs for it two
+// workgroups sweep a first segment, 64 V columns each.
 template <typename act_t>
 __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefillParams p) {
   static_assert(LEAN_LDS_BYTES <= FUSED_LDS_BYTES, "one array serves both sweeps");
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
-  const int pairs = p.seg.max_segments * p.HV, grid = gridDim.x / 2;
-  const bool second = (int)blockIdx.x >= grid;             // (behind all others in the grid)
-  const int pair = xcd_grouped_index(second ? blockIdx.x - grid : blockIdx.x, p.HV / p.H, pairs);
+  const int ratio = p.HV / p.H;
+  const bool second = blockIdx.x >= p.split_grid;          // (behind all others in the grid: one for every sequence's first segment)
+  const int pair = second ? xcd_grouped_index(blockIdx.x - p.split_grid, ratio, p.N * p.HV)
+                          : xcd_grouped_index(blockIdx.x, ratio, p.seg.max_segments * p.HV);
   if (pair < 0) return;
-  const int s = pair / p.HV, segments = p.seg.seq_seg_off[p.N];
-  if (s >= segments) return;
-  const bool first = s == p.seg.seq_seg_off[p.seg.seg_seq[s]], halves = segments * p.HV <= CUS;
-  if (first && halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * pair + (second ? 1 : 0));
-  else if (second) return;
-  else if (first) fused_sweep<act_t, 2, true>(p, lds_all, pair);
-  else lean_sweep<act_t>(p, lds_all, pair);
+  const int item = pair / p.HV, hv = pair - item * p.HV, count = segment_count(p);
+  const SweptSegments s = swept_segments(count, true);
+  const int workgroups = __builtin_amdgcn_readlane(wave_inclusive_scan(s.swept + (count > 0)), 63) * p.HV;
+  const bool halves = workgroups <= CUS;
+  SweptSegment segment = swept_segment(s, count, false, item);
+  if (second) {
+    const int n_count = __builtin_amdgcn_readlane(count, item);
+    segment = SweptSegment{halves && n_count > 0 ? item : -1, 0, n_count, p.seg.seq_seg_off[item]};
+  }
+  if (segment.sequence < 0) return;
+  if (segment.index > 0) lean_sweep<act_t>(p, lds_all, segment, hv);
+  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + second, segment);
+  else fused_sweep<act_t, 2, true>(p, lds_all, hv, segment);
 }
 
 struct GdnWorkspaceLayout {
@@ -1552,8 +1565,7 @@ static int gdn_prefill_run(
   p.a = a; p.b = b; p.stride_a = stride_a; p.stride_b = stride_b;
   p.A_log = A_log; p.dt_bias = dt_bias; p.g_in = g_in; p.beta_in = beta_in;
   p.cu_seqlens = cu_seqlens; p.N = N; p.T = T; p.scale = scale; p.normalize_qk = normalize_qk;
-  p.h0 = h0; p.h0_indices = h0_indices; p.h0_slot_stride = h0_slot_stride;
-  p.ht = ht; p.ht_indices = ht_indices; p.ht_slot_stride = ht_slot_stride;
+  p.states = SweepStates{h0, h0_indices, h0_slot_stride, ht, ht_indices, ht_slot_stride};
   p.o = o;
   p.seq_chunk_off = reinterpret_cast<int32_t*>(ws + L.seq_chunk_off);
   p.chunk_seq = reinterpret_cast<int32_t*>(ws + L.chunk_seq);
@@ -1662,7 +1674,8 @@ static int gdn_prefill_run(
       },
       [&](unsigned grid) {
         if (p.pass == 1) {        // first sweep over segments
-          const unsigned g = 2 * xcd_grouped_grid(grid / 2, (unsigned)(HV / H));
+          p.split_grid = xcd_grouped_grid(grid, (unsigned)(HV / H));
+          const unsigned g = p.split_grid + xcd_grouped_grid((unsigned)N * HV, (unsigned)(HV / H));
           if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
           else hipLaunchKernelGGL(gdn_first_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
         } else {

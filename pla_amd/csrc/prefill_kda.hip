@@ -516,7 +516,7 @@ __device__ __forceinline__ float* kda_state_out(const KdaPrefillParams& p, int n
   return slot >= 0 ? p.ht + (int64_t)slot * p.ht_slot_stride + (int64_t)head * 16384 : nullptr;
 }
 
-// The chain of logical index `index`: (sequence, head), or (segment, head) in the second sweep over segments.
+// The chain of logical index `index`: (sequence, head), or (segment, head) of those that the second sweep runs.
 __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index, int lane) {
   Chain c{};
   const int item = index / p.H;
@@ -530,13 +530,13 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
     c.fin = kda_state_out(p, item, c.head);
     return c;
   }
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0 || (s.index == 0 && s.count > 1)) return c;      // (the first sweep was done with it)
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, p.split_from, true, item, lane);
+  if (s.sequence < 0) return c;
   c.token = s.token;
   c.tokens = s.tokens;
   c.slot = s.slot;
   // the caller's state for a sequence of one segment, else what its predecessor ends in
-  c.init = s.count == 1 ? kda_state_in(p, s.sequence, c.head) : p.seg.B + (int64_t)(index - p.H) * 16384;
+  c.init = s.count == 1 ? kda_state_in(p, s.sequence, c.head) : p.seg.B + ((int64_t)(s.number - 1) * p.H + c.head) * 16384;
   if (s.index + 1 == s.count) c.fin = kda_state_out(p, s.sequence, c.head);
   return c;
 }
@@ -616,14 +616,14 @@ __global__ __launch_bounds__(64 * (8 + FEEDERS), 1) void kda_first_sweep_kernel(
   __shared__ union { KdaLds<true> out; KdaLds<false> lean; } lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = blockIdx.x / p.H;
-  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg.seg_chunks, p.split_from, item, lane);
-  if (s.sequence < 0 || s.index + 1 == s.count) return;
-  const int64_t tile = (int64_t)blockIdx.x * 16384;
+  const Segment s = inline_segment(p.cu_seqlens, p.N, p.T, p.seg, p.split_from, false, item, lane);
+  if (s.sequence < 0) return;
   Chain chain{};
   chain.token = s.token;
   chain.tokens = s.tokens;
   chain.slot = s.slot;
   chain.head = blockIdx.x - item * p.H;
+  const int64_t tile = ((int64_t)s.number * p.H + chain.head) * 16384;
   if (s.index == 0) {
     ring_reset(&lds.out.flags);
     chain.init = kda_state_in(p, s.sequence, chain.head);

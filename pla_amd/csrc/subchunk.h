@@ -226,16 +226,17 @@ struct Chain {
 // Sub-chunk i of sequence n is number first_slot + i among the prepared ones of a call: sequences do not overlap in it, whatever
 // their lengths, and no table is needed.
 __device__ __forceinline__ int64_t first_slot(int n, int token) { return token / SUB + n; }
-// Segment s of a split call (count_segments).  sequence < 0: the call has fewer segments.
-struct Segment { int sequence, index, count, token, tokens; int64_t slot; };
-__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, int seg_chunks, int split_from, int s, int lane) {
-  const SegmentCounts c = count_segments(cu_seqlens, N, T, seg_chunks, split_from, lane);
-  Segment r{-1, 0, 0, 0, 0, 0};
-  const unsigned long long owner = __ballot(s >= c.before && s < c.before + c.count);
-  if (owner == 0) return r;
-  r.sequence = __builtin_amdgcn_readfirstlane(__ffsll((long long)owner) - 1);
-  r.index = s - __builtin_amdgcn_readlane(c.before, r.sequence);
-  r.count = __builtin_amdgcn_readlane(c.count, r.sequence);
+// Segment `i` of those that a sweep over the segments of a split call runs (swept_segment).  sequence < 0: it runs fewer.
+struct Segment { int sequence, index, count, number, token, tokens; int64_t slot; };
+__device__ __forceinline__ Segment inline_segment(const int32_t* cu_seqlens, int N, int T, const SegmentTable& t, int split_from, bool second, int i, int lane) {
+  const SegmentCounts c = count_segments(cu_seqlens, N, T, t.seg_chunks, split_from, lane);
+  const SweptSegment s = swept_segment(swept_segments(c.count, second), c.count, second, i);
+  Segment r{-1, 0, 0, 0, 0, 0, 0};
+  if (s.sequence < 0 || s.number >= t.max_segments) return r;      // (number: offsets that do not fit the workspace)
+  r.sequence = s.sequence;
+  r.index = s.index;
+  r.count = s.count;
+  r.number = s.number;
   const int skipped = r.index * c.chunks * CHUNK;
   r.token = __builtin_amdgcn_readlane(c.tokens.x, r.sequence) + skipped;
   r.slot = first_slot(r.sequence, r.token - skipped) + skipped / SUB;
