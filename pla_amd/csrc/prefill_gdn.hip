@@ -79,7 +79,6 @@ struct GdnPrefillParams {
   int inline_tables;     // at most 64 whole sequences: kernels work the chunk tables out themselves (no table kernel)
   int tail_blocks;       // workgroups appended to the preparation grid that zero the output rows beyond the last sequence
   int store_kn;          // gdn_wsolve_kernel stores the normalised K rows (kn) for the sweeps to copy, else 1 / |k|
-  // gdn_first_sweep_kernel: the workgroups from `split_grid` on take the second halves of first segments
   // gdn_fused_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long)
   // as two halves, the others those of seq_order[n_long .. N) whole
   unsigned split_grid; int n_long;
@@ -1350,30 +1349,32 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
 }
 
 // First sweep over segments: first segments for good, with output, from their real start states (which takes as long per
-// chunk as the two roles of the others), those behind them for their summaries.  Where all of them together leave CUs for it two
-// workgroups sweep a first segment, 64 V columns each.
+// chunk as the two roles of the others), those behind them for their summaries.  Where all of them together leave half of the CUs idle
+// two workgroups sweep a first segment, 64 V columns each, the second ones ahead in the grid.  That is for calls in which no sequence
+// is split (1000 + 1050 tokens of 16 value heads 65.5 -> 54.9 us).  Among split ones it changes less than 1 % on half a chip (59.7 / 60.8
+// without / with it, 2100 tokens of 8 value heads) and costs on a full one (16 384 tokens of 16 value heads, 256 workgroups: first
+// sweep 64.8 us without, 79.4 with the second ones behind in the grid; the call 171.6 without, 174.5 with them ahead).
 template <typename act_t>
 __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefillParams p) {
   static_assert(LEAN_LDS_BYTES <= FUSED_LDS_BYTES, "one array serves both sweeps");
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
-  const int ratio = p.HV / p.H;
-  const bool second = blockIdx.x >= p.split_grid;          // (behind all others in the grid: one for every sequence's first segment)
-  const int pair = second ? xcd_grouped_index(blockIdx.x - p.split_grid, ratio, p.N * p.HV)
-                          : xcd_grouped_index(blockIdx.x, ratio, p.seg.max_segments * p.HV);
+  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, (p.N + p.seg.max_segments) * p.HV);
   if (pair < 0) return;
-  const int item = pair / p.HV, hv = pair - item * p.HV, count = segment_count(p);
+  const int count = segment_count(p), hv = pair % p.HV;
   const SweptSegments s = swept_segments(count, true);
-  const int workgroups = __builtin_amdgcn_readlane(wave_inclusive_scan(s.swept + (count > 0)), 63) * p.HV;
-  const bool halves = workgroups <= CUS;
+  const int sequences = __popcll(__ballot(count > 0)), segments = __builtin_amdgcn_readlane(wave_inclusive_scan(s.swept), 63);
+  const bool halves = (sequences + segments) * p.HV <= CUS / 2;
+  const int item = pair / p.HV - (halves ? sequences : 0);
   SweptSegment segment = swept_segment(s, count, false, item);
-  if (second) {
-    const int n_count = __builtin_amdgcn_readlane(count, item);
-    segment = SweptSegment{halves && n_count > 0 ? item : -1, 0, n_count, p.seg.seq_seg_off[item]};
+  if (item < 0) {                                            // (second half of a first segment)
+    const int before = __popcll(__ballot(count > 0) & ((1ull << (threadIdx.x & 63)) - 1));
+    const int n = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(count > 0 && before == item + sequences)) - 1);
+    segment = SweptSegment{n, 0, __builtin_amdgcn_readlane(count, n), p.seg.seq_seg_off[n]};
   }
   if (segment.sequence < 0) return;
   if (segment.index > 0) lean_sweep<act_t>(p, lds_all, segment, hv);
-  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + second, segment);
+  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + (item < 0), segment);
   else fused_sweep<act_t, 2, true>(p, lds_all, hv, segment);
 }
 
@@ -1674,8 +1675,7 @@ static int gdn_prefill_run(
       },
       [&](unsigned grid) {
         if (p.pass == 1) {        // first sweep over segments
-          p.split_grid = xcd_grouped_grid(grid, (unsigned)(HV / H));
-          const unsigned g = p.split_grid + xcd_grouped_grid((unsigned)N * HV, (unsigned)(HV / H));
+          const unsigned g = xcd_grouped_grid(grid + (unsigned)N * HV, (unsigned)(HV / H));
           if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
           else hipLaunchKernelGGL(gdn_first_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
         } else {
