@@ -395,6 +395,13 @@ int pla_gdn_prefill_launch_raw(
 int pla_gdn_prefill_halved_sequences(const int32_t* raw_cu_seqlens, int N, int T, int H, int HV);
 
 /*
+ * Chunks (of 64 tokens) per segment of a GDN prefill call whose sequences are split, 0: none is.  *split_from (NULL: not
+ * wanted) receives the chunks from which on the longest of several sequences has the device split any (0: whatever they are).
+ * Host arithmetic only, for tests and for callers who log the plan.
+ */
+int pla_gdn_prefill_segment_chunks(int T, int N, int H, int HV, int* split_from);
+
+/*
  * pla_gdn_prefill_launch for callers that cannot allocate (code under hipGraph capture, tight serving
  * loops, harnesses that forbid hipMalloc): same arguments without the workspace pair, same results bit
  * for bit.  No counterpart in the reference.  The workspace is an array inside the library, one per GPU

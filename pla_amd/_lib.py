@@ -140,6 +140,8 @@ def load():
     lib.pla_last_error.argtypes = []
     lib.pla_gdn_prefill_workspace_bytes.restype = _c_i64
     lib.pla_gdn_prefill_workspace_bytes.argtypes = [_c_int, _c_int, _c_int, _c_int]
+    lib.pla_gdn_prefill_segment_chunks.restype = _c_int
+    lib.pla_gdn_prefill_segment_chunks.argtypes = [_c_int, _c_int, _c_int, _c_int, _c_p]
     lib.pla_gdn_prefill_halved_sequences.restype = _c_int
     lib.pla_gdn_prefill_halved_sequences.argtypes = [_c_p, _c_int, _c_int, _c_int, _c_int]
     lib.pla_kda_commit_launches.restype = _c_int

@@ -285,6 +285,12 @@ inline unsigned xcd_grouped_grid(unsigned total, unsigned group) {
   const unsigned groups = (total + group - 1) / group;
   return (groups + XCDS - 1) / XCDS * XCDS * group;
 }
+// Workgroups, a CU each, that the chip takes at once under this map: whole groups only on an XCD.
+constexpr int CUS = 256;
+inline int xcd_grouped_capacity(int group) {
+  const int cus = CUS / XCDS;
+  return group > cus ? CUS : XCDS * (cus / group) * group;
+}
 __device__ __forceinline__ int xcd_grouped_index(int hw_index, int group, int total) {
   const int xcd = hw_index % XCDS, t = hw_index / XCDS;
   const int member = t % group, g = (t / group) * XCDS + xcd;
@@ -609,8 +615,6 @@ static __global__ __launch_bounds__(256, 1) void segment_combine_kernel(SegmentT
     }
   }
 }
-
-constexpr int CUS = 256;
 
 // Zero the rows of a dense [T, heads, 128] 16-bit output that lie beyond the last sequence (workgroup `block` of `blocks`).
 __device__ __forceinline__ void zero_tail(uint16_t* o, const int32_t* cu_seqlens, int N, int T, int heads, int block, int blocks) {

@@ -1406,7 +1406,9 @@ static int mixed_sweep_from_offsets(const int32_t* raw_cu_seqlens, int N, int HV
 // chunks is priced in us from the call's longest sequence (L chunks; of several the host has the mean only, which random lengths
 // exceed by about half): 3.8 s for the two sweeps where the second one runs as halves ((segment, head) pairs on half of the CUs at
 // most), 5 s otherwise, 2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep,
-// which runs one segment less per sequence than there are (of N sequences it counts a third of that).  One sequence is split where
+// which runs one segment less per sequence than there are (of N sequences it counts a third of that).  The value heads of a q/k head
+// go to one XCD (xcd_grouped_index), so where 32 CUs are no multiple of them there are less than 256 pairs at once (16 384 tokens, 12
+// value heads of 4, 252 pairs 207 us, 240 SPLIT12; 30 000, 6 of 2, 252 pairs 206, 240 SPLIT6).  One sequence is split where
 // that is below 16 + 1.75 L, with 33 for the launches and 0.06 per thousand tokens and heads for the keys it stores.  us per call,
 // s = 4 / 5 / 6 / 8 / 10 / 12 / 16 / not split: one of 2048 tokens, 16 value heads 67.8 / 68.9 / - / - / - / - / - / 72.7; 32 heads 78.8 / 76.6 / 78.5 /
 // 78.5 / 85.9 / - / - / 76.1; 64 heads - / - / - / 90.1 / 97.3 / - / - / 76.6; 3000, 48 heads - / - / - / 107.5 / 112.0 / 117.6 / - / 113.5; 4096, 16
@@ -1416,16 +1418,17 @@ static int mixed_sweep_from_offsets(const int32_t* raw_cu_seqlens, int N, int HV
 // (segment_map) and the first sweep takes them all: us split / not, 1000 + 1050 tokens of 16 heads 62.5 / 53.5; three of 700, 12 heads
 // 68.5 / 48.0; four of 400 to 600, 16 heads 58.1 / 43.6.
 struct GdnSplit { int chunks, from; };      // SegmentTable::seg_chunks (0: not split), split_from
-static GdnSplit gdn_split(int T, int N, int HV) {
+static GdnSplit gdn_split(int T, int N, int H, int HV) {
   if ((int64_t)N * HV > 64 || T / CHUNK < 32) return GdnSplit{0, 0};
-  const int chunks = N == 1 ? (T - 1) / CHUNK + 1 : T / CHUNK, per_head = CUS / HV + (N == 1 ? 1 : N / 3);
+  const int ratio = std::max(1, HV / H), pairs = xcd_grouped_capacity(ratio), half_pairs = xcd_grouped_capacity(2 * ratio) / 2;
+  const int chunks = N == 1 ? (T - 1) / CHUNK + 1 : T / CHUNK, per_head = pairs / HV + (N == 1 ? 1 : N / 3);
   const double longest = N == 1 ? chunks : std::min<double>(chunks, 1.5 * chunks / N);
   const int least = std::max(3, (chunks + per_head - 1) / per_head);
   int best = 0;
   double best_price = 0.;
   for (int s = least; s <= least + 16; ++s) {
     const double swept = (N == 1 ? (chunks - 1) / s : std::max(0., (double)chunks / s - 0.5 * N)) * HV;
-    const double price = (swept <= CUS / 2 ? 3.8 : 5.) * s + 2. * longest / s;
+    const double price = (swept <= half_pairs ? 3.8 : 5.) * s + 2. * longest / s;
     if (best == 0 || price < best_price) best_price = price, best = s;
   }
   const double fixed = 17. + 6e-5 * T * HV, sweeps = best_price - 2. * longest / best;
@@ -1472,7 +1475,7 @@ static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chu
 // The plan of a call is one for all entry points, so where segments as short as that would outgrow the library's own array, calls
 // small enough for it with segments of 16 chunks (of three tiles each, which it has always taken) get the shortest that fit.
 static GdnWorkspaceLayout gdn_layout(int T, int N, int H, int HV, bool allow_stages = true) {
-  const GdnSplit split = gdn_split(T, N, HV);
+  const GdnSplit split = gdn_split(T, N, H, HV);
   const size_t tile = (size_t)HV * 16384 * 4, before = 3 * (size_t)(T / CHUNK / 16 + N + 1) * tile;
   GdnWorkspaceLayout L = gdn_layout_of(T, N, H, HV, split.chunks, allow_stages);
   if (split.chunks > 0 && gdn_layout_of(T, N, H, HV, 0, false).total + before <= PLA_GDN_PREFILL_STATIC_BYTES)
@@ -1716,7 +1719,7 @@ static int gdn_prefill_run(
         segments += std::max(0, nc - 1) / L.seg_chunks;
       }
     }
-    if (segments * HV <= 128) {
+    if (2 * segments * HV <= xcd_grouped_capacity(2 * (HV / H))) {
       const unsigned g = xcd_grouped_grid(2 * (unsigned)L.max_segments * HV, 2 * (unsigned)(HV / H));
       if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
       else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
@@ -1759,6 +1762,14 @@ extern "C" int pla_gdn_prefill_launch_raw(
                          cu_seqlens, N, T, scale, normalize_qk, h0, h0_indices, h0_slot_stride, ht, ht_indices,
                          ht_slot_stride, o, workspace, workspace_bytes, false, gcum_out, beta_out, H, HV, K, V, act_dtype,
                          stream, raw_cu_seqlens);
+}
+
+extern "C" int pla_gdn_prefill_segment_chunks(int T, int N, int H, int HV, int* split_from) {
+  if (split_from != nullptr) *split_from = 0;
+  if (T <= 0 || N <= 0 || H <= 0 || HV < H || HV % H != 0) return 0;
+  const GdnWorkspaceLayout L = gdn_layout(T, N, H, HV);
+  if (split_from != nullptr) *split_from = L.split_from;
+  return L.seg_chunks;
 }
 
 extern "C" int pla_gdn_prefill_halved_sequences(const int32_t* raw_cu_seqlens, int N, int T, int H, int HV) {

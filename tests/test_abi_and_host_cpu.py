@@ -90,6 +90,30 @@ def test_plan_of_the_halved_sequences_is_host_arithmetic():
     assert lib.pla_kda_prefill_halved_sequences(None, 5, 1000, 32) == 0
 
 
+def test_segments_of_one_sequence_fit_the_chip_at_once():
+    """Each sweep over the segments of a split GDN sequence runs one workgroup per (segment, value head), of one segment less
+    than there are, and those of the value heads of a q/k head on one of the eight XCDs (32 CUs each): no XCD gets more of
+    them than it has CUs."""
+    from pla_amd import _lib
+    lib = _lib.load()
+    planned = 0
+    for H, HV in ((1, 1), (1, 2), (2, 4), (1, 8), (2, 6), (4, 12), (1, 6), (2, 10), (4, 8), (4, 32), (8, 16), (8, 24), (16, 32),
+                  (16, 48), (16, 64)):
+        for T in (2048, 2049, 3000, 4159, 8192, 12000, 16384, 30000, 65536):
+            chunks = -(-T // 64)
+            s = lib.pla_gdn_prefill_segment_chunks(T, 1, H, HV, None)
+            if s == 0:
+                continue
+            planned += 1
+            groups = (-(-chunks // s) - 1) * H                   # of the HV / H pairs that share an XCD
+            assert -(-groups // 8) * (HV // H) <= 32, (T, H, HV, s)
+    assert planned > 100
+    line = ctypes.c_int(-1)
+    assert lib.pla_gdn_prefill_segment_chunks(2646, 8, 1, 2, ctypes.byref(line)) >= 3 and line.value > 0
+    assert lib.pla_gdn_prefill_segment_chunks(2646, 64, 1, 2, ctypes.byref(line)) == 0 and line.value == 0
+    assert lib.pla_gdn_prefill_segment_chunks(4096, 1, 4, 6, None) == 0 and lib.pla_gdn_prefill_segment_chunks(0, 1, 1, 1, None) == 0
+
+
 def test_native_entry_points_reject_bad_arguments_without_a_gpu():
     """Argument checks run before any launch, so they are testable on a CPU-only host."""
     from pla_amd import _lib
