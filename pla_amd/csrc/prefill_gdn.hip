@@ -1408,7 +1408,7 @@ static int mixed_sweep_from_offsets(const int32_t* raw_cu_seqlens, int N, int HV
 // most), 5 s otherwise, 2 a segment for the combine step.  Segments are at least as long as gives every CU one pair of a sweep,
 // which runs one segment less per sequence than there are (of N sequences it counts a third of that).  The value heads of a q/k head
 // go to one XCD (xcd_grouped_index), so where 32 CUs are no multiple of them there are less than 256 pairs at once (16 384 tokens, 12
-// value heads of 4, 252 pairs 207 us, 240 SPLIT12; 30 000, 6 of 2, 252 pairs 206, 240 SPLIT6).  One sequence is split where
+// value heads of 4, 252 pairs 207 us, 240 157; 30 000, 6 of 2, 252 pairs 206, 234 194).  One sequence is split where
 // that is below 16 + 1.75 L, with 33 for the launches and 0.06 per thousand tokens and heads for the keys it stores.  us per call,
 // s = 4 / 5 / 6 / 8 / 10 / 12 / 16 / not split: one of 2048 tokens, 16 value heads 67.8 / 68.9 / - / - / - / - / - / 72.7; 32 heads 78.8 / 76.6 / 78.5 /
 // 78.5 / 85.9 / - / - / 76.1; 64 heads - / - / - / 90.1 / 97.3 / - / - / 76.6; 3000, 48 heads - / - / - / 107.5 / 112.0 / 117.6 / - / 113.5; 4096, 16
