@@ -519,9 +519,13 @@ __device__ __forceinline__ void segment_map(const int32_t* seq_chunk_off, int N,
 // the next - in the place of its B.  A step S <- S M + B is a 16 x 128 x 128 product per workgroup on the FP32 MFMA
 // (v_mfma_f32_16x16x4_f32, exact products, FP32 accumulation): wavefront w owns columns 32 w .. 32 w + 31 as two
 // accumulator tiles that start from B; the A operand is the workgroup's 16 rows of S from LDS (lane (r, kb) takes
-// S[r][16 s + 4 kb + e] for step (s, e)), the B operand the matching row of M straight from memory (lane (c, kb):
-// M[16 s + 4 kb + e][column c], 64 contiguous bytes per group of 16 lanes).  M and B do not depend on the state, so those
-// of the next segment are requested before the products of this one: a step then waits for its products, not for memory.
+// S[r][16 s + 4 kb + e] for step (s, e)), the B operand the matching row of M straight from memory (lane (c, kb): columns 2 c
+// and 2 c + 1 of the wavefront's in the two tiles, eight bytes of row 16 s + 4 kb + e, 128 contiguous bytes per group of 16
+// lanes).  M and B do not depend on the state, so those of the next segment are requested during the products of this one, whose 64
+// MFMAs (32 cycles each) are what bounds a step: 1.28 us.  A wavefront issues in order, so requests ahead of the products
+// delay them, and the compiler waits by a count of those still out, of which the hardware counts 63.  17 858 + 20 774 tokens of 3 heads, 46
+// segments: 67.7 us with M requested where it is used, 70.9 with 72 requests of four bytes ahead of the products, left out at the
+// end (every other step then waited for all of them), 81 with 36 of eight bytes, 59.5 with one of those at every second MFMA.
 constexpr int COMBINE_SPLIT = 8;
 template <bool TABLE>
 static __global__ __launch_bounds__(256, 1) void segment_combine_kernel(SegmentTable t, const int32_t* cu_seqlens, int N, int T, int heads, int split_from) {
@@ -548,72 +552,65 @@ static __global__ __launch_bounds__(256, 1) void segment_combine_kernel(SegmentT
   if (end - first < 3) return;                 // no middle segment: the second one starts from the first one's B
   __shared__ __align__(16) float S[2][16][132];
   const int c = lane & 15, kb = lane >> 4;
-  const int col0 = 32 * wave + c;              // this lane's column of accumulator tile 0 (tile 1: + 16)
-  // place of accumulator element (tile cb, row v) inside a [128, 128] tile
-  auto at = [&](int cb, int v) { return (int64_t)(16 * part + 4 * kb + v) * 128 + col0 + 16 * cb; };
+  const int col0 = 32 * wave + 2 * c;          // this lane's column of accumulator tile 0 (tile 1: + 1)
+  // place of accumulator elements (tile 0 and 1, row v) inside a [128, 128] tile
+  auto at = [&](int v) { return (int64_t)(16 * part + 4 * kb + v) * 128 + col0; };
   auto tile_of = [&](int seg) { return ((int64_t)seg * heads + h) * 16384; };
-  struct Operands { float m[2][32]; f32x4_t b[2]; };
-  auto request = [&](int seg, Operands& x) {
-    const float* const Mt = t.M + tile_of(seg);
-    const float* const Bt = t.B + tile_of(seg);
+  struct Operands { float2 m[32], b[4]; };
+  auto request_b = [&](int seg, Operands& x) {
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x.b[cb][v] = Bt[at(cb, v)];
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) x.m[cb][4 * s8 + e] = Mt[(int64_t)(16 * s8 + 4 * kb + e) * 128 + col0 + 16 * cb];
+    for (int v = 0; v < 4; ++v) x.b[v] = *reinterpret_cast<const float2*>(t.B + tile_of(seg) + at(v));
+  };
+  const float* const M_lane = t.M + 4 * kb * 128 + col0;
+  auto request_m = [&](int seg, Operands& x, int i) {          // row 16 (i / 4) + 4 kb + i % 4
+    x.m[i] = *reinterpret_cast<const float2*>(M_lane + tile_of(seg) + (16 * (i >> 2) + (i & 3)) * 128);
   };
   f32x4_t acc[2];
-  {
-    const float* src = t.B + tile_of(first);
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[cb][v] = src[at(cb, v)];
+  for (int v = 0; v < 4; ++v) {
+    const float2 b = *reinterpret_cast<const float2*>(t.B + tile_of(first) + at(v));
+    acc[0][v] = b.x;
+    acc[1][v] = b.y;
   }
-  const int last = end - 1;                    // the last segment has no summary
+  const int last = end - 1;                    // the last segment has no summary (its tiles may be requested, and are not used)
   // S in LDS is double buffered by the parity of the step: one barrier a step
-  auto step = [&](int seg, const Operands& x, float (&Sp)[16][132]) {
+  auto step = [&](int seg, const Operands& x, Operands& next, float (&Sp)[16][132]) {
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        Sp[4 * kb + v][col0 + 16 * cb] = acc[cb][v];
-        acc[cb][v] = x.b[cb][v];
-      }
+    for (int v = 0; v < 4; ++v) *reinterpret_cast<float2*>(&Sp[4 * kb + v][col0]) = make_float2(acc[0][v], acc[1][v]);
     lds_barrier();
     float4 a[8];
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8) a[s8] = *reinterpret_cast<const float4*>(&Sp[c][16 * s8 + 4 * kb]);
 #pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8)
+    for (int v = 0; v < 4; ++v) {
+      acc[0][v] = x.b[v].x;
+      acc[1][v] = x.b[v].y;
+      asm volatile("" : "+v"(acc[0][v]), "+v"(acc[1][v]));      // (here: the compiler would wait for them in the step before)
+    }
+    request_b(seg + 1, next);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float av = e == 0 ? a[s8].x : e == 1 ? a[s8].y : e == 2 ? a[s8].z : a[s8].w;
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x.m[cb][4 * s8 + e], acc[cb], 0, 0, 0);
-      }
+    for (int i = 0; i < 32; ++i) {
+      const float4 q = a[i >> 2];
+      const float av = (i & 3) == 0 ? q.x : (i & 3) == 1 ? q.y : (i & 3) == 2 ? q.z : q.w;
+      request_m(seg + 1, next, i);
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x.m[i].x, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x.m[i].y, acc[1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     float* const dst = t.B + tile_of(seg);
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) dst[at(cb, v)] = acc[cb][v];
+    for (int v = 0; v < 4; ++v) *reinterpret_cast<float2*>(dst + at(v)) = make_float2(acc[0][v], acc[1][v]);
   };
   Operands even, odd;
-  request(first + 1, even);
-  for (int seg = first + 1; seg < last; seg += 2) {
-    if (seg + 1 < last) request(seg + 1, odd);
-    step(seg, even, S[0]);
-    if (seg + 1 < last) {
-      if (seg + 2 < last) request(seg + 2, even);
-      step(seg + 1, odd, S[1]);
-    }
+  request_b(first + 1, even);
+#pragma unroll
+  for (int i = 0; i < 32; ++i) request_m(first + 1, even, i);
+  int seg = first + 1;
+  for (; seg + 1 < last; seg += 2) {
+    step(seg, even, odd, S[0]);
+    step(seg + 1, odd, even, S[1]);
   }
+  if (seg < last) step(seg, even, odd, S[0]);
 }
 
 // Zero the rows of a dense [T, heads, 128] 16-bit output that lie beyond the last sequence (workgroup `block` of `blocks`).
