@@ -138,10 +138,7 @@ __global__ __launch_bounds__(64 * WAVES) void gdn_wsolve_kernel(const GdnPrefill
     const int extra = blockIdx.x - main_blocks;
     const int builders = p.seg.seg_chunks > 0 ? 1 : 0;
     if (extra < builders) {
-      chunk_map(p.cu_seqlens, p.N, p.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len);
-      __threadfence();
-      __syncthreads();
-      segment_map(p.seq_chunk_off, p.N, p.seg);
+      segment_map(p.cu_seqlens, p.N, p.seq_chunk_off, p.seg);
     } else {
       zero_tail(reinterpret_cast<uint16_t*>(p.o), p.cu_seqlens, p.N, p.T, p.HV, extra - builders, p.tail_blocks - builders);
     }
@@ -1349,38 +1346,37 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
 }
 
 // First sweep over segments: first segments for good, with output, from their real start states (which takes as long per
-// chunk as the two roles of the others), those behind them for their summaries.  Where all of them together leave half of the CUs idle
-// two workgroups sweep a first segment, 64 V columns each, the second ones ahead in the grid.  That is for calls in which no sequence
-// is split (1000 + 1050 tokens of 16 value heads 65.5 -> 54.9 us).  Among split ones it changes less than 1 % on half a chip (59.7 / 60.8
-// without / with it, 2100 tokens of 8 value heads) and costs on a full one (16 384 tokens of 16 value heads, 256 workgroups: first
-// sweep 64.8 us without, 79.4 with the second ones behind in the grid; the call 171.6 without, 174.5 with them ahead).
+// chunk as the two roles of the others), those behind them for their summaries.  Where no sequence turns out to be split two
+// workgroups sweep each, 64 V columns each (1000 + 1050 tokens of 16 value heads 65.5 -> 54.9 us), the second ones a multiple of eight
+// sequences behind the first ones in the grid: on the same XCD, whose L2 then has the tiles of both (six sequences of 414 to 446 tokens, 8 value
+// heads, 37.0 -> 34.9 us).  Among split sequences that changes less than 1 % on half a chip (2100 tokens of 8 value heads 59.7 / 60.8 without
+// / with it) and costs on a full one (16 384 tokens of 16 value heads, 256 workgroups: first sweep 64.8 / 79.4).
+__host__ __device__ __forceinline__ int round_up8(int n) { return (n + 7) & ~7; }
+__host__ __device__ __forceinline__ int first_sweep_items(int N, int max_segments) {
+  const int halves = round_up8(N) + N;
+  return max_segments > halves ? max_segments : halves;
+}
 template <typename act_t>
 __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefillParams p) {
   static_assert(LEAN_LDS_BYTES <= FUSED_LDS_BYTES, "one array serves both sweeps");
   __shared__ __align__(1024) unsigned char lds_all[FUSED_LDS_BYTES];
   // the value heads of a q/k head copy the same K rows: on one XCD they come from memory once
-  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, (p.N + p.seg.max_segments) * p.HV);
+  const int pair = xcd_grouped_index(blockIdx.x, p.HV / p.H, first_sweep_items(p.N, p.seg.max_segments) * p.HV);
   if (pair < 0) return;
-  const int count = segment_count(p), hv = pair % p.HV;
+  const int count = segment_count(p), item = pair / p.HV, hv = pair - item * p.HV;
   const SweptSegments s = swept_segments(count, true);
-  const int sequences = __popcll(__ballot(count > 0)), segments = __builtin_amdgcn_readlane(wave_inclusive_scan(s.swept), 63);
-  const bool halves = (sequences + segments) * p.HV <= CUS / 2;
-  const int item = pair / p.HV - (halves ? sequences : 0);
-  SweptSegment segment = swept_segment(s, count, false, item);
-  if (item < 0) {                                            // (second half of a first segment)
-    const int before = __popcll(__ballot(count > 0) & ((1ull << (threadIdx.x & 63)) - 1));
-    const int n = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(count > 0 && before == item + sequences)) - 1);
-    segment = SweptSegment{n, 0, __builtin_amdgcn_readlane(count, n), p.seg.seq_seg_off[n]};
-  }
+  const int sequences = __popcll(__ballot(count > 0)), second_halves = round_up8(sequences);
+  const bool halves = __ballot(count > 1) == 0, second = halves && item >= second_halves;
+  const SweptSegment segment = swept_segment(s, count, false, second ? item - second_halves : item);
   if (segment.sequence < 0) return;
   if (segment.index > 0) lean_sweep<act_t>(p, lds_all, segment, hv);
-  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + (item < 0), segment);
+  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + second, segment);
   else fused_sweep<act_t, 2, true>(p, lds_all, hv, segment);
 }
 
 struct GdnWorkspaceLayout {
   size_t seq_chunk_off, chunk_seq, chunk_tok, chunk_len, q_rows, k_rows, kn, kinv, gtile, W;
-  size_t seq_seg_off, seg_seq, seg_c0, seg_nc, segM, segB, identity;
+  size_t seq_seg_off, seg_c0, seg_nc, segM, segB, identity;
   size_t order, stage_begin, carry, total;
   int NC_max, seg_chunks, max_segments, split_from, stages;
 };
@@ -1455,7 +1451,6 @@ static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chu
   L.max_segments = seg_chunks == 0 ? 0 : N == 1 ? (T - 1) / CHUNK / seg_chunks + 1 : (T / CHUNK + N) / seg_chunks + N;
   if (L.seg_chunks > 0) {
     L.seq_seg_off = take((size_t)(N + 1) * 4);
-    L.seg_seq = take((size_t)L.max_segments * 4);
     L.seg_c0 = take((size_t)L.max_segments * 4);
     L.seg_nc = take((size_t)L.max_segments * 4);
     const size_t states = (size_t)L.max_segments * HV * 16384 * 4;
@@ -1607,7 +1602,6 @@ static int gdn_prefill_run(
   if (segmented) {
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
     p.seg.seq_seg_off = reinterpret_cast<int32_t*>(ws + L.seq_seg_off);
-    p.seg.seg_seq = reinterpret_cast<int32_t*>(ws + L.seg_seq);
     p.seg.seg_c0 = reinterpret_cast<int32_t*>(ws + L.seg_c0);
     p.seg.seg_nc = reinterpret_cast<int32_t*>(ws + L.seg_nc);
     p.seg.M = reinterpret_cast<float*>(ws + L.segM);
