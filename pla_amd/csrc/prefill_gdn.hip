@@ -1672,7 +1672,7 @@ static int gdn_prefill_run(
       },
       [&](unsigned grid) {
         if (p.pass == 1) {        // first sweep over segments
-          const unsigned g = xcd_grouped_grid(grid + (unsigned)N * HV, (unsigned)(HV / H));
+          const unsigned g = xcd_grouped_grid((unsigned)first_sweep_items(N, L.max_segments) * HV, (unsigned)(HV / H));
           if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
           else hipLaunchKernelGGL(gdn_first_sweep_kernel<bf16_t>, dim3(g), dim3(512), 0, s, p);
         } else {
