@@ -1594,10 +1594,12 @@ static int gdn_prefill_run(
   const bool v_halves = !segmented && (int64_t)N * HV <= 128;
   // Normalised K rows in memory take the scaling of the keys from the sweeps of every value head and cost the preparation a
   // tile per q/k head and chunk.  They pay where the chip is not full (128 chains at most: 3 short prompts 24.0 -> 22.6 us, one of
-  // 1100 tokens, 32 value heads 56.2 -> 51.0) and from three value heads a q/k head on (six ragged prompts, 48 of 16 heads 177 ->
+  // 1100 tokens, 32 value heads 56.2 -> 51.0), with one or three value heads a q/k head, of which the preparation shares no tile, from
+  // the second chunk of a sequence on (copied / formed: 16 of 64 tokens, 6 of 2 18.5 / 18.0, 2 of 60, 48 of 16 18.5 / 18.1, but 3 of 128, 6 of
+  // 2 19.1 / 19.3); on a full chip they pay from three value heads a q/k head on (six ragged prompts, 48 of 16 heads 177 ->
   // 171; eight of 512, 24 of 8 48.8 -> 47.3); of two the write shows (eight of 2048, 32 of 16 170 -> 184).  The sweeps over
   // segments read them anyway.
-  const bool kn = segmented || v_halves || HV >= 3 * H;
+  const bool kn = segmented || (v_halves ? HV / H % 2 == 0 || T > CHUNK * (int64_t)N : HV >= 3 * H);
   p.store_kn = kn;
   if (segmented) {
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
@@ -1688,8 +1690,8 @@ static int gdn_prefill_run(
             else hipLaunchKernelGGL((kn ? gdn_fused_sweep_mixed_kernel<bf16_t, true> : gdn_fused_sweep_mixed_kernel<bf16_t, false>), dim3(g), dim3(512), 0, s, p);
           } else if (v_halves) {
             const unsigned g = xcd_grouped_grid(2 * grid, 2 * (unsigned)(HV / H));
-            if (half_act) hipLaunchKernelGGL((gdn_fused_sweep_kernel<f16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
-            else hipLaunchKernelGGL((gdn_fused_sweep_kernel<bf16_t, 1, true>), dim3(g), dim3(512), 0, s, p);
+            if (half_act) hipLaunchKernelGGL((kn ? gdn_fused_sweep_kernel<f16_t, 1, true> : gdn_fused_sweep_kernel<f16_t, 1, false>), dim3(g), dim3(512), 0, s, p);
+            else hipLaunchKernelGGL((kn ? gdn_fused_sweep_kernel<bf16_t, 1, true> : gdn_fused_sweep_kernel<bf16_t, 1, false>), dim3(g), dim3(512), 0, s, p);
           } else {
             const unsigned g = xcd_grouped_grid(grid, (unsigned)(HV / H));
             if (half_act) hipLaunchKernelGGL((kn ? gdn_fused_sweep_kernel<f16_t, 2, true> : gdn_fused_sweep_kernel<f16_t, 2, false>), dim3(g), dim3(512), 0, s, p);

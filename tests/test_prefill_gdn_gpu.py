@@ -298,6 +298,28 @@ def test_gdn_prefill_keys_copied_or_formed_by_the_sweep(H, HV):
         assert torch.equal(r[2][0], o[0, lo:hi]) and torch.equal(w["initial_state"][int(idx[n])], pool[int(idx[n])]), n
 
 
+@pytest.mark.parametrize("H,HV", [(2, 6), (3, 3), (2, 4)])
+def test_gdn_prefill_keys_of_one_chunk_sequences(H, HV):
+    """At most 128 chains: with one or three value heads a q/k head the sweeps form the keys of calls of one chunk a sequence
+    and copy those of longer ones, with two they always copy them.  The same sequences with a longer one behind them keep
+    their bits; against the oracle."""
+    from pla_amd.workloads import gdn_prefill_packed
+    lengths = [64, 17, 1, 0, 300]
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=8, seed=40 + HV)
+    pool0 = w["initial_state"].clone()
+    _, _, o, _, final = _run_workload(w)
+    T, N = sum(lengths[:4]), 4
+    short = dict(w, packed_qkv=w["packed_qkv"][:T], raw_gate_a=w["raw_gate_a"][:T], raw_beta_b=w["raw_beta_b"][:T],
+                 cu_seqlens=w["cu_seqlens"][:N + 1], raw_cu_seqlens=w["raw_cu_seqlens"][:N + 1],
+                 initial_state_indices=w["initial_state_indices"][:N])
+    w["initial_state"].copy_(pool0)
+    _, _, o_short, _, final_short = _run_workload(short)
+    torch.cuda.synchronize()
+    assert torch.equal(o_short[0], o[0, :T]) and torch.equal(final_short, final[:N])
+    w["initial_state"].copy_(pool0)
+    _check(w, fast=True)
+
+
 @pytest.mark.parametrize("lengths,tail_pad,H,HV", [
     ([2048], 0, 1, 4), ([2049], 3, 2, 4),                              # segments of three chunks; a last one of one token
     ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2),                  # one, two, three and more segments a sequence
