@@ -292,8 +292,8 @@ int pla_kda_commit_launch(
     int token_capacity, int64_t block_row_stride, int64_t block_col_stride, int64_t block_size,
     int32_t* candidate, int32_t* plan, void* stream);
 
-/* The form pla_kda_commit_launch takes for a batch whose plan shares no memory with its inputs (host arithmetic): 1 for one
- * launch, 3 for plan, fold and conv windows as parts of their own (of which the latter two share a launch). */
+/* Whether pla_kda_commit_launch is one launch for a batch whose plan shares no memory with its inputs (host arithmetic): 1, or 3
+ * where the plan is a launch of its own.  (3 is no count: fold and conv windows, two launches once, share the second one.) */
 int pla_kda_commit_launches(int batch, int heads, int layers);
 
 /*

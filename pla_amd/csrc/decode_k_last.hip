@@ -1046,11 +1046,14 @@ extern "C" int pla_kda_fold_native_launch(
   return launch_fold(p, PLA_BF16, stream, layers);
 }
 
-// Up to this many state tiles the paged commit is one launch.  There a workgroup's plan costs a trip to memory or two beside
-// the trip for its tile and saves a launch; with more tiles than the chip holds workgroups every round pays for it.
-// us at one launch / at three, the conv windows apart from the fold (windows of 3-8 tokens; with a block table in brackets):
-//     8 tiles  6.8 / 9.1 (7.8 / 9.8)      240 tiles 11.6 / 13.9 (12.7 / 14.6)   480 tiles 24.9 / 23.4 (25.8 / 24.1)
-//    96 tiles 10.6 / 12.4 (11.6 / 13.0)   320 tiles 17.4 / 18.0 (18.4 / 18.5)   504 tiles 24.7 / 24.5 (26.7 / 25.0)
+// Up to this many state tiles the paged commit is one launch, beyond it two: the plan, then the fold with the conv windows.  In
+// one launch a workgroup's plan costs a trip to memory or two beside the trip for its tile; with more tiles than the chip
+// holds workgroups every round pays for it.  us at one launch / at two (windows of four tokens; of eight in brackets):
+//     8 tiles  5.4 / 6.1                 288 tiles 14.8 / 16.2                384 tiles 19.5 / 17.4 (20.3 / 19.2)
+//    96 tiles  8.8 / 9.1 (11.2 / 11.6)   320 tiles 15.1 / 15.4 (16.9 / 18.3)  480 tiles 20.8 / 20.7
+//   240 tiles 11.7 / 11.9 (15.6 / 15.5)  336 tiles 14.7 / 15.8                504 tiles 21.7 / 20.8 (25.6 / 26.5)
+// With a block table, of which the plan reads a row for every request, the two are even up to 288 tiles and two launches ahead from
+// 336 on (320 tiles 15.7 / 15.6, 336 12.3 / 11.3, 504 19.9 / 14.7; many of these requests commit nothing).
 constexpr int64_t COMMIT_ONE_LAUNCH_TILES = 320;
 
 extern "C" int pla_kda_commit_launches(int batch, int heads, int layers) {

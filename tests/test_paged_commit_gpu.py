@@ -1,5 +1,5 @@
-"""The paged commit in one launch against plan, fold and conv windows in three, bit for bit (the arithmetic of a tile is the
-same), on both sides of the line between them; and the plan of large batches, whose look-ups are spread over workgroups, against
+"""The paged commit, in one launch or with its plan ahead, against plan, fold and conv windows in three, bit for bit (the arithmetic
+of a tile is the same), on both sides of the line between them; and the plan of large batches, whose look-ups are spread over workgroups, against
 the oracle."""
 import pytest
 import torch
@@ -49,14 +49,15 @@ def _three_launches(ctx, sampled, source, offsets, mapping, table, computed, tok
 
 
 # one request; few tiles (8 rows per wavefront) and more (16 rows); more requests than threads of a workgroup; the largest
-# number of tiles of one launch, and one request more than that
+# number of tiles of one launch, and one request more than that; beyond it the conv windows stand behind the tiles of the fold, with 16
+# and with 32 rows per wavefront, in both layouts, with whole workgroups of channels and with a remainder
 @pytest.mark.parametrize("requests,heads,q,n_layers,layout,capacity", [
     (1, 1, 1, 1, "SD", 1), (5, 3, 4, 2, "DS", 9), (17, 6, 8, 2, "SD", 20), (260, 1, 2, 1, "DS", 300), (20, 8, 3, 2, "SD", 20),
-    (21, 8, 3, 2, "SD", 21)])
+    (21, 8, 3, 2, "SD", 21), (115, 3, 4, 1, "DS", 120), (64, 8, 3, 2, "SD", 64), (180, 3, 2, 1, "SD", 181), (70, 4, 8, 2, "DS", 70)])
 @pytest.mark.parametrize("mode", ["plain", "mapping", "align", "mapping 64 bits", "align 64 bits"])
 def test_commit_in_one_launch_equals_three(requests, heads, q, n_layers, layout, capacity, mode):
     from pla_amd import _lib
-    assert _lib.load().pla_kda_commit_launches(requests, heads, n_layers) == (3 if requests == 21 else 1)
+    assert _lib.load().pla_kda_commit_launches(requests, heads, n_layers) == (3 if requests * heads * n_layers > 320 else 1)
     mode, dtype = mode.split()[0], torch.int64 if "64" in mode else torch.int32
     ctx, layers, source, offsets, slots, gen = _context(requests, heads, q, n_layers, layout, capacity, 31 + requests)
     ri = lambda lo, hi, n: torch.randint(lo, hi, (n,), generator=gen)
