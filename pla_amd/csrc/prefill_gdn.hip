@@ -78,6 +78,7 @@ struct GdnPrefillParams {
   int H, HV, NC_max;
   int inline_tables;     // at most 64 whole sequences: kernels work the chunk tables out themselves (no table kernel)
   int tail_blocks;       // workgroups appended to the preparation grid that zero the output rows beyond the last sequence
+  int o_past_caches;     // the sweeps of 128 columns a workgroup store their outputs past the caches
   int store_kn;          // gdn_wsolve_kernel stores the normalised K rows (kn) for the sweeps to copy, else 1 / |k|
   // gdn_fused_sweep_mixed_kernel: the first `split_grid` workgroups sweep the chains of sequences seq_order[0 .. n_long)
   // as two halves, the others those of seq_order[n_long .. N) whole
@@ -1275,8 +1276,18 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
             w[2 * nb + 1] = pack2<act_t>(OT[nb][ni][2], OT[nb][ni][3]);
           }
           uint16_t* const at = dst + (int64_t)16 * ni * p.HV * 128;
-          if constexpr (NB == 2) __builtin_nontemporal_store(u32x4_t{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4_t*>(at));
-          else *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
+          if constexpr (NB == 2) {
+            const u32x4_t row = {w[0], w[1], w[2], w[3]};
+            if (p.o_past_caches) {
+              // (as assembly: the compiler makes one ordinary store of a non-temporal one here and that below.  s_nop: the two
+              // wait states before a vector instruction may write the data registers of a store this wide)
+              asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" :: "v"(at), "v"(row) : "memory");
+            } else {
+              *reinterpret_cast<u32x4_t*>(at) = row;
+            }
+          } else {
+            *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
+          }
         }
       }
       SB();
@@ -1373,6 +1384,13 @@ __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefil
   else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + second, segment);
   else fused_sweep<act_t, 2, true>(p, lds_all, hv, segment);
 }
+
+// Outputs of up to this size are left to the caches, from where the kernel behind the call reads them; larger ones are stored past
+// them.  us per call / of the call and an elementwise kernel that reads its output, past the caches against through them: 13 MB
+// (eight of 200 tokens, 32 value heads) 36.6 / 43.3, 37.5 / 43.0; 25 (six of 500) 47.5 / 59.3, 47.9 / 58.3; 33 (eight of 500) 52.7 / 66.9,
+// 52.3 / 65.4; 66 (eight of 1000) 85.7 / 114.6, 89.5 / 116.1; 98 (six of 1500), the call alone, 103.5, 111.1; 134 (eight of 2048) 174 /
+// 223, 174 / 220.
+constexpr int64_t OUTPUT_IN_CACHES = (int64_t)48 << 20;
 
 struct GdnWorkspaceLayout {
   size_t seq_chunk_off, chunk_seq, chunk_tok, chunk_len, q_rows, k_rows, kn, kinv, gtile, W;
@@ -1601,6 +1619,7 @@ static int gdn_prefill_run(
   // segments read them anyway.
   const bool kn = segmented || (v_halves ? HV / H % 2 == 0 || T > CHUNK * (int64_t)N : HV >= 3 * H);
   p.store_kn = kn;
+  p.o_past_caches = (int64_t)T * HV * 256 > OUTPUT_IN_CACHES;
   if (segmented) {
     // few, long sequences: sweep their segments concurrently (two sweeps and a combine step)
     p.seg.seq_seg_off = reinterpret_cast<int32_t*>(ws + L.seq_seg_off);

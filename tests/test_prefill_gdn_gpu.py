@@ -298,6 +298,30 @@ def test_gdn_prefill_keys_copied_or_formed_by_the_sweep(H, HV):
         assert torch.equal(r[2][0], o[0, lo:hi]) and torch.equal(w["initial_state"][int(idx[n])], pool[int(idx[n])]), n
 
 
+@pytest.mark.parametrize("H,HV", [(16, 32), (8, 24)])
+def test_gdn_prefill_outputs_on_both_sides_of_the_caches(H, HV):
+    """Outputs of more than 48 MiB are stored past the caches, smaller ones through them: seven sequences in one call on the far side
+    have the bits of the first five and the last two in calls of their own, on the near side, all of them of more than 128 chains
+    and with tail chunks."""
+    from pla_amd.workloads import gdn_prefill_packed
+    tokens = (48 << 20) // (256 * HV)
+    lengths = [tokens // 7 + d for d in (5, -60, 0, 33, 1, 64, 7)]
+    T, split = sum(lengths), 5
+    assert T * HV * 256 > 48 << 20 > sum(lengths[:split]) * HV * 256
+    w = gdn_prefill_packed(lengths + [0] * 4, H=H, HV=HV, pool_slots=12, seed=70 + HV)
+    pool0 = w["initial_state"].clone()
+    _, _, o, _, final = _run_workload(w)
+    cut = w["_meta"]["offsets"][split]
+    cu, idx = w["cu_seqlens"], w["initial_state_indices"]
+    for rows, offsets, of in ((slice(0, cut), cu[:split + 1], slice(0, split)), (slice(cut, T), cu[split:] - cut, slice(split, None))):
+        part = {k: w[k][rows].contiguous() for k in ("packed_qkv", "raw_gate_a", "raw_beta_b")}
+        w["initial_state"].copy_(pool0)
+        _, _, o_part, _, final_part = _run_workload(dict(w, **part, cu_seqlens=offsets.contiguous(), initial_state_indices=idx[of].contiguous(),
+                                                         raw_cu_seqlens=None))
+        torch.cuda.synchronize()
+        assert torch.equal(o_part[0], o[0, rows]) and torch.equal(final_part, final[of])
+
+
 @pytest.mark.parametrize("H,HV", [(2, 6), (3, 3), (2, 4)])
 def test_gdn_prefill_keys_of_one_chunk_sequences(H, HV):
     """At most 128 chains: with one or three value heads a q/k head the sweeps form the keys of calls of one chunk a sequence
