@@ -193,7 +193,7 @@ struct SegmentTable {
 struct StageTable {
   int32_t* order;         // [chunks] global chunk ids, all of stage 0 first, then stage 1, ...
   int32_t* stage_begin;   // [MAX_STAGES + 2]: offsets into `order` per stage, then (last word) the number of stages in effect
-  float* carry;           // [N, heads, V, K] (whole sequences; segments carry in their own tiles)
+  float* carry;           // [N, heads, V, K]
   int stages;             // 0: not staged
 };
 constexpr int MAX_STAGES = 2;
@@ -220,18 +220,15 @@ __host__ __device__ __forceinline__ int stage_cut(int nc, int s, int plan) {
   return (int)((int64_t)nc * (s < S ? s : S) / S);
 }
 
-// Single workgroup of 256 threads with (stages + 1) * n_items_max + 1 words of LDS at `pair_begin`.  The items are sequences (`counts` null: item i holds chunks
-// starts[i] .. starts[i + 1]) or segments (chunks starts[i] .. starts[i] + counts[i]); `n_items` is read
-// on the device.  (Stage, item) pairs count their chunks, a serial prefix places them, then every pair
+// Single workgroup of 256 threads with (stages + 1) * N + 1 words of LDS at `pair_begin`.  Sequence i holds chunks starts[i] ..
+// starts[i + 1].  (Stage, sequence) pairs count their chunks, a serial prefix places them, then every pair
 // writes its own chunk ids.
-__device__ __forceinline__ void stage_map(const int32_t* starts, const int32_t* counts, const int32_t* n_items_ptr,
-                                          int n_items_max, int NC_max, StageTable t, int32_t* pair_begin) {
-  // pair_begin: [stages * n_items_max + 1], then n_items_max chunk counts
+__device__ __forceinline__ void stage_map(const int32_t* starts, int N, int NC_max, StageTable t, int32_t* pair_begin) {
+  // pair_begin: [stages * N + 1], then N chunk counts
   const int S = t.stages;
-  const int n_items = n_items_ptr ? min(*n_items_ptr, n_items_max) : n_items_max;
-  int32_t* const count = pair_begin + S * n_items_max + 1;
+  int32_t* const count = pair_begin + S * N + 1;
   __shared__ int stages_in_effect;
-  for (int i = threadIdx.x; i < n_items; i += blockDim.x) count[i] = counts ? counts[i] : starts[i + 1] - starts[i];
+  for (int i = threadIdx.x; i < N; i += blockDim.x) count[i] = starts[i + 1] - starts[i];
   __syncthreads();
   auto count_of = [&](int i) { return count[i]; };
   if (threadIdx.x == 0) {
@@ -242,16 +239,16 @@ __device__ __forceinline__ void stage_map(const int32_t* starts, const int32_t* 
     // One stage then takes everything, the others stay empty.
     int64_t total = 0;
     int longest = 0;
-    for (int i = 0; i < n_items; ++i) { total += count_of(i); longest = max(longest, count_of(i)); }
-    const int E = stage_plan(total, n_items, longest, S);                  // the plan word: stages in effect and the cut
+    for (int i = 0; i < N; ++i) { total += count_of(i); longest = max(longest, count_of(i)); }
+    const int E = stage_plan(total, N, longest, S);                  // the plan word: stages in effect and the cut
     stages_in_effect = E;
     t.stage_begin[MAX_STAGES + 1] = E;
     int k = 0;
     for (int s = 0; s < S; ++s) {
       t.stage_begin[s] = k;
-      for (int i = 0; i < n_items; ++i) {
+      for (int i = 0; i < N; ++i) {
         const int nc = count_of(i);
-        pair_begin[s * n_items + i] = k;
+        pair_begin[s * N + i] = k;
         k += stage_cut(nc, s + 1, E) - stage_cut(nc, s, E);
       }
     }
@@ -259,8 +256,8 @@ __device__ __forceinline__ void stage_map(const int32_t* starts, const int32_t* 
   }
   __syncthreads();
   const int E = stages_in_effect;
-  for (int pair = threadIdx.x >> 3; pair < S * n_items; pair += blockDim.x >> 3) {      // eight threads per pair
-    const int s = pair / n_items, i = pair - s * n_items;
+  for (int pair = threadIdx.x >> 3; pair < S * N; pair += blockDim.x >> 3) {      // eight threads per pair
+    const int s = pair / N, i = pair - s * N;
     const int nc = count_of(i), lo = stage_cut(nc, s, E), hi = stage_cut(nc, s + 1, E);
     const int base = pair_begin[pair];
     for (int cc = lo + (threadIdx.x & 7); cc < hi; cc += 8)
@@ -608,40 +605,30 @@ __device__ __forceinline__ void zero_tail(uint16_t* o, const int32_t* cu_seqlens
     o[i] = 0;
 }
 
-// All tables of a call in one launch.  Workgroup 0 builds the chunk table, then (split calls) the segment
-// table, then (pipelined calls) the stage table; each step reads what the previous one wrote, through
-// memory, after a device-scope fence and a barrier of that one workgroup.  The other workgroups zero the
-// output rows beyond the last sequence.  Dynamic LDS: (stages + 1) * stage_items + 1 words.
+// The tables of a call of more than 64 sequences in one launch.  Workgroup 0 builds the chunk table, then (pipelined calls) the
+// stage table from it, through memory, after a device-scope fence and a barrier of that one workgroup.  The other workgroups zero the
+// output rows beyond the last sequence.  Dynamic LDS: (stages + 1) * N + 1 words.
 constexpr int TABLE_WORKGROUPS = 1 + 64;
 static __global__ __launch_bounds__(256) void prefill_tables_kernel(
     const int32_t* cu_seqlens, int N, int T, int NC_max, int32_t* seq_chunk_off, int32_t* chunk_seq,
-    int32_t* chunk_tok, int32_t* chunk_len, SegmentTable seg, StageTable stg, int stage_items, uint16_t* o, int heads) {
+    int32_t* chunk_tok, int32_t* chunk_len, StageTable stg, uint16_t* o, int heads) {
   extern __shared__ int32_t table_lds[];
   if (blockIdx.x > 0) {
     zero_tail(o, cu_seqlens, N, T, heads, blockIdx.x - 1, gridDim.x - 1);
     return;
   }
   chunk_map(cu_seqlens, N, NC_max, seq_chunk_off, chunk_seq, chunk_tok, chunk_len);
-  const bool segmented = seg.seg_chunks > 0;
-  if (segmented) {
-    __threadfence();
-    __syncthreads();
-    segment_map(cu_seqlens, N, seq_chunk_off, seg);
-  }
   if (stg.stages > 0) {
     __threadfence();
     __syncthreads();
-    stage_map(segmented ? seg.seg_c0 : seq_chunk_off, segmented ? seg.seg_nc : nullptr,
-              segmented ? seg.seq_seg_off + N : nullptr, stage_items, NC_max, stg, table_lds);
+    stage_map(seq_chunk_off, N, NC_max, stg, table_lds);
   }
 }
 inline void launch_tables(hipStream_t s, const int32_t* cu_seqlens, int N, int T, int NC_max, int32_t* seq_chunk_off,
-                          int32_t* chunk_seq, int32_t* chunk_tok, int32_t* chunk_len, const SegmentTable& seg,
-                          const StageTable& stg, int stage_items, void* o, int heads) {
-  const size_t lds = stg.stages > 0 ? (size_t)((stg.stages + 1) * stage_items + 1) * 4 : 0;
+                          int32_t* chunk_seq, int32_t* chunk_tok, int32_t* chunk_len, const StageTable& stg, void* o, int heads) {
+  const size_t lds = stg.stages > 0 ? (size_t)((stg.stages + 1) * N + 1) * 4 : 0;
   hipLaunchKernelGGL(prefill_tables_kernel, dim3(TABLE_WORKGROUPS), dim3(256), lds, s, cu_seqlens, N, T, NC_max,
-                     seq_chunk_off, chunk_seq, chunk_tok, chunk_len, seg, stg, stage_items,
-                     reinterpret_cast<uint16_t*>(o), heads);
+                     seq_chunk_off, chunk_seq, chunk_tok, chunk_len, stg, reinterpret_cast<uint16_t*>(o), heads);
 }
 
 inline size_t align_up256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -771,25 +758,21 @@ inline int mixed_sweep_plan(const int* r, int N, int HV, unsigned char* order, d
 // fills again), and the preparation only hides under a sweep on CUs that chains which ended early have left.
 // (Segmented calls already keep every CU busy with sweeps - staging them was measured for GDN: 0.57 -> 0.66 ms for
 // one sequence of 16 384 tokens -; the KDA path has no stages: its sweeps form their operands themselves.)
-inline int pick_stages(int T, int N, int heads, int seg_chunks) {
-  if (seg_chunks > 0) return 0;
+inline int pick_stages(int T, int N, int heads) {
   // (the stage map keeps (stages + 1) counters per sequence in LDS: at most 2048 sequences)
   return ((int64_t)N * heads >= 128 && T / CHUNK >= 16 * N && N <= 2048) ? MAX_STAGES : 0;
 }
 
 // Launch order of a prefill call, shared by both paths.  `prepare(stream)` launches the per-chunk
-// kernels of stage *stage_field, `sweep(grid)` the sequential kernel for (*pass_field, *stage_field).
+// kernels of stage *stage_field, `sweep()` the sequential kernel of that stage.
 // Stage 0 is prepared on the caller's stream, alone; the side stream (a SideStreamLease the caller holds for the
 // time of the call) prepares the other stages underneath the sweeps and is joined before the last sweep starts.
 template <typename Prepare, typename Sweep>
-inline bool launch_pipeline(hipStream_t s, int stages, SideStream* side, bool segmented, unsigned grid_whole,
-                            unsigned grid_segments, int* pass_field, int* stage_field, Prepare prepare, Sweep sweep) {
-  *pass_field = segmented ? 1 : 0;
-  const unsigned grid = segmented ? grid_segments : grid_whole;
+inline bool launch_pipeline(hipStream_t s, int stages, SideStream* side, int* stage_field, Prepare prepare, Sweep sweep) {
   if (stages == 0) {
     *stage_field = 0;
     prepare(s);
-    sweep(grid);
+    sweep();
     return true;
   }
   if (side == nullptr) return false;             // (callers stage a call only with a side stream in hand)
@@ -807,7 +790,7 @@ inline bool launch_pipeline(hipStream_t s, int stages, SideStream* side, bool se
   for (int st = 0; st < stages; ++st) {
     *stage_field = st;
     if (st > 0) ok = ok && hipStreamWaitEvent(s, side->ready[st], 0) == hipSuccess;
-    sweep(grid);
+    sweep();
   }
   return ok;
 }

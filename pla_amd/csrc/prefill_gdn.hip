@@ -1476,11 +1476,11 @@ static GdnWorkspaceLayout gdn_layout_of(int T, int N, int H, int HV, int seg_chu
     L.identity = take(16384 * 4);
   }
   // pipeline the preparation with the sweeps in stages where that pays
-  L.stages = allow_stages ? pick_stages(T, N, HV, L.seg_chunks) : 0;
+  L.stages = allow_stages ? pick_stages(T, N, HV) : 0;
   if (L.stages > 0) {
     L.order = take((size_t)L.NC_max * 4);
     L.stage_begin = take((size_t)(MAX_STAGES + 2) * 4);
-    L.carry = L.seg_chunks > 0 ? 0 : take((size_t)N * HV * 16384 * 4);
+    L.carry = take((size_t)N * HV * 16384 * 4);
   }
   L.total = off;
   return L;
@@ -1653,7 +1653,7 @@ static int gdn_prefill_run(
   if (stages > 0) {
     p.stg.order = reinterpret_cast<int32_t*>(ws + L.order);
     p.stg.stage_begin = reinterpret_cast<int32_t*>(ws + L.stage_begin);
-    p.stg.carry = segmented ? nullptr : reinterpret_cast<float*>(ws + L.carry);
+    p.stg.carry = reinterpret_cast<float*>(ws + L.carry);
     p.stg.stages = stages;
   }
   // Ragged whole sequences whose offsets the host holds: the last (or only) sweep runs the chains of the longest
@@ -1672,10 +1672,10 @@ static int gdn_prefill_run(
   // preparation does, and one workgroup appended to it writes the chunk and segment tables for the sweeps.
   p.inline_tables = N <= INLINE_TABLE_SEQUENCES;
   if (!p.inline_tables)
-    launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.seg, p.stg,
-                  segmented ? L.max_segments : N, o, HV);
+    launch_tables(s, cu_seqlens, N, T, L.NC_max, p.seq_chunk_off, p.chunk_seq, p.chunk_tok, p.chunk_len, p.stg, o, HV);
+  p.pass = segmented ? 1 : 0;
   const bool ok = launch_pipeline(
-      s, stages, lease.get(), segmented, (unsigned)N * HV, (unsigned)L.max_segments * HV, &p.pass, &p.stage,
+      s, stages, lease.get(), &p.stage,
       [&](hipStream_t ps) {
         const int ratio = HV / H;       // value heads per q/k head: as many wavefronts of a workgroup share K and Q
         const int waves = ratio % 4 == 0 ? 4 : ratio % 2 == 0 ? 2 : 1;
@@ -1691,7 +1691,8 @@ static int gdn_prefill_run(
           else hipLaunchKernelGGL((gdn_wsolve_kernel<bf16_t, 1>), grid, block, 0, ps, p);
         }
       },
-      [&](unsigned grid) {
+      [&]() {
+        const unsigned grid = (unsigned)N * HV;
         if (p.pass == 1) {        // first sweep over segments
           const unsigned g = xcd_grouped_grid((unsigned)first_sweep_items(N, L.max_segments) * HV, (unsigned)(HV / H));
           if (half_act) hipLaunchKernelGGL(gdn_first_sweep_kernel<f16_t>, dim3(g), dim3(512), 0, s, p);
