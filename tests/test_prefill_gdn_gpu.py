@@ -258,10 +258,10 @@ def test_config3_gdn_prefill_32k_varlen(seed, tokens):
 @pytest.mark.parametrize("lengths,tail_pad,H,HV", [([2500, 0, 1111, 40], 5, 1, 2), ([4096], 0, 2, 2), ([1030, 2049], 0, 1, 4),
                                                     ([16384], 0, 16, 32)])
 def test_gdn_prefill_split_sequences_match_oracle(lengths, tail_pad, H, HV):
-    """Calls with few (sequence, head) chains and long sequences are split into 16-chunk segments that
-    are swept concurrently (zero-state and identity sweeps, a combine step, a second sweep): ragged
-    lengths, an empty sequence, a sequence shorter than one segment, indexed pool, against the oracle.  The last case is
-    the reference report's single 16 384-token sequence of 32 value heads (8 segments of 32 chunks per head)."""
+    """Calls with few (sequence, head) chains and long sequences are split into segments that are swept concurrently (first
+    sweep, a combine step, a second sweep): ragged lengths, an empty sequence, a sequence shorter than one segment, indexed
+    pool, against the oracle.  The last case is the reference report's single 16 384-token sequence of 32 value heads (nine
+    segments of 29 chunks per head)."""
     from pla_amd import _lib
     from pla_amd.workloads import gdn_prefill_packed
     T, N = sum(lengths) + tail_pad, len(lengths)
@@ -344,18 +344,59 @@ def test_gdn_prefill_keys_of_one_chunk_sequences(H, HV):
     _check(w, fast=True)
 
 
-@pytest.mark.parametrize("lengths,tail_pad,H,HV", [
-    ([2048], 0, 1, 4), ([2049], 3, 2, 4),                              # segments of three chunks; a last one of one token
-    ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2),                  # one, two, three and more segments a sequence
-    ([3000, 5], 0, 8, 32), ([4159], 0, 16, 64),                        # second sweep over whole pairs; few, long segments
-    ([700, 760, 650], 2, 4, 12), ([2000, 1, 129], 0, 12, 12)])         # none split by the device; one on the line
-def test_gdn_prefill_segments_at_their_edges(lengths, tail_pad, H, HV):
+def _segments(lengths, tail_pad, H, HV):
+    """Segments per sequence as the call plans them (0 chunks a segment: never split; the device splits from a longest sequence on)."""
+    import ctypes
+    from pla_amd import _lib
+    line = ctypes.c_int()
+    chunks = _lib.load().pla_gdn_prefill_segment_chunks(sum(lengths) + tail_pad, len(lengths), H, HV, ctypes.byref(line))
+    assert chunks > 0
+    of = [-(-n // 64) for n in lengths]
+    return [-(-c // chunks) if max(of) >= line.value else min(c, 1) for c in of]
+
+
+@pytest.mark.parametrize("lengths,tail_pad,H,HV,segments", [
+    ([2048], 0, 1, 4, [8]), ([2049], 3, 2, 4, [9]),                    # segments of four chunks; a last one of one token
+    ([191, 192, 193, 0, 1, 384, 385, 2600], 0, 1, 2, [1, 1, 2, 0, 1, 2, 3, 14]),      # of three: ends short of one's, at it, beyond it
+    ([2600, 385, 193, 0, 577, 1], 0, 2, 6, [14, 3, 2, 0, 4, 1]),       # the longest first, three heads on an XCD
+    ([3000, 5], 0, 8, 32, [8, 1]), ([4159], 0, 16, 64, [5]),           # of six; few, long ones
+    ([700, 760, 650], 2, 4, 12, [1, 1, 1]),                            # none split by the device
+    ([191, 192, 193, 0, 1, 384, 385, 1300], 0, 1, 2, [1, 1, 1, 0, 1, 1, 1, 1])])
+def test_gdn_prefill_segments_at_their_edges(lengths, tail_pad, H, HV, segments):
     """A first segment of a split sequence is swept once, with output; the combine step only concerns the segments between
     the first and the last: sequences of one, of two and of many segments, ends one token beyond a segment's and one short of
     it.  Against the oracle, at the bounds of the whole file."""
     from pla_amd.workloads import gdn_prefill_packed
+    assert _segments(lengths, tail_pad, H, HV) == segments
     w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 3, seed=50 + sum(lengths), tail_pad=tail_pad)
     _check(w, fast=True)
+
+
+@pytest.mark.parametrize("lengths,split", [([1664, 100, 364], False), ([1665, 100, 364], True), ([1664, 1664, 1], False),
+                                           ([1665, 1664, 1], True)])
+def test_gdn_prefill_split_by_the_longest_sequence(lengths, split):
+    """Several sequences are split where the longest reaches a number of chunks that the plan names: calls one chunk below it and
+    at it, against the oracle.  A call has the bits of one of more than 64 chains, which is never split, exactly where nothing is
+    split (gates so weak that the state outlives a segment: sums in another order show)."""
+    from pla_amd.workloads import gdn_prefill_packed
+    H, HV = 1, 2
+    assert (max(_segments(lengths, 0, H, HV)) > 1) == split
+    w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=len(lengths) + 3, seed=sum(lengths))
+    w["A_log"] = torch.full_like(w["A_log"], -5.0)
+    pool0 = w["initial_state"].clone()
+    _check(w, fast=True)
+    w["initial_state"].copy_(pool0)
+    _, _, o, _, final = _run_workload(w)
+    copies = 64 // (HV * len(lengths)) + 1
+    T, packed = sum(lengths), w["packed_qkv"]
+    q, k, v = packed[:, :128 * H], packed[:, 128 * H:256 * H], packed[:, 256 * H:]
+    wide = dict(w, packed_qkv=torch.cat([q.repeat(1, copies), k.repeat(1, copies), v.repeat(1, copies)], 1), num_qk_heads=H * copies,
+                num_v_heads=HV * copies, raw_gate_a=w["raw_gate_a"].repeat(1, copies), raw_beta_b=w["raw_beta_b"].repeat(1, copies),
+                A_log=w["A_log"].repeat(copies), dt_bias=w["dt_bias"].repeat(copies), initial_state=pool0.repeat(1, copies, 1, 1))
+    _, _, o_wide, _, final_wide = _run_workload(wide)
+    torch.cuda.synchronize()
+    same = torch.equal(o_wide[0, :, :HV], o[0]) and torch.equal(final_wide[:, :HV], final)
+    assert same == (not split)
 
 
 def test_gdn_prefill_staged_pipeline_matches_oracle_and_unstaged_bits():
