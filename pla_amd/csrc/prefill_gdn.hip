@@ -725,8 +725,8 @@ constexpr int FUSED_OFF_K = FUSED_OFF_Q + 2 * TILE128_HALVES * 2, FUSED_OFF_V = 
 constexpr int FUSED_LDS_BYTES = FUSED_OFF_V + 2 * TILE128_HALVES * 2;
 
 // The sweep of one workgroup.  `wide`: 2 / NB x the chain's logical index (sequence x HV + value head, or that of `segment` among
-// those of a sweep over segments) plus, for NB = 1, the half of the V columns it takes.
-template <typename act_t, int NB, bool KN>
+// those of a sweep over segments) plus, for NB = 1, the half of the V columns it takes.  PAST: outputs are stored past the caches.
+template <typename act_t, int NB, bool KN, bool PAST>
 __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int wide,
                                             const SweptSegment& segment = SweptSegment{-1, 0, 0, 0}) {
   constexpr int CW = 4, AUX = 4;
@@ -738,7 +738,8 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   // the chunks of this workgroup's sequence: from the tables, or worked out here (every wavefront for itself)
   int3 inline_chunks{-1, 0, 0};
   int seq_first_chunk = 0, seq_first_token = 0, seq_end_token = 0;
-  const bool inline_tables = p.inline_tables && p.pass == 0;         // segments are looked up in the segment table
+  const bool whole = !KN || p.pass == 0;                             // (sweeps over segments copy the keys)
+  const bool inline_tables = p.inline_tables && whole;               // segments are looked up in the segment table
   if (inline_tables) {
     const InlineSequences seqs = inline_sequences(p.cu_seqlens, p.N, p.stg.stages, lane);
     const int n0 = __builtin_amdgcn_readfirstlane(block / p.HV);
@@ -747,9 +748,9 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
     seq_end_token = seq_first_token + __builtin_amdgcn_readlane(seqs.len, n0);
     inline_chunks = int3{seq_first_chunk, min(seq_first_chunk + __builtin_amdgcn_readlane(seqs.nc, n0), p.NC_max), seqs.E};
   }
-  const SweepRole role = p.pass == 0 ? sequence_role(block, p.HV, p.seq_chunk_off, p.stg, p.stage, p.states, inline_chunks)
-                                     : segment_role(p.pass == 1 ? SegmentSweep::FIRST_OUT : SegmentSweep::LATER, segment, block % p.HV,
-                                                    p.HV, p.seg, p.states);
+  const SweepRole role = whole ? sequence_role(block, p.HV, p.seq_chunk_off, p.stg, p.stage, p.states, inline_chunks)
+                               : segment_role(p.pass == 1 ? SegmentSweep::FIRST_OUT : SegmentSweep::LATER, segment, block % p.HV,
+                                              p.HV, p.seg, p.states);
   if (!role.active) return;
   const int n = role.n, hv = role.head, c_begin = role.c_begin, c_end = role.c_end;
   const int h = hv / (p.HV / p.H);
@@ -1278,13 +1279,8 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
           uint16_t* const at = dst + (int64_t)16 * ni * p.HV * 128;
           if constexpr (NB == 2) {
             const u32x4_t row = {w[0], w[1], w[2], w[3]};
-            if (p.o_past_caches) {
-              // (as assembly: the compiler makes one ordinary store of a non-temporal one here and that below.  s_nop: the two
-              // wait states before a vector instruction may write the data registers of a store this wide)
-              asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" :: "v"(at), "v"(row) : "memory");
-            } else {
-              *reinterpret_cast<u32x4_t*>(at) = row;
-            }
+            if constexpr (PAST) __builtin_nontemporal_store(row, reinterpret_cast<u32x4_t*>(at));
+            else *reinterpret_cast<u32x4_t*>(at) = row;
           } else {
             *reinterpret_cast<uint2*>(at) = make_uint2(w[0], w[1]);
           }
@@ -1322,6 +1318,7 @@ __device__ __forceinline__ int segment_count(const GdnPrefillParams& p) {
 
 // One workgroup per (sequence, value head), or per (segment, value head) in the second sweep over segments (NB = 2);
 // NB = 1: two per chain, 64 V columns each (the columns of V are independent: same bits).
+// (The sweep is compiled for both kinds of output store: with a branch at each store eight ragged prompts took 404.2 us, now 402.7.)
 template <typename act_t, int NB, bool KN>
 __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_kernel(const GdnPrefillParams p) {
   constexpr int HALVES = 2 / NB;
@@ -1333,7 +1330,8 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_kernel(const GdnPrefil
     const int count = segment_count(p);
     segment = swept_segment(swept_segments(count, false), count, true, wide / HALVES / p.HV);
   }
-  fused_sweep<act_t, NB, KN>(p, lds_all, wide, segment);
+  if (NB == 2 && p.o_past_caches) fused_sweep<act_t, NB, KN, NB == 2>(p, lds_all, wide, segment);
+  else fused_sweep<act_t, NB, KN, false>(p, lds_all, wide, segment);
 }
 
 // Whole sequences of unequal length, swept in one launch whose longest chains decide how long it lasts while the CUs
@@ -1347,12 +1345,13 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
     const int wide = xcd_grouped_index(blockIdx.x, 2 * ratio, 2 * p.n_long * p.HV);
     if (wide < 0) return;
     const int chain = wide >> 1, k = chain / p.HV;
-    fused_sweep<act_t, 1, KN>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
+    fused_sweep<act_t, 1, KN, false>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
   } else {
     const int chain = xcd_grouped_index(blockIdx.x - p.split_grid, ratio, (p.N - p.n_long) * p.HV);
     if (chain < 0) return;
-    const int k = chain / p.HV;
-    fused_sweep<act_t, 2, KN>(p, lds_all, p.seq_order[p.n_long + k] * p.HV + chain - k * p.HV);
+    const int k = chain / p.HV, wide = p.seq_order[p.n_long + k] * p.HV + chain - k * p.HV;
+    if (p.o_past_caches) fused_sweep<act_t, 2, KN, true>(p, lds_all, wide);
+    else fused_sweep<act_t, 2, KN, false>(p, lds_all, wide);
   }
 }
 
@@ -1381,8 +1380,9 @@ __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefil
   const SweptSegment segment = swept_segment(s, count, false, second ? item - second_halves : item);
   if (segment.sequence < 0) return;
   if (segment.index > 0) lean_sweep<act_t>(p, lds_all, segment, hv);
-  else if (halves) fused_sweep<act_t, 1, true>(p, lds_all, 2 * hv + second, segment);
-  else fused_sweep<act_t, 2, true>(p, lds_all, hv, segment);
+  else if (halves) fused_sweep<act_t, 1, true, false>(p, lds_all, 2 * hv + second, segment);
+  else if (p.o_past_caches) fused_sweep<act_t, 2, true, true>(p, lds_all, hv, segment);
+  else fused_sweep<act_t, 2, true, false>(p, lds_all, hv, segment);
 }
 
 // Outputs of up to this size are left to the caches, from where the kernel behind the call reads them; larger ones are stored past
