@@ -541,9 +541,11 @@ __device__ __forceinline__ Chain kda_chain(const KdaPrefillParams& p, int index,
   return c;
 }
 
-// The final state of an empty sequence, which no chain reaches: the one it starts from (or zero), by the workgroups that sweep
-// (sequence, head) `index`, or that segment and head, last.  (Copied ahead of the launch, for every sequence, it is a launch and up to 7 us: 18
-// sequences of 12 heads, 28 MB.)
+// The final state of an empty sequence, which no chain reaches: the one it starts from (or zero), by the workgroups of
+// (sequence, head) `index`, or of that segment and head.  (Copied ahead of the launch, for every sequence, it is a launch and up to 7 us: 18
+// sequences of 12 heads, 28 MB.)  In the kernel of ragged sequences it stands BEHIND the sweep: ahead of it the two bodies came out
+// slower (21 short sequences of 48 heads 108.7 us without it, 109.5 ahead, 106.5 behind; 18 of 12 heads 57.8 / 58.6 / 57.1); in the others
+// ahead (364 + 124 tokens of 16 heads 30.0 / 30.4 / 30.7, 65 536 of 32 heads 1573 / 1574 / 1582).
 template <int NB>
 __device__ __forceinline__ void kda_empty_state(const KdaPrefillParams& p, int index, int half) {
   const int n = index / p.H, head = index - n * p.H;
@@ -556,15 +558,18 @@ __device__ __forceinline__ void kda_empty_state(const KdaPrefillParams& p, int i
 }
 
 constexpr int FEEDERS = 4;                         // producing or copying wavefronts of a workgroup
-template <int NB, bool PREPARED>
+template <int NB, bool PREPARED, bool BEHIND>
 __device__ __forceinline__ void kda_sweep(const KdaPrefillParams& p, KdaLds<true>& lds, int index, int half) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const Chain chain = kda_chain(p, index, lane);
-  if (p.empty_states && (p.pass == 2 || chain.tokens == 0)) kda_empty_state<NB>(p, index, half);
-  if (chain.tokens == 0) return;
-  if (wave < 4) kda_compute<NB, true>(p, lds, chain, lane, 64 * half + 16 * NB * wave);
-  else if (PREPARED) kda_copy<true, FEEDERS>(p, lds, chain, lane, wave - 4, 4);
-  else kda_produce<true, FEEDERS>(p, lds, chain, lane, wave - 4, 4);
+  if (!BEHIND && p.empty_states && (p.pass == 2 || chain.tokens == 0)) kda_empty_state<NB>(p, index, half);
+  if (chain.tokens > 0) {
+    if (wave < 4) kda_compute<NB, true>(p, lds, chain, lane, 64 * half + 16 * NB * wave);
+    else if (PREPARED) kda_copy<true, FEEDERS>(p, lds, chain, lane, wave - 4, 4);
+    else kda_produce<true, FEEDERS>(p, lds, chain, lane, wave - 4, 4);
+    if (!BEHIND || p.pass == 0) return;
+  }
+  if (BEHIND && p.empty_states) kda_empty_state<NB>(p, index, half);
 }
 
 // The rows of o beyond the last sequence, dealt to all workgroups of a launch.
@@ -582,7 +587,7 @@ __global__ __launch_bounds__(64 * (4 + FEEDERS), 1) void kda_sweep_kernel(const 
   const int chains = (p.pass == 2 ? p.seg.max_segments : p.N) * p.H;
   const int wide = NB == 2 ? (int)blockIdx.x : xcd_grouped_index(blockIdx.x, 2, 2 * chains);
   if (wide < 0) return;
-  kda_sweep<NB, PREPARED>(p, lds, NB == 2 ? wide : wide >> 1, NB == 2 ? 0 : wide & 1);
+  kda_sweep<NB, PREPARED, false>(p, lds, NB == 2 ? wide : wide >> 1, NB == 2 ? 0 : wide & 1);
 }
 
 // Ragged whole sequences: the chains of the longest sequences as two halves (first in the grid: workgroups are
@@ -595,12 +600,12 @@ __global__ __launch_bounds__(64 * (4 + FEEDERS), 1) void kda_sweep_mixed_kernel(
     const int wide = xcd_grouped_index(blockIdx.x, 2, 2 * p.n_long * p.H);
     if (wide < 0) return;
     const int chain = wide >> 1, k = chain / p.H;
-    kda_sweep<1, false>(p, lds, p.seq_order[k] * p.H + chain - k * p.H, wide & 1);
+    kda_sweep<1, false, true>(p, lds, p.seq_order[k] * p.H + chain - k * p.H, wide & 1);
   } else {
     const int chain = blockIdx.x - p.split_grid;
     if (chain >= (p.N - p.n_long) * p.H) return;
     const int k = chain / p.H;
-    kda_sweep<2, false>(p, lds, p.seq_order[p.n_long + k] * p.H + chain - k * p.H, 0);
+    kda_sweep<2, false, true>(p, lds, p.seq_order[p.n_long + k] * p.H + chain - k * p.H, 0);
   }
 }
 
