@@ -164,7 +164,7 @@ __device__ __forceinline__ void chunk_map(const int32_t* cu_seqlens, int N, int 
 // B is the state the segment produces from a zero state and M (K x K) is what it produces from the
 // identity with all values v = 0 (rows of the k-last state transform independently).  So:
 //   pass 1   A first segment runs from the caller's state, with output: it is done with, and the state it ends in is
-//            its B (or, where it is the whole sequence, the final state); every segment between the first and the last
+//            its B (or, where it is the whole sequence, the final state; KDA leaves such a one to pass 2); every segment between the first and the last
 //            of its sequence runs twice without output, from zero (-> B) and from the identity with v = 0 (-> M); the
 //            last segment does not run: nothing needs its summary
 //   combine  per (sequence, head): the state each middle segment ends in, S <- S M + B in FP32, in the place of its B
@@ -343,7 +343,7 @@ __device__ __forceinline__ SweepRole sequence_role(int block, int heads, const i
 // sequences: lane n holds sequence n, prefix sums run over the lanes.  A kernel that does this at its start needs no
 // table kernel before it (one launch and its gap less on the critical path of a call) and no dependent trips to
 // memory for its tile: one load of cu_seqlens per lane.  The results equal chunk_map / stage_map / staged_chunk /
-// select_sweep(pass 0) for the same offsets, including the rule that keeps a single stage for chains of nearly equal
+// sequence_role for the same offsets, including the rule that keeps a single stage for chains of nearly equal
 // length.  All 64 lanes of the wavefront must call these functions together.
 constexpr int INLINE_TABLE_SEQUENCES = 64;
 // Inclusive scan over the 64 lanes by DPP: six moves in the vector pipe instead of six dependent LDS permutes, which

@@ -20,10 +20,10 @@
 // near 1, U = W X cancels heavily and the state is the work of the last few tokens, so a single rounding of
 // those two shows unaveraged (final-state rel-L2 1e-3 .. 3.5e-3 in a float64 simulation of the rounding
 // points, 2.5e-4 .. 2.7e-4 with the pairs; random keys: 3.7e-4 .. 4.8e-4 single, bound 1e-3).  Every rounding
-// saturates at +-65504, the fp16 range, instead of producing infinities.
+// of an operand saturates at +-65504, the fp16 range, instead of producing infinities.
 //
 // Kernels:
-//   prefill_tables_kernel    chunk / segment / stage tables from cu_seqlens (device side, graph-capturable)
+//   prefill_tables_kernel    chunk and stage tables of calls of more than 64 sequences (device side, graph-capturable)
 //   gdn_align_rows_kernel    q / k rows that start on 4-byte boundaries only are copied into dense buffers first
 //   gdn_wsolve_kernel        preparation, one wavefront per (chunk, value head): gate, beta and their chunk-local
 //                            cumsum, the decay-factor tile, normalised K, K K^T on MFMA, the inverse of I + L by
@@ -697,7 +697,7 @@ __device__ __forceinline__ void lean_sweep(const GdnPrefillParams& p, unsigned c
 //     KS = K S^T,  X = V - e^G (.) KS,  U = W X                  (W as an fp16 hi + lo pair)
 //     O^T = scale e^G (.) (S Q^T) + U^T P^T  -> rows of o         (the output product is formed transposed: a lane
 //                                                                  then holds four adjacent V columns of one token
-//                                                                  and stores them as 8 bytes, no LDS tile)
+//                                                                  of a column block: 16 bytes of both with NB = 2)
 //     S^T = e^{G_last} S^T + K^T (e^{G_last - G} (.) U)          (U as an fp16 hi + lo pair)
 // Wavefronts 0-3 compute, each on its own 32 V columns of S^T, nothing crossing wavefronts (the chain K S^T -> X -> U
 // -> S^T stays in registers; the query product is formed after U, so its accumulators and those of K S^T never live

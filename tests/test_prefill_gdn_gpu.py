@@ -268,6 +268,7 @@ def test_gdn_prefill_split_sequences_match_oracle(lengths, tail_pad, H, HV):
     size = _lib.load().pla_gdn_prefill_workspace_bytes
     unsplit_per_head = size(T, N, 65 * H, 65 * HV) / (65 * HV)      # more than 64 chains are never split
     assert size(T, N, H, HV) > 1.1 * HV * unsplit_per_head           # so this call carries the segment buffers
+    assert max(_segments(lengths, tail_pad, H, HV)) > 1              # and the device splits its longest sequence
     w = gdn_prefill_packed(lengths, H=H, HV=HV, pool_slots=N + 3, seed=99 + T, tail_pad=tail_pad)
     _check(w, fast=True)
 
