@@ -725,8 +725,10 @@ constexpr int FUSED_OFF_K = FUSED_OFF_Q + 2 * TILE128_HALVES * 2, FUSED_OFF_V = 
 constexpr int FUSED_LDS_BYTES = FUSED_OFF_V + 2 * TILE128_HALVES * 2;
 
 // The sweep of one workgroup.  `wide`: 2 / NB x the chain's logical index (sequence x HV + value head, or that of `segment` among
-// those of a sweep over segments) plus, for NB = 1, the half of the V columns it takes.  PAST: outputs are stored past the caches.
-template <typename act_t, int NB, bool KN, bool PAST>
+// those of a sweep over segments) plus, for NB = 1, the half of the V columns it takes.  PARTS: the kernel also sweeps
+// segments (others do not ask at run time which they do: 22 sequences of 3 to 18 tokens, 48 value heads, 72.7 -> 67.6 us).  PAST: outputs are
+// stored past the caches.
+template <typename act_t, int NB, bool KN, bool PARTS, bool PAST>
 __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned char* const lds_all, const int wide,
                                             const SweptSegment& segment = SweptSegment{-1, 0, 0, 0}) {
   constexpr int CW = 4, AUX = 4;
@@ -738,7 +740,7 @@ __device__ __forceinline__ void fused_sweep(const GdnPrefillParams& p, unsigned 
   // the chunks of this workgroup's sequence: from the tables, or worked out here (every wavefront for itself)
   int3 inline_chunks{-1, 0, 0};
   int seq_first_chunk = 0, seq_first_token = 0, seq_end_token = 0;
-  const bool whole = !KN || p.pass == 0;                             // (sweeps over segments copy the keys)
+  const bool whole = !PARTS || p.pass == 0;
   const bool inline_tables = p.inline_tables && whole;               // segments are looked up in the segment table
   if (inline_tables) {
     const InlineSequences seqs = inline_sequences(p.cu_seqlens, p.N, p.stg.stages, lane);
@@ -1330,8 +1332,8 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_kernel(const GdnPrefil
     const int count = segment_count(p);
     segment = swept_segment(swept_segments(count, false), count, true, wide / HALVES / p.HV);
   }
-  if (NB == 2 && p.o_past_caches) fused_sweep<act_t, NB, KN, NB == 2>(p, lds_all, wide, segment);
-  else fused_sweep<act_t, NB, KN, false>(p, lds_all, wide, segment);
+  if (NB == 2 && p.o_past_caches) fused_sweep<act_t, NB, KN, KN, NB == 2>(p, lds_all, wide, segment);
+  else fused_sweep<act_t, NB, KN, KN, false>(p, lds_all, wide, segment);
 }
 
 // Whole sequences of unequal length, swept in one launch whose longest chains decide how long it lasts while the CUs
@@ -1345,13 +1347,13 @@ __global__ __launch_bounds__(512, 1) void gdn_fused_sweep_mixed_kernel(const Gdn
     const int wide = xcd_grouped_index(blockIdx.x, 2 * ratio, 2 * p.n_long * p.HV);
     if (wide < 0) return;
     const int chain = wide >> 1, k = chain / p.HV;
-    fused_sweep<act_t, 1, KN, false>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
+    fused_sweep<act_t, 1, KN, false, false>(p, lds_all, 2 * (p.seq_order[k] * p.HV + chain - k * p.HV) + (wide & 1));
   } else {
     const int chain = xcd_grouped_index(blockIdx.x - p.split_grid, ratio, (p.N - p.n_long) * p.HV);
     if (chain < 0) return;
     const int k = chain / p.HV, wide = p.seq_order[p.n_long + k] * p.HV + chain - k * p.HV;
-    if (p.o_past_caches) fused_sweep<act_t, 2, KN, true>(p, lds_all, wide);
-    else fused_sweep<act_t, 2, KN, false>(p, lds_all, wide);
+    if (p.o_past_caches) fused_sweep<act_t, 2, KN, false, true>(p, lds_all, wide);
+    else fused_sweep<act_t, 2, KN, false, false>(p, lds_all, wide);
   }
 }
 
@@ -1380,9 +1382,9 @@ __global__ __launch_bounds__(512, 1) void gdn_first_sweep_kernel(const GdnPrefil
   const SweptSegment segment = swept_segment(s, count, false, second ? item - second_halves : item);
   if (segment.sequence < 0) return;
   if (segment.index > 0) lean_sweep<act_t>(p, lds_all, segment, hv);
-  else if (halves) fused_sweep<act_t, 1, true, false>(p, lds_all, 2 * hv + second, segment);
-  else if (p.o_past_caches) fused_sweep<act_t, 2, true, true>(p, lds_all, hv, segment);
-  else fused_sweep<act_t, 2, true, false>(p, lds_all, hv, segment);
+  else if (halves) fused_sweep<act_t, 1, true, true, false>(p, lds_all, 2 * hv + second, segment);
+  else if (p.o_past_caches) fused_sweep<act_t, 2, true, true, true>(p, lds_all, hv, segment);
+  else fused_sweep<act_t, 2, true, true, false>(p, lds_all, hv, segment);
 }
 
 // Outputs of up to this size are left to the caches, from where the kernel behind the call reads them; larger ones are stored past
